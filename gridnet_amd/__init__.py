@@ -13,6 +13,7 @@ import torch
 import torch.nn as nn
 
 try:
+    from . import native as _n
     from .backend_cuda import GatedGridnetCudaOp, GridnetCudaOp
     from .layernorm import GridLayerNorm, grid_layer_norm
     _IMPORT_ERROR = None
@@ -40,6 +41,12 @@ def gridnet_step(weight, bias, residual_scale, init_activations, inner_iteration
     if block_size not in SUPPORTED_BLOCK_SIZES:
         raise NotImplementedError(
             f"gridnet block_size {block_size} not supported by the HIP kernels (4 or 8)")
+    # the native operator takes calls that are in order; what it declines goes to the Python one,
+    # which handles the empty batch and raises for the rest
+    out = _n.ops.step(weight, bias, residual_scale, init_activations, inner_iterations, block_size,
+                      eps, normalize, activation)
+    if out is not None:
+        return out
     return GridnetCudaOp.apply(weight, bias, residual_scale, init_activations, inner_iterations,
                                block_size, eps, normalize, activation)
 
@@ -55,6 +62,9 @@ def gated_gridnet_step(weight, bias, init_activations, inner_iterations: int, bl
     if block_size not in SUPPORTED_BLOCK_SIZES:
         raise NotImplementedError(
             f"gridnet block_size {block_size} not supported by the HIP kernels (4 or 8)")
+    out = _n.ops.gated_step(weight, bias, init_activations, inner_iterations, block_size, activation)
+    if out is not None:
+        return out
     return GatedGridnetCudaOp.apply(weight, bias, init_activations, inner_iterations, block_size,
                                     activation)
 

@@ -1,5 +1,5 @@
-"""Build recipe for libgridnet_hip.so and the benchmark's libgridnet_probe.so (gfx950 only, hipcc,
-in-tree).
+"""Build recipe for libgridnet_hip.so, the torch operators on it (_torch_ops.so) and the benchmark's
+libgridnet_probe.so (gfx950 only, hipcc and the host compiler, in-tree).
 
 Usage: ``python -m gridnet_amd.build`` or ``gridnet_amd.build.build()``.
 """
@@ -16,6 +16,10 @@ SOURCES = ["api.hip", "step_generic.hip", "step_fast.hip", "fwd_rows.hip", "bwd_
 # machine ceilings for bench.py: not part of the product library (it allocates and synchronises)
 PROBE_LIB = os.path.join(HERE, "libgridnet_probe.so")
 PROBE_SOURCES = ["probe.hip"]
+
+# the torch operators: host code against torch's headers, which finds libgridnet_hip.so when it is bound
+TORCH_OPS = os.path.join(HERE, "_torch_ops.so")
+TORCH_OPS_SOURCE = "torch_ops.cpp"
 
 # -packed-fp32-ops is switched OFF on purpose: hipcc -O3 otherwise forms v_pk_*_f32 from
 # ordinary float code.
@@ -35,6 +39,22 @@ FILE_FLAGS = {
     # an iteration later; the atomic optimizer would make it a wave reduction that waits at once
     "chain_bwd.hip": ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],
 }
+
+
+def build_torch_ops(out: str, verbose: bool) -> None:
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    includes = [*include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", *(f"-I{p}" for p in includes),
+           os.path.join(CSRC, TORCH_OPS_SOURCE), "-o", out, *(f"-L{p}" for p in library_paths()),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
 
 
 def build(verbose: bool = True, extra_flags=(), out=None, objdir=None) -> str:
@@ -59,8 +79,10 @@ def build(verbose: bool = True, extra_flags=(), out=None, objdir=None) -> str:
             print(out)
         return obj
 
-    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + len(PROBE_SOURCES))) as pool:
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + len(PROBE_SOURCES) + 1)) as pool:
+        ops = pool.submit(build_torch_ops, os.path.join(os.path.dirname(out), os.path.basename(TORCH_OPS)), verbose)
         all_objs = list(pool.map(compile_one, SOURCES + PROBE_SOURCES))
+        ops.result()
     objs, probe_objs = all_objs[:len(SOURCES)], all_objs[len(SOURCES):]
     probe_out = os.path.join(os.path.dirname(out), os.path.basename(PROBE_LIB))
     for target, members in ((out, objs), (probe_out, probe_objs)):

@@ -64,7 +64,9 @@ class GridLayerNormFn(torch.autograd.Function):
 
 
 def grid_layer_norm(x, weight, bias, eps: float = 1e-5):
-    return GridLayerNormFn.apply(x, weight, bias, eps)
+    # as in gridnet_amd.gridnet_step: natively where the call is in order
+    out = _n.ops.layer_norm(x, weight, bias, eps)
+    return out if out is not None else GridLayerNormFn.apply(x, weight, bias, eps)
 
 
 class GridLayerNorm(nn.Module):

@@ -135,6 +135,13 @@ try:
 except AttributeError as exc:  # an older build of the library without some entry point
     raise ImportError(f"{LIB_PATH} is stale ({exc}): rebuild with `python -m gridnet_amd.build`") from exc
 
+try:
+    from . import _torch_ops as ops  # the autograd operators, natively (csrc/torch_ops.cpp)
+except ImportError as exc:
+    raise ImportError(f"gridnet_amd/_torch_ops.so is missing or does not load ({exc}): build it with "
+                      "`python -m gridnet_amd.build`") from exc
+ops.bind(LIB_PATH)
+
 
 def last_error() -> str:
     return lib.gridnet_hip_last_error().decode()

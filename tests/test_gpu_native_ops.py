@@ -1,0 +1,58 @@
+"""The native operators (csrc/torch_ops.cpp) against the Python ones on the same kernels: same bits,
+forward and gradients; calls they decline reach the Python operator's checks."""
+
+import pytest
+import torch
+
+from helpers import make_acts, make_params
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("op", ["step", "gated", "norm"])
+def test_native_operator_equals_the_python_operator(op, batch, dtype):
+    import gridnet_amd as ga
+    from gridnet_amd.layernorm import GridLayerNormFn
+
+    w, b, r = (t.to(DEV, dtype) for t in make_params((8, 16, 8), seed=3))
+    x, gy = (make_acts(batch, (8, 16, 8), seed=s).to(DEV, dtype) for s in (4, 5))
+    if op == "step":
+        native, python, params = ga.gridnet_step, ga.GridnetCudaOp.apply, [w, b, r, x]
+        rest = (2, 8, 1e-5, True, "silu")
+    elif op == "gated":
+        native, python = ga.gated_gridnet_step, ga.GatedGridnetCudaOp.apply
+        params, rest = [torch.stack([w, w.flip(0)], 1), torch.stack([b, r]), x], (2, 8, "tanh")
+    else:
+        native, python, params, rest = ga.grid_layer_norm, GridLayerNormFn.apply, [x, r, b], (1e-5,)
+    results = []
+    for f in (native, python):
+        leaves = [p.clone().requires_grad_(True) for p in params]
+        y = f(*leaves, *rest)
+        y.backward(gy)
+        results.append([y.detach(), *[p.grad for p in leaves]])
+    tol = dict(rtol=0, atol=0) if dtype is torch.float32 or op == "norm" else dict(rtol=1e-12, atol=1e-12)
+    for got, want in zip(*results):  # fp64 dx is built with atomics
+        torch.testing.assert_close(got, want, **tol)
+    with torch.no_grad():
+        assert not native(*params, *rest).requires_grad
+
+
+def test_native_step_refuses_what_the_python_operator_refuses():
+    import gridnet_amd as ga
+
+    w, b, r = (t.to(DEV) for t in make_params((8, 8, 8), seed=3))
+    x = make_acts(2, (8, 8, 8), seed=4).to(DEV)
+    with pytest.raises(AssertionError, match="mismatching dtypes"):
+        ga.gridnet_step(w, b.double(), r, x, 1, 8)
+    assert ga.gridnet_step(w, b, r, x[:0], 1, 8).shape == (0, 8, 8, 8)
+    y = ga.gridnet_step(w.requires_grad_(True), b, r, x, 1, 8)
+    with pytest.raises(RuntimeError, match="outGrads must be contiguous"):
+        y.sum().backward()  # an expanded gradient
+    y = ga.gridnet_step(w, b, r, x, 1, 8)
+    with torch.no_grad():
+        w.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward(torch.ones_like(y))

@@ -324,7 +324,9 @@ static int check_fused(const StepArgs &a, bool backward) {
 
 static size_t fused_forward_workspace(const StepArgs &a) {
     const size_t nblk = (size_t)(a.M / a.block_size) * (a.N / a.block_size) * (a.K / a.block_size);
-    return (size_t)a.B * nblk * step_fast_forward_parts(a.block_size) * 2 * sizeof(float);
+    size_t pairs = nblk * step_fast_forward_parts(a.block_size);
+    if (fwd_rows_supports(a) && (size_t)fwd_rows_pairs(a) > pairs) pairs = (size_t)fwd_rows_pairs(a);
+    return (size_t)a.B * pairs * 2 * sizeof(float);
 }
 
 // backward workspace: [D of every cell | partial sums of the cross-block kernel]
@@ -334,6 +336,7 @@ static size_t fused_backward_dsum(const StepArgs &a) {
 static size_t fused_backward_parts(const StepArgs &a) {
     const size_t nblk = (size_t)(a.M / a.block_size) * (a.N / a.block_size) * (a.K / a.block_size);
     size_t pairs = nblk * step_fast_backward_parts(a.block_size);
+    if ((size_t)step_fast_cross_pairs(a) > pairs) pairs = (size_t)step_fast_cross_pairs(a);
     if (bwd_rows_supports(a)) {  // one inner iteration, by rows: a pair per wave of its first kernel
         StepArgs plain = a;
         plain.ln.residual = 0;

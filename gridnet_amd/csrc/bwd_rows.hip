@@ -33,6 +33,7 @@
 // LN / RES as in step_bwd_fast (LnFold): x is normalised while its rows are committed; dy passes
 // the backward of the LayerNorm behind the step as it is loaded (dgamma, dbeta fall out); the
 // residual loop adds G'' and stores G', and its direct part of dx is G' - G' = 0.
+// PAD: rows of other than 16, 32 or 64 cells, as in cross_rows.hip.
 
 #include "common.h"
 #include "fast_tiles.h"
@@ -46,13 +47,13 @@ namespace {
 constexpr int kTube = 4;                          // the tube is 4 x 4 grid rows
 constexpr int kWinRows = (kTube + 2) * (kTube + 2);  // rows in and around it
 
-template <int ACT, bool LN, bool RES>
+template <int ACT, bool LN, bool RES, bool PAD>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 3)))
 void bwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, const float *__restrict__ scale,
               const float *__restrict__ x, const float *__restrict__ dy, float *__restrict__ dweight,
               float *__restrict__ dbias, float *__restrict__ dscale, float *__restrict__ dx,
               float *__restrict__ delta_out, int B, int M, int N, int K, int ntube, int nchunk, int chunk_len,
-              int param_mode, int dx_accumulate, LnFold ln, long slab_stride) {
+              int param_mode, int dx_accumulate, LnFold ln, long slab_stride, int lanes) {
     static_assert(LN || !RES, "the residual form comes with the folded LayerNorm");
     // [2 stages][36 rows][K]; LN: then gamma and beta of the 36 rows
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -69,8 +70,9 @@ void bwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
             ln.dbeta += off;
         }
     }
-    const int kb = K / 2, nt = 16 * kb, tid = threadIdx.x;  // kb: threads along a row
-    const int bk = tid % kb, r = tid / kb, ci = r / kTube, cj = r % kTube;
+    const int kb = K / 2, kl = PAD ? lanes : kb, nt = 16 * kl, tid = threadIdx.x;  // kb: pieces, kl: lanes of a row
+    const bool live = !PAD || tid % kl < kb;
+    const int bk = PAD ? min(tid % kl, kb - 1) : tid % kb, r = tid / kl, ci = r / kTube, cj = r % kTube;
     const int nbj = N / kTube, p0 = (tube / nbj) * kTube, q0 = (tube % nbj) * kTube;
     const long cells = (long)M * N * K;
     const int grow = ((p0 + ci) * N + (q0 + cj)) * K + 2 * bk;  // this thread's two cells
@@ -264,9 +266,15 @@ void bwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
             out[c] = (RES ? 0.f : g[c]) + (dx_accumulate ? keep[c] : 0.f);
         }
         const long o = (long)s * cells + grow;
-        store_cells<2>(delta_out + o, delta);
-        store_cells<2>(dx + o, out);
-        if (RES && ln.g_out) store_cells<2>(ln.g_out + o, gin);
+        if (PAD) {
+            keep_here(delta);
+            keep_here(out);
+        }
+        if (live) {
+            store_cells<2>(delta_out + o, delta);
+            store_cells<2>(dx + o, out);
+            if (RES && ln.g_out) store_cells<2>(ln.g_out + o, gin);
+        }
         if (LN && !RES) {
             if (sums_here) {
                 float t1 = 0.f, t2 = 0.f;
@@ -275,6 +283,7 @@ void bwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
                     t1 = fmaf(gam[c], out[c], fmaf(delta[c], wgam[c], t1));
                     t2 = fmaf(out[c], own[c] - bet[c], fmaf(delta[c], u[c] - bwb[c], t2));
                 }
+                if (PAD && !live) t1 = t2 = 0.f;
                 const float w1 = slot_wave_sum<64>(t1), w2 = slot_wave_sum<64>(t2);
                 if ((tid & 63) == 0) {
                     float *to = ln.x_part + (((long)s * ntube + tube) * (nt / 64) + tid / 64) * 2;
@@ -291,6 +300,7 @@ void bwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
         });
     }
     // ---- parameter gradients: plain stores of whole rows ----
+    if (PAD && !live) return;
 #pragma unroll
     for (int pq = 0; pq < 9; ++pq) {
         nw[pq * 3][0] *= keep_first;
@@ -322,30 +332,34 @@ void bwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
     }
 }
 
-bool k_ok(int K) { return K == 16 || K == 32 || K == 64; }
+bool k_ok(int K) { return K % 4 == 0 && K >= 8 && K <= 64; }
 
-template <int ACT, bool LN, bool RES> int launch(const StepArgs &a, hipStream_t st) {
-    auto kern = bwd_rows<ACT, LN, RES>;
+// Chunks of the batch: enough workgroups to fill the chip, none shorter than eight elements (every
+// chunk writes a copy of the gradient arrays, which is then read again), but where that gives fewer
+// workgroups than the chip has CUs, down to three elements (32^3, batch 16: 25.4 us with two
+// chunks, 23.9 with four; batch 64: 32.9 us with eight, 35.4 with twelve).
+int batch_chunks(int B, int ntube, int per_cu, int &chunk_len) {
+    const int cus = plan_device_cus();
+    const int n = plan_row_chunks(B, ntube, per_cu * cus, 8, chunk_len);
+    return n * ntube >= cus ? n : plan_row_chunks(B, ntube, cus, kRowsMinWalk, chunk_len);
+}
+
+template <int ACT, bool LN, bool RES, bool PAD> int launch_rows(const StepArgs &a, hipStream_t st) {
+    auto kern = bwd_rows<ACT, LN, RES, PAD>;
     const long cells = (long)a.M * a.N * a.K;
-    const int nt = 8 * a.K, ntube = (a.M / kTube) * (a.N / kTube);
+    const int lanes = row_lanes(a.K, 2), nt = 16 * lanes, ntube = (a.M / kTube) * (a.N / kTube);
     const size_t lds = (size_t)(LN ? 4 : 2) * kWinRows * a.K * sizeof(float);
-    static int per_cu_cache[3] = {0, 0, 0};  // per instantiation, by K
-    int &per_cu = per_cu_cache[a.K == 16 ? 0 : a.K == 32 ? 1 : 2];
+    static int per_cu_cache[64 / 4 + 1];  // per instantiation, by K
+    int &per_cu = per_cu_cache[a.K / 4];
     if (per_cu == 0) {
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, nt, lds) != hipSuccess || n < 1) n = 1;
         per_cu = n;
     }
-    // chunks of the batch: enough workgroups to fill the chip, none shorter than eight elements,
-    // and no more than there is room for copies of the gradient arrays
-    int nchunk = per_cu * plan_device_cus() / ntube;
-    if (nchunk > a.B / 8) nchunk = a.B / 8;
     const long slab_floats = kStepSlabPlanes * cells;
+    int chunk_len, nchunk = batch_chunks(a.B, ntube, per_cu, chunk_len);
     const int room = plan_slab_capacity(a.slabs, a.slab_bytes, slab_floats);
-    if (nchunk > room) nchunk = room;
-    if (nchunk < 2) nchunk = 1;
-    const int chunk_len = (a.B + nchunk - 1) / nchunk;
-    nchunk = (a.B + chunk_len - 1) / chunk_len;
+    if (nchunk > room) nchunk = plan_row_chunks(a.B, ntube, (room > 1 ? room : 1) * ntube, 1, chunk_len);
     const bool split = nchunk > 1;
     const bool new_params = (a.flags & GRIDNET_OVERWRITE_PARAMS) != 0;
     const int param_mode = split || new_params ? kParamStore : kParamAddExclusive;
@@ -360,8 +374,9 @@ template <int ACT, bool LN, bool RES> int launch(const StepArgs &a, hipStream_t 
                        (const float *)a.bias, (const float *)a.scale, (const float *)a.x, (const float *)a.dy,
                        split ? slab : (float *)a.dweight, split ? slab + 27 * cells : (float *)a.dbias,
                        split ? slab + 28 * cells : (float *)a.dscale, (float *)a.dx, (float *)a.workspace, a.B, a.M,
-                       a.N, a.K, ntube, nchunk, chunk_len, param_mode, dx_accumulate, ln, split ? slab_floats : 0L);
+                       a.N, a.K, ntube, nchunk, chunk_len, param_mode, dx_accumulate, ln, split ? slab_floats : 0L, lanes);
     if (int rc = check_launch("bwd_rows")) return rc;
+    TailJob tail{};
     if (split) {
         SlabTargets t{};
         t.dst[0] = (float *)a.dweight; t.end[0] = 27 * cells;
@@ -373,17 +388,19 @@ template <int ACT, bool LN, bool RES> int launch(const StepArgs &a, hipStream_t 
             t.dst[4] = a.ln.dbeta;  t.end[4] = 31 * cells;
             t.count = 5;
         }
-        // the LayerNorm sums the kernel above left per wave are finished by spare workgroups of this one
-        SumsJob job{nullptr, 0, 0, 0, nullptr};
-        if (bwd_rows_leaves_sums(a)) job = SumsJob{a.ln.x_part, bwd_rows_pairs(a), a.B, cells, a.ln.x_sums};
-        if (int rc = plan_reduce_slabs(slab, nchunk, slab_floats, t, new_params ? 0 : 1, st, job)) return rc;
-    } else if (bwd_rows_leaves_sums(a)) {
-        if (int rc = layernorm_finalize_sums(a.ln.x_part, bwd_rows_pairs(a), cells, a.ln.x_sums, a.B, st)) return rc;
+        tail = plan_tail_job(slab, nchunk, slab_floats, t, new_params ? 0 : 1, cross_rows_threads(a));
     }
+    // the LayerNorm sums the kernel above left per wave
+    if (bwd_rows_leaves_sums(a)) tail.sums = SumsJob{a.ln.x_part, bwd_rows_pairs(a), a.B, cells, a.ln.x_sums};
     // dx holds its direct part, the scratch tensor delta: the sum over the neighbours' deltas, all
     // 27 taps of it; the LayerNorm sums of the finished rows only where the kernel above left them out
     const bool sums_here = LN && !RES && a.ln.x_stats && a.ln.x_part;
-    return cross_rows_full_launch(a, st, !sums_here);
+    return cross_rows_full_launch(a, tail, st, !sums_here);
+}
+
+template <int ACT, bool LN, bool RES> int launch(const StepArgs &a, hipStream_t st) {
+    return row_lanes(a.K, 2) * 2 == a.K ? launch_rows<ACT, LN, RES, false>(a, st)
+                                        : launch_rows<ACT, LN, RES, true>(a, st);
 }
 
 template <int ACT> int dispatch(const StepArgs &a, hipStream_t st) {
@@ -405,15 +422,15 @@ bool bwd_rows_leaves_sums(const StepArgs &a) {
 
 int bwd_rows_pairs(const StepArgs &a) {
     if (a.ln.residual) return cross_rows_pairs(a);
-    return (a.M / kTube) * (a.N / kTube) * (8 * a.K / 64);
+    return (a.M / kTube) * (a.N / kTube) * (16 * row_lanes(a.K, 2) / 64);
 }
 
 // room for per-chunk copies of the gradient arrays that lets the batch be split as far as the
-// kernel likes (three workgroups per CU, none with fewer than eight elements)
+// kernel likes (with at most three workgroups per CU)
 size_t bwd_rows_slab_bytes(const StepArgs &a) {
-    const long ntube = (long)(a.M / kTube) * (a.N / kTube);
-    long chunks = 3L * plan_device_cus() / ntube;
-    if (chunks > a.B / 8) chunks = a.B / 8;
+    const int ntube = (a.M / kTube) * (a.N / kTube);
+    int chunk_len;
+    const long chunks = batch_chunks(a.B, ntube, 3, chunk_len);
     if (chunks < 2) return 0;
     return (size_t)chunks * kStepSlabPlanes * a.M * a.N * a.K * sizeof(float);
 }

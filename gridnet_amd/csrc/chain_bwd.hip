@@ -950,6 +950,7 @@ template <int ACT, bool DEFER, bool WIDE> int launch_chain(const StepArgs &a, hi
     k.B = a.B; k.M = a.M; k.N = a.N; k.K = a.K; k.inner = a.inner;
     hipLaunchKernelGGL(kern, dim3(padded_grid(k.nblk, k.nchunk)), dim3(256), lds, st, k);
     if (int rc = check_launch("chain_bwd")) return rc;
+    TailJob tail{};
     if (split) {
         SlabTargets t{};
         t.dst[0] = (float *)a.dweight; t.end[0] = 27 * cells;
@@ -958,11 +959,12 @@ template <int ACT, bool DEFER, bool WIDE> int launch_chain(const StepArgs &a, hi
         t.dst[3] = a.ln.dgamma;        t.end[3] = 30 * cells;
         t.dst[4] = a.ln.dbeta;         t.end[4] = 31 * cells;
         t.count = 5;
-        if (int rc = plan_reduce_slabs(slab, k.nchunk, slab_floats, t, new_params ? 0 : 1, st)) return rc;
+        tail = plan_tail_job(slab, k.nchunk, slab_floats, t, new_params ? 0 : 1,
+                             !DEFER && cross_rows_supports(a) ? cross_rows_threads(a) : 256);
     }
-    if (DEFER) return GRIDNET_OK;
+    if (DEFER) return plan_launch_tail_job(tail, st);
     // dx is wanted finished: the cross-block kernel completes it from D (same blocks, same chunks)
-    return step_cross_launch(a, k.nchunk, k.chunk_len, st);
+    return step_cross_launch(a, k.nchunk, k.chunk_len, tail, st);
 }
 
 // What the first step of a one-launch chain leaves in its records is added to dx here: the

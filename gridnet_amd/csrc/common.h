@@ -121,22 +121,22 @@ template <typename T> __device__ __forceinline__ T block_sum(T v, T *scratch, in
 }
 
 // ---- device: the last step of the LayerNorm backward's two sums --------------------------
-// (s1_i, s2_i), `parts` pairs of sample b -> (sum s1 / n, sum s2 / n), by one workgroup of THREADS
-// threads: doubles, a fixed order.  `red` is LDS, one pair per wave.  A kernel of its own in
+// (s1_i, s2_i), `parts` pairs of sample b -> (sum s1 / n, sum s2 / n), by one workgroup of at most THREADS
+// threads (`nthreads`, a multiple of the wave width, where it is fewer): doubles, a fixed order.  `red` is LDS, one pair per wave.  A kernel of its own in
 // layernorm.hip; also run by spare workgroups of the kernel that adds up the gradient copies.
 constexpr int kFinUnroll = 4;  // pairs a thread requests before it uses any
 template <int THREADS>
 __device__ __forceinline__ void finalize_sums_of_sample(const float *__restrict__ part, int parts, long n,
                                                         float *__restrict__ sums, int b,
-                                                        double (*red)[2]) {
+                                                        double (*red)[2], int nthreads = THREADS) {
     const int tid = threadIdx.x;
     const float2 *ps = reinterpret_cast<const float2 *>(part) + (long)b * parts;
     double s1 = 0.0, s2 = 0.0;
-    for (int i0 = tid; i0 < parts; i0 += THREADS * kFinUnroll) {
+    for (int i0 = tid; i0 < parts; i0 += nthreads * kFinUnroll) {
         float2 v[kFinUnroll];
 #pragma unroll
         for (int k = 0; k < kFinUnroll; ++k) {
-            const int i = i0 + k * THREADS;
+            const int i = i0 + k * nthreads;
             v[k] = i < parts ? ps[i] : make_float2(0.f, 0.f);
         }
 #pragma unroll
@@ -154,7 +154,7 @@ __device__ __forceinline__ void finalize_sums_of_sample(const float *__restrict_
     __syncthreads();
     if (tid == 0) {
         s1 = s2 = 0.0;
-        for (int w = 0; w < THREADS / kWave; ++w) {
+        for (int w = 0; w < nthreads / kWave; ++w) {
             s1 += red[w][0];
             s2 += red[w][1];
         }

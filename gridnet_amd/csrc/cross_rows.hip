@@ -25,6 +25,11 @@
 // columns of blocks around them: their (Q, R) travel through LDS with the D rows.
 // SETS = 2: the gated variant of the update (weight [27, 2, M, N, K]): two D tensors, one behind
 // the other in `dsum`, each with its own set of mirrored weights; the cell receives the sum.
+// PAD: rows of other than 16, 32, 64 or 128 cells take the next power of two of lanes each, so that
+// no row straddles two waves; the spare lanes idle (they repeat the row's last piece and store
+// nothing).  Against the kernel dealt by block face that served such rows, step_bwd_cross, at
+// 40 x 48 x 56, batch 13, one inner iteration: 55 -> 30 us for the whole backward; gated at 40^3,
+// batch 6: 49 -> 46 us.
 
 #include "common.h"
 #include "fast_tiles.h"
@@ -45,21 +50,28 @@ template <int BS> struct Tube {
 // FULL: ALL taps, not only those that leave the block: the second kernel of the backward of a step
 // with one inner iteration (bwd_rows.hip), where `dsum` holds delta of every cell and dx the
 // direct part of the gradient.
-template <int BS, bool LN, bool NORM = false, int SETS = 1, bool FULL = false>
+template <int BS, bool LN, bool NORM, int SETS, bool FULL, bool PAD>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(SETS == 1 ? 3 : 2, SETS == 1 ? 3 : 2)))
 void cross_rows(const float *__restrict__ weight, const float *__restrict__ x,
                 const float *__restrict__ dsum, float *__restrict__ dx, int B, int M, int N, int K,
-                int ntube, int nchunk, int chunk_len, LnFold ln, const float *__restrict__ qr) {
+                int ntube, int nchunk, int chunk_len, LnFold ln, const float *__restrict__ qr, int lanes,
+                TailJob tail) {
     using TB = Tube<BS>;
     static_assert(!(NORM && LN), "the folded LayerNorm comes without normalisation");
     static_assert(SETS == 1 || !(LN || NORM), "the gated update has no variants");
     // [2 stages][SETS][TB::ROWS][K]; NORM: then [2 stages][3 x 3 columns of blocks][K / BS + 2] (Q, R) pairs
     extern __shared__ __attribute__((aligned(16))) float lds[];
 
+    const int main_grid = padded_grid(ntube, nchunk);
+    if ((int)blockIdx.x >= main_grid) {  // behind them: what the kernel before left to be finished
+        run_tail_job<512>(tail, blockIdx.x - main_grid, blockDim.x, reinterpret_cast<double (*)[2]>(lds));
+        return;
+    }
     int tube, chunk;
     if (!split_block_id(blockIdx.x, ntube, nchunk, tube, chunk)) return;  // grid padding
-    const int kb = K / 4, nt = 16 * kb, tid = threadIdx.x;  // kb: threads along a row
-    const int bk = tid % kb, r = tid / kb, ci = r / TB::RJ, cj = r % TB::RJ;
+    const int kb = K / 4, kl = PAD ? lanes : kb, nt = 16 * kl, tid = threadIdx.x;  // kb: pieces, kl: lanes of a row
+    const bool live = !PAD || tid % kl < kb;
+    const int bk = PAD ? min(tid % kl, kb - 1) : tid % kb, r = tid / kl, ci = r / TB::RJ, cj = r % TB::RJ;
     const int nbj = N / TB::RJ, p0 = (tube / nbj) * TB::RI, q0 = (tube % nbj) * TB::RJ;
     // where the thread's row and its first cell lie inside their block
     const int bi = (p0 + ci) % BS, bj = cj, bk0 = (4 * bk) % BS;
@@ -117,7 +129,7 @@ void cross_rows(const float *__restrict__ weight, const float *__restrict__ x,
         goff[e] = ok[e] ? (gi * N + gj) * K + 4 * bk : grow;  // anything valid when not used
         loff[e] = row * K + 4 * bk;
     }
-    const bool has_last = r + 16 * (RPT - 1) < TB::ROWS;
+    const bool has_last = r + 16 * (RPT - 1) < TB::ROWS && live;
     const int own_row = (ci + 1) * TB::WJ + (cj + 1);
 
     // NORM: (Q, R) of the blocks in the 3 x 3 columns around the tube's own, a row of K / BS blocks
@@ -178,7 +190,7 @@ void cross_rows(const float *__restrict__ weight, const float *__restrict__ x,
                 float v[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] = ok[e] ? dbuf[k][e][q] : 0.f;
-                store_cells<4>(stage + k * TB::ROWS * K + loff[e], v);
+                if (live) store_cells<4>(stage + k * TB::ROWS * K + loff[e], v);
             }
         const float2 *qst = qrs + ((s - s0) & 1) * 9 * qrow;
         if (NORM && tid < 9 * nbk)
@@ -241,7 +253,8 @@ void cross_rows(const float *__restrict__ weight, const float *__restrict__ x,
                 if (c == 3 && bk0 + 3 == BS - 1) g[c] += fmaf(-xc[c], sq[2], sr[2]);
             }
         }
-        store_cells<4>(dx + (long)s * cells + grow, g);
+        if (PAD) keep_here(g);
+        if (live) store_cells<4>(dx + (long)s * cells + grow, g);
         if (ln_in) {
             float t1 = 0.f, t2 = 0.f;
 #pragma unroll
@@ -250,6 +263,7 @@ void cross_rows(const float *__restrict__ weight, const float *__restrict__ x,
                 t1 += a;
                 t2 = fmaf(a, (xc[c] - mean) * rstd, t2);
             }
+            if (PAD && !live) t1 = t2 = 0.f;
             const float w1 = slot_wave_sum<64>(t1), w2 = slot_wave_sum<64>(t2);
             if ((tid & 63) == 0) {
                 const int nwave = nt / 64;
@@ -261,13 +275,13 @@ void cross_rows(const float *__restrict__ weight, const float *__restrict__ x,
     }
 }
 
-bool k_ok(int K) { return K == 16 || K == 32 || K == 64 || K == 128; }
+bool k_ok(int K) { return K % 4 == 0 && K >= 8 && K <= 128; }
 
-template <int BS, bool LN, bool NORM = false, int SETS = 1, bool FULL = false>
-int launch(const StepArgs &a, const float *dsum, hipStream_t st) {
+template <int BS, bool LN, bool NORM, int SETS, bool FULL, bool PAD>
+int launch_rows(const StepArgs &a, const float *dsum, const TailJob &tail, hipStream_t st) {
     using TB = Tube<BS>;
-    auto kern = cross_rows<BS, LN, NORM, SETS, FULL>;
-    const int nt = 4 * a.K, ntube = (a.M / TB::RI) * (a.N / TB::RJ);
+    auto kern = cross_rows<BS, LN, NORM, SETS, FULL, PAD>;
+    const int lanes = row_lanes(a.K, 4), nt = 16 * lanes, ntube = (a.M / TB::RI) * (a.N / TB::RJ);
     const size_t lds = ((size_t)2 * SETS * TB::ROWS * a.K + (NORM ? 2 * 9 * (a.K / BS + 2) * 2 : 0)) * sizeof(float);
     static bool big_lds_enabled = false;  // per instantiation
     if (lds > 64 * 1024 && !big_lds_enabled) {
@@ -279,31 +293,32 @@ int launch(const StepArgs &a, const float *dsum, hipStream_t st) {
     }
     // NORM: (Q, R) per (element, block) behind the D tensor in the workspace
     const float *qr = NORM ? dsum + (size_t)a.B * a.M * a.N * a.K : nullptr;
-    static int per_cu_cache[4] = {0, 0, 0, 0};  // per instantiation, by K
-    int &per_cu = per_cu_cache[a.K == 16 ? 0 : a.K == 32 ? 1 : a.K == 64 ? 2 : 3];
+    static int per_cu_cache[128 / 4 + 1];  // per instantiation, by K
+    int &per_cu = per_cu_cache[a.K / 4];
     if (per_cu == 0) {
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, nt, lds) != hipSuccess || n < 1) n = 1;
         per_cu = n;
     }
-    // chunks of the batch: enough workgroups to fill the chip, but none that walks fewer than
-    // eight elements for its one fetch of the weights
-    int nchunk = per_cu * plan_device_cus() / ntube;
-    if (nchunk > a.B / 8) nchunk = a.B / 8;
-    if (nchunk < 1) nchunk = 1;
-    const int chunk_len = (a.B + nchunk - 1) / nchunk;
-    nchunk = (a.B + chunk_len - 1) / chunk_len;
-    hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, nchunk)), dim3(nt), lds, st, (const float *)a.weight,
-                       (const float *)a.x, dsum, (float *)a.dx, a.B, a.M, a.N, a.K,
-                       ntube, nchunk, chunk_len, a.ln, qr);
+    int chunk_len;
+    const int nchunk = plan_row_chunks(a.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, chunk_len);
+    hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, nchunk) + tail.blocks()), dim3(nt), lds, st,
+                       (const float *)a.weight, (const float *)a.x, dsum, (float *)a.dx, a.B, a.M, a.N, a.K,
+                       ntube, nchunk, chunk_len, a.ln, qr, lanes, tail);
     return check_launch("cross_rows");
 }
 
-template <int BS> int dispatch(const StepArgs &a, hipStream_t st) {
+template <int BS, bool LN, bool NORM = false, int SETS = 1, bool FULL = false>
+int launch(const StepArgs &a, const float *dsum, const TailJob &tail, hipStream_t st) {
+    if (row_lanes(a.K, 4) * 4 == a.K) return launch_rows<BS, LN, NORM, SETS, FULL, false>(a, dsum, tail, st);
+    return launch_rows<BS, LN, NORM, SETS, FULL, true>(a, dsum, tail, st);
+}
+
+template <int BS> int dispatch(const StepArgs &a, const TailJob &tail, hipStream_t st) {
     const float *dsum = (const float *)a.workspace;
-    if (a.normalize) return launch<BS, false, true>(a, dsum, st);
-    if (a.ln.gamma) return launch<BS, true>(a, dsum, st);
-    return launch<BS, false>(a, dsum, st);
+    if (a.normalize) return launch<BS, false, true>(a, dsum, tail, st);
+    if (a.ln.gamma) return launch<BS, true>(a, dsum, tail, st);
+    return launch<BS, false>(a, dsum, tail, st);
 }
 
 }  // namespace
@@ -314,18 +329,18 @@ bool cross_rows_supports(const StepArgs &a) {
            a.M % bs == 0 && a.N % bs == 0;
 }
 
-// one pair per wave: 16 grid rows of K / 4 threads each per workgroup
-int cross_rows_pairs(const StepArgs &a) { return (a.M * a.N / 16) * (4 * a.K / 64); }
+// one pair per wave, 16 grid rows per workgroup
+int cross_rows_pairs(const StepArgs &a) { return (a.M * a.N / 16) * (16 * row_lanes(a.K, 4) / 64); }
 
-int cross_rows_launch(const StepArgs &a, hipStream_t st) {
-    return a.block_size == 8 ? dispatch<8>(a, st) : dispatch<4>(a, st);
+int cross_rows_launch(const StepArgs &a, const TailJob &tail, hipStream_t st) {
+    return a.block_size == 8 ? dispatch<8>(a, tail, st) : dispatch<4>(a, tail, st);
 }
 
 // all 27 taps (the second kernel of bwd_rows.hip); the block size does not enter then
-int cross_rows_full_launch(const StepArgs &a, hipStream_t st, bool ln_sums) {
+int cross_rows_full_launch(const StepArgs &a, const TailJob &tail, hipStream_t st, bool ln_sums) {
     const float *dsum = (const float *)a.workspace;
-    return a.ln.gamma && ln_sums ? launch<4, true, false, 1, true>(a, dsum, st)
-                                 : launch<4, false, false, 1, true>(a, dsum, st);
+    return a.ln.gamma && ln_sums ? launch<4, true, false, 1, true>(a, dsum, tail, st)
+                                 : launch<4, false, false, 1, true>(a, dsum, tail, st);
 }
 
 // the gated update: weight [27, 2, M, N, K], D0 and D1 of every cell behind one another in `dsum`
@@ -333,8 +348,8 @@ bool cross_rows_gated_supports(const StepArgs &a) {
     const int bs = a.block_size;
     return a.dtype == GRIDNET_F32 && (bs == 4 || bs == 8) && k_ok(a.K) && a.M % bs == 0 && a.N % bs == 0;
 }
-int cross_rows_gated_launch(const StepArgs &a, const float *dsum, hipStream_t st) {
-    return a.block_size == 8 ? launch<8, false, false, 2>(a, dsum, st) : launch<4, false, false, 2>(a, dsum, st);
+int cross_rows_gated_launch(const StepArgs &a, const float *dsum, const TailJob &tail, hipStream_t st) {
+    return a.block_size == 8 ? launch<8, false, false, 2>(a, dsum, tail, st) : launch<4, false, false, 2>(a, dsum, tail, st);
 }
 
 }  // namespace gridnet

@@ -206,6 +206,14 @@ template <int CPT> __device__ __forceinline__ void store_cells(float *p, const f
     }
 }
 
+// The values of v are worked out before this point and not, as the compiler otherwise does, behind a
+// branch that only stores them: there the weights of a whole stencil would have to stay live across
+// what lies between (72 spilled registers in the row-wise kernels with idle lanes).
+template <int CPT> __device__ __forceinline__ void keep_here(float (&v)[CPT]) {
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) asm volatile("" : "+v"(v[c]));
+}
+
 template <int CPT> __device__ __forceinline__ void add_cells(float *p, const float (&v)[CPT]) {
     float old[CPT];
     load_cells<CPT>(p, old);

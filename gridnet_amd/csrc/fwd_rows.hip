@@ -17,6 +17,8 @@
 // are committed to LDS, gamma and beta of the tube's rows waiting in LDS beside them; every wave
 // leaves (mean, M2) of its 256 results.  RES: the residual form of the loop, the result is the
 // RAW input plus the update.
+// PAD: rows of other than 16, 32, 64 or 128 cells, as in cross_rows.hip (padded to a power of two of
+// lanes, the spare lanes idle).
 
 #include "common.h"
 #include "fast_tiles.h"
@@ -31,11 +33,11 @@ constexpr int kRowsTube = 4;                                  // the tube is 4 x
 constexpr int kRowsWin = (kRowsTube + 2) * (kRowsTube + 2);  // rows in and around it
 constexpr int kRowsRpt = (kRowsWin + 15) / 16;               // rows a thread moves
 
-template <int ACT, bool LN, bool RES>
+template <int ACT, bool LN, bool RES, bool PAD>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RES ? 2 : 3, 3)))  // RES: four more values per thread
 void fwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, const float *__restrict__ scale,
               const float *__restrict__ x, float *__restrict__ y, int B, int M, int N, int K, int ntube,
-              int nchunk, int chunk_len, LnFold ln) {
+              int nchunk, int chunk_len, LnFold ln, int lanes) {
     static_assert(LN || !RES, "the residual form comes with the folded LayerNorm");
     // [2 stages][36 rows][K]; LN: then gamma and beta of the 36 rows
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -44,8 +46,9 @@ void fwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
     if (!split_block_id(ln.walk_reverse ? reversed_on_its_xcd(blockIdx.x, gridDim.x) : blockIdx.x, ntube, nchunk,
                         tube, chunk))
         return;  // grid padding
-    const int kb = K / 4, nt = 16 * kb, tid = threadIdx.x;  // kb: threads along a row
-    const int bk = tid % kb, r = tid / kb, ci = r / kRowsTube, cj = r % kRowsTube;
+    const int kb = K / 4, kl = PAD ? lanes : kb, nt = 16 * kl, tid = threadIdx.x;  // kb: pieces, kl: lanes of a row
+    const bool live = !PAD || tid % kl < kb;
+    const int bk = PAD ? min(tid % kl, kb - 1) : tid % kb, r = tid / kl, ci = r / kRowsTube, cj = r % kRowsTube;
     const int nbj = N / kRowsTube, p0 = (tube / nbj) * kRowsTube, q0 = (tube % nbj) * kRowsTube;
     const long cells = (long)M * N * K;
     const int grow = ((p0 + ci) * N + (q0 + cj)) * K + 4 * bk;  // this thread's four cells
@@ -126,7 +129,7 @@ void fwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] = ok[e] ? xbuf[e][q] : 0.f;
             }
-            store_cells<4>(stage + loff[e], v);
+            if (live) store_cells<4>(stage + loff[e], v);
         }
         float base[4];
 #pragma unroll
@@ -161,8 +164,23 @@ void fwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
         float out[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) out[c] = fmaf(rv[c], Act<ACT, float>::f(u[c]), RES ? base[c] : own[c]);
-        store_cells<4>(y + (long)s * cells + grow, out);
-        if (LN && ln.y_part) {
+        if (PAD) keep_here(out);
+        if (live) store_cells<4>(y + (long)s * cells + grow, out);
+        if (LN && ln.y_part && PAD) {
+            // one (mean, M2) pair per wave over its live lanes
+            const float cells_here = (float)(64 / kl * kb * 4);
+            const float sum = live ? (out[0] + out[1]) + (out[2] + out[3]) : 0.f;
+            const float mean = slot_wave_sum<64>(sum) / cells_here;
+            float m2 = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) m2 = fmaf(out[c] - mean, out[c] - mean, m2);
+            m2 = slot_wave_sum<64>(live ? m2 : 0.f);
+            if ((tid & 63) == 0) {
+                float *to = ln.y_part + (((long)s * ntube + tube) * (nt / 64) + tid / 64) * 2;
+                to[0] = mean;
+                to[1] = m2;
+            }
+        } else if (LN && ln.y_part) {
             // statistics of the result for the LayerNorm that follows: one (mean, M2) pair per wave
             const float sum = (out[0] + out[1]) + (out[2] + out[3]);
             const float mean = row16_sum(sum) * (1.f / 64);
@@ -182,11 +200,11 @@ void fwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
     }
 }
 
-bool k_ok(int K) { return K == 16 || K == 32 || K == 64 || K == 128; }
+bool k_ok(int K) { return K % 4 == 0 && K >= 8 && K <= 128; }
 
-template <int ACT, bool LN, bool RES> int launch(const StepArgs &a, hipStream_t st) {
-    auto kern = fwd_rows<ACT, LN, RES>;
-    const int nt = 4 * a.K, ntube = (a.M / kRowsTube) * (a.N / kRowsTube);
+template <int ACT, bool LN, bool RES, bool PAD> int launch_rows(const StepArgs &a, hipStream_t st) {
+    auto kern = fwd_rows<ACT, LN, RES, PAD>;
+    const int lanes = row_lanes(a.K, 4), nt = 16 * lanes, ntube = (a.M / kRowsTube) * (a.N / kRowsTube);
     const size_t lds = (size_t)(LN ? 4 : 2) * kRowsWin * a.K * sizeof(float);
     static bool big_lds_enabled = false;  // per instantiation
     if (lds > 64 * 1024 && !big_lds_enabled) {
@@ -196,26 +214,27 @@ template <int ACT, bool LN, bool RES> int launch(const StepArgs &a, hipStream_t 
         }
         big_lds_enabled = true;
     }
-    static int per_cu_cache[4] = {0, 0, 0, 0};  // per instantiation, by K
-    int &per_cu = per_cu_cache[a.K == 16 ? 0 : a.K == 32 ? 1 : a.K == 64 ? 2 : 3];
+    static int per_cu_cache[128 / 4 + 1];  // per instantiation, by K
+    int &per_cu = per_cu_cache[a.K / 4];
     if (per_cu == 0) {
         int n = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, nt, lds) != hipSuccess || n < 1) n = 1;
         per_cu = n;
     }
-    // chunks of the batch: enough workgroups to fill the chip, but none that walks fewer than
-    // eight elements for its one fetch of the weights (32^3 grid, batch 256: chunks of 11 beat
-    // chunks of 16, 32 and 64 elements, 10.33 against 10.42, 11.9 and 14.3 ms per 64-step training
-    // step: what limits the kernel is the trip to memory per element, and more workgroups hide it)
-    int nchunk = per_cu * plan_device_cus() / ntube;
-    if (nchunk > a.B / 8) nchunk = a.B / 8;
-    if (nchunk < 1) nchunk = 1;
-    const int chunk_len = (a.B + nchunk - 1) / nchunk;
-    nchunk = (a.B + chunk_len - 1) / chunk_len;
+    // (32^3 grid, batch 256: chunks of 11 beat chunks of 16, 32 and 64 elements, 10.33 against 10.42,
+    // 11.9 and 14.3 ms per 64-step training step: what limits the kernel is the trip to memory per
+    // element, and more workgroups hide it)
+    int chunk_len;
+    const int nchunk = plan_row_chunks(a.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, chunk_len);
     hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, nchunk)), dim3(nt), lds, st, (const float *)a.weight,
                        (const float *)a.bias, (const float *)a.scale, (const float *)a.x, (float *)a.y, a.B, a.M,
-                       a.N, a.K, ntube, nchunk, chunk_len, a.ln);
+                       a.N, a.K, ntube, nchunk, chunk_len, a.ln, lanes);
     return check_launch("fwd_rows");
+}
+
+template <int ACT, bool LN, bool RES> int launch(const StepArgs &a, hipStream_t st) {
+    return row_lanes(a.K, 4) * 4 == a.K ? launch_rows<ACT, LN, RES, false>(a, st)
+                                        : launch_rows<ACT, LN, RES, true>(a, st);
 }
 
 template <int ACT> int dispatch(const StepArgs &a, hipStream_t st) {
@@ -231,8 +250,9 @@ bool fwd_rows_supports(const StepArgs &a) {
            k_ok(a.K) && a.M % 4 == 0 && a.N % 4 == 0;
 }
 
-// (mean, M2) pairs per sample that it leaves in a.ln.y_part, each over 256 cells
-int fwd_rows_pairs(const StepArgs &a) { return (int)((long)a.M * a.N * a.K / 256); }
+// (mean, M2) pairs per sample that it leaves in a.ln.y_part: one per wave, over its live lanes' cells
+int fwd_rows_pairs(const StepArgs &a) { return (a.M * a.N / 16) * (16 * row_lanes(a.K, 4) / 64); }
+int fwd_rows_pair_count(const StepArgs &a) { return 64 / row_lanes(a.K, 4) * a.K; }
 
 int fwd_rows_launch(const StepArgs &a, hipStream_t st) {
     switch (a.activation) {

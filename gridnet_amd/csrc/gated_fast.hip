@@ -488,15 +488,17 @@ template <int BS, int NSLOT, int ACT> int launch_bwd(const StepArgs &a, hipStrea
                        (float *)a.workspace, a.B, a.M, a.N, a.K, a.inner, nblk, nchunk, chunk_len,
                        param_mode, dx_accumulate, split ? slab_floats : 0L);
     if (int rc = check_launch("gated_bwd_fast")) return rc;
+    TailJob tail{};
     if (split) {
         SlabTargets t{};
         t.dst[0] = (float *)a.dweight; t.end[0] = 54 * cells;
         t.dst[1] = (float *)a.dbias;   t.end[1] = 56 * cells;
         t.count = 2;
-        if (int rc = plan_reduce_slabs(slab, nchunk, slab_floats, t, new_params ? 0 : 1, st)) return rc;
+        tail = plan_tail_job(slab, nchunk, slab_floats, t, new_params ? 0 : 1,
+                             cross_rows_gated_supports(a) ? cross_rows_threads(a) : 256);
     }
     // same blocks, same batch chunks; the parameter gradients are complete, dx is not yet
-    return gated_cross_launch(a, (const float *)a.workspace, nchunk, chunk_len, st);
+    return gated_cross_launch(a, (const float *)a.workspace, nchunk, chunk_len, tail, st);
 }
 
 template <bool BWD, int ACT> int dispatch_bs(const StepArgs &a, hipStream_t st) {

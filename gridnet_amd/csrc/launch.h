@@ -82,6 +82,44 @@ enum ParamMode {
     kParamAtomic = 2         // several workgroups (batch chunks) share the cells (generic kernels only)
 };
 
+// The caller's gradient arrays and where each ends within one copy of them (see plan.h)
+struct SlabTargets {
+    float *dst[5];   // the caller's gradient arrays, in slab order
+    long end[5];     // end of each array within a slab, in floats (multiples of 4)
+    int count;
+};
+
+// The last step of the LayerNorm backward's sums (common.h), one workgroup per sample, where those
+// sums are ready when the gradient copies are.  It saves a launch of its own (4.4 us, a thirtieth
+// of a training step with one inner iteration).
+struct SumsJob {
+    const float *part;  // [B, parts, 2]
+    int parts, B;       // B = 0: no job
+    long n;
+    float *sums;        // [B, 2]
+};
+
+// The addition of the gradient copies, and a SumsJob, as work for spare workgroups of another
+// kernel: what the first kernel of a backward left behind is finished beside its second kernel
+// (cross_rows) instead of in a launch of its own, whose 8 us on a 32^3 grid were mostly start and end.
+struct TailJob {
+    const float *slabs;
+    int ncopies, accumulate, reduce_blocks;  // reduce_blocks = 0: no copies
+    long stride, total4;                     // total4: 16-byte vectors in a copy
+    SlabTargets t;
+    SumsJob sums;
+    int blocks() const { return reduce_blocks + sums.B; }
+};
+
+// Threads along a grid row of the row-wise kernels, with `cpt` cells per thread: the row's own number
+// where that is a power of two, the next one above it otherwise (rows then start where waves do,
+// the spare lanes idle: an eighth of them at rows of 56 cells, three eighths at 40)
+inline int row_lanes(int K, int cpt) {
+    int lanes = 4;
+    while (lanes * cpt < K) lanes *= 2;
+    return lanes;
+}
+
 struct LayerNormArgs {
     int dtype;
     const void *x, *gamma, *beta, *dy, *mean_in, *rstd_in;
@@ -114,13 +152,14 @@ int step_fast_backward_pairs(const StepArgs &a);  // pairs per sample that the b
 int step_fast_cross_pairs(const StepArgs &a);     // the same for step_cross_launch alone (behind chain_bwd)
 
 // fwd_rows.hip: the forward of a step with ONE inner iteration, dealt by whole K-rows (fp32, normalize
-// off, K of 16, 32, 64 or 128; the folded LayerNorm and the residual form as a.ln says)
+// off, K up to 128; the folded LayerNorm and the residual form as a.ln says)
 bool fwd_rows_supports(const StepArgs &a);
-int fwd_rows_pairs(const StepArgs &a);  // (mean, M2) pairs per sample in a.ln.y_part, 256 cells each
+int fwd_rows_pairs(const StepArgs &a);  // (mean, M2) pairs per sample in a.ln.y_part ...
+int fwd_rows_pair_count(const StepArgs &a);  // ... and the cells behind each
 int fwd_rows_launch(const StepArgs &a, hipStream_t st);
 
 // bwd_rows.hip: the backward of a step with ONE inner iteration by whole K-rows (with
-// cross_rows_full_launch behind it); fp32, normalize off, K of 16, 32 or 64; a.slabs as for
+// cross_rows_full_launch behind it); fp32, normalize off, K up to 64; a.slabs as for
 // step_backward_fast
 bool bwd_rows_supports(const StepArgs &a);
 size_t bwd_rows_slab_bytes(const StepArgs &a);
@@ -132,19 +171,20 @@ int bwd_rows_pairs(const StepArgs &a);
 bool bwd_rows_leaves_sums(const StepArgs &a);
 
 // cross_rows.hip: the cross-block part of the backward for 4^3 blocks, dealt by whole K-rows
-// (a.workspace holds D, a.dx the block-local part; LayerNorm fold as a.ln says); K of 16, 32, 64
-// or 128, normalize off
+// (a.workspace holds D, a.dx the block-local part; LayerNorm fold as a.ln says); K up to 128
 bool cross_rows_supports(const StepArgs &a);
+inline int cross_rows_threads(const StepArgs &a) { return 16 * row_lanes(a.K, 4); }
 int cross_rows_pairs(const StepArgs &a);  // LayerNorm sum pairs per sample that it leaves in a.ln.x_part
-int cross_rows_launch(const StepArgs &a, hipStream_t st);
+// `tail`: work that the kernel before left (gradient copies, LayerNorm sums), done by spare workgroups
+int cross_rows_launch(const StepArgs &a, const TailJob &tail, hipStream_t st);
 // all 27 taps, for bwd_rows.hip; ln_sums: with the LayerNorm sums of the finished rows (a.ln.x_part)
-int cross_rows_full_launch(const StepArgs &a, hipStream_t st, bool ln_sums);
+int cross_rows_full_launch(const StepArgs &a, const TailJob &tail, hipStream_t st, bool ln_sums);
 bool cross_rows_gated_supports(const StepArgs &a);  // the gated update: two weight sets, D0 and D1 in `dsum`
-int cross_rows_gated_launch(const StepArgs &a, const float *dsum, hipStream_t st);
+int cross_rows_gated_launch(const StepArgs &a, const float *dsum, const TailJob &tail, hipStream_t st);
 
 // step_fast.hip: the cross-block kernel alone (8^3 blocks, folded LayerNorm arguments in a.ln, the
 // D tensor in a.workspace), for chain_bwd.hip
-int step_cross_launch(const StepArgs &a, int nchunk, int chunk_len, hipStream_t st);
+int step_cross_launch(const StepArgs &a, int nchunk, int chunk_len, const TailJob &tail, hipStream_t st);
 
 // chain_bwd.hip: backward of one step of a chain with the cross-block part deferred to the step
 // before (a.ln.halo_in / halo_out); fp32, 8^3 blocks, 1..8 inner iterations, normalize off
@@ -172,7 +212,8 @@ size_t chain_all_workspace(const ChainAll &c);
 int chain_backward_all(const ChainAll &c, hipStream_t st);
 
 // step_fast.hip: the cross-block kernel on two weight sets, for gated_fast.hip
-int gated_cross_launch(const StepArgs &a, const float *dsum, int nchunk, int chunk_len, hipStream_t st);
+int gated_cross_launch(const StepArgs &a, const float *dsum, int nchunk, int chunk_len, const TailJob &tail,
+                       hipStream_t st);
 
 // gated_fast.hip: fp32, block sizes 4 and 8, as many inner iterations as the LDS holds
 bool gated_fast_supports(const StepArgs &a, bool backward);

@@ -36,6 +36,20 @@ void plan_batch_chunks(int B, int nblk, int nslot, int resident, bool whole, int
     nchunk = (B + chunk_len - 1) / chunk_len;
 }
 
+// The same for the row-wise kernels: at most `resident` workgroups, none that walks fewer than
+// `min_walk` elements for its one fetch of the weights.  Three keep the fetch below the walk and still
+// spread a small batch over the chip (forward / second kernel of the backward; 32^3, one inner
+// iteration, batch 64: 8.8 us at 3, 9.8 at 2 and 11.2 at 8; 40 x 48 x 56, batch 13: 18.6, 17.9
+// and 31.9); at large batches `resident` decides.
+constexpr int kRowsMinWalk = 3;
+int plan_row_chunks(int B, int ntube, int resident, int min_walk, int &chunk_len) {
+    int nchunk = resident / ntube;
+    if (nchunk > B / min_walk) nchunk = B / min_walk;
+    if (nchunk < 1) nchunk = 1;
+    chunk_len = (B + nchunk - 1) / nchunk;
+    return (B + chunk_len - 1) / chunk_len;
+}
+
 __global__ void plan_fill_zero_f32(float *p, long n) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long stride = (long)gridDim.x * blockDim.x;
@@ -56,48 +70,44 @@ int plan_fill_zero(float *p, long n, hipStream_t st) {
 // "slab": the arrays one behind the other, `planes` x cells floats) with plain stores, and one
 // small kernel adds the copies in chunk order into the caller's arrays: no atomics, the same bits
 // on every run.
-struct SlabTargets {
-    float *dst[5];   // the caller's gradient arrays, in slab order
-    long end[5];     // end of each array within a slab, in floats (multiples of 4)
-    int count;
-};
 
 // The slabs are 256-byte aligned and read as 16-byte vectors.  The caller's arrays are accessed as
 // 16-byte vectors too although the C ABI asks them to be aligned to their element size only:
 // gfx950 serves global accesses at any 4-byte alignment (a misaligned vector costs a second
 // request, nothing else); tests/test_gpu_alignment.py runs this with arrays 4 bytes off.
-// Work for spare workgroups of the kernel below: the last step of the LayerNorm backward's sums
-// (common.h), one workgroup per sample, where those sums are ready when the gradient copies are.
-// It saves a launch of its own (4.4 us, a thirtieth of a training step with one inner iteration).
-struct SumsJob {
-    const float *part;  // [B, parts, 2]
-    int parts, B;       // B = 0: no job
-    long n;
-    float *sums;        // [B, 2]
-};
-
-__global__ __launch_bounds__(256) void plan_reduce_slabs_f32(const float *slabs, int ncopies, long stride,
-                                                             SlabTargets t, long total4, int accumulate,
-                                                             int reduce_blocks, SumsJob job) {
-    if ((int)blockIdx.x >= reduce_blocks) {
-        __shared__ double red[256 / kWave][2];
-        finalize_sums_of_sample<256>(job.part, job.parts, job.n, job.sums, blockIdx.x - reduce_blocks, red);
+constexpr int kTailAhead = 4;
+// workgroup `block` of the job's; `red` is LDS, one pair of doubles per wave of the caller's workgroup
+template <int THREADS>
+__device__ __forceinline__ void run_tail_job(const TailJob &job, int block, int nthreads, double (*red)[2]) {
+    if (block >= job.reduce_blocks) {
+        finalize_sums_of_sample<THREADS>(job.sums.part, job.sums.parts, job.sums.n, job.sums.sums,
+                                         block - job.reduce_blocks, red, nthreads);
         return;
     }
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long step = (long)reduce_blocks * blockDim.x;
-    for (; i < total4; i += step) {
+    long i = (long)block * nthreads + threadIdx.x;
+    const long step = (long)job.reduce_blocks * nthreads;
+    for (; i < job.total4; i += step) {
         const long at = 4 * i;
-        float4 sum = *reinterpret_cast<const float4 *>(slabs + at);
-        for (int q = 1; q < ncopies; ++q) {
-            const float4 v = *reinterpret_cast<const float4 *>(slabs + q * stride + at);
-            sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int q0 = 0; q0 < job.ncopies; q0 += kTailAhead) {
+            // several copies requested before any is added: the kernel this runs beside leaves it few
+            // waves (past the last copy the requests repeat it)
+            float4 v[kTailAhead];
+#pragma unroll
+            for (int k = 0; k < kTailAhead; ++k)
+                v[k] = *reinterpret_cast<const float4 *>(job.slabs + min(q0 + k, job.ncopies - 1) * job.stride + at);
+#pragma unroll
+            for (int k = 0; k < kTailAhead; ++k) {
+                const bool have = q0 + k < job.ncopies;
+                sum.x += have ? v[k].x : 0.f; sum.y += have ? v[k].y : 0.f;
+                sum.z += have ? v[k].z : 0.f; sum.w += have ? v[k].w : 0.f;
+            }
         }
         int k = 0;
         long begin = 0;
-        while (k + 1 < t.count && at >= t.end[k]) begin = t.end[k++];
-        float4 *to = reinterpret_cast<float4 *>(t.dst[k] + (at - begin));
-        if (accumulate) {
+        while (k + 1 < job.t.count && at >= job.t.end[k]) begin = job.t.end[k++];
+        float4 *to = reinterpret_cast<float4 *>(job.t.dst[k] + (at - begin));
+        if (job.accumulate) {
             const float4 old = *to;
             sum.x += old.x; sum.y += old.y; sum.z += old.z; sum.w += old.w;
         }
@@ -121,13 +131,31 @@ int plan_slab_capacity(const void *slabs, size_t slab_bytes, long slab_floats) {
 constexpr int kSplitMinSaved = 2;
 int plan_split_room(int room, int B, int chunk_len) { return B - chunk_len < kSplitMinSaved ? 1 : room; }
 
-int plan_reduce_slabs(const float *slabs, int ncopies, long stride, const SlabTargets &t, int accumulate,
-                      hipStream_t st, const SumsJob &job = SumsJob{nullptr, 0, 0, 0, nullptr}) {
-    const long total4 = t.end[t.count - 1] / 4;
-    long blocks = (total4 + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(plan_reduce_slabs_f32, dim3((unsigned)(blocks + job.B)), dim3(256), 0, st, slabs, ncopies,
-                       stride, t, total4, accumulate, (int)blocks, job);
+// `nthreads`: threads per workgroup of the kernel that will run the job.  Its workgroups take as
+// many vectors per thread as keeps them below the number the chip holds.
+TailJob plan_tail_job(const float *slabs, int ncopies, long stride, const SlabTargets &t, int accumulate,
+                      int nthreads) {
+    TailJob job{};
+    job.slabs = slabs;
+    job.ncopies = ncopies;
+    job.accumulate = accumulate;
+    job.stride = stride;
+    job.total4 = t.end[t.count - 1] / 4;
+    job.t = t;
+    const long blocks = (job.total4 + nthreads - 1) / nthreads;
+    job.reduce_blocks = (int)(blocks > 4096 ? 4096 : blocks);
+    return job;
+}
+
+__global__ __launch_bounds__(256) void plan_run_tail_job(TailJob job) {
+    __shared__ double red[256 / kWave][2];
+    run_tail_job<256>(job, blockIdx.x, 256, red);
+}
+
+// as a kernel of its own, where there is no second kernel to take it along
+int plan_launch_tail_job(const TailJob &job, hipStream_t st) {
+    if (job.blocks() == 0) return GRIDNET_OK;
+    hipLaunchKernelGGL(plan_run_tail_job, dim3((unsigned)job.blocks()), dim3(256), 0, st, job);
     return check_launch("reduce_slabs");
 }
 

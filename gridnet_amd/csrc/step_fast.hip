@@ -32,7 +32,7 @@
 //     x_halo * D: the first kernel adds it once per element.  What the cells of NEIGHBOURING
 //     blocks receive needs the neighbours' D: the first kernel leaves D of every cell in a
 //     scratch tensor and a second kernel works it out and completes dx, in a fixed order:
-//     cross_rows (cross_rows.hip), dealt by whole grid rows, for rows of 16, 32, 64 or 128 cells;
+//     cross_rows (cross_rows.hip), dealt by whole grid rows, for rows of up to 128 cells;
 //     step_bwd_cross, dealt by block face from the D window with its real halo, for the rest.
 // Forward with 8^3 blocks: the same mapping over a window stored in two parts, so that every LDS
 // access of the inner loop is aligned and free of bank conflicts (step_fwd_split).
@@ -1807,6 +1807,8 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
                        (float *)a.workspace, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk, p.chunk_len,
                        param_mode, dx_accumulate, ln, (float)a.eps, qr, split ? slab_floats : 0L);
     if (int rc = check_launch("step_bwd_fast")) return rc;
+    const bool by_rows = cross_rows_supports(a);
+    TailJob tail{};
     if (split) {
         SlabTargets t{};
         t.dst[0] = (float *)a.dweight; t.end[0] = 27 * cells;
@@ -1818,12 +1820,13 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
             t.dst[4] = a.ln.dbeta;  t.end[4] = 31 * cells;
             t.count = 5;
         }
-        if (int rc = plan_reduce_slabs(slab, p.nchunk, slab_floats, t, new_params ? 0 : 1, st)) return rc;
+        tail = plan_tail_job(slab, p.nchunk, slab_floats, t, new_params ? 0 : 1, by_rows ? cross_rows_threads(a) : 256);
     }
     // same blocks, same batch chunks; the parameter gradients are complete, dx is not yet
     constexpr int XSLOT = BS == 8 ? kCrossSlots8 : kCrossSlots4;
     constexpr int XE = BS == 8 ? kCrossElems8 : kCrossElems4;
-    if (cross_rows_supports(a)) return cross_rows_launch(a, st);  // by whole K-rows
+    if (by_rows) return cross_rows_launch(a, tail, st);  // by whole K-rows
+    if (int rc = plan_launch_tail_job(tail, st)) return rc;
     hipLaunchKernelGGL((step_bwd_cross<BS, XSLOT, XE, LN, false, NORM>), dim3(padded_grid(p.nblk, p.nchunk)),
                        dim3(6 * BS * BS * XSLOT), 0, st, (const float *)a.weight,
                        (const float *)a.x, (const float *)a.workspace, (float *)a.dx, a.B, a.M, a.N,
@@ -1867,8 +1870,9 @@ template <bool BWD> int dispatch(const StepArgs &a, hipStream_t st) {
 
 // The cross-block kernel alone, completing a dx whose block-local part another kernel wrote
 // (8^3 blocks; the LayerNorm fold as a.ln says; D in a.workspace).
-int step_cross_launch(const StepArgs &a, int nchunk, int chunk_len, hipStream_t st) {
-    if (cross_rows_supports(a)) return cross_rows_launch(a, st);
+int step_cross_launch(const StepArgs &a, int nchunk, int chunk_len, const TailJob &tail, hipStream_t st) {
+    if (cross_rows_supports(a)) return cross_rows_launch(a, tail, st);
+    if (int rc = plan_launch_tail_job(tail, st)) return rc;
     const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
     hipLaunchKernelGGL((step_bwd_cross<8, kCrossSlots8, kCrossElems8, true>), dim3(padded_grid(nblk, nchunk)),
                        dim3(6 * 64 * kCrossSlots8), 0, st, (const float *)a.weight, (const float *)a.x,
@@ -1879,8 +1883,10 @@ int step_cross_launch(const StepArgs &a, int nchunk, int chunk_len, hipStream_t 
 
 // The cross-block kernel for the gated update: D0 and D1 of every cell behind one another in
 // `dsum`, weight [27, 2, M, N, K]; same blocks and batch chunks as the kernel that left them.
-int gated_cross_launch(const StepArgs &a, const float *dsum, int nchunk, int chunk_len, hipStream_t st) {
-    if (cross_rows_gated_supports(a)) return cross_rows_gated_launch(a, dsum, st);
+int gated_cross_launch(const StepArgs &a, const float *dsum, int nchunk, int chunk_len, const TailJob &tail,
+                       hipStream_t st) {
+    if (cross_rows_gated_supports(a)) return cross_rows_gated_launch(a, dsum, tail, st);
+    if (int rc = plan_launch_tail_job(tail, st)) return rc;
     const int bs = a.block_size;
     const int nblk = (a.M / bs) * (a.N / bs) * (a.K / bs);
     const LnFold none{};
@@ -1912,7 +1918,7 @@ int step_fast_forward_pairs(const StepArgs &a) {
     return (a.M / a.block_size) * (a.N / a.block_size) * (a.K / a.block_size) * step_fast_forward_parts(a.block_size);
 }
 int step_fast_forward_pair_count(const StepArgs &a) {
-    return fwd_rows_supports(a) ? 256 : step_fast_forward_part_count(a.block_size);
+    return fwd_rows_supports(a) ? fwd_rows_pair_count(a) : step_fast_forward_part_count(a.block_size);
 }
 int step_fast_backward_parts(int block_size) { return block_size == 8 ? 2 : 1; }
 int step_fast_backward_pairs(const StepArgs &a) {

@@ -607,6 +607,54 @@ int gridnet_hip_chain_set_spin_limit(int limit) {
     return old;
 }
 
+int gridnet_hip_chain_forward_all_supported(int dtype, int B, int M, int N, int K, int inner, int outer,
+                                            int block_size, int normalize) {
+    if (dtype != GRIDNET_F32 || block_size != 8 || normalize) return 0;
+    return chain_fwd_supports(B, M, N, K, inner, outer) ? 1 : 0;
+}
+
+size_t gridnet_hip_chain_forward_all_workspace_bytes(int B, int M, int N, int K) {
+    if (B <= 0 || M <= 0 || N <= 0 || K <= 0 || M % 8 || N % 8 || K % 8) return 0;
+    ChainFwd c{};
+    c.B = B; c.M = M; c.N = N; c.K = K;
+    return chain_fwd_workspace(c);
+}
+
+int gridnet_hip_chain_forward_all(int dtype, const void *weight, const void *bias, const void *scale,
+                                  const void *gamma, const void *beta, const void *x0, void *y_raw,
+                                  void *stats, void *out, int B, int M, int N, int K, int inner, int outer,
+                                  int block_size, double ln_eps, int activation, void *workspace,
+                                  size_t workspace_bytes, void *stream) {
+    StepArgs a{};
+    a.dtype = dtype; a.weight = weight; a.bias = bias; a.scale = scale; a.x = x0; a.y = out;
+    a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner; a.block_size = block_size;
+    a.activation = activation;
+    if (dtype != GRIDNET_F32 || block_size != 8)
+        return fail(GRIDNET_ERR_ARGUMENT, "the one-launch chain is float32 with block_size 8 (dtype id %d, block_size %d)",
+                    dtype, block_size);
+    if (int rc = check_step(a, false)) return rc;
+    if (!chain_fwd_supports(B, M, N, K, inner, outer))
+        return fail(GRIDNET_ERR_ARGUMENT,
+                    "the one-launch forward does not cover this problem (B=%d grid %dx%dx%d inner=%d outer=%d): "
+                    "see gridnet_hip_chain_forward_all_supported; use gridnet_hip_fused_forward",
+                    B, M, N, K, inner, outer);
+    if (!gamma || !beta || (y_raw == nullptr) != (stats == nullptr))
+        return fail(GRIDNET_ERR_ARGUMENT, "null pointer (y_raw and stats go together: both or neither)");
+    ChainFwd c{};
+    c.weight = (const float *)weight; c.bias = (const float *)bias; c.scale = (const float *)scale;
+    c.gamma = (const float *)gamma; c.beta = (const float *)beta; c.x0 = (const float *)x0;
+    c.y_all = (float *)y_raw; c.stats = (float *)stats; c.out = (float *)out;
+    c.B = B; c.M = M; c.N = N; c.K = K; c.inner = inner; c.outer = outer; c.activation = activation;
+    c.eps = ln_eps;
+    c.workspace = workspace; c.workspace_bytes = workspace_bytes;
+    c.spin_limit = chain_spin_limit;
+    const size_t need = chain_fwd_workspace(c);
+    if (!workspace || workspace_bytes < need)
+        return fail(GRIDNET_ERR_WORKSPACE, "the one-launch forward needs %zu bytes of workspace, got %zu", need,
+                    workspace ? workspace_bytes : (size_t)0);
+    return chain_forward_all(c, (hipStream_t)stream);
+}
+
 int gridnet_hip_chain_all_supported(int dtype, int B, int M, int N, int K, int inner, int outer,
                                     int block_size, int normalize) {
     if (dtype != GRIDNET_F32 || block_size != 8 || normalize) return 0;

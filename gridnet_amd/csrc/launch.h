@@ -211,6 +211,23 @@ bool chain_all_supports(int B, int M, int N, int K, int inner, int outer);
 size_t chain_all_workspace(const ChainAll &c);
 int chain_backward_all(const ChainAll &c, hipStream_t st);
 
+// chain_fwd.hip: the forward of a whole chain of `outer` steps (one parameter set, the plain loop) in
+// one launch of resident workgroups, where blocks x batch elements are few enough for that; fp32, 8^3
+// blocks, normalize off.
+struct ChainFwd {
+    const float *weight, *bias, *scale, *gamma, *beta, *x0;
+    float *y_all, *stats;  // [outer,B,M,N,K] raw outputs and [outer,B,2] statistics for a backward, or null
+    float *out;            // [B,M,N,K]
+    int B, M, N, K, inner, outer, activation;
+    double eps;
+    void *workspace;
+    size_t workspace_bytes;
+    int spin_limit;  // as in ChainAll
+};
+bool chain_fwd_supports(int B, int M, int N, int K, int inner, int outer);
+size_t chain_fwd_workspace(const ChainFwd &c);
+int chain_forward_all(const ChainFwd &c, hipStream_t st);
+
 // step_fast.hip: the cross-block kernel on two weight sets, for gated_fast.hip
 int gated_cross_launch(const StepArgs &a, const float *dsum, int nchunk, int chunk_len, const TailJob &tail,
                        hipStream_t st);

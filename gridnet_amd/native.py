@@ -125,6 +125,12 @@ def _load():
     lib.gridnet_hip_chain_all_workspace_bytes.argtypes = [i] * 7
     lib.gridnet_hip_chain_backward_all.restype = i
     lib.gridnet_hip_chain_backward_all.argtypes = [i] + [p] * 15 + [i] * 9 + [p, z, p]
+    lib.gridnet_hip_chain_forward_all_supported.restype = i
+    lib.gridnet_hip_chain_forward_all_supported.argtypes = [i] * 9
+    lib.gridnet_hip_chain_forward_all_workspace_bytes.restype = z
+    lib.gridnet_hip_chain_forward_all_workspace_bytes.argtypes = [i] * 4
+    lib.gridnet_hip_chain_forward_all.restype = i
+    lib.gridnet_hip_chain_forward_all.argtypes = [i] + [p] * 9 + [i] * 7 + [d, i, p, z, p]
     lib.gridnet_hip_chain_set_spin_limit.restype = i
     lib.gridnet_hip_chain_set_spin_limit.argtypes = [i]
     return lib

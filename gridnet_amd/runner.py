@@ -27,6 +27,10 @@ weights and gradient accumulators from step to step and signal each other throug
 waits are bounded; ``chain_all_status()`` (which synchronises) tells whether one ran out, in which
 case ``backward`` must be repeated with ``chain_all`` off -- ``backward_checked`` does both.
 
+Where blocks and batch are few enough to be resident at once (a 32^3 grid at up to 16 samples) the
+forward of a chain with one parameter set is one launch too (``gridnet_hip_chain_forward_all``;
+``forward_all=False``: never).
+
 ``weight``, ``bias`` and ``scale`` may each be a list of ``outer`` tensors: one parameter set
 per outer step (the reference's ``--separate_params``, gridnet/scripts/train_imagenet.py:54-58).
 ``backward`` then returns lists of gradients for them, one entry per step.
@@ -46,7 +50,7 @@ class BodyRunner:
                  block_size: int, activation: str = "leaky_relu", normalize: bool = False,
                  eps: float = 1e-5, ln_eps: float = 1e-5, backward: bool = True,
                  fused: bool = False, outer_residual: bool = False, chain=None,
-                 chain_all=None):
+                 chain_all=None, forward_all=None):
         self.separate = isinstance(weight, (list, tuple))
         if self.separate:
             if not (len(weight) == len(bias) == len(scale) == outer):
@@ -74,9 +78,14 @@ class BodyRunner:
         # What a mode never touches is not allocated: the fused chain keeps the raw outputs s[*]
         # and one h (the final result; forward only, a second buffer to alternate with), the
         # residual chain every h and two s (free buffers for its backward).
+        self.forward_all = bool(
+            fused and not outer_residual and not self.separate and forward_all is not False and
+            _n.lib.gridnet_hip_chain_forward_all_supported(
+                self.dt, batch, self.M, self.N, self.K, inner, outer, block_size, self.normalize))
         n_h, n_s = keep + 1, keep
         if fused and not outer_residual:
-            n_h = 1 if backward else 2
+            n_h = 1 if backward or self.forward_all else 2
+            n_s = 0 if self.forward_all and not backward else n_s
         if fused and outer_residual:
             n_s = 2 if backward else 1
         self.h = [torch.empty(shape, device=dev, dtype=dtype) for _ in range(n_h)]
@@ -111,8 +120,12 @@ class BodyRunner:
             if weight.dtype != torch.float32 or normalize or inner < 1:
                 raise RuntimeError("the fused body covers float32, normalize=False, inner >= 1")
             self.stats = torch.empty(max(keep, 2), batch, 2, device=dev, dtype=dtype)
-            self.fw_ws_bytes = _n.lib.gridnet_hip_fused_workspace_bytes(
-                batch, self.M, self.N, self.K, inner, block_size, 0)
+            if self.forward_all:
+                self.fw_ws_bytes = _n.lib.gridnet_hip_chain_forward_all_workspace_bytes(
+                    batch, self.M, self.N, self.K)
+            else:
+                self.fw_ws_bytes = _n.lib.gridnet_hip_fused_workspace_bytes(
+                    batch, self.M, self.N, self.K, inner, block_size, 0)
             self.fw_ws = _n.workspace(self.fw_ws_bytes, dev)
             if outer_residual:  # statistics of h_0 .. h_outer, and a LayerNorm output nobody reads
                 self.stats = torch.empty(keep + 1, batch, 2, device=dev, dtype=dtype)
@@ -188,6 +201,15 @@ class BodyRunner:
         stream = _n.current_stream(self.w)
         keep = self.has_backward
         self.x0 = x0
+        if self.forward_all:
+            self._mark("step_fwd", 0)
+            _n.check(_n.lib.gridnet_hip_chain_forward_all(
+                self.dt, *self._params(0), self.gamma.data_ptr(), self.beta.data_ptr(), x0.data_ptr(),
+                self.s_all.data_ptr() if keep else None, self.stats.data_ptr() if keep else None,
+                self.h[0].data_ptr(), self.B, self.M, self.N, self.K, self.inner, self.outer, self.bs,
+                self.ln_eps, self.act, self.fw_ws.data_ptr(), self.fw_ws_bytes, stream))
+            self._mark("step_fwd", 1)
+            return self.h[0]
         x, x_stats = x0, None
         for j in range(self.outer):
             # forward only: nothing is kept, two raw buffers and two statistics rows alternate

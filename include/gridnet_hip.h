@@ -352,6 +352,23 @@ int gridnet_hip_chain_backward_all(int dtype, const void *weight, const void *bi
                                    void *dbeta, void *dx, int B, int M, int N, int K, int inner,
                                    int outer, int block_size, int activation, int flags,
                                    void *workspace, size_t workspace_bytes, void *stream);
+/*
+ * ---- The forward of a whole chain in one launch, for small problems ------------------------------
+ * The same loop forward, h = LayerNorm(step(h)) `outer` times: out [B,M,N,K].  y_raw [outer,B,M,N,K]
+ * and stats [outer,B,2] receive what a backward needs, or are both NULL.  float32, normalize = false,
+ * block_size 8, inner >= 1, outer >= 2, and few enough (block, batch element) pairs to be resident at
+ * once; gridnet_hip_chain_forward_all_supported() tells.  Launched cooperatively; its waits are
+ * bounded, and should one run out a second kernel on the same stream computes the chain again without
+ * waits: the results are complete either way.
+ */
+int gridnet_hip_chain_forward_all_supported(int dtype, int B, int M, int N, int K, int inner, int outer,
+                                            int block_size, int normalize);
+size_t gridnet_hip_chain_forward_all_workspace_bytes(int B, int M, int N, int K);
+int gridnet_hip_chain_forward_all(int dtype, const void *weight, const void *bias, const void *scale,
+                                  const void *gamma, const void *beta, const void *x0, void *y_raw,
+                                  void *stats, void *out, int B, int M, int N, int K, int inner, int outer,
+                                  int block_size, double ln_eps, int activation, void *workspace,
+                                  size_t workspace_bytes, void *stream);
 /* How often a wait inside the one-launch chain kernels polls before it gives up (default 200000,
  * about a second).  A negative value makes the kernels never signal completion to each other, so
  * that every wait runs out after -limit polls: the give-up path, for tests.  Returns the old value. */

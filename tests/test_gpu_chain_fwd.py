@@ -1,0 +1,74 @@
+"""The forward of a whole chain in one launch (csrc/chain_fwd.hip) against the CPU oracle in fp64: one
+block and many, grids that are no cubes, numbers of outer steps on both sides of the ring of four, the
+backward behind it (which reads the raw outputs and statistics it left), and the second kernel
+that takes over when a wait runs out."""
+
+import pytest
+import torch
+
+from helpers import assert_close, make_acts, make_params
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+NAMES = ("y", "dweight", "dbias", "dscale", "dgamma", "dbeta", "dx0")
+
+
+def run_chain(shape, batch, inner, outer, activation, backward=True, **kw):
+    from gridnet_amd.runner import BodyRunner
+
+    print(f"chain_fwd {shape} B={batch} inner={inner} outer={outer} {activation} {kw}", flush=True)
+    g = torch.Generator().manual_seed(5)
+    params = [*make_params(shape, seed=4), 1 + 0.2 * torch.randn(shape, generator=g), 0.2 * torch.randn(shape, generator=g)]
+    x, gy = make_acts(batch, shape, seed=6), make_acts(batch, shape, seed=7)
+    run = BodyRunner(*(t.to(DEV) for t in params), batch, inner, outer, 8, activation, fused=True, backward=backward, **kw)
+    got = [run.forward(x.to(DEV)).clone()]
+    if backward:
+        got += [t.clone() for t in run.backward(gy.to(DEV))]
+    torch.cuda.synchronize()
+    return run, params, x, gy, got
+
+
+@pytest.mark.parametrize("shape,batch,inner,outer,activation", [
+    ((8, 8, 8), 1, 1, 2, "silu"), ((8, 8, 8), 5, 3, 5, "tanh"), ((8, 16, 24), 3, 2, 3, "silu"),
+    ((16, 8, 40), 2, 1, 6, "tanh"), ((32, 32, 32), 1, 1, 9, "silu"), ((32, 32, 32), 3, 2, 4, "silu"),
+    ((40, 48, 56), 1, 1, 3, "tanh")], ids=str)
+def test_against_oracle(shape, batch, inner, outer, activation):
+    from oracle.network import network_forward_backward
+
+    run, params, x, gy, got = run_chain(shape, batch, inner, outer, activation)
+    assert run.forward_all
+    want = network_forward_backward([t.double() for t in params], x.double(), gy.double(), inner_iterations=inner,
+                                    outer_iterations=outer, block_size=8, activation=activation)
+    for name, a, e in zip(NAMES, got, want):
+        assert_close(a, e, rtol=2e-4, atol=2e-5, what=name)
+    again = run_chain(shape, batch, inner, outer, activation, backward=False)[-1]
+    assert torch.equal(again[0], got[0])
+
+
+def test_a_wait_that_runs_out_is_repaired():
+    from gridnet_amd import native as n
+
+    args = ((16, 8, 24), 3, 2, 5, "silu")
+    want = run_chain(*args, forward_all=False)[-1]
+    old = n.lib.gridnet_hip_chain_set_spin_limit(-20)  # nobody publishes: every wait runs out
+    try:
+        run, *_, got = run_chain(*args, chain_all=False)
+    finally:
+        n.lib.gridnet_hip_chain_set_spin_limit(old)
+    assert run.forward_all
+    for name, a, e in zip(NAMES, got, want):
+        assert_close(a, e, rtol=1e-5, atol=1e-5, what=name)
+
+
+def test_the_largest_batch_and_one_more():
+    run = run_chain((16, 16, 16), 1, 1, 2, "relu", backward=False)[0]
+    batch = 1
+    from gridnet_amd import native as n
+
+    while n.lib.gridnet_hip_chain_forward_all_supported(0, batch + 1, 16, 16, 16, 1, 5, 8, 0):
+        batch += 1
+    for b in (batch, batch + 1):
+        run, *_, got = run_chain((16, 16, 16), b, 1, 5, "silu", backward=False)
+        assert run.forward_all == (b == batch)
+        want = run_chain((16, 16, 16), b, 1, 5, "silu", backward=False, forward_all=False)[-1]
+        assert_close(got[0], want[0], rtol=1e-5, atol=1e-5, what=f"batch {b}")

@@ -107,7 +107,10 @@ def gpu_run(wl, steps, warmup, fused, graph_replay=True, chain_all=None, chain=N
         assert p0 == 0 and p1 == 1
         spans.setdefault(name, []).append(e0.elapsed_time(e1) * 1e-3)
     kernel_s = {k: sum(v) / len(v) for k, v in spans.items()}
-    return wall, graph_s, kernel_s, bool(getattr(run, "chain_all", False))
+    # entry points that take all outer steps in one call
+    whole = {name for name, flags in (("step_fwd", ("forward_all", "rows")), ("step_bwd", ("chain_all", "rows")))
+             if any(getattr(run, f, False) for f in flags)}
+    return wall, graph_s, kernel_s, whole
 
 
 def what_binds(hbm_frac, valu_busy_pct, lds_busy_frac):
@@ -279,15 +282,14 @@ def main():
             sys.exit("bench.py: --outer-residual runs through the fused entry points (no --path steps, no --normalize)")
         wl = dataclasses.replace(wl, name=wl.name + " outer_residual")
     fused = args.path == "fused" and not wl.normalize and wl.inner >= 1
-    wall, graph_s, kernel_s, one_launch = gpu_run(wl, args.steps, args.warmup, fused, not args.no_graph,
+    wall, graph_s, kernel_s, whole = gpu_run(wl, args.steps, args.warmup, fused, not args.no_graph,
                                       {"auto": None, "on": True, "off": False}[args.chain_all],
                                       {"auto": None, "on": True, "off": False}[args.chain], args.outer_residual)
     bytes_ = wl.algorithmic_bytes()
     if fused:  # a fused entry point does the work of the step AND of the LayerNorm beside it
         bytes_["step_fwd"] += bytes_["ln_fwd"]
         bytes_["step_bwd"] += bytes_["ln_bwd"]
-    # the one-launch chain backward takes all outer steps in ONE call
-    steps_per_call = {"step_bwd": wl.outer} if one_launch else {}
+    steps_per_call = {name: wl.outer for name in whole}
     for k, n_steps in steps_per_call.items():
         bytes_[k] *= n_steps
     dominant = max(kernel_s, key=lambda k: kernel_s[k])
@@ -352,7 +354,7 @@ def main():
         "config": {"workload": wl.name, "activation": wl.activation, "normalize": wl.normalize,
                    "pass": "fwd+bwd" if wl.backward else "fwd",
                    "path": ("fused step+LayerNorm entry points" + (", backward of the chain in one launch"
-                                                                   if one_launch else ""))
+                                                                   if dominant in whole else ""))
                            if fused else "step and LayerNorm calls"},
         "timing": {"headline": "eager wall clock over the timed steps, synchronised on both sides",
                    "eager_ms_per_step": wall * 1e3,

@@ -622,8 +622,8 @@ size_t gridnet_hip_chain_forward_all_workspace_bytes(int B, int M, int N, int K)
 
 int gridnet_hip_chain_forward_all(int dtype, const void *weight, const void *bias, const void *scale,
                                   const void *gamma, const void *beta, const void *x0, void *y_raw,
-                                  void *stats, void *out, int B, int M, int N, int K, int inner, int outer,
-                                  int block_size, double ln_eps, int activation, void *workspace,
+                                  void *stats, void *saved, void *out, int B, int M, int N, int K, int inner,
+                                  int outer, int block_size, double ln_eps, int activation, void *workspace,
                                   size_t workspace_bytes, void *stream) {
     StepArgs a{};
     a.dtype = dtype; a.weight = weight; a.bias = bias; a.scale = scale; a.x = x0; a.y = out;
@@ -643,6 +643,8 @@ int gridnet_hip_chain_forward_all(int dtype, const void *weight, const void *bia
     ChainFwd c{};
     c.weight = (const float *)weight; c.bias = (const float *)bias; c.scale = (const float *)scale;
     c.gamma = (const float *)gamma; c.beta = (const float *)beta; c.x0 = (const float *)x0;
+    if (saved && inner != 1) return fail(GRIDNET_ERR_ARGUMENT, "pre-activations are saved for one inner iteration only");
+    c.saved = (float *)saved;
     c.y_all = (float *)y_raw; c.stats = (float *)stats; c.out = (float *)out;
     c.B = B; c.M = M; c.N = N; c.K = K; c.inner = inner; c.outer = outer; c.activation = activation;
     c.eps = ln_eps;
@@ -653,6 +655,77 @@ int gridnet_hip_chain_forward_all(int dtype, const void *weight, const void *bia
         return fail(GRIDNET_ERR_WORKSPACE, "the one-launch forward needs %zu bytes of workspace, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
     return chain_forward_all(c, (hipStream_t)stream);
+}
+
+int gridnet_hip_rows_chain_supported(int dtype, int M, int N, int K, int inner, int normalize, int gated) {
+    if (dtype != GRIDNET_F32 || inner != 1 || normalize) return 0;
+    return rows_chain_supports(M, N, K, gated != 0) ? 1 : 0;
+}
+
+size_t gridnet_hip_rows_chain_workspace_bytes(int B, int M, int N, int K, int gated, int keep, int backward) {
+    if (B <= 0 || !rows_chain_supports(M, N, K, gated != 0)) return 0;
+    RowsChain c{};
+    c.B = B; c.M = M; c.N = N; c.K = K; c.gated = gated != 0; c.keep = keep != 0;
+    return rows_chain_workspace(c, backward != 0) + 256;  // the caller's may start at any address
+}
+
+static int check_rows_chain(RowsChain &c, bool backward, void *workspace, size_t workspace_bytes) {
+    StepArgs a{};
+    a.dtype = GRIDNET_F32; a.weight = c.weight; a.bias = c.bias;
+    a.B = c.B; a.M = c.M; a.N = c.N; a.K = c.K; a.inner = 1; a.block_size = 4; a.activation = c.activation;
+    a.scale = c.gated ? c.gamma : c.scale;
+    a.x = c.x0; a.y = c.out; a.dy = c.dy;
+    a.dweight = c.dweight; a.dbias = c.dbias; a.dscale = c.gated ? c.dgamma : c.dscale; a.dx = c.dx;
+    if (backward) a.bias = c.gamma;  // not read there
+    if (int rc = check_step(a, backward)) return rc;
+    if (!rows_chain_supports(c.M, c.N, c.K, c.gated))
+        return fail(GRIDNET_ERR_ARGUMENT, "the row-wise chain does not cover a %dx%dx%d grid: see "
+                    "gridnet_hip_rows_chain_supported", c.M, c.N, c.K);
+    if (c.outer < 1) return fail(GRIDNET_ERR_ARGUMENT, "outer must be at least 1, got %d", c.outer);
+    if (c.B == 0) return GRIDNET_OK;
+    if (!c.gamma || !c.beta) return fail(GRIDNET_ERR_ARGUMENT, "null pointer");
+    c.keep = c.y_raw != nullptr;
+    if ((backward && !c.keep) || c.keep != (c.stats != nullptr) || c.keep != (c.saved != nullptr))
+        return fail(GRIDNET_ERR_ARGUMENT, "y_raw, stats and saved go together: all or none, all for a backward");
+    if (backward && (!c.dgamma || !c.dbeta)) return fail(GRIDNET_ERR_ARGUMENT, "null pointer");
+    const size_t need = rows_chain_workspace(c, backward) + 256;
+    if (!workspace || workspace_bytes < need)
+        return fail(GRIDNET_ERR_WORKSPACE, "the row-wise chain needs %zu bytes of workspace, got %zu", need,
+                    workspace ? workspace_bytes : (size_t)0);
+    c.workspace = (void *)(((uintptr_t)workspace + 255) / 256 * 256);
+    return GRIDNET_OK;
+}
+
+int gridnet_hip_rows_chain_forward(const void *weight, const void *bias, const void *scale, const void *gamma,
+                                   const void *beta, const void *x0, void *y_raw, void *stats, void *saved,
+                                   void *out, int B, int M, int N, int K, int outer, int gated, double ln_eps,
+                                   int activation, void *workspace, size_t workspace_bytes, void *stream) {
+    RowsChain c{};
+    c.weight = (const float *)weight; c.bias = (const float *)bias; c.scale = (const float *)scale;
+    c.gamma = (const float *)gamma; c.beta = (const float *)beta; c.x0 = (const float *)x0;
+    c.y_raw = (float *)y_raw; c.stats = (float *)stats; c.saved = (float *)saved; c.out = (float *)out;
+    c.B = B; c.M = M; c.N = N; c.K = K; c.outer = outer; c.activation = activation; c.gated = gated != 0;
+    c.eps = ln_eps;
+    if (int rc = check_rows_chain(c, false, workspace, workspace_bytes)) return rc;
+    return B == 0 ? GRIDNET_OK : rows_chain_forward(c, (hipStream_t)stream);
+}
+
+int gridnet_hip_rows_chain_backward(const void *weight, const void *scale, const void *gamma, const void *beta,
+                                    const void *x0, const void *y_raw, const void *stats, const void *saved,
+                                    const void *dy, void *dweight, void *dbias, void *dscale, void *dgamma,
+                                    void *dbeta, void *dx, int B, int M, int N, int K, int outer, int gated,
+                                    int activation, int flags, void *workspace, size_t workspace_bytes,
+                                    void *stream) {
+    RowsChain c{};
+    c.weight = (const float *)weight; c.scale = (const float *)scale;
+    c.gamma = (const float *)gamma; c.beta = (const float *)beta; c.x0 = (const float *)x0;
+    c.y_raw = (float *)y_raw; c.stats = (float *)stats; c.saved = (float *)saved; c.dy = (const float *)dy;
+    c.dweight = (float *)dweight; c.dbias = (float *)dbias; c.dscale = (float *)dscale;
+    c.dgamma = (float *)dgamma; c.dbeta = (float *)dbeta; c.dx = (float *)dx;
+    c.B = B; c.M = M; c.N = N; c.K = K; c.outer = outer; c.activation = activation; c.gated = gated != 0;
+    c.flags = flags;
+    if (int rc = check_rows_chain(c, true, workspace, workspace_bytes)) return rc;
+    return B == 0 ? GRIDNET_OK : rows_chain_backward(c, (hipStream_t)stream);
 }
 
 int gridnet_hip_chain_all_supported(int dtype, int B, int M, int N, int K, int inner, int outer,

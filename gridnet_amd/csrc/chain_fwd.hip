@@ -46,6 +46,7 @@ struct ChainFwdArgs {
     const float *weight, *bias, *scale, *gamma, *beta, *x0;
     float *y_all;   // [outer,B,cells] raw outputs, or null
     float *stats;   // [outer,B,2], or null
+    float *saved;   // [outer,B,cells] pre-activations of the last inner iteration, or null
     float *out;     // [B,cells]: LayerNorm of the last raw output
     unsigned *status;
     unsigned long long *parts;  // [kRing][B][nblk][kGroups]: (mean, M2)
@@ -104,7 +105,7 @@ __device__ __forceinline__ void load_weights(const float *weight, int cells, int
 // first.
 template <int ACT>
 __device__ __forceinline__ float advance(float (*win)[kWindow], int at, int dir, const float (&w)[27], float bias,
-                                         float scale, float x, int inner) {
+                                         float scale, float x, int inner, float &last_u) {
     for (int it = 0; it < inner; ++it) {
         const float *row = win[it & 1] + at, *from[3] = {row - dir, row, row + dir};
         float u = bias;
@@ -112,30 +113,13 @@ __device__ __forceinline__ float advance(float (*win)[kWindow], int at, int dir,
         for (int t = 0; t < 27; ++t)
             u = fmaf(w[t], from[t % 3][(t / 9 - 1) * kSide * kSide + (t / 3 % 3 - 1) * kSide], u);
         x = fmaf(scale, Act<ACT, float>::f(u), x);
+        last_u = u;
         if (it + 1 < inner) {
             win[(it + 1) & 1][at] = x;
             lds_barrier();
         }
     }
     return x;
-}
-
-// wave_sum for doubles on the vector ALU: rotations within the rows of 16 lanes, then across the rows
-// by readlane.  The shuffles of the general one go through LDS, eighteen trips of them here in a row
-// (0.5 us of a step).
-__device__ __forceinline__ double wave_sum_dpp(double v) {
-    const auto rotated = [](double d, auto move) {
-        return __hiloint2double(move(__double2hiint(d)), move(__double2loint(d)));
-    };
-    v += rotated(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x128, 0xf, 0xf, false); });
-    v += rotated(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x124, 0xf, 0xf, false); });
-    v += rotated(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x122, 0xf, 0xf, false); });
-    v += rotated(v, [](int x) { return __builtin_amdgcn_update_dpp(0, x, 0x121, 0xf, 0xf, false); });
-    const auto row = [&](int lane) {
-        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                                __builtin_amdgcn_readlane(__double2loint(v), lane));
-    };
-    return (row(0) + row(16)) + (row(32) + row(48));
 }
 
 // Statistics of the block's values as the kernels for 8^3 blocks leave them, bit for bit: two groups of
@@ -158,9 +142,7 @@ __device__ __forceinline__ unsigned long long group_moments(const float *values,
     return (unsigned long long)__float_as_uint(mean) | (unsigned long long)__float_as_uint(m2) << 32;
 }
 
-// Sums over the groups of an element: means, M2, squares of the means; then its statistics.  1 / sqrt by
-// the hardware's estimate and two Newton steps in double: a relative error below 1e-12 in a quarter
-// of the instructions.
+// Sums over the groups of an element: means, M2, squares of the means; then its statistics.
 struct GroupSums {
     double m = 0.0, q = 0.0, mm = 0.0;
     __device__ __forceinline__ void add(unsigned long long word) {
@@ -177,12 +159,8 @@ struct GroupSums {
     __device__ __forceinline__ void finish(double inv_groups, double eps, float &mean, float &rstd) const {
         const double centre = m * inv_groups;
         const double var = fma(q * inv_groups, 1.0 / kGroupCells, fma(-centre, centre, mm * inv_groups));
-        const double v = (var > 0.0 ? var : 0.0) + eps;
-        double r = __builtin_amdgcn_rsq(v);
-        r = r * fma(-0.5 * v * r, r, 1.5);
-        r = r * fma(-0.5 * v * r, r, 1.5);
         mean = (float)centre;
-        rstd = (float)r;
+        rstd = (float)rsqrt_newton((var > 0.0 ? var : 0.0) + eps);
     }
 };
 
@@ -262,7 +240,8 @@ template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd(Chain
         win[0][p.at] = x;
         if (p.edge_at >= 0) win[0][p.edge_at] = win[1][p.edge_at] = e;
         lds_barrier();
-        own = advance<ACT>(win, p.at, dir, w, bias, scale, x, a.inner);
+        float u;
+        own = advance<ACT>(win, p.at, dir, w, bias, scale, x, a.inner, u);
         st_agent(ring + (j & (kRing - 1)) * slot_cells + p.cell, own);
         values[tid] = own;
         lds_barrier();
@@ -272,6 +251,7 @@ template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd(Chain
                 st_agent(parts + (j & (kRing - 1)) * slot_parts + kGroups * blk + wave, word);
         }
         if (a.y_all) a.y_all[(long)j * slot_cells + (long)s * cells + p.cell] = own;
+        if (a.saved) a.saved[(long)j * slot_cells + (long)s * cells + p.cell] = u;
     }
 }
 
@@ -304,9 +284,11 @@ template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd_repai
             win[0][p.at] = x;
             if (p.edge_at >= 0) win[0][p.edge_at] = win[1][p.edge_at] = e;
             __syncthreads();
-            const float y = advance<ACT>(win, p.at, dir, w, a.bias[p.cell], a.scale[p.cell], x, a.inner);
+            float u;
+            const float y = advance<ACT>(win, p.at, dir, w, a.bias[p.cell], a.scale[p.cell], x, a.inner, u);
             to[p.cell] = y;
             if (a.y_all) a.y_all[(long)j * slot_cells + mine + p.cell] = y;
+            if (a.saved) a.saved[(long)j * slot_cells + mine + p.cell] = u;
             values[tid] = y;
             __syncthreads();
             if (tid / 64 < kGroups) {
@@ -345,7 +327,7 @@ template <int ACT> int launch_chain_fwd(const ChainFwd &c, hipStream_t st) {
     char *ws = (char *)(((uintptr_t)c.workspace + kAlign - 1) / kAlign * kAlign);
     ChainFwdArgs a{};
     a.weight = c.weight; a.bias = c.bias; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta; a.x0 = c.x0;
-    a.y_all = c.y_all; a.stats = c.stats; a.out = c.out;
+    a.y_all = c.y_all; a.stats = c.stats; a.saved = c.saved; a.out = c.out;
     a.status = (unsigned *)ws;
     a.parts = (unsigned long long *)(ws + kStatusBytes);
     a.ring = (float *)(ws + kStatusBytes + parts_bytes(c));

@@ -1,0 +1,729 @@
+// A chain of steps with ONE inner iteration each, h = LayerNorm(step(h)) `outer` times, by whole K-rows:
+// one kernel per step and direction, for the plain update and for the gated one.
+//
+// With one inner iteration a step is a 27-tap stencil over the whole grid (see fwd_rows.hip) and a few
+// operations per byte: what a step costs is the tensors it moves, and beside that the launches and
+// small kernels between the steps.  What this file does about them:
+//   * The forward of a chain that is to be differentiated keeps what the backward would recompute from
+//     27 taps (plain: the pre-activation u; gated: d/d(pre), d/d(gate pre-activation) and the gate, each
+//     per unit of gradient).  With it the deltas of a cell are a few operations on values of that cell
+//     alone, so a workgroup forms them for its tube of 4 x 4 rows AND the rows around it, and the
+//     backward of a step is one kernel: no delta tensor between two kernels, no partial dx written and
+//     read back, one stencil instead of two (5 passes over activations against 8).
+//   * The weight gradients come from the same stencil over delta: x[c] delta[c + off_t] is the gradient
+//     of the neighbour's weight 26 - t, and no other cell contributes to it.
+//   * Where the batch is split over workgroups every chunk keeps ONE copy of the gradient arrays for the
+//     whole chain, each step adding to what the step before left; the copies are added up once.
+// (The pairs per wave behind the LayerNorms' per-sample numbers are merged by small kernels between the
+// steps, 4.7 us each.  Merged by the workgroups that need them, one wave an element ahead, they cost
+// the kernels 11 us forward and 24 us backward: everybody waits for that wave at the barrier.)
+// 32^3, batch 256, silu, per step: forward 27.5 + 4.6 us (the merging kernel), backward 58 + 29 us
+// with fwd_rows, bwd_rows and cross_rows.
+
+#include "common.h"
+#include "fast_tiles.h"
+#include "launch.h"
+#include "plan.h"
+
+namespace gridnet {
+
+namespace {
+
+constexpr int kTube = 4, kSide = kTube + 2, kWinRows = kSide * kSide;
+
+// sigmoid and activation of the gated update, as gated_fast.hip
+template <int ACT> __device__ __forceinline__ void gate_parts(float pre, float gp, float &a, float &d, float &gate) {
+    gate = sigmoid_stable(gp);
+    Act<ACT, float>::fd(pre, a, d);
+}
+
+// What both kernels know about a thread's place: its row of the tube, its CPT cells of it.
+template <int CPT> struct RowPlace {
+    int kl, r, ci, cj, bk, p0, q0, grow;
+    bool first, last;
+    __device__ __forceinline__ RowPlace(int tid, int tube, int N, int K) {
+        kl = K / CPT;
+        r = tid / kl;
+        bk = tid % kl;
+        ci = r / kTube;
+        cj = r % kTube;
+        const int nbj = N / kTube;
+        p0 = tube / nbj * kTube;
+        q0 = tube % nbj * kTube;
+        grow = ((p0 + ci) * N + q0 + cj) * K + CPT * bk;
+        first = bk == 0;
+        last = bk == kl - 1;
+    }
+};
+
+// CPT floats at a byte offset of this lane behind a pointer that is the same for the whole wave: an
+// addressing mode; an element index per lane is widened, scaled and added in vector registers.
+template <int CPT> __device__ __forceinline__ void load_at(const float *base, unsigned bytes, float (&v)[CPT]) {
+    load_cells<CPT>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + bytes), v);
+}
+template <int CPT> __device__ __forceinline__ void store_at(float *base, unsigned bytes, const float (&v)[CPT]) {
+    store_cells<CPT>(reinterpret_cast<float *>(reinterpret_cast<char *>(base) + bytes), v);
+}
+// a pair of per-sample numbers, as load_ahead
+__device__ __forceinline__ float2 load_pair_ahead(const float *pairs, int sample) {
+    unsigned zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    return *reinterpret_cast<const float2 *>(reinterpret_cast<const char *>(pairs + 2L * sample) + zero);
+}
+
+struct RowsFwdArgs {
+    const float *weight, *bias, *scale, *gamma, *beta, *x;
+    const float *x_stats;   // the LayerNorm in front of the step (null: x is used as it is)
+    float *y, *y_part;
+    float *saved;           // plain: [B,cells]; gated: [3][B,cells]; or null
+    int B, M, N, K, ntube, nchunk, chunk_len;
+};
+
+// PLAIN: four cells and 108 weights per thread; GATED: two cells and 2 x 54.  Everything else as
+// fwd_rows.hip: six by six rows in LDS, two stages, one barrier per batch element.
+template <int ACT, int SETS, bool SAVE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(SETS == 1 ? 3 : 2, 3)))
+void rows_fwd(RowsFwdArgs a) {
+    constexpr int CPT = 4 / SETS, RPT = 3;
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][36][K], gamma rows, beta rows
+    int tube, chunk;
+    if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
+    const int tid = threadIdx.x, M = a.M, N = a.N, K = a.K, nw = blockDim.x / 64, wave = tid / 64;
+    const RowPlace<CPT> p(tid, tube, N, K);
+    const long cells = (long)M * N * K;
+    const bool ln_in = a.x_stats != nullptr;
+    const int s0 = chunk * a.chunk_len, s1 = min(a.B, s0 + a.chunk_len);
+
+    float w[SETS][9][3][CPT], bv[SETS][CPT], rv[CPT];
+#pragma unroll
+    for (int pq = 0; pq < 9; ++pq)
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+            for (int k = 0; k < SETS; ++k) {
+                load_cells<CPT>(a.weight + ((pq * 3 + cc) * SETS + k) * cells + p.grow, w[k][pq][cc]);
+            }
+#pragma unroll
+    for (int k = 0; k < SETS; ++k) load_cells<CPT>(a.bias + k * cells + p.grow, bv[k]);
+    if (SETS == 1) load_cells<CPT>(a.scale + p.grow, rv);
+    const float keep_first = p.first ? 0.f : 1.f, keep_last = p.last ? 0.f : 1.f;
+#pragma unroll
+    for (int k = 0; k < SETS; ++k)
+#pragma unroll
+        for (int pq = 0; pq < 9; ++pq) {
+            w[k][pq][0][0] *= keep_first;
+            w[k][pq][2][CPT - 1] *= keep_last;
+        }
+
+    int goff[RPT], loff[RPT];
+    bool ok[RPT];
+    float *gam_rows = lds + 2 * kWinRows * K, *bet_rows = gam_rows + kWinRows * K;
+#pragma unroll
+    for (int e = 0; e < RPT; ++e) {
+        const int row = p.r + 16 * e, wi = row / kSide, wj = row % kSide;
+        const int gi = p.p0 + wi - 1, gj = p.q0 + wj - 1;
+        ok[e] = row < kWinRows && gi >= 0 && gi < M && gj >= 0 && gj < N;
+        goff[e] = ok[e] ? (gi * N + gj) * K + CPT * p.bk : p.grow;  // anything valid when not used
+        loff[e] = row * K + CPT * p.bk;
+        if (ln_in && row < kWinRows) {  // zeros outside the grid: no test per element then
+            float gq[CPT], bq[CPT];
+            load_cells<CPT>(a.gamma + goff[e], gq);
+            load_cells<CPT>(a.beta + goff[e], bq);
+#pragma unroll
+            for (int q = 0; q < CPT; ++q) {
+                gq[q] = ok[e] ? gq[q] : 0.f;
+                bq[q] = ok[e] ? bq[q] : 0.f;
+            }
+            store_cells<CPT>(gam_rows + loff[e], gq);
+            store_cells<CPT>(bet_rows + loff[e], bq);
+        }
+    }
+    const bool has_last = p.r + 16 * (RPT - 1) < kWinRows;
+    const int own_row = (p.ci + 1) * kSide + p.cj + 1;
+    wait_global_loads();
+
+    float xbuf[RPT][CPT];
+    float2 next_stat = make_float2(0.f, 1.f);
+    auto fetch = [&](int s) {
+        const float *x = a.x + (long)s * cells;
+        if (ln_in) next_stat = load_pair_ahead(a.x_stats, s);
+#pragma unroll
+        for (int e = 0; e < RPT; ++e) load_at<CPT>(x, 4u * (unsigned)goff[e], xbuf[e]);
+    };
+    if (s0 < s1) fetch(s0);
+    for (int s = s0; s < s1; ++s) {
+        float *stage = lds + ((s - s0) & 1) * kWinRows * K;
+        const float xmean = next_stat.x, xrstd = next_stat.y;
+#pragma unroll
+        for (int e = 0; e < RPT; ++e) {
+            if (e == RPT - 1 && !has_last) break;
+            float v[CPT];
+            if (ln_in) {
+                float gq[CPT], bq[CPT];
+                load_cells<CPT>(gam_rows + loff[e], gq);
+                load_cells<CPT>(bet_rows + loff[e], bq);
+#pragma unroll
+                for (int q = 0; q < CPT; ++q) v[q] = fmaf((xbuf[e][q] - xmean) * xrstd, gq[q], bq[q]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < CPT; ++q) v[q] = ok[e] ? xbuf[e][q] : 0.f;
+            }
+            store_cells<CPT>(stage + loff[e], v);
+        }
+        lds_barrier();  // the stage is complete; the other one's readers are done
+        fetch(min(s + 1, s1 - 1));
+        __builtin_amdgcn_sched_barrier(0);  // the requests leave now, with the whole stencil in front of their use
+        float u[SETS][CPT], own[CPT];
+#pragma unroll
+        for (int k = 0; k < SETS; ++k)
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) u[k][c] = bv[k][c];
+#pragma unroll
+        for (int pq = 0; pq < 9; ++pq) {
+            const int di = pq / 3 - 1, dj = pq % 3 - 1;
+            float d[CPT + 2], mid[CPT];
+            load_cells<CPT>(stage + (own_row + di * kSide + dj) * K + CPT * p.bk, mid);
+            d[0] = lane_before(mid[CPT - 1]);
+            d[CPT + 1] = lane_after(mid[0]);
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) d[c + 1] = mid[c];
+            if (pq == 4) {
+#pragma unroll
+                for (int c = 0; c < CPT; ++c) own[c] = mid[c];
+            }
+#pragma unroll
+            for (int k = 0; k < SETS; ++k)
+#pragma unroll
+                for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+                    for (int c = 0; c < CPT; ++c) u[k][c] = fmaf(w[k][pq][cc][c], d[c + cc], u[k][c]);
+        }
+        const long at = (long)s * cells;
+        const unsigned o = 4u * (unsigned)p.grow;
+        float out[CPT];
+        if (SETS == 1) {
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) out[c] = fmaf(rv[c], Act<ACT, float>::f(u[0][c]), own[c]);
+            if (SAVE) store_at<CPT>(a.saved + at, o, u[0]);
+        } else {
+            float f0[CPT], f1[CPT], gate[CPT];
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) {
+                float act, d;
+                gate_parts<ACT>(u[0][c], u[SETS - 1][c], act, d, gate[c]);
+                out[c] = fmaf(gate[c], own[c] - act, act);
+                f0[c] = (1.f - gate[c]) * d;
+                f1[c] = (own[c] - act) * gate[c] * (1.f - gate[c]);
+            }
+            if (SAVE) {
+                store_at<CPT>(a.saved + at, o, f0);
+                store_at<CPT>(a.saved + (long)a.B * cells + at, o, f1);
+                store_at<CPT>(a.saved + 2L * a.B * cells + at, o, gate);
+            }
+        }
+        store_at<CPT>(a.y + at, o, out);
+        // one (mean, M2) pair per wave
+        float sum = out[0];
+#pragma unroll
+        for (int c = 1; c < CPT; ++c) sum += out[c];
+        if (CPT == 4) sum = (out[0] + out[1]) + (out[CPT - 2] + out[CPT - 1]);  // in fwd_rows' order
+        const float mean = row16_sum(sum) * (1.f / (16 * CPT));
+        float m2 = 0.f;
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) m2 = fmaf(out[c] - mean, out[c] - mean, m2);
+        m2 = row16_sum(m2);
+        float wave_mean, wave_m2;
+        slot_wave_moments<64>(mean, m2, 16 * CPT, wave_mean, wave_m2);
+        if ((tid & 63) == 0) {
+            float *to = a.y_part + (((long)s * a.ntube + tube) * nw + wave) * 2;
+            to[0] = wave_mean;
+            to[1] = wave_m2;
+        }
+    }
+}
+
+struct RowsBwdArgs {
+    const float *weight, *scale, *gamma, *beta;
+    const float *dy;                // gradient with respect to LayerNorm(y)
+    const float *y, *y_stats;
+    const float *y_sums;            // the LayerNorm backward's two sums per sample
+    const float *saved;
+    const float *x, *x_stats;       // the step's input: raw, and the statistics of the LayerNorm on it (null: as it is)
+    float *dx, *x_part;             // x_part: pairs for the LayerNorm on x, or null
+    float *dweight, *dbias, *dscale, *dgamma, *dbeta;
+    long slab_stride;               // a copy of the gradient arrays per batch chunk (0: the arrays themselves)
+    int accumulate;                 // on top of what the gradient arrays hold
+    int B, M, N, K, ntube, nchunk, chunk_len;
+};
+
+// PLAIN: two cells per thread, GATED: one; 54 mirrored weights and 54 gradient accumulators for each set
+// and two cells.  A thread moves its own row and one or two of the 20 rows around the tube.
+template <int ACT, int SETS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_bwd(RowsBwdArgs a) {
+    constexpr int CPT = 2 / SETS;
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K]
+    int tube, chunk;
+    if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
+    const int tid = threadIdx.x, M = a.M, N = a.N, K = a.K, nw = blockDim.x / 64, wave = tid / 64;
+    const RowPlace<CPT> p(tid, tube, N, K);
+    const long cells = (long)M * N * K, tensor = (long)a.B * cells;
+    const bool ln_in = a.x_stats != nullptr;
+    const int s0 = chunk * a.chunk_len, s1 = min(a.B, s0 + a.chunk_len);
+    const long slab = chunk * a.slab_stride;
+    float *dweight = a.dweight + slab;
+
+    // ---- mirrored weights W[26 - t, c + off_t] and the gradients of those weights ----
+    // A tap's weights for the thread's cells lie along K, one cell off its own for dk = -1 / +1: aligned
+    // pieces, the missing end from the lane next door (cross_rows.hip).
+    float v[SETS][9][3][CPT], nv[SETS][9][3][CPT];
+    auto shift_in = [&](float (&piece)[CPT], int cc) {
+        if (cc == 0) {
+            const float before = lane_before(piece[CPT - 1]);
+            if (CPT == 2) piece[CPT - 1] = piece[0];
+            piece[0] = before;
+        } else if (cc == 2) {
+            const float after = lane_after(piece[0]);
+            if (CPT == 2) piece[0] = piece[CPT - 1];
+            piece[CPT - 1] = after;
+        }
+    };
+    // all requests first (in one stretch: behind a test per tap each would wait for the one before)
+    auto load_planes = [&](const float *planes, float (&to)[SETS][9][3][CPT]) {
+#pragma unroll
+        for (int pq = 0; pq < 9; ++pq) {
+            const int gi = p.p0 + p.ci + pq / 3 - 1, gj = p.q0 + p.cj + pq % 3 - 1;
+            const bool row_ok = gi >= 0 && gi < M && gj >= 0 && gj < N;
+            const unsigned base = 4u * (unsigned)(p.grow + (row_ok ? ((pq / 3 - 1) * N + pq % 3 - 1) * K : 0));
+#pragma unroll
+            for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+                for (int k = 0; k < SETS; ++k)
+                    load_at<CPT>(planes + ((26 - (pq * 3 + cc)) * SETS + k) * cells, base, to[k][pq][cc]);
+        }
+    };
+    load_planes(a.weight, v);
+    if (a.accumulate) {
+        load_planes(dweight, nv);
+    } else {
+#pragma unroll
+        for (int k = 0; k < SETS; ++k)
+#pragma unroll
+            for (int t = 0; t < 27; ++t)
+#pragma unroll
+                for (int c = 0; c < CPT; ++c) nv[k][t / 3][t % 3][c] = 0.f;
+    }
+    float gam[CPT], bet[CPT], rv[CPT] = {}, db[SETS][CPT], dr[CPT] = {}, dgam[CPT], dbet[CPT];
+    load_cells<CPT>(a.gamma + p.grow, gam);
+    load_cells<CPT>(a.beta + p.grow, bet);
+    if (SETS == 1) load_cells<CPT>(a.scale + p.grow, rv);
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+        dgam[c] = dbet[c] = 0.f;
+#pragma unroll
+        for (int k = 0; k < SETS; ++k) db[k][c] = 0.f;
+    }
+    if (a.accumulate) {
+#pragma unroll
+        for (int k = 0; k < SETS; ++k) load_cells<CPT>(a.dbias + slab + k * cells + p.grow, db[k]);
+        if (SETS == 1) load_cells<CPT>(a.dscale + slab + p.grow, dr);
+        load_cells<CPT>(a.dgamma + slab + p.grow, dgam);
+        load_cells<CPT>(a.dbeta + slab + p.grow, dbet);
+    }
+
+    // ---- the rows around the tube that this thread moves: number r and, the first four rows, 16 + r ----
+    int hoff[2], hat[2];
+    bool hok[2];
+    float hgam[2][CPT], hrv[2][CPT] = {};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const int h = min(p.r + 16 * e, 19);
+        const int wi = h < 12 ? h / 6 * (kSide - 1) : 1 + (h - 12) / 2, wj = h < 12 ? h % 6 : (h - 12) % 2 * (kSide - 1);
+        const int gi = p.p0 + wi - 1, gj = p.q0 + wj - 1;
+        hok[e] = gi >= 0 && gi < M && gj >= 0 && gj < N;
+        hoff[e] = hok[e] ? (gi * N + gj) * K + CPT * p.bk : p.grow;  // anything valid when not used
+        hat[e] = (wi * kSide + wj) * K + CPT * p.bk;
+        load_cells<CPT>(a.gamma + hoff[e], hgam[e]);
+        if (SETS == 1) load_cells<CPT>(a.scale + hoff[e], hrv[e]);
+    }
+    const bool second = p.r < 4;  // whole waves or parts of them
+    const int own_row = (p.ci + 1) * kSide + p.cj + 1, own_at = own_row * K + CPT * p.bk;
+    wait_global_loads();
+#pragma unroll
+    for (int pq = 0; pq < 9; ++pq) {
+        const int gi = p.p0 + p.ci + pq / 3 - 1, gj = p.q0 + p.cj + pq % 3 - 1;
+        const float keep = gi >= 0 && gi < M && gj >= 0 && gj < N ? 1.f : 0.f;
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+            for (int k = 0; k < SETS; ++k) {
+                shift_in(v[k][pq][cc], cc);
+                shift_in(nv[k][pq][cc], cc);
+#pragma unroll
+                for (int c = 0; c < CPT; ++c) v[k][pq][cc][c] *= keep;
+                if (cc == 0 && p.first) v[k][pq][cc][0] = 0.f;
+                if (cc == 2 && p.last) v[k][pq][cc][CPT - 1] = 0.f;
+            }
+    }
+
+    // what an element needs, requested one element ahead: dy, y and the saved factors of the cell (plain:
+    // u; gated: f0, f1, and of the own cells the gate)
+    constexpr int NF = SETS;
+    float bdy[3][CPT], by[3][CPT], bf[3][NF][CPT], bgate[CPT] = {}, bx[CPT];
+    float2 next_y, next_sums, next_x;
+    const unsigned own_off = 4u * (unsigned)p.grow;
+    const unsigned off[3] = {own_off, 4u * (unsigned)hoff[0], 4u * (unsigned)hoff[1]};
+    const float *x_stats = ln_in ? a.x_stats : a.y_stats;  // loaded in any case: no branch among the requests
+    auto fetch = [&](int s) {
+        const long at = (long)s * cells;
+        next_y = load_pair_ahead(a.y_stats, s);
+        next_sums = load_pair_ahead(a.y_sums, s);
+        next_x = load_pair_ahead(x_stats, s);
+        load_at<CPT>(a.x + at, own_off, bx);
+        if (SETS == 2) load_at<CPT>(a.saved + 2 * tensor + at, own_off, bgate);
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            load_at<CPT>(a.dy + at, off[e], bdy[e]);
+            load_at<CPT>(a.y + at, off[e], by[e]);
+#pragma unroll
+            for (int k = 0; k < NF; ++k) load_at<CPT>(a.saved + k * tensor + at, off[e], bf[e][k]);
+        }
+    };
+    float out[CPT];
+    if (s0 < s1) fetch(s0);
+    for (int s = s0; s < s1; ++s) {
+        float *stage = lds + ((s - s0) & 1) * SETS * kWinRows * K;
+        const float ymean = next_y.x, yrstd = next_y.y, c1 = next_sums.x, c2 = next_sums.y;
+        // through the LayerNorm's backward: the gradient with respect to the step's raw output
+        auto raw_gradient = [&](float dy, float y, float gamma, float &yh) {
+            yh = (y - ymean) * yrstd;
+            return yrstd * (gamma * dy - c1 - yh * c2);
+        };
+        float direct[CPT], xh[CPT], xn[CPT];
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) {
+            xn[c] = (bx[c] - next_x.x) * next_x.y;
+            xh[c] = ln_in ? fmaf(xn[c], gam[c], bet[c]) : bx[c];
+        }
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            if (e == 2 && !second) break;
+            float delta[SETS][CPT];
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) {
+                float yh;
+                const float g = raw_gradient(bdy[e][c], by[e][c], e == 0 ? gam[c] : hgam[e - 1 < 0 ? 0 : e - 1][c], yh);
+                const bool in_grid = e == 0 || hok[e - 1 < 0 ? 0 : e - 1];
+                if (SETS == 1) {
+                    float f, d;
+                    Act<ACT, float>::fd(bf[e][0][c], f, d);
+                    delta[0][c] = in_grid ? d * g * (e == 0 ? rv[c] : hrv[e - 1 < 0 ? 0 : e - 1][c]) : 0.f;
+                    if (e == 0) dr[c] = fmaf(f, g, dr[c]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < SETS; ++k) delta[k][c] = in_grid ? g * bf[e][k][c] : 0.f;
+                }
+                if (e == 0) {
+                    direct[c] = SETS == 1 ? g : bgate[c] * g;
+                    dgam[c] = fmaf(bdy[e][c], yh, dgam[c]);
+                    dbet[c] += bdy[e][c];
+#pragma unroll
+                    for (int k = 0; k < SETS; ++k) db[k][c] += delta[k][c];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < SETS; ++k)
+                store_cells<CPT>(stage + k * kWinRows * K + (e == 0 ? own_at : hat[e - 1 < 0 ? 0 : e - 1]), delta[k]);
+        }
+        // worked out in front of the requests that replace what they come from (behind them, the compiler
+        // has to wait for the first of those)
+        keep_here(xn);
+        keep_here(xh);
+        keep_here(direct);
+        lds_barrier();  // the stage is complete; the other one's readers are done
+        // The result of the element before leaves here, ahead of the requests: the memory counter is in
+        // order, and a store behind them would be waited for with the last of them.
+        if (s > s0) store_at<CPT>(a.dx + (long)(s - 1) * cells, own_off, out);
+        fetch(min(s + 1, s1 - 1));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) out[c] = direct[c];
+#pragma unroll
+        for (int k = 0; k < SETS; ++k)
+#pragma unroll
+            for (int pq = 0; pq < 9; ++pq) {
+                const int di = pq / 3 - 1, dj = pq % 3 - 1;
+                float d[CPT + 2], mid[CPT];
+                load_cells<CPT>(stage + k * kWinRows * K + own_at + (di * kSide + dj) * K, mid);
+                d[0] = lane_before(mid[CPT - 1]);
+                d[CPT + 1] = lane_after(mid[0]);
+#pragma unroll
+                for (int c = 0; c < CPT; ++c) d[c + 1] = mid[c];
+#pragma unroll
+                for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+                    for (int c = 0; c < CPT; ++c) {
+                        out[c] = fmaf(v[k][pq][cc][c], d[c + cc], out[c]);
+                        nv[k][pq][cc][c] = fmaf(xh[c], d[c + cc], nv[k][pq][cc][c]);
+                    }
+            }
+        if (a.x_part) {  // the sums of the LayerNorm on x, one pair per wave
+            float t1 = 0.f, t2 = 0.f;
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) {
+                const float go = gam[c] * out[c];
+                t1 += go;
+                t2 = fmaf(go, xn[c], t2);
+            }
+            t1 = slot_wave_sum<64>(t1);
+            t2 = slot_wave_sum<64>(t2);
+            if ((tid & 63) == 0) {
+                float *to = a.x_part + (((long)s * a.ntube + tube) * nw + wave) * 2;
+                to[0] = t1;
+                to[1] = t2;
+            }
+        }
+    }
+
+    if (s0 < s1) store_at<CPT>(a.dx + (long)(s1 - 1) * cells, own_off, out);
+
+    // ---- parameter gradients: the shifts of the set-up back again, aligned stores of whole rows ----
+#pragma unroll
+    for (int pq = 0; pq < 9; ++pq) {
+        const int gi = p.p0 + p.ci + pq / 3 - 1, gj = p.q0 + p.cj + pq % 3 - 1;
+        const bool row_ok = gi >= 0 && gi < M && gj >= 0 && gj < N;
+        const int base = (gi * N + gj) * K + CPT * p.bk;
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+            for (int k = 0; k < SETS; ++k) {
+                const float (&n)[CPT] = nv[k][pq][cc];
+                float piece[CPT];
+                if (cc == 1) {
+#pragma unroll
+                    for (int c = 0; c < CPT; ++c) piece[c] = n[c];
+                } else if (cc == 0) {  // from the cell after; behind the row's last cell there is none
+                    const float after = lane_after(n[0]);
+                    if (CPT == 2) piece[0] = n[CPT - 1];
+                    piece[CPT - 1] = p.last ? 0.f : after;
+                } else {
+                    const float before = lane_before(n[CPT - 1]);
+                    if (CPT == 2) piece[CPT - 1] = n[0];
+                    piece[0] = p.first ? 0.f : before;
+                }
+                const int t = pq * 3 + cc;
+                float *to = dweight + (long)((26 - t) * SETS + k) * cells + base;
+                if (row_ok && a.accumulate && ((cc == 0 && p.last) || (cc == 2 && p.first))) {
+                    // the weight that reads outside the grid keeps what its gradient holds
+                    if (CPT == 2) to[cc == 0 ? 0 : CPT - 1] = piece[cc == 0 ? 0 : CPT - 1];
+                } else if (row_ok) {
+                    store_cells<CPT>(to, piece);
+                } else if (!a.accumulate) {  // the own weight of tap t reads outside the grid: no gradient
+#pragma unroll
+                    for (int c = 0; c < CPT; ++c) piece[c] = 0.f;
+                    store_cells<CPT>(dweight + (long)(t * SETS + k) * cells + p.grow, piece);
+                }
+            }
+    }
+#pragma unroll
+    for (int k = 0; k < SETS; ++k) store_cells<CPT>(a.dbias + slab + k * cells + p.grow, db[k]);
+    if (SETS == 1) store_cells<CPT>(a.dscale + slab + p.grow, dr);
+    store_cells<CPT>(a.dgamma + slab + p.grow, dgam);
+    store_cells<CPT>(a.dbeta + slab + p.grow, dbet);
+}
+
+// ---- host side -------------------------------------------------------------------------------
+int sets_of(const RowsChain &c) { return c.gated ? 2 : 1; }
+long cells_of(const RowsChain &c) { return (long)c.M * c.N * c.K; }
+int tubes_of(const RowsChain &c) { return c.M / kTube * (c.N / kTube); }
+int fwd_threads(const RowsChain &c) { return 16 * c.K * sets_of(c) / 4; }
+int bwd_threads(const RowsChain &c) { return 16 * c.K * sets_of(c) / 2; }
+int fwd_pairs(const RowsChain &c) { return tubes_of(c) * fwd_threads(c) / 64; }
+int bwd_pairs(const RowsChain &c) { return tubes_of(c) * bwd_threads(c) / 64; }
+size_t align_up(size_t v) { return (v + 255) / 256 * 256; }
+size_t part_bytes(int B, int pairs) { return align_up((size_t)B * pairs * 2 * sizeof(float)); }
+
+template <typename K> int workgroups_per_cu(K kern, int threads, size_t lds) {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)kern, threads, lds) != hipSuccess || n < 1) n = 1;
+    return n;
+}
+template <typename K> int allow_lds(K kern, size_t lds) {
+    if (lds > 64 * 1024 &&
+        hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(GRIDNET_ERR_LAUNCH, "chain_rows: cannot enable %zu bytes of LDS", lds);
+    }
+    return GRIDNET_OK;
+}
+
+template <int ACT, int SETS, bool SAVE> int run_forward(const RowsChain &c, hipStream_t st) {
+    auto kern = rows_fwd<ACT, SETS, SAVE>;
+    const long cells = cells_of(c), tensor = (long)c.B * cells;
+    const int ntube = tubes_of(c), nt = fwd_threads(c), pairs = fwd_pairs(c);
+    const size_t lds = 4 * (size_t)kWinRows * c.K * sizeof(float);
+    static int per_cu_cache[128 / 4 + 1];  // per instantiation, by K
+    int &per_cu = per_cu_cache[c.K / 4];
+    if (per_cu == 0) {
+        if (int rc = allow_lds(kern, lds)) return rc;
+        per_cu = workgroups_per_cu(kern, nt, lds);
+    }
+    RowsFwdArgs a{};
+    a.nchunk = plan_row_chunks(c.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, a.chunk_len);
+    a.weight = c.weight; a.bias = c.bias; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
+    a.B = c.B; a.M = c.M; a.N = c.N; a.K = c.K; a.ntube = ntube;
+    // workspace: the pairs; and, where nothing is kept, statistics and two raw tensors
+    char *ws = (char *)c.workspace;
+    a.y_part = (float *)ws;
+    ws += part_bytes(c.B, pairs);
+    float *own_stats = (float *)ws, *own_y = (float *)(ws + align_up((size_t)2 * c.B * sizeof(float)));
+    for (int j = 0; j < c.outer; ++j) {
+        float *stats = c.stats ? c.stats + (long)j * 2 * c.B : own_stats;
+        a.x = j ? a.y : c.x0;
+        a.y = c.y_raw ? c.y_raw + j * tensor : own_y + (j & 1) * tensor;
+        a.saved = SAVE ? c.saved + (long)j * (SETS == 1 ? 1 : 3) * tensor : nullptr;
+        hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, a.nchunk)), dim3(nt), lds, st, a);
+        if (int rc = check_launch("rows_fwd")) return rc;
+        if (int rc = layernorm_finalize_stats(a.y_part, pairs, (int)(cells / pairs), stats, c.B, c.eps, st)) return rc;
+        a.x_stats = stats;
+    }
+    return layernorm_apply_stats(a.y, a.x_stats, c.gamma, c.beta, c.out, c.B, cells, st);
+}
+
+// at least eight elements per copy of the gradient arrays, but where that leaves CUs without a
+// workgroup, down to three (as bwd_rows.hip)
+int bwd_chunks(const RowsChain &c, int per_cu, int &chunk_len) {
+    const int cus = plan_device_cus(), ntube = tubes_of(c);
+    const int n = plan_row_chunks(c.B, ntube, per_cu * cus, 8, chunk_len);
+    return n * ntube >= cus ? n : plan_row_chunks(c.B, ntube, cus, kRowsMinWalk, chunk_len);
+}
+constexpr int kBwdMostPerCu = 4;
+int grad_planes(const RowsChain &c) { return c.gated ? 58 : 31; }
+
+template <int ACT, int SETS> int run_backward(const RowsChain &c, hipStream_t st) {
+    auto kern = rows_bwd<ACT, SETS>;
+    const long cells = cells_of(c), tensor = (long)c.B * cells;
+    const int ntube = tubes_of(c), nt = bwd_threads(c), pairs = bwd_pairs(c);
+    const size_t lds = 2 * (size_t)SETS * kWinRows * c.K * sizeof(float);
+    static int per_cu_cache[64 / 4 + 1];  // per instantiation, by K
+    int &per_cu = per_cu_cache[c.K / 4];
+    if (per_cu == 0) {
+        const int n = workgroups_per_cu(kern, nt, lds);
+        per_cu = n < kBwdMostPerCu ? n : kBwdMostPerCu;
+    }
+    RowsBwdArgs a{};
+    a.nchunk = bwd_chunks(c, per_cu, a.chunk_len);
+    a.weight = c.weight; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
+    a.B = c.B; a.M = c.M; a.N = c.N; a.K = c.K; a.ntube = ntube;
+    // workspace: the pairs, the sums, scratch of the last LayerNorm's sums, a second dx, the copies
+    char *ws = (char *)c.workspace;
+    float *part = (float *)ws;
+    ws += part_bytes(c.B, pairs);
+    float *sums = (float *)ws;
+    ws += align_up((size_t)2 * c.B * sizeof(float));
+    float *scratch = (float *)ws;
+    ws += align_up(layernorm_workspace(GRIDNET_F32, c.B, cells));
+    float *other_dx = (float *)ws;
+    ws += align_up((size_t)tensor * sizeof(float));
+    float *slabs = (float *)ws;
+    const int wplanes = 27 * SETS;
+    const long slab_floats = grad_planes(c) * cells;
+    const bool split = a.nchunk > 1, add = (c.flags & GRIDNET_OVERWRITE_PARAMS) == 0;
+    SlabTargets t{};
+    int k = 0;
+    auto target = [&](float *dst, long planes) {
+        t.dst[k] = dst;
+        t.end[k] = (k ? t.end[k - 1] : 0) + planes * cells;
+        ++k;
+    };
+    target(c.dweight, wplanes);
+    target(c.dbias, SETS);
+    if (SETS == 1) target(c.dscale, 1);
+    target(c.dgamma, 1);
+    target(c.dbeta, 1);
+    t.count = k;
+    if (split) {
+        a.dweight = slabs;
+        a.dbias = a.dweight + wplanes * cells;
+        a.dscale = SETS == 1 ? a.dbias + cells : nullptr;
+        a.dgamma = a.dbias + 2 * cells;  // plain: behind the scale; gated: behind the second bias
+        a.dbeta = a.dgamma + cells;
+        a.slab_stride = slab_floats;
+    } else {
+        a.dweight = c.dweight; a.dbias = c.dbias; a.dscale = c.dscale; a.dgamma = c.dgamma; a.dbeta = c.dbeta;
+    }
+    const long last = c.outer - 1;
+    if (int rc = layernorm_backward_sums(c.dy, c.y_raw + last * tensor, c.stats + last * 2 * c.B, c.gamma, sums, c.B, cells,
+                                         scratch, st))
+        return rc;
+    a.dy = c.dy;
+    a.y_sums = sums;
+    for (long j = last; j >= 0; --j) {
+        a.y = c.y_raw + j * tensor;
+        a.y_stats = c.stats + j * 2 * c.B;
+        a.saved = c.saved + j * (SETS == 1 ? 1 : 3) * tensor;
+        a.x = j ? c.y_raw + (j - 1) * tensor : c.x0;
+        a.x_stats = j ? c.stats + (j - 1) * 2 * c.B : nullptr;
+        a.x_part = j ? part : nullptr;
+        a.dx = j & 1 ? other_dx : c.dx;
+        a.accumulate = j < last || (!split && add);
+        hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, a.nchunk)), dim3(nt), lds, st, a);
+        if (int rc = check_launch("rows_bwd")) return rc;
+        a.dy = a.dx;
+        if (j)
+            if (int rc = layernorm_finalize_sums(part, pairs, cells, sums, c.B, st)) return rc;
+    }
+    if (!split) return GRIDNET_OK;
+    return plan_launch_tail_job(plan_tail_job(slabs, a.nchunk, slab_floats, t, add ? 1 : 0, 256), st);
+}
+
+template <int SETS, bool SAVE> int forward_act(const RowsChain &c, hipStream_t st) {
+    switch (c.activation) {
+        case GRIDNET_ACT_RELU: return run_forward<GRIDNET_ACT_RELU, SETS, SAVE>(c, st);
+        case GRIDNET_ACT_LEAKY_RELU: return run_forward<GRIDNET_ACT_LEAKY_RELU, SETS, SAVE>(c, st);
+        case GRIDNET_ACT_SILU: return run_forward<GRIDNET_ACT_SILU, SETS, SAVE>(c, st);
+        case GRIDNET_ACT_TANH: return run_forward<GRIDNET_ACT_TANH, SETS, SAVE>(c, st);
+    }
+    return fail(GRIDNET_ERR_ACTIVATION, "unknown activation function: id %d", c.activation);
+}
+template <int SETS> int backward_act(const RowsChain &c, hipStream_t st) {
+    switch (c.activation) {
+        case GRIDNET_ACT_RELU: return run_backward<GRIDNET_ACT_RELU, SETS>(c, st);
+        case GRIDNET_ACT_LEAKY_RELU: return run_backward<GRIDNET_ACT_LEAKY_RELU, SETS>(c, st);
+        case GRIDNET_ACT_SILU: return run_backward<GRIDNET_ACT_SILU, SETS>(c, st);
+        case GRIDNET_ACT_TANH: return run_backward<GRIDNET_ACT_TANH, SETS>(c, st);
+    }
+    return fail(GRIDNET_ERR_ACTIVATION, "unknown activation function: id %d", c.activation);
+}
+
+}  // namespace
+
+// Rows that are a power of two of lanes in both kernels; with two weight sets a row of 64 cells would
+// take a workgroup of 1024 threads, whose waves have half the registers this needs.
+bool rows_chain_supports(int M, int N, int K, bool gated) {
+    if (M <= 0 || N <= 0 || M % kTube || N % kTube || (long)M * N * K * 54 >= (1L << 31)) return false;
+    return K == 16 || K == 32 || (K == 64 && !gated);
+}
+
+size_t rows_chain_workspace(const RowsChain &c, bool backward) {
+    if (!backward) {
+        size_t n = part_bytes(c.B, fwd_pairs(c)) + align_up((size_t)2 * c.B * sizeof(float));
+        if (!c.keep) n += 2 * (size_t)c.B * cells_of(c) * sizeof(float);
+        return n;
+    }
+    int chunk_len;
+    const int chunks = bwd_chunks(c, kBwdMostPerCu, chunk_len);
+    return part_bytes(c.B, bwd_pairs(c)) + align_up((size_t)2 * c.B * sizeof(float)) +
+           align_up(layernorm_workspace(GRIDNET_F32, c.B, cells_of(c))) + align_up((size_t)c.B * cells_of(c) * sizeof(float)) +
+           (chunks > 1 ? (size_t)chunks * grad_planes(c) * cells_of(c) * sizeof(float) : 0);
+}
+
+int rows_chain_forward(const RowsChain &c, hipStream_t st) {
+    if (c.gated) return c.saved ? forward_act<2, true>(c, st) : forward_act<2, false>(c, st);
+    return c.saved ? forward_act<1, true>(c, st) : forward_act<1, false>(c, st);
+}
+
+int rows_chain_backward(const RowsChain &c, hipStream_t st) {
+    return c.gated ? backward_act<2>(c, st) : backward_act<1>(c, st);
+}
+
+}  // namespace gridnet

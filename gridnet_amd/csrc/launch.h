@@ -217,6 +217,7 @@ int chain_backward_all(const ChainAll &c, hipStream_t st);
 struct ChainFwd {
     const float *weight, *bias, *scale, *gamma, *beta, *x0;
     float *y_all, *stats;  // [outer,B,M,N,K] raw outputs and [outer,B,2] statistics for a backward, or null
+    float *saved;          // one inner iteration: [outer,B,M,N,K] pre-activations (see RowsChain), or null
     float *out;            // [B,M,N,K]
     int B, M, N, K, inner, outer, activation;
     double eps;
@@ -227,6 +228,24 @@ struct ChainFwd {
 bool chain_fwd_supports(int B, int M, int N, int K, int inner, int outer);
 size_t chain_fwd_workspace(const ChainFwd &c);
 int chain_forward_all(const ChainFwd &c, hipStream_t st);
+
+// chain_rows.hip: a chain of `outer` steps with one inner iteration each (one parameter set, the plain
+// loop), one kernel per step and direction by whole K-rows, plain or gated; fp32, normalize off.
+struct RowsChain {
+    const float *weight, *bias, *scale, *gamma, *beta, *x0;  // gated: no scale
+    float *y_raw, *stats, *saved;  // [outer,B,cells], [outer,B,2], [outer,B,cells] (gated: [outer,3,B,cells]), or all null
+    float *out;                    // forward: [B,cells]
+    const float *dy;               // backward
+    float *dweight, *dbias, *dscale, *dgamma, *dbeta, *dx;
+    int B, M, N, K, outer, activation, flags;
+    bool gated, keep;              // keep: y_raw, stats and saved are given
+    double eps;
+    void *workspace;
+};
+bool rows_chain_supports(int M, int N, int K, bool gated);
+size_t rows_chain_workspace(const RowsChain &c, bool backward);
+int rows_chain_forward(const RowsChain &c, hipStream_t st);
+int rows_chain_backward(const RowsChain &c, hipStream_t st);
 
 // step_fast.hip: the cross-block kernel on two weight sets, for gated_fast.hip
 int gated_cross_launch(const StepArgs &a, const float *dsum, int nchunk, int chunk_len, const TailJob &tail,

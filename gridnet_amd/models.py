@@ -21,7 +21,7 @@ import torch.nn as nn
 
 from . import GatedGridnet, Gridnet
 from .layernorm import GridLayerNorm
-from .network import fused_body
+from .network import fused_body, gated_body
 
 
 class Readout(nn.Module):
@@ -76,6 +76,8 @@ class MnistGridModel(nn.Module):
         h = self.embed(batch)
         if self.fused_body:
             return self.readout(fused_body(h, self.network, self.norm, self.outer_iters))
+        if isinstance(self.network, GatedGridnet):
+            return self.readout(gated_body(h, self.network, self.norm, self.outer_iters))
         for _ in range(self.outer_iters):
             h = self.norm(self.network(h))
         return self.readout(h)

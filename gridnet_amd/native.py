@@ -51,6 +51,13 @@ EXPORTS = (
     "gridnet_hip_chain_all_supported",
     "gridnet_hip_chain_all_workspace_bytes",
     "gridnet_hip_chain_backward_all",
+    "gridnet_hip_chain_forward_all_supported",
+    "gridnet_hip_chain_forward_all_workspace_bytes",
+    "gridnet_hip_chain_forward_all",
+    "gridnet_hip_rows_chain_supported",
+    "gridnet_hip_rows_chain_workspace_bytes",
+    "gridnet_hip_rows_chain_forward",
+    "gridnet_hip_rows_chain_backward",
     "gridnet_hip_chain_set_spin_limit",
 )
 
@@ -130,7 +137,15 @@ def _load():
     lib.gridnet_hip_chain_forward_all_workspace_bytes.restype = z
     lib.gridnet_hip_chain_forward_all_workspace_bytes.argtypes = [i] * 4
     lib.gridnet_hip_chain_forward_all.restype = i
-    lib.gridnet_hip_chain_forward_all.argtypes = [i] + [p] * 9 + [i] * 7 + [d, i, p, z, p]
+    lib.gridnet_hip_chain_forward_all.argtypes = [i] + [p] * 10 + [i] * 7 + [d, i, p, z, p]
+    lib.gridnet_hip_rows_chain_supported.restype = i
+    lib.gridnet_hip_rows_chain_supported.argtypes = [i] * 7
+    lib.gridnet_hip_rows_chain_workspace_bytes.restype = z
+    lib.gridnet_hip_rows_chain_workspace_bytes.argtypes = [i] * 7
+    lib.gridnet_hip_rows_chain_forward.restype = i
+    lib.gridnet_hip_rows_chain_forward.argtypes = [p] * 10 + [i] * 6 + [d, i, p, z, p]
+    lib.gridnet_hip_rows_chain_backward.restype = i
+    lib.gridnet_hip_rows_chain_backward.argtypes = [p] * 15 + [i] * 8 + [p, z, p]
     lib.gridnet_hip_chain_set_spin_limit.restype = i
     lib.gridnet_hip_chain_set_spin_limit.argtypes = [i]
     return lib

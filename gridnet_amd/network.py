@@ -86,6 +86,85 @@ def fused_body(h, network, norm, outer_iterations: int, outer_residual: bool = F
                              first.block_size, first.activation, outer_residual, *params)
 
 
+class GatedBodyOp(torch.autograd.Function):
+    """The loop over a gated step with one inner iteration and its LayerNorm as one autograd node, on
+    ``gridnet_hip_rows_chain_*``: a kernel per step and direction, the LayerNorm and the accumulation of
+    the shared parameters' gradients inside them."""
+
+    @staticmethod
+    def forward(ctx, x0, weight, bias, gamma, beta, outer_iterations, activation, eps):
+        from . import native as _n
+
+        x0 = x0.contiguous()
+        batch, (m, n, k) = x0.shape[0], x0.shape[1:]
+        keep = any(ctx.needs_input_grad)
+        act = _n.activation_id(activation)
+        out = torch.empty_like(x0)
+        y_raw = stats = saved = None
+        if keep:
+            y_raw = torch.empty((outer_iterations, *x0.shape), dtype=x0.dtype, device=x0.device)
+            saved = torch.empty((outer_iterations, 3, *x0.shape), dtype=x0.dtype, device=x0.device)
+            stats = torch.empty((outer_iterations, batch, 2), dtype=x0.dtype, device=x0.device)
+        with torch.cuda.device(x0.device):
+            nbytes = _n.lib.gridnet_hip_rows_chain_workspace_bytes(batch, m, n, k, 1, int(keep), 0)
+            ws = _n.workspace(nbytes, x0.device)
+            _n.check(_n.lib.gridnet_hip_rows_chain_forward(
+                weight.data_ptr(), bias.data_ptr(), None, gamma.data_ptr(), beta.data_ptr(), x0.data_ptr(),
+                *([t.data_ptr() for t in (y_raw, stats, saved)] if keep else [None] * 3), out.data_ptr(),
+                batch, m, n, k, outer_iterations, 1, float(eps), act, ws.data_ptr(), nbytes,
+                _n.current_stream(x0)))
+        if keep:
+            ctx.save_for_backward(x0, weight, bias, gamma, beta, y_raw, stats, saved)
+            ctx.outer_iterations, ctx.act = outer_iterations, act
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_out):
+        from . import native as _n
+
+        x0, weight, bias, gamma, beta, y_raw, stats, saved = ctx.saved_tensors
+        batch, (m, n, k) = x0.shape[0], x0.shape[1:]
+        dy = grad_out.contiguous()
+        grads = [torch.empty_like(t) for t in (x0, weight, bias, gamma, beta)]
+        dx, dw, db, dgamma, dbeta = (t.data_ptr() for t in grads)
+        with torch.cuda.device(x0.device):
+            nbytes = _n.lib.gridnet_hip_rows_chain_workspace_bytes(batch, m, n, k, 1, 1, 1)
+            ws = _n.workspace(nbytes, x0.device)
+            _n.check(_n.lib.gridnet_hip_rows_chain_backward(
+                weight.data_ptr(), None, gamma.data_ptr(), beta.data_ptr(), x0.data_ptr(), y_raw.data_ptr(),
+                stats.data_ptr(), saved.data_ptr(), dy.data_ptr(), dw, db, None, dgamma, dbeta, dx,
+                batch, m, n, k, ctx.outer_iterations, 1, ctx.act, _n.OVERWRITE_PARAMS, ws.data_ptr(), nbytes,
+                _n.current_stream(x0)))
+        return (*grads, None, None, None)
+
+
+def _bare(module):
+    """No hook would miss a call that goes round ``module.forward``."""
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
+                module._backward_pre_hooks)
+
+
+def gated_body(h, network, norm, outer_iterations: int):
+    """``outer_iterations`` x (``network``, ``norm``) on ``h``: a :class:`gridnet_amd.GatedGridnet` and a
+    :class:`gridnet_amd.GridLayerNorm`, through :class:`GatedBodyOp` where that covers the problem and one
+    after the other where it does not."""
+    from . import native as _n
+
+    params = (network.weight, network.bias, norm.weight, norm.bias)
+    shape = tuple(network.bias.shape[1:])
+    if (outer_iterations >= 1 and h.is_cuda and h.shape[0] > 0 and tuple(h.shape[1:]) == shape and
+            h.dtype == torch.float32 and _bare(network) and _bare(norm) and
+            network.block_size in (4, 8) and not any(n % network.block_size for n in shape) and
+            network.weight.shape == (27, 2, *shape) and norm.weight.shape == shape and norm.bias.shape == shape and
+            all(t.is_contiguous() and t.dtype == h.dtype and t.device == h.device for t in params) and
+            _n.lib.gridnet_hip_rows_chain_supported(_n.F32, *shape, network.inner_iterations, 0, 1)):
+        return GatedBodyOp.apply(h, *params, outer_iterations, network.activation, norm.eps)
+    for _ in range(outer_iterations):
+        h = norm(network(h))
+    return h
+
+
 class GridnetBody(nn.Module):
     def __init__(self, shape, inner_iterations: int, outer_iterations: int, block_size: int,
                  device, activation: str = "leaky_relu", normalize: bool = False,

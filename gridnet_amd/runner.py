@@ -31,6 +31,10 @@ Where blocks and batch are few enough to be resident at once (a 32^3 grid at up 
 forward of a chain with one parameter set is one launch too (``gridnet_hip_chain_forward_all``;
 ``forward_all=False``: never).
 
+With one inner iteration per step, one parameter set and rows of 16, 32 or 64 cells a chain takes one kernel per
+step and direction (``gridnet_hip_rows_chain_*``; ``rows=False``: never); its forward keeps the
+pre-activations as well, one more tensor per step.
+
 ``weight``, ``bias`` and ``scale`` may each be a list of ``outer`` tensors: one parameter set
 per outer step (the reference's ``--separate_params``, gridnet/scripts/train_imagenet.py:54-58).
 ``backward`` then returns lists of gradients for them, one entry per step.
@@ -50,7 +54,7 @@ class BodyRunner:
                  block_size: int, activation: str = "leaky_relu", normalize: bool = False,
                  eps: float = 1e-5, ln_eps: float = 1e-5, backward: bool = True,
                  fused: bool = False, outer_residual: bool = False, chain=None,
-                 chain_all=None, forward_all=None):
+                 chain_all=None, forward_all=None, rows=None):
         self.separate = isinstance(weight, (list, tuple))
         if self.separate:
             if not (len(weight) == len(bias) == len(scale) == outer):
@@ -82,10 +86,16 @@ class BodyRunner:
             fused and not outer_residual and not self.separate and forward_all is not False and
             _n.lib.gridnet_hip_chain_forward_all_supported(
                 self.dt, batch, self.M, self.N, self.K, inner, outer, block_size, self.normalize))
+        # chain or chain_all=True asks for the one backward or the other
+        self.rows = bool(
+            fused and not outer_residual and not self.separate and rows is not False and
+            not (backward and (chain or chain_all)) and
+            _n.lib.gridnet_hip_rows_chain_supported(self.dt, self.M, self.N, self.K, inner, self.normalize, 0))
         n_h, n_s = keep + 1, keep
         if fused and not outer_residual:
-            n_h = 1 if backward or self.forward_all else 2
-            n_s = 0 if self.forward_all and not backward else n_s
+            whole = self.forward_all or self.rows  # keep the values between the steps themselves
+            n_h = 1 if backward or whole else 2
+            n_s = 0 if whole and not backward else n_s
         if fused and outer_residual:
             n_s = 2 if backward else 1
         self.h = [torch.empty(shape, device=dev, dtype=dtype) for _ in range(n_h)]
@@ -123,6 +133,9 @@ class BodyRunner:
             if self.forward_all:
                 self.fw_ws_bytes = _n.lib.gridnet_hip_chain_forward_all_workspace_bytes(
                     batch, self.M, self.N, self.K)
+            elif self.rows:
+                self.fw_ws_bytes = _n.lib.gridnet_hip_rows_chain_workspace_bytes(
+                    batch, self.M, self.N, self.K, 0, int(backward), 0)
             else:
                 self.fw_ws_bytes = _n.lib.gridnet_hip_fused_workspace_bytes(
                     batch, self.M, self.N, self.K, inner, block_size, 0)
@@ -132,10 +145,15 @@ class BodyRunner:
                 self.unused = torch.empty(shape, device=dev, dtype=dtype)
             if backward:
                 self.sums = torch.empty(keep, batch, 2, device=dev, dtype=dtype)
-                self.fb_ws_bytes = _n.lib.gridnet_hip_fused_workspace_bytes(
-                    batch, self.M, self.N, self.K, inner, block_size, 1)
+                if self.rows:
+                    self.saved = torch.empty_like(self.s_all)
+                    self.fb_ws_bytes = _n.lib.gridnet_hip_rows_chain_workspace_bytes(
+                        batch, self.M, self.N, self.K, 0, 1, 1)
+                else:
+                    self.fb_ws_bytes = _n.lib.gridnet_hip_fused_workspace_bytes(
+                        batch, self.M, self.N, self.K, inner, block_size, 1)
                 self.fb_ws = _n.workspace(self.fb_ws_bytes, dev)
-        chain_ok = bool(chain is not False and fused and backward and not outer_residual and
+        chain_ok = bool(chain is not False and fused and backward and not outer_residual and not self.rows and
                         _n.lib.gridnet_hip_chain_supported(self.dt, inner, block_size, self.normalize))
         rows = self.K <= 128  # what the row-wise cross-block kernel takes
         self.chain = chain_ok and (chain is True or not rows)
@@ -206,8 +224,17 @@ class BodyRunner:
             _n.check(_n.lib.gridnet_hip_chain_forward_all(
                 self.dt, *self._params(0), self.gamma.data_ptr(), self.beta.data_ptr(), x0.data_ptr(),
                 self.s_all.data_ptr() if keep else None, self.stats.data_ptr() if keep else None,
-                self.h[0].data_ptr(), self.B, self.M, self.N, self.K, self.inner, self.outer, self.bs,
+                self.saved.data_ptr() if keep and self.rows else None, self.h[0].data_ptr(), self.B, self.M, self.N, self.K, self.inner, self.outer, self.bs,
                 self.ln_eps, self.act, self.fw_ws.data_ptr(), self.fw_ws_bytes, stream))
+            self._mark("step_fwd", 1)
+            return self.h[0]
+        if self.rows:
+            kept = [t.data_ptr() for t in (self.s_all, self.stats, self.saved)] if keep else [None] * 3
+            self._mark("step_fwd", 0)
+            _n.check(_n.lib.gridnet_hip_rows_chain_forward(
+                *self._params(0), self.gamma.data_ptr(), self.beta.data_ptr(), x0.data_ptr(), *kept,
+                self.h[0].data_ptr(), self.B, self.M, self.N, self.K, self.outer, 0, self.ln_eps, self.act,
+                self.fw_ws.data_ptr(), self.fw_ws_bytes, stream))
             self._mark("step_fwd", 1)
             return self.h[0]
         x, x_stats = x0, None
@@ -331,7 +358,21 @@ class BodyRunner:
         self._mark("step_bwd", 1)
         return (*self._param_grads(), self.dgamma, self.dbeta, self.ga)
 
+    def _rows_backward(self, grad_out):
+        stream = _n.current_stream(self.w)
+        w, _, r = self._params(0)
+        self._mark("step_bwd", 0)
+        _n.check(_n.lib.gridnet_hip_rows_chain_backward(
+            w, r, self.gamma.data_ptr(), self.beta.data_ptr(), self.x0.data_ptr(), self.s_all.data_ptr(),
+            self.stats.data_ptr(), self.saved.data_ptr(), grad_out.data_ptr(), *self._grads(0),
+            self.dgamma.data_ptr(), self.dbeta.data_ptr(), self.ga.data_ptr(), self.B, self.M, self.N, self.K,
+            self.outer, 0, self.act, _n.OVERWRITE_PARAMS, self.fb_ws.data_ptr(), self.fb_ws_bytes, stream))
+        self._mark("step_bwd", 1)
+        return (*self._param_grads(), self.dgamma, self.dbeta, self.ga)
+
     def _fused_backward(self, grad_out):
+        if self.rows:
+            return self._rows_backward(grad_out)
         if self.chain_all:
             return self._chain_all_backward(grad_out)
         stream = _n.current_stream(self.w)

@@ -355,7 +355,8 @@ int gridnet_hip_chain_backward_all(int dtype, const void *weight, const void *bi
 /*
  * ---- The forward of a whole chain in one launch, for small problems ------------------------------
  * The same loop forward, h = LayerNorm(step(h)) `outer` times: out [B,M,N,K].  y_raw [outer,B,M,N,K]
- * and stats [outer,B,2] receive what a backward needs, or are both NULL.  float32, normalize = false,
+ * and stats [outer,B,2] receive what a backward needs, or are both NULL; saved [outer,B,M,N,K], with one
+ * inner iteration, what gridnet_hip_rows_chain_backward needs beside them, or NULL.  float32, normalize = false,
  * block_size 8, inner >= 1, outer >= 2, and few enough (block, batch element) pairs to be resident at
  * once; gridnet_hip_chain_forward_all_supported() tells.  Launched cooperatively; its waits are
  * bounded, and should one run out a second kernel on the same stream computes the chain again without
@@ -366,9 +367,34 @@ int gridnet_hip_chain_forward_all_supported(int dtype, int B, int M, int N, int 
 size_t gridnet_hip_chain_forward_all_workspace_bytes(int B, int M, int N, int K);
 int gridnet_hip_chain_forward_all(int dtype, const void *weight, const void *bias, const void *scale,
                                   const void *gamma, const void *beta, const void *x0, void *y_raw,
-                                  void *stats, void *out, int B, int M, int N, int K, int inner, int outer,
-                                  int block_size, double ln_eps, int activation, void *workspace,
+                                  void *stats, void *saved, void *out, int B, int M, int N, int K, int inner,
+                                  int outer, int block_size, double ln_eps, int activation, void *workspace,
                                   size_t workspace_bytes, void *stream);
+
+/*
+ * ---- A chain of steps with one inner iteration, by whole rows ------------------------------------
+ * The same loop with one inner iteration per step (the block size does not enter then), plain
+ * (gated = 0: weight [27,M,N,K], bias, scale [M,N,K]) or with the gated step (weight [27,2,M,N,K], bias
+ * [2,M,N,K], scale and dscale ignored).  One kernel per step and direction.
+ *   y_raw [outer,B,M,N,K], stats [outer,B,2], saved   what the backward needs, or all NULL (forward only);
+ *         saved is [outer,B,M,N,K] (plain) or [outer,3,B,M,N,K] (gated), opaque
+ *   out   [B,M,N,K]        LayerNorm of the last step's output
+ *   dy, dx, d...           as gridnet_hip_chain_backward_all; GRIDNET_OVERWRITE_PARAMS as there
+ * float32, normalize = false, grids that gridnet_hip_rows_chain_supported() names (rows of 16 or 32
+ * cells; plain: 64 too).  Nothing is atomic: the same bits on every run.
+ */
+int gridnet_hip_rows_chain_supported(int dtype, int M, int N, int K, int inner, int normalize, int gated);
+size_t gridnet_hip_rows_chain_workspace_bytes(int B, int M, int N, int K, int gated, int keep, int backward);
+int gridnet_hip_rows_chain_forward(const void *weight, const void *bias, const void *scale, const void *gamma,
+                                   const void *beta, const void *x0, void *y_raw, void *stats, void *saved,
+                                   void *out, int B, int M, int N, int K, int outer, int gated, double ln_eps,
+                                   int activation, void *workspace, size_t workspace_bytes, void *stream);
+int gridnet_hip_rows_chain_backward(const void *weight, const void *scale, const void *gamma, const void *beta,
+                                    const void *x0, const void *y_raw, const void *stats, const void *saved,
+                                    const void *dy, void *dweight, void *dbias, void *dscale, void *dgamma,
+                                    void *dbeta, void *dx, int B, int M, int N, int K, int outer, int gated,
+                                    int activation, int flags, void *workspace, size_t workspace_bytes,
+                                    void *stream);
 /* How often a wait inside the one-launch chain kernels polls before it gives up (default 200000,
  * about a second).  A negative value makes the kernels never signal completion to each other, so
  * that every wait runs out after -limit polls: the give-up path, for tests.  Returns the old value. */

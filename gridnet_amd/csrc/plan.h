@@ -122,14 +122,10 @@ int plan_slab_capacity(const void *slabs, size_t slab_bytes, long slab_floats) {
     return n > 65535 ? 65535 : (int)n;
 }
 
-// Splitting the batch of a block costs one more kernel and a pass over a copy of the gradient
-// arrays per chunk.  Back to back on a stream the split is never slower (32^3 grid, 8^3 blocks,
-// 4 inner iterations: 28.6 against 29.9 us at batch 2, 30.8 against 34.7 us at batch 3, 48 against
-// 91 us at batch 16); a caller that waits for every call sees the extra launch instead, and at
-// batch 2 -- the shape of the reference's own benchmark -- the unsplit call returns 9 % sooner.
-// So the batch is split when that shortens the walk of a workgroup by two elements or more.
-constexpr int kSplitMinSaved = 2;
-int plan_split_room(int room, int B, int chunk_len) { return B - chunk_len < kSplitMinSaved ? 1 : room; }
+// A split costs a pass over a copy of the gradient arrays per chunk, but no launch: the copies are added
+// up beside the second kernel of the backward (TailJob).  So the batch is split as far as it goes: 32^3,
+// batch 2, ten inner iterations with normalize, forward + backward 70 us with both elements in one
+// workgroup, 51 us with one in each.
 
 // `nthreads`: threads per workgroup of the kernel that will run the job.  Its workgroups take as
 // many vectors per thread as keeps them below the number the chip holds.

@@ -31,18 +31,20 @@ namespace {
 
 constexpr int kTube = 4, kSide = kTube + 2, kWinRows = kSide * kSide;
 
-// sigmoid and activation of the gated update, as gated_fast.hip
+// Sigmoid and activation of the gated update, as gated_fast.hip.  (Shorter ones, on the hardware's exp2
+// and reciprocal with one Newton step each, took 5 us off the forward; over a chain of 64 steps their
+// errors, a fifth larger, left the chain's input gradient 1e-5 off where these leave 1e-6.)
 template <int ACT> __device__ __forceinline__ void gate_parts(float pre, float gp, float &a, float &d, float &gate) {
     gate = sigmoid_stable(gp);
     Act<ACT, float>::fd(pre, a, d);
 }
 
 // What both kernels know about a thread's place: its row of the tube, its CPT cells of it.
-template <int CPT> struct RowPlace {
-    int kl, r, ci, cj, bk, p0, q0, grow;
+template <int CPT, int K> struct RowPlace {
+    static constexpr int kl = K / CPT;
+    int r, ci, cj, bk, p0, q0, grow;
     bool first, last;
-    __device__ __forceinline__ RowPlace(int tid, int tube, int N, int K) {
-        kl = K / CPT;
+    __device__ __forceinline__ RowPlace(int tid, int tube, int N) {
         r = tid / kl;
         bk = tid % kl;
         ci = r / kTube;
@@ -57,18 +59,41 @@ template <int CPT> struct RowPlace {
 };
 
 // CPT floats at a byte offset of this lane behind a pointer that is the same for the whole wave: an
-// addressing mode; an element index per lane is widened, scaled and added in vector registers.
+// addressing mode; an element index per lane is widened, scaled and added in vector registers.  Both
+// are opaque: the compiler otherwise widens the offset ahead of the loop, or adds to it what the tensors'
+// pointers share, and is back at vector additions, one per load.
+#define GRIDNET_GLOBAL __attribute__((address_space(1)))
+template <int CPT> struct CellVector { typedef float type __attribute__((ext_vector_type(CPT), aligned(4))); };
+template <> struct CellVector<1> { typedef float type; };
 template <int CPT> __device__ __forceinline__ void load_at(const float *base, unsigned bytes, float (&v)[CPT]) {
-    load_cells<CPT>(reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + bytes), v);
+    typedef typename CellVector<CPT>::type V;
+    const GRIDNET_GLOBAL char *from = (const GRIDNET_GLOBAL char *)base;
+    asm volatile("" : "+s"(from), "+v"(bytes));
+    const V got = *(const GRIDNET_GLOBAL V *)(from + bytes);
+    if constexpr (CPT == 1) v[0] = got;
+    else
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) v[c] = got[c];
 }
 template <int CPT> __device__ __forceinline__ void store_at(float *base, unsigned bytes, const float (&v)[CPT]) {
-    store_cells<CPT>(reinterpret_cast<float *>(reinterpret_cast<char *>(base) + bytes), v);
+    typedef typename CellVector<CPT>::type V;
+    GRIDNET_GLOBAL char *to = (GRIDNET_GLOBAL char *)base;
+    asm volatile("" : "+s"(to), "+v"(bytes));
+    V put;
+    if constexpr (CPT == 1) put = v[0];
+    else
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) put[c] = v[c];
+    *(GRIDNET_GLOBAL V *)(to + bytes) = put;
 }
+#undef GRIDNET_GLOBAL
 // a pair of per-sample numbers, as load_ahead
 __device__ __forceinline__ float2 load_pair_ahead(const float *pairs, int sample) {
     unsigned zero;
     asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
-    return *reinterpret_cast<const float2 *>(reinterpret_cast<const char *>(pairs + 2L * sample) + zero);
+    float v[2];
+    load_at<2>(pairs + 2L * sample, zero, v);
+    return make_float2(v[0], v[1]);
 }
 
 struct RowsFwdArgs {
@@ -76,20 +101,20 @@ struct RowsFwdArgs {
     const float *x_stats;   // the LayerNorm in front of the step (null: x is used as it is)
     float *y, *y_part;
     float *saved;           // plain: [B,cells]; gated: [3][B,cells]; or null
-    int B, M, N, K, ntube, nchunk, chunk_len;
+    int B, M, N, ntube, nchunk, chunk_len;
 };
 
 // PLAIN: four cells and 108 weights per thread; GATED: two cells and 2 x 54.  Everything else as
 // fwd_rows.hip: six by six rows in LDS, two stages, one barrier per batch element.
-template <int ACT, int SETS, bool SAVE>
+template <int ACT, int SETS, bool SAVE, int K>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(SETS == 1 ? 3 : 2, 3)))
 void rows_fwd(RowsFwdArgs a) {
     constexpr int CPT = 4 / SETS, RPT = 3;
     extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][36][K], gamma rows, beta rows
     int tube, chunk;
     if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
-    const int tid = threadIdx.x, M = a.M, N = a.N, K = a.K, nw = blockDim.x / 64, wave = tid / 64;
-    const RowPlace<CPT> p(tid, tube, N, K);
+    const int tid = threadIdx.x, M = a.M, N = a.N, nw = blockDim.x / 64, wave = tid / 64;
+    const RowPlace<CPT, K> p(tid, tube, N);
     const long cells = (long)M * N * K;
     const bool ln_in = a.x_stats != nullptr;
     const int s0 = chunk * a.chunk_len, s1 = min(a.B, s0 + a.chunk_len);
@@ -242,6 +267,45 @@ void rows_fwd(RowsFwdArgs a) {
     }
 }
 
+// One row of delta against the mirrored weights and against x: out[c] += v[t][c] d and n[t][c] += x[c] d for
+// the d of the cell before (t = 0), at (1) and behind (2).  The neighbouring lanes' values are DPP
+// operands of the multiply-adds; the compiler makes moves of them, a quarter of this kernel's
+// instructions with one cell per thread.  A DPP operand must not be a vector ALU result of the two
+// instructions before: the products that take none stand in front.
+#define GRIDNET_BEFORE " wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+#define GRIDNET_BEHIND " wave_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+__device__ __forceinline__ void row_products(const float (&d)[1], const float (&v)[3][1], const float (&x)[1],
+                                             float (&out)[1], float (&n)[3][1]) {
+    asm("v_fmac_f32 %0, %4, %6\n\t"
+        "v_fmac_f32 %2, %4, %8\n\t"
+        "v_fmac_f32_dpp %0, %4, %5" GRIDNET_BEFORE
+        "v_fmac_f32_dpp %1, %4, %8" GRIDNET_BEFORE
+        "v_fmac_f32_dpp %0, %4, %7" GRIDNET_BEHIND
+        "v_fmac_f32_dpp %3, %4, %8" GRIDNET_BEHIND
+        : "+v"(out[0]), "+v"(n[0][0]), "+v"(n[1][0]), "+v"(n[2][0])
+        : "v"(d[0]), "v"(v[0][0]), "v"(v[1][0]), "v"(v[2][0]), "v"(x[0]));
+}
+__device__ __forceinline__ void row_products(const float (&d)[2], const float (&v)[3][2], const float (&x)[2],
+                                             float (&out)[2], float (&n)[3][2]) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        out[c] = fmaf(v[1][c], d[c], out[c]);
+        n[1][c] = fmaf(x[c], d[c], n[1][c]);
+    }
+    n[0][1] = fmaf(x[1], d[0], n[0][1]);
+    n[2][0] = fmaf(x[0], d[1], n[2][0]);
+    asm("v_fmac_f32 %0, %5, %8\n\t"
+        "v_fmac_f32 %1, %4, %7\n\t"
+        "v_fmac_f32_dpp %0, %5, %6" GRIDNET_BEFORE
+        "v_fmac_f32_dpp %2, %5, %10" GRIDNET_BEFORE
+        "v_fmac_f32_dpp %1, %4, %9" GRIDNET_BEHIND
+        "v_fmac_f32_dpp %3, %4, %11" GRIDNET_BEHIND
+        : "+v"(out[0]), "+v"(out[1]), "+v"(n[0][0]), "+v"(n[2][1])
+        : "v"(d[0]), "v"(d[1]), "v"(v[0][0]), "v"(v[0][1]), "v"(v[2][0]), "v"(v[2][1]), "v"(x[0]), "v"(x[1]));
+}
+#undef GRIDNET_BEFORE
+#undef GRIDNET_BEHIND
+
 struct RowsBwdArgs {
     const float *weight, *scale, *gamma, *beta;
     const float *dy;                // gradient with respect to LayerNorm(y)
@@ -253,19 +317,19 @@ struct RowsBwdArgs {
     float *dweight, *dbias, *dscale, *dgamma, *dbeta;
     long slab_stride;               // a copy of the gradient arrays per batch chunk (0: the arrays themselves)
     int accumulate;                 // on top of what the gradient arrays hold
-    int B, M, N, K, ntube, nchunk, chunk_len;
+    int B, M, N, ntube, nchunk, chunk_len;
 };
 
 // PLAIN: two cells per thread, GATED: one; 54 mirrored weights and 54 gradient accumulators for each set
 // and two cells.  A thread moves its own row and one or two of the 20 rows around the tube.
-template <int ACT, int SETS>
+template <int ACT, int SETS, int K>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_bwd(RowsBwdArgs a) {
     constexpr int CPT = 2 / SETS;
     extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K]
     int tube, chunk;
     if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
-    const int tid = threadIdx.x, M = a.M, N = a.N, K = a.K, nw = blockDim.x / 64, wave = tid / 64;
-    const RowPlace<CPT> p(tid, tube, N, K);
+    const int tid = threadIdx.x, M = a.M, N = a.N, nw = blockDim.x / 64, wave = tid / 64;
+    const RowPlace<CPT, K> p(tid, tube, N);
     const long cells = (long)M * N * K, tensor = (long)a.B * cells;
     const bool ln_in = a.x_stats != nullptr;
     const int s0 = chunk * a.chunk_len, s1 = min(a.B, s0 + a.chunk_len);
@@ -452,19 +516,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int pq = 0; pq < 9; ++pq) {
                 const int di = pq / 3 - 1, dj = pq % 3 - 1;
-                float d[CPT + 2], mid[CPT];
+                float mid[CPT];
                 load_cells<CPT>(stage + k * kWinRows * K + own_at + (di * kSide + dj) * K, mid);
-                d[0] = lane_before(mid[CPT - 1]);
-                d[CPT + 1] = lane_after(mid[0]);
-#pragma unroll
-                for (int c = 0; c < CPT; ++c) d[c + 1] = mid[c];
-#pragma unroll
-                for (int cc = 0; cc < 3; ++cc)
-#pragma unroll
-                    for (int c = 0; c < CPT; ++c) {
-                        out[c] = fmaf(v[k][pq][cc][c], d[c + cc], out[c]);
-                        nv[k][pq][cc][c] = fmaf(xh[c], d[c + cc], nv[k][pq][cc][c]);
-                    }
+                row_products(mid, v[k][pq], xh, out, nv[k][pq]);
             }
         if (a.x_part) {  // the sums of the LayerNorm on x, one pair per wave
             float t1 = 0.f, t2 = 0.f;
@@ -556,13 +610,12 @@ template <typename K> int allow_lds(K kern, size_t lds) {
     return GRIDNET_OK;
 }
 
-template <int ACT, int SETS, bool SAVE> int run_forward(const RowsChain &c, hipStream_t st) {
-    auto kern = rows_fwd<ACT, SETS, SAVE>;
+template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &c, hipStream_t st) {
+    auto kern = rows_fwd<ACT, SETS, SAVE, K>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
     const int ntube = tubes_of(c), nt = fwd_threads(c), pairs = fwd_pairs(c);
     const size_t lds = 4 * (size_t)kWinRows * c.K * sizeof(float);
-    static int per_cu_cache[128 / 4 + 1];  // per instantiation, by K
-    int &per_cu = per_cu_cache[c.K / 4];
+    static int per_cu = 0;  // per instantiation
     if (per_cu == 0) {
         if (int rc = allow_lds(kern, lds)) return rc;
         per_cu = workgroups_per_cu(kern, nt, lds);
@@ -570,7 +623,7 @@ template <int ACT, int SETS, bool SAVE> int run_forward(const RowsChain &c, hipS
     RowsFwdArgs a{};
     a.nchunk = plan_row_chunks(c.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, a.chunk_len);
     a.weight = c.weight; a.bias = c.bias; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
-    a.B = c.B; a.M = c.M; a.N = c.N; a.K = c.K; a.ntube = ntube;
+    a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
     // workspace: the pairs; and, where nothing is kept, statistics and two raw tensors
     char *ws = (char *)c.workspace;
     a.y_part = (float *)ws;
@@ -599,13 +652,12 @@ int bwd_chunks(const RowsChain &c, int per_cu, int &chunk_len) {
 constexpr int kBwdMostPerCu = 4;
 int grad_planes(const RowsChain &c) { return c.gated ? 58 : 31; }
 
-template <int ACT, int SETS> int run_backward(const RowsChain &c, hipStream_t st) {
-    auto kern = rows_bwd<ACT, SETS>;
+template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStream_t st) {
+    auto kern = rows_bwd<ACT, SETS, K>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
     const int ntube = tubes_of(c), nt = bwd_threads(c), pairs = bwd_pairs(c);
     const size_t lds = 2 * (size_t)SETS * kWinRows * c.K * sizeof(float);
-    static int per_cu_cache[64 / 4 + 1];  // per instantiation, by K
-    int &per_cu = per_cu_cache[c.K / 4];
+    static int per_cu = 0;  // per instantiation
     if (per_cu == 0) {
         const int n = workgroups_per_cu(kern, nt, lds);
         per_cu = n < kBwdMostPerCu ? n : kBwdMostPerCu;
@@ -613,7 +665,7 @@ template <int ACT, int SETS> int run_backward(const RowsChain &c, hipStream_t st
     RowsBwdArgs a{};
     a.nchunk = bwd_chunks(c, per_cu, a.chunk_len);
     a.weight = c.weight; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
-    a.B = c.B; a.M = c.M; a.N = c.N; a.K = c.K; a.ntube = ntube;
+    a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
     // workspace: the pairs, the sums, scratch of the last LayerNorm's sums, a second dx, the copies
     char *ws = (char *)c.workspace;
     float *part = (float *)ws;
@@ -676,21 +728,35 @@ template <int ACT, int SETS> int run_backward(const RowsChain &c, hipStream_t st
     return plan_launch_tail_job(plan_tail_job(slabs, a.nchunk, slab_floats, t, add ? 1 : 0, 256), st);
 }
 
+template <int ACT, int SETS, bool SAVE> int forward_rows(const RowsChain &c, hipStream_t st) {
+    if (c.K == 16) return run_forward<ACT, SETS, SAVE, 16>(c, st);
+    if (c.K == 32) return run_forward<ACT, SETS, SAVE, 32>(c, st);
+    if constexpr (SETS == 1) return run_forward<ACT, SETS, SAVE, 64>(c, st);
+    return fail(GRIDNET_ERR_ARGUMENT, "rows of %d cells", c.K);
+}
+template <int ACT, int SETS> int backward_rows(const RowsChain &c, hipStream_t st) {
+    if (c.K == 16) return run_backward<ACT, SETS, 16>(c, st);
+    if (c.K == 32) return run_backward<ACT, SETS, 32>(c, st);
+    if constexpr (SETS == 1) return run_backward<ACT, SETS, 64>(c, st);
+    return fail(GRIDNET_ERR_ARGUMENT, "rows of %d cells", c.K);
+}
 template <int SETS, bool SAVE> int forward_act(const RowsChain &c, hipStream_t st) {
     switch (c.activation) {
-        case GRIDNET_ACT_RELU: return run_forward<GRIDNET_ACT_RELU, SETS, SAVE>(c, st);
-        case GRIDNET_ACT_LEAKY_RELU: return run_forward<GRIDNET_ACT_LEAKY_RELU, SETS, SAVE>(c, st);
-        case GRIDNET_ACT_SILU: return run_forward<GRIDNET_ACT_SILU, SETS, SAVE>(c, st);
-        case GRIDNET_ACT_TANH: return run_forward<GRIDNET_ACT_TANH, SETS, SAVE>(c, st);
+        case GRIDNET_ACT_RELU: return forward_rows<GRIDNET_ACT_RELU, SETS, SAVE>(c, st);
+        case GRIDNET_ACT_LEAKY_RELU: return forward_rows<GRIDNET_ACT_LEAKY_RELU, SETS, SAVE>(c, st);
+        case GRIDNET_ACT_SILU: return forward_rows<GRIDNET_ACT_SILU, SETS, SAVE>(c, st);
+        case GRIDNET_ACT_TANH: return forward_rows<GRIDNET_ACT_TANH, SETS, SAVE>(c, st);
     }
     return fail(GRIDNET_ERR_ACTIVATION, "unknown activation function: id %d", c.activation);
 }
+// The gated backward works on saved factors: no activation in it.
 template <int SETS> int backward_act(const RowsChain &c, hipStream_t st) {
+    if constexpr (SETS == 2) return backward_rows<GRIDNET_ACT_RELU, SETS>(c, st);
     switch (c.activation) {
-        case GRIDNET_ACT_RELU: return run_backward<GRIDNET_ACT_RELU, SETS>(c, st);
-        case GRIDNET_ACT_LEAKY_RELU: return run_backward<GRIDNET_ACT_LEAKY_RELU, SETS>(c, st);
-        case GRIDNET_ACT_SILU: return run_backward<GRIDNET_ACT_SILU, SETS>(c, st);
-        case GRIDNET_ACT_TANH: return run_backward<GRIDNET_ACT_TANH, SETS>(c, st);
+        case GRIDNET_ACT_RELU: return backward_rows<GRIDNET_ACT_RELU, SETS>(c, st);
+        case GRIDNET_ACT_LEAKY_RELU: return backward_rows<GRIDNET_ACT_LEAKY_RELU, SETS>(c, st);
+        case GRIDNET_ACT_SILU: return backward_rows<GRIDNET_ACT_SILU, SETS>(c, st);
+        case GRIDNET_ACT_TANH: return backward_rows<GRIDNET_ACT_TANH, SETS>(c, st);
     }
     return fail(GRIDNET_ERR_ACTIVATION, "unknown activation function: id %d", c.activation);
 }

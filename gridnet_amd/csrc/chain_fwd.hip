@@ -39,7 +39,7 @@ namespace {
 
 constexpr int kSide = 10, kWindow = kSide * kSide * kSide, kShellCells = 488;
 constexpr int kCfThreads = 512;
-constexpr int kRing = 4;
+constexpr int kRing = 4, kAhead = 2;
 constexpr unsigned kEmpty = 0xffffffffu;
 
 struct ChainFwdArgs {
@@ -197,14 +197,20 @@ template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd(Chain
             float v = want ? ld_agent(from + p.edge) : 0.f;
             if (wave == 0) {
                 GroupSums sums;
-                for (int i = lane; i < kGroups * a.nblk; i += 64) {
-                    unsigned long long word = ld_agent(pf + i);
-                    while (word == ~0ull && budget > 0) {
-                        if (--budget == 0) st_agent(a.status, 1u);
-                        __builtin_amdgcn_s_sleep(1);
-                        word = ld_agent(pf + i);
+                const int nwords = kGroups * a.nblk;
+                for (int i0 = lane; i0 < nwords; i0 += 64 * kAhead) {
+                    unsigned long long word[kAhead];  // requested together: one trip to memory
+#pragma unroll
+                    for (int k = 0; k < kAhead; ++k) word[k] = ld_agent(pf + min(i0 + 64 * k, nwords - 1));
+#pragma unroll
+                    for (int k = 0; k < kAhead; ++k) {
+                        while (word[k] == ~0ull && budget > 0) {
+                            if (--budget == 0) st_agent(a.status, 1u);
+                            __builtin_amdgcn_s_sleep(1);
+                            word[k] = ld_agent(pf + min(i0 + 64 * k, nwords - 1));
+                        }
+                        if (i0 + 64 * k < nwords) sums.add(word[k]);
                     }
-                    sums.add(word);
                 }
                 sums.over_wave();
                 float mean, rstd;

@@ -325,7 +325,7 @@ struct RowsBwdArgs {
 template <int ACT, int SETS, int K>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_bwd(RowsBwdArgs a) {
     constexpr int CPT = 2 / SETS;
-    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K]
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K], then gamma and (plain) scale of the rows
     int tube, chunk;
     if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
     const int tid = threadIdx.x, M = a.M, N = a.N, nw = blockDim.x / 64, wave = tid / 64;
@@ -397,7 +397,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // ---- the rows around the tube that this thread moves: number r and, the first four rows, 16 + r ----
     int hoff[2], hat[2];
     bool hok[2];
-    float hgam[2][CPT], hrv[2][CPT] = {};
+    // gamma and scale of a thread's rows wait in LDS (each thread reads what it wrote); the scale is zero
+    // outside the grid
+    float *gam_rows = lds + 2 * SETS * kWinRows * K, *scale_rows = gam_rows + kWinRows * K;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
         const int h = min(p.r + 16 * e, 19);
@@ -406,11 +408,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         hok[e] = gi >= 0 && gi < M && gj >= 0 && gj < N;
         hoff[e] = hok[e] ? (gi * N + gj) * K + CPT * p.bk : p.grow;  // anything valid when not used
         hat[e] = (wi * kSide + wj) * K + CPT * p.bk;
-        load_cells<CPT>(a.gamma + hoff[e], hgam[e]);
-        if (SETS == 1) load_cells<CPT>(a.scale + hoff[e], hrv[e]);
+        float t[CPT];
+        load_cells<CPT>(a.gamma + hoff[e], t);
+        if (e == 0 || p.r < 4) store_cells<CPT>(gam_rows + hat[e], t);
+        if (SETS == 1) {
+            load_cells<CPT>(a.scale + hoff[e], t);
+#pragma unroll
+            for (int c = 0; c < CPT; ++c) t[c] = hok[e] ? t[c] : 0.f;
+            if (e == 0 || p.r < 4) store_cells<CPT>(scale_rows + hat[e], t);
+        }
     }
     const bool second = p.r < 4;  // whole waves or parts of them
     const int own_row = (p.ci + 1) * kSide + p.cj + 1, own_at = own_row * K + CPT * p.bk;
+    store_cells<CPT>(gam_rows + own_at, gam);
+    if (SETS == 1) store_cells<CPT>(scale_rows + own_at, rv);
     wait_global_loads();
 #pragma unroll
     for (int pq = 0; pq < 9; ++pq) {
@@ -429,34 +440,35 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
     }
 
-    // what an element needs, requested one element ahead: dy, y and the saved factors of the cell (plain:
+    // what an element needs, requested TWO elements ahead: dy, y and the saved factors of the cell (plain:
     // u; gated: f0, f1, and of the own cells the gate)
     constexpr int NF = SETS;
-    float bdy[3][CPT], by[3][CPT], bf[3][NF][CPT], bgate[CPT] = {}, bx[CPT];
-    float2 next_y, next_sums, next_x;
+    struct Ahead {
+        float dy[3][CPT], y[3][CPT], f[3][NF][CPT], gate[CPT], x[CPT];
+        float numbers;  // of the sample, by lane: statistics of y, the two sums, statistics of x
+    };
     const unsigned own_off = 4u * (unsigned)p.grow;
     const unsigned off[3] = {own_off, 4u * (unsigned)hoff[0], 4u * (unsigned)hoff[1]};
-    const float *x_stats = ln_in ? a.x_stats : a.y_stats;  // loaded in any case: no branch among the requests
-    auto fetch = [&](int s) {
+    const int lane = tid & 63;
+    const float *number = lane < 2 ? a.y_stats + lane : lane < 4 ? a.y_sums + (lane - 2) : lane < 6 && ln_in ? a.x_stats + (lane - 4) : a.y_stats;
+    auto fetch = [&](int s, Ahead &n) {
         const long at = (long)s * cells;
-        next_y = load_pair_ahead(a.y_stats, s);
-        next_sums = load_pair_ahead(a.y_sums, s);
-        next_x = load_pair_ahead(x_stats, s);
-        load_at<CPT>(a.x + at, own_off, bx);
-        if (SETS == 2) load_at<CPT>(a.saved + 2 * tensor + at, own_off, bgate);
+        n.numbers = number[2 * s];
+        load_at<CPT>(a.x + at, own_off, n.x);
+        if (SETS == 2) load_at<CPT>(a.saved + 2 * tensor + at, own_off, n.gate);
 #pragma unroll
         for (int e = 0; e < 3; ++e) {
-            load_at<CPT>(a.dy + at, off[e], bdy[e]);
-            load_at<CPT>(a.y + at, off[e], by[e]);
+            load_at<CPT>(a.dy + at, off[e], n.dy[e]);
+            load_at<CPT>(a.y + at, off[e], n.y[e]);
 #pragma unroll
-            for (int k = 0; k < NF; ++k) load_at<CPT>(a.saved + k * tensor + at, off[e], bf[e][k]);
+            for (int k = 0; k < NF; ++k) load_at<CPT>(a.saved + k * tensor + at, off[e], n.f[e][k]);
         }
     };
     float out[CPT];
-    if (s0 < s1) fetch(s0);
-    for (int s = s0; s < s1; ++s) {
-        float *stage = lds + ((s - s0) & 1) * SETS * kWinRows * K;
-        const float ymean = next_y.x, yrstd = next_y.y, c1 = next_sums.x, c2 = next_sums.y;
+    auto element = [&](int s, float *stage, Ahead &n) {
+        auto number_of = [&](int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.numbers), k)); };
+        const float ymean = number_of(0), yrstd = number_of(1), c1 = number_of(2), c2 = number_of(3);
+        const float xmean = number_of(4), xrstd = number_of(5);
         // through the LayerNorm's backward: the gradient with respect to the step's raw output
         auto raw_gradient = [&](float dy, float y, float gamma, float &yh) {
             yh = (y - ymean) * yrstd;
@@ -465,38 +477,44 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         float direct[CPT], xh[CPT], xn[CPT];
 #pragma unroll
         for (int c = 0; c < CPT; ++c) {
-            xn[c] = (bx[c] - next_x.x) * next_x.y;
-            xh[c] = ln_in ? fmaf(xn[c], gam[c], bet[c]) : bx[c];
+            xn[c] = (n.x[c] - xmean) * xrstd;
         }
+        float g_own[CPT];
+        load_cells<CPT>(gam_rows + own_at, g_own);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) xh[c] = ln_in ? fmaf(xn[c], g_own[c], bet[c]) : n.x[c];
 #pragma unroll
         for (int e = 0; e < 3; ++e) {
             if (e == 2 && !second) break;
-            float delta[SETS][CPT];
+            float delta[SETS][CPT], gq[CPT], rq[CPT];
+            const int at = e == 0 ? own_at : hat[e - 1 < 0 ? 0 : e - 1];
+            load_cells<CPT>(gam_rows + at, gq);
+            if (SETS == 1) load_cells<CPT>(scale_rows + at, rq);
 #pragma unroll
             for (int c = 0; c < CPT; ++c) {
                 float yh;
-                const float g = raw_gradient(bdy[e][c], by[e][c], e == 0 ? gam[c] : hgam[e - 1 < 0 ? 0 : e - 1][c], yh);
-                const bool in_grid = e == 0 || hok[e - 1 < 0 ? 0 : e - 1];
+                const float g = raw_gradient(n.dy[e][c], n.y[e][c], gq[c], yh);
+                const bool in_grid = SETS == 1 || e == 0 || hok[e - 1 < 0 ? 0 : e - 1];
                 if (SETS == 1) {
                     float f, d;
-                    Act<ACT, float>::fd(bf[e][0][c], f, d);
-                    delta[0][c] = in_grid ? d * g * (e == 0 ? rv[c] : hrv[e - 1 < 0 ? 0 : e - 1][c]) : 0.f;
+                    Act<ACT, float>::fd(n.f[e][0][c], f, d);
+                    delta[0][c] = d * g * rq[c];
                     if (e == 0) dr[c] = fmaf(f, g, dr[c]);
                 } else {
 #pragma unroll
-                    for (int k = 0; k < SETS; ++k) delta[k][c] = in_grid ? g * bf[e][k][c] : 0.f;
+                    for (int k = 0; k < SETS; ++k) delta[k][c] = in_grid ? g * n.f[e][k][c] : 0.f;
                 }
                 if (e == 0) {
-                    direct[c] = SETS == 1 ? g : bgate[c] * g;
-                    dgam[c] = fmaf(bdy[e][c], yh, dgam[c]);
-                    dbet[c] += bdy[e][c];
+                    direct[c] = SETS == 1 ? g : n.gate[c] * g;
+                    dgam[c] = fmaf(n.dy[e][c], yh, dgam[c]);
+                    dbet[c] += n.dy[e][c];
 #pragma unroll
                     for (int k = 0; k < SETS; ++k) db[k][c] += delta[k][c];
                 }
             }
 #pragma unroll
             for (int k = 0; k < SETS; ++k)
-                store_cells<CPT>(stage + k * kWinRows * K + (e == 0 ? own_at : hat[e - 1 < 0 ? 0 : e - 1]), delta[k]);
+                store_cells<CPT>(stage + k * kWinRows * K + at, delta[k]);
         }
         // worked out in front of the requests that replace what they come from (behind them, the compiler
         // has to wait for the first of those)
@@ -507,7 +525,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // The result of the element before leaves here, ahead of the requests: the memory counter is in
         // order, and a store behind them would be waited for with the last of them.
         if (s > s0) store_at<CPT>(a.dx + (long)(s - 1) * cells, own_off, out);
-        fetch(min(s + 1, s1 - 1));
+        fetch(min(s + 2, s1 - 1), n);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int c = 0; c < CPT; ++c) out[c] = direct[c];
@@ -521,10 +539,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 row_products(mid, v[k][pq], xh, out, nv[k][pq]);
             }
         if (a.x_part) {  // the sums of the LayerNorm on x, one pair per wave
-            float t1 = 0.f, t2 = 0.f;
+            float t1 = 0.f, t2 = 0.f, g_own[CPT];
+            load_cells<CPT>(gam_rows + own_at, g_own);
 #pragma unroll
             for (int c = 0; c < CPT; ++c) {
-                const float go = gam[c] * out[c];
+                const float go = g_own[c] * out[c];
                 t1 += go;
                 t2 = fmaf(go, xn[c], t2);
             }
@@ -536,8 +555,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 to[1] = t2;
             }
         }
+    };
+    float *stages[2] = {lds, lds + SETS * kWinRows * K};
+    Ahead even, odd;
+    fetch(min(s0, a.B - 1), even);
+    fetch(min(s0 + 1, a.B - 1), odd);
+    // in pairs: with a test between the two the compiler counts on fewer requests in flight, and waits for all
+    int s = s0;
+    for (; s + 1 < s1; s += 2) {
+        element(s, stages[0], even);
+        element(s + 1, stages[1], odd);
     }
-
+    if (s < s1) element(s, stages[0], even);
     if (s0 < s1) store_at<CPT>(a.dx + (long)(s1 - 1) * cells, own_off, out);
 
     // ---- parameter gradients: the shifts of the set-up back again, aligned stores of whole rows ----
@@ -656,7 +685,7 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
     auto kern = rows_bwd<ACT, SETS, K>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
     const int ntube = tubes_of(c), nt = bwd_threads(c), pairs = bwd_pairs(c);
-    const size_t lds = 2 * (size_t)SETS * kWinRows * c.K * sizeof(float);
+    const size_t lds = (2 * SETS + 1 + (SETS == 1)) * (size_t)kWinRows * K * sizeof(float);
     static int per_cu = 0;  // per instantiation
     if (per_cu == 0) {
         const int n = workgroups_per_cu(kern, nt, lds);

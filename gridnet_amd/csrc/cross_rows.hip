@@ -301,7 +301,8 @@ int launch_rows(const StepArgs &a, const float *dsum, const TailJob &tail, hipSt
         per_cu = n;
     }
     int chunk_len;
-    const int nchunk = plan_row_chunks(a.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, chunk_len);
+    int nchunk = plan_row_chunks(a.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, chunk_len);
+    plan_even_rounds(a.B, ntube, 1, per_cu * plan_device_cus(), kRowsMinWalk, nchunk, chunk_len);
     hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, nchunk) + tail.blocks()), dim3(nt), lds, st,
                        (const float *)a.weight, (const float *)a.x, dsum, (float *)a.dx, a.B, a.M, a.N, a.K,
                        ntube, nchunk, chunk_len, a.ln, qr, lanes, tail);

@@ -225,7 +225,8 @@ template <int ACT, bool LN, bool RES, bool PAD> int launch_rows(const StepArgs &
     // 11.9 and 14.3 ms per 64-step training step: what limits the kernel is the trip to memory per
     // element, and more workgroups hide it)
     int chunk_len;
-    const int nchunk = plan_row_chunks(a.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, chunk_len);
+    int nchunk = plan_row_chunks(a.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, chunk_len);
+    plan_even_rounds(a.B, ntube, 1, per_cu * plan_device_cus(), kRowsMinWalk, nchunk, chunk_len);
     hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, nchunk)), dim3(nt), lds, st, (const float *)a.weight,
                        (const float *)a.bias, (const float *)a.scale, (const float *)a.x, (float *)a.y, a.B, a.M,
                        a.N, a.K, ntube, nchunk, chunk_len, a.ln, lanes);
@@ -243,11 +244,30 @@ template <int ACT> int dispatch(const StepArgs &a, hipStream_t st) {
     return launch<ACT, false, false>(a, st);
 }
 
+// Rows above 64 cells run as workgroups of 512 lanes, of which a CU holds one: there the share of the
+// chip that works, live lanes x workgroups of the rounds they take, decides against the kernel by
+// blocks.  us by rows / by blocks in a chain, in a residual one and without LayerNorm:
+//   48 x 64 x 96,  batch 32, share .56: 60 / 49, 53 / 57, 33 / 38
+//   40 x 48 x 80,  batch 32, share .58: 34 / 36, 31 / 41, 19 / 29
+//   64 x 64 x 104, batch 16, share .81: 40 / 43, 37 / 52, 23 / 33
+//   64 x 64 x 128, batch 16, share 1:   37 / 47
+//   48 x 88 x 88,  batch 37, share .35: 122 / 65, 109 / 72, 68 / 48
+// Shorter rows share a CU, and win or lose a few per cent at the smallest batches.
+bool fills_chip(const StepArgs &a) {
+    const int lanes = row_lanes(a.K, 4), ntube = (a.M / kRowsTube) * (a.N / kRowsTube), cus = plan_device_cus();
+    if (lanes <= 16 || a.B < 1) return true;
+    int chunk_len;
+    const long groups = (long)ntube * plan_row_chunks(a.B, ntube, cus, kRowsMinWalk, chunk_len);
+    const long room = (groups + cus - 1) / cus * cus;
+    const long share = 100 * groups * (a.K / 4) / (room * lanes);
+    return share >= (a.ln.gamma && !a.ln.residual ? 75 : 45);
+}
+
 }  // namespace
 
 bool fwd_rows_supports(const StepArgs &a) {
     return a.dtype == GRIDNET_F32 && a.inner == 1 && !a.normalize && (a.block_size == 4 || a.block_size == 8) &&
-           k_ok(a.K) && a.M % 4 == 0 && a.N % 4 == 0;
+           k_ok(a.K) && a.M % 4 == 0 && a.N % 4 == 0 && fills_chip(a);
 }
 
 // (mean, M2) pairs per sample that it leaves in a.ln.y_part: one per wave, over its live lanes' cells

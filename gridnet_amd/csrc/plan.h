@@ -36,7 +36,29 @@ void plan_batch_chunks(int B, int nblk, int nslot, int resident, bool whole, int
     nchunk = (B + chunk_len - 1) / chunk_len;
 }
 
-// The same for the row-wise kernels: at most `resident` workgroups, none that walks fewer than
+// Where the chip holds fewer than two workgroups per block the rule above takes one or two chunks and
+// can leave the last round of workgroups nearly empty.  Shorter chunks make that round cheaper, and
+// cost a fetch of the weights each, which is worth about `fetch` turns of the walk.  Takes another number of
+// chunks where rounds x (turns + fetch) says at least a tenth less, so never on grids that fill
+// their rounds already.  For kernels that keep no copy of anything per chunk.  (Forward, four inner
+// iterations: 80 x 80 x 72, batch 32, 129.7 us in one chunk, 116.6 in three; 96^3, batch 16, 129.1
+// and 120.6.)
+void plan_even_rounds(int B, int ngroup, int nslot, int resident, int min_walk, int &nchunk, int &chunk_len) {
+    constexpr long fetch = 3;
+    if ((long)nchunk * ngroup * 10 > 9L * resident && nchunk * ngroup <= resident) return;
+    auto cost = [&](int n, int len) { return ((long)n * ngroup + resident - 1) / resident * (len / nslot + fetch); };
+    const long now = cost(nchunk, chunk_len);
+    long best = now - now / 10;
+    for (int n = 1; n <= 8 && n <= B / min_walk; ++n) {
+        int len = (B + n - 1) / n;
+        len = (len + nslot - 1) / nslot * nslot;
+        const int m = (B + len - 1) / len;
+        const long c = cost(m, len);
+        if (c < best) best = c, nchunk = m, chunk_len = len;
+    }
+}
+
+// As plan_batch_chunks, for the row-wise kernels: at most `resident` workgroups, none that walks fewer than
 // `min_walk` elements for its one fetch of the weights.  Three keep the fetch below the walk and still
 // spread a small batch over the chip (forward / second kernel of the backward; 32^3, one inner
 // iteration, batch 64: 8.8 us at 3, 9.8 at 2 and 11.2 at 8; 40 x 48 x 56, batch 13: 18.6, 17.9

@@ -1670,6 +1670,8 @@ Plan make_plan(const StepArgs &a, int nslot, int resident, bool whole_batch_per_
     return p;
 }
 
+constexpr int kMinForwardWalk = 4;  // elements that a chunk made shorter to even the rounds still walks
+
 template <int BS, int CPT, int NSLOT, int ACT, bool LN, bool RES = false, bool NORM = false>
 int launch_fwd_ln(const StepArgs &a, hipStream_t st) {
     using TL = Tile<BS, CPT>;
@@ -1682,7 +1684,8 @@ int launch_fwd_ln(const StepArgs &a, hipStream_t st) {
             n = 1;
         per_cu = n;
     }
-    const Plan p = make_plan(a, NSLOT, per_cu * device_cus(), false);
+    Plan p = make_plan(a, NSLOT, per_cu * device_cus(), false);
+    plan_even_rounds(a.B, p.nblk, NSLOT, per_cu * device_cus(), kMinForwardWalk, p.nchunk, p.chunk_len);
     hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(TL::TPS * NSLOT), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
                        (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
@@ -1698,7 +1701,8 @@ int launch_fwd_split(const StepArgs &a, hipStream_t st) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 128, 0) != hipSuccess || n < 1) n = 1;
         per_cu = n;
     }
-    const Plan p = make_plan(a, 1, per_cu * device_cus(), false);
+    Plan p = make_plan(a, 1, per_cu * device_cus(), false);
+    plan_even_rounds(a.B, p.nblk, 1, per_cu * device_cus(), kMinForwardWalk, p.nchunk, p.chunk_len);
     hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(128), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
                        (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
@@ -1713,7 +1717,8 @@ template <int ACT> int launch_fwd_pair(const StepArgs &a, hipStream_t st) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kern, 128, 0) != hipSuccess || n < 1) n = 1;
         per_cu = n;
     }
-    const Plan p = make_plan(a, 2, per_cu * device_cus(), false);
+    Plan p = make_plan(a, 2, per_cu * device_cus(), false);
+    plan_even_rounds(a.B, p.nblk, 2, per_cu * device_cus(), kMinForwardWalk, p.nchunk, p.chunk_len);
     hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(128), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
                        (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,

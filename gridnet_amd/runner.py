@@ -14,8 +14,9 @@ With ``fused=True`` and a problem it covers (float32, 8^3 blocks, up to 8 inner 
 backward of a chain can go through ``gridnet_hip_chain_backward``: the backward hands what
 crosses a block boundary from step to step instead of finishing every dx (one kernel per step
 instead of two).  Same results to rounding.  ``chain=None`` (the default) takes it where the
-two-kernel backward would have to deal its cross-block part by block face (rows of more than 128
-cells); where that part goes by whole rows the two kernels are the faster pair
+two-kernel backward would deal its cross-block part by block face (rows of more than 128 cells) or
+by rows that leave lanes idle (72 to 120 cells; 80 x 80 x 72, batch 32, 421 against 463 us per
+step); where that part goes by whole rows the two kernels are the faster pair
 (64^3 grid, batch 32, 12 steps: 3.12 against 3.19 ms per training step).  ``True``: wherever the
 library supports it; ``False``: never (nor the one launch below).
 
@@ -155,7 +156,9 @@ class BodyRunner:
                 self.fb_ws = _n.workspace(self.fb_ws_bytes, dev)
         chain_ok = bool(chain is not False and fused and backward and not outer_residual and not self.rows and
                         _n.lib.gridnet_hip_chain_supported(self.dt, inner, block_size, self.normalize))
-        rows = self.K <= 128  # what the row-wise cross-block kernel takes
+        # where the row-wise cross-block kernel beats the hand-over: above 64 cells a row's workgroup has a
+        # CU to itself, and only rows of 128 use all of it
+        rows = self.K <= 64 or self.K == 128
         self.chain = chain_ok and (chain is True or not rows)
         if self.chain:
             # two buffers that the backward calls of neighbouring steps hand their cross-block

@@ -74,3 +74,33 @@ def test_gated_step(shape, bs, batch, inner):
         results.append([y, *[t.grad for t in leaves]])
     for name, a, e in zip(("y", "dweight", "dbias", "dx"), *results):
         assert_close(a, e, what=name)
+
+
+# Grids of about one round of workgroups: the rule that gives rows of more than 64 cells to the kernel
+# by rows or to the one by blocks, and chunks made shorter to even the rounds.  Samples do not mix, so
+# a batch has to give what its samples give in twos; the first two are held against the oracle.
+@pytest.mark.parametrize("residual", [False, True], ids=["plain", "residual"])
+@pytest.mark.parametrize("shape,bs,batch,inner", [((48, 64, 96), 8, 4, 1), ((40, 48, 72), 8, 9, 1),
+                                                  ((48, 88, 88), 8, 37, 1), ((80, 80, 72), 8, 33, 2),
+                                                  ((52, 52, 52), 4, 21, 2)])
+def test_rounds(shape, bs, batch, inner, residual):
+    from gridnet_amd.runner import BodyRunner
+    from oracle.network import network_forward_backward
+
+    w, b, r = make_params(shape, seed=12)
+    g = torch.Generator().manual_seed(13)
+    params = [w, b, r, 1 + 0.2 * torch.randn(shape, generator=g), 0.2 * torch.randn(shape, generator=g)]
+    x = make_acts(batch, shape, seed=14)
+
+    def forward(rows):
+        run = BodyRunner(*(t.to(DEV) for t in params), len(rows), inner, 2, bs, "silu", fused=True,
+                         backward=False, outer_residual=residual)
+        return run.forward(rows.to(DEV)).cpu()
+
+    got = forward(x)
+    for i in range(0, batch, 2):
+        assert_close(got[i:i + 2], forward(x[i:i + 2]), what=f"samples from {i}")
+    want = network_forward_backward([t.double() for t in params], x[:2].double(), x[:2].double(),
+                                    inner_iterations=inner, outer_iterations=2, block_size=bs,
+                                    activation="silu", outer_residual=residual)[0]
+    assert_close(got[:2], want, rtol=2e-4, atol=2e-5, what="y")

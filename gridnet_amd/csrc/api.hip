@@ -459,7 +459,7 @@ static int fused_backward(int dtype, const void *weight, const void *bias, const
     a.dweight = dweight; a.dbias = dbias; a.dscale = dscale; a.dx = dx;
     a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner; a.block_size = block_size;
     a.activation = activation;
-    a.flags = (flags & GRIDNET_OVERWRITE_PARAMS) | GRIDNET_OVERWRITE_DX;  // dx is always written
+    a.flags = (flags & (GRIDNET_OVERWRITE_PARAMS | GRIDNET_OVERWRITE_STEP_PARAMS)) | GRIDNET_OVERWRITE_DX;  // dx is always written
     a.ln.gamma = (const float *)gamma;  // before the checks: the LDS budget depends on it
     if (int rc = check_fused(a, true)) return rc;
     if (B == 0) return GRIDNET_OK;
@@ -556,7 +556,7 @@ int gridnet_hip_chain_backward(int dtype, const void *weight, const void *bias, 
     a.x = x; a.dy = dy; a.dweight = dweight; a.dbias = dbias; a.dscale = dscale; a.dx = dx;
     a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner; a.block_size = block_size;
     a.activation = activation;
-    a.flags = (flags & GRIDNET_OVERWRITE_PARAMS) | GRIDNET_OVERWRITE_DX;  // dx is always written
+    a.flags = (flags & (GRIDNET_OVERWRITE_PARAMS | GRIDNET_OVERWRITE_STEP_PARAMS)) | GRIDNET_OVERWRITE_DX;  // dx is always written
     a.ln.gamma = (const float *)gamma;
     if (!chain_supports(a))
         return fail(GRIDNET_ERR_ARGUMENT,

@@ -306,21 +306,21 @@ void bwd_rows(const float *__restrict__ weight, const float *__restrict__ bias, 
         nw[pq * 3][0] *= keep_first;
         nw[pq * 3 + 2][1] *= keep_last;
     }
+    auto add_old = [&](const float *from, float (&v)[2]) {
+        float old[2];
+        load_cells<2>(from + grow, old);
+        v[0] += old[0];
+        v[1] += old[1];
+    };
     if (param_mode == kParamAddExclusive) {  // add-in-place mode: on top of what the buffers hold
-        auto add_old = [&](const float *from, float (&v)[2]) {
-            float old[2];
-            load_cells<2>(from + grow, old);
-            v[0] += old[0];
-            v[1] += old[1];
-        };
 #pragma unroll
         for (int t = 0; t < 27; ++t) add_old(dweight + t * cells, nw[t]);
         add_old(dbias, db);
         add_old(dscale, dr);
-        if (LN) {
-            add_old(ln.dgamma, dgam);
-            add_old(ln.dbeta, dbet);
-        }
+    }
+    if (LN && ln.accumulate) {
+        add_old(ln.dgamma, dgam);
+        add_old(ln.dbeta, dbet);
     }
 #pragma unroll
     for (int t = 0; t < 27; ++t) store_cells<2>(dweight + t * cells + grow, nw[t]);
@@ -361,10 +361,11 @@ template <int ACT, bool LN, bool RES, bool PAD> int launch_rows(const StepArgs &
     const int room = plan_slab_capacity(a.slabs, a.slab_bytes, slab_floats);
     if (nchunk > room) nchunk = plan_row_chunks(a.B, ntube, (room > 1 ? room : 1) * ntube, 1, chunk_len);
     const bool split = nchunk > 1;
-    const bool new_params = (a.flags & GRIDNET_OVERWRITE_PARAMS) != 0;
+    const bool new_params = (a.flags & (GRIDNET_OVERWRITE_PARAMS | GRIDNET_OVERWRITE_STEP_PARAMS)) != 0;
     const int param_mode = split || new_params ? kParamStore : kParamAddExclusive;
     float *slab = (float *)a.slabs;
     LnFold ln = a.ln;
+    ln.accumulate = !split && !(a.flags & GRIDNET_OVERWRITE_PARAMS);
     if (split && LN) {
         ln.dgamma = slab + 29 * cells;
         ln.dbeta = slab + 30 * cells;
@@ -388,7 +389,7 @@ template <int ACT, bool LN, bool RES, bool PAD> int launch_rows(const StepArgs &
             t.dst[4] = a.ln.dbeta;  t.end[4] = 31 * cells;
             t.count = 5;
         }
-        tail = plan_tail_job(slab, nchunk, slab_floats, t, new_params ? 0 : 1, cross_rows_threads(a));
+        tail = plan_tail_job(slab, nchunk, slab_floats, t, plan_accumulate_mask(a.flags), cross_rows_threads(a));
     }
     // the LayerNorm sums the kernel above left per wave
     if (bwd_rows_leaves_sums(a)) tail.sums = SumsJob{a.ln.x_part, bwd_rows_pairs(a), a.B, cells, a.ln.x_sums};

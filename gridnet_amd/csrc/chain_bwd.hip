@@ -112,6 +112,7 @@ struct ChainBwdArgs {
     float *out2;               // DEFER: halo_out [B, nblk, 488]; otherwise D [B, cells]
     float *x_part;             // DEFER: [B, nblk, 2] sums for the LayerNorm in front of this step
     int B, M, N, K, inner, nblk, nchunk, chunk_len, param_mode;
+    int norm_accumulate;       // dgamma and dbeta are added to what is there, whatever param_mode says
     long slab_stride;          // split batch: floats between the chunks' copies of the gradient arrays, else 0
     // ---- ALL: every step of the chain in one launch (see chain_bwd) ----
     // y_raw and y_stats then point at step 0's and the steps lie step_floats / 2 B floats apart;
@@ -421,8 +422,10 @@ void chain_bwd(const ChainBwdArgs a) {
             for (int c = 0; c < CPT; ++c) nw[t][c] = (a.dweight + slab_off)[owner_of(t, c)];
         load_cells<CPT>((a.dbias + slab_off) + pl.gc, db);
         load_cells<CPT>((a.dscale + slab_off) + pl.gc, dr);
-        load_cells<CPT>((a.dgamma + slab_off) + pl.gc, dgam);
-        load_cells<CPT>((a.dbeta + slab_off) + pl.gc, dbet);
+    }
+    if (a.norm_accumulate) {
+        load_cells<CPT>((a.dgamma + slab_offset()) + pl.gc, dgam);
+        load_cells<CPT>((a.dbeta + slab_offset()) + pl.gc, dbet);
     }
     auto acc_ref = [&](int k) -> float & { return reinterpret_cast<float *>(ctab)[(kTabAcc + k) * 256 + tid]; };
 #pragma unroll
@@ -921,7 +924,7 @@ template <int ACT, bool DEFER, bool WIDE> int launch_chain(const StepArgs &a, hi
     // a workgroup: plain stores for the parameter gradients, bitwise reproducible
     const bool whole = k.nblk >= plan_device_cus();
     plan_batch_chunks(a.B, k.nblk, 1, per_cu * plan_device_cus(), whole, k.nchunk, k.chunk_len);
-    const bool new_params = (a.flags & GRIDNET_OVERWRITE_PARAMS) != 0;
+    const bool new_params = (a.flags & (GRIDNET_OVERWRITE_PARAMS | GRIDNET_OVERWRITE_STEP_PARAMS)) != 0;
     // A split batch: every chunk gets a copy of the gradient arrays in the scratch; with less
     // room than chunks the batch is split less (down to not at all).
     const long slab_floats = kStepSlabPlanes * cells;
@@ -932,6 +935,7 @@ template <int ACT, bool DEFER, bool WIDE> int launch_chain(const StepArgs &a, hi
     }
     const bool split = k.nchunk > 1;
     k.param_mode = split || new_params ? kParamStore : kParamAddExclusive;
+    k.norm_accumulate = !split && !(a.flags & GRIDNET_OVERWRITE_PARAMS);
     k.slab_stride = split ? slab_floats : 0;
     float *slab = (float *)a.slabs;
     k.weight = (const float *)a.weight; k.bias = (const float *)a.bias; k.scale = (const float *)a.scale;
@@ -959,7 +963,7 @@ template <int ACT, bool DEFER, bool WIDE> int launch_chain(const StepArgs &a, hi
         t.dst[3] = a.ln.dgamma;        t.end[3] = 30 * cells;
         t.dst[4] = a.ln.dbeta;         t.end[4] = 31 * cells;
         t.count = 5;
-        tail = plan_tail_job(slab, k.nchunk, slab_floats, t, new_params ? 0 : 1,
+        tail = plan_tail_job(slab, k.nchunk, slab_floats, t, plan_accumulate_mask(a.flags),
                              !DEFER && cross_rows_supports(a) ? cross_rows_threads(a) : 256);
     }
     if (DEFER) return plan_launch_tail_job(tail, st);
@@ -1057,6 +1061,7 @@ template <int ACT, bool WIDE> int launch_chain_all(const ChainAll &c, hipStream_
     k.nchunk = 1;
     k.chunk_len = c.B;
     k.param_mode = (c.flags & GRIDNET_OVERWRITE_PARAMS) ? kParamStore : kParamAddExclusive;
+    k.norm_accumulate = k.param_mode == kParamAddExclusive;
     k.weight = c.weight; k.bias = c.bias; k.scale = c.scale; k.gamma = c.gamma; k.beta = c.beta;
     k.x0 = c.x0; k.y_raw = c.y_raw; k.y_stats = c.stats; k.sums = (float *)(ws + l.sums_at); k.dy = c.dy;
     k.dweight = c.dweight; k.dbias = c.dbias; k.dscale = c.dscale; k.dgamma = c.dgamma; k.dbeta = c.dbeta;

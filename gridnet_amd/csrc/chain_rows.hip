@@ -754,7 +754,7 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
             if (int rc = layernorm_finalize_sums(part, pairs, cells, sums, c.B, st)) return rc;
     }
     if (!split) return GRIDNET_OK;
-    return plan_launch_tail_job(plan_tail_job(slabs, a.nchunk, slab_floats, t, add ? 1 : 0, 256), st);
+    return plan_launch_tail_job(plan_tail_job(slabs, a.nchunk, slab_floats, t, add ? ~0 : 0, 256), st);
 }
 
 template <int ACT, int SETS, bool SAVE> int forward_rows(const RowsChain &c, hipStream_t st) {

@@ -494,7 +494,7 @@ template <int BS, int NSLOT, int ACT> int launch_bwd(const StepArgs &a, hipStrea
         t.dst[0] = (float *)a.dweight; t.end[0] = 54 * cells;
         t.dst[1] = (float *)a.dbias;   t.end[1] = 56 * cells;
         t.count = 2;
-        tail = plan_tail_job(slab, nchunk, slab_floats, t, new_params ? 0 : 1,
+        tail = plan_tail_job(slab, nchunk, slab_floats, t, plan_accumulate_mask(a.flags),
                              cross_rows_gated_supports(a) ? cross_rows_threads(a) : 256);
     }
     // same blocks, same batch chunks; the parameter gradients are complete, dx is not yet

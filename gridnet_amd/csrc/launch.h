@@ -22,7 +22,8 @@ struct LnFold {
     const float *y_raw;         // [B,M,N,K] this step's forward output before its LayerNorm
     const float *y_stats;       // [B,2]
     const float *y_sums;        // [B,2]: mean(g), mean(g * yhat) with g = gamma * incoming gradient
-    float *dgamma, *dbeta;      // [M,N,K], summed over the batch, committed like dbias
+    float *dgamma, *dbeta;      // [M,N,K], summed over the batch
+    int accumulate;             // they are added to what is there, whatever dbias is (set by the launcher)
     float *x_part;              // partial sums for the LayerNorm backward of x: [B, nblk, parts, 2]
     float *x_sums;              // [B,2] or null: where a backward that finishes the sums itself leaves them
                                 // (bwd_rows_leaves_sums); otherwise the caller finalizes x_part
@@ -104,7 +105,8 @@ struct SumsJob {
 // (cross_rows) instead of in a launch of its own, whose 8 us on a 32^3 grid were mostly start and end.
 struct TailJob {
     const float *slabs;
-    int ncopies, accumulate, reduce_blocks;  // reduce_blocks = 0: no copies
+    int ncopies, reduce_blocks;  // reduce_blocks = 0: no copies
+    int accumulate;              // bit k: target k is added to
     long stride, total4;                     // total4: 16-byte vectors in a copy
     SlabTargets t;
     SumsJob sums;

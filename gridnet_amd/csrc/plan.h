@@ -129,7 +129,7 @@ __device__ __forceinline__ void run_tail_job(const TailJob &job, int block, int 
         long begin = 0;
         while (k + 1 < job.t.count && at >= job.t.end[k]) begin = job.t.end[k++];
         float4 *to = reinterpret_cast<float4 *>(job.t.dst[k] + (at - begin));
-        if (job.accumulate) {
+        if (job.accumulate >> k & 1) {
             const float4 old = *to;
             sum.x += old.x; sum.y += old.y; sum.z += old.z; sum.w += old.w;
         }
@@ -148,6 +148,13 @@ int plan_slab_capacity(const void *slabs, size_t slab_bytes, long slab_floats) {
 // up beside the second kernel of the backward (TailJob).  So the batch is split as far as it goes: 32^3,
 // batch 2, ten inner iterations with normalize, forward + backward 70 us with both elements in one
 // workgroup, 51 us with one in each.
+
+// Which targets of a split backward are added to rather than written (dweight, dbias, dscale, then
+// dgamma and dbeta), by the caller's flags.
+int plan_accumulate_mask(int flags) {
+    if (flags & GRIDNET_OVERWRITE_PARAMS) return 0;
+    return (flags & GRIDNET_OVERWRITE_STEP_PARAMS) ? 8 | 16 : ~0;
+}
 
 // `nthreads`: threads per workgroup of the kernel that will run the job.  Its workgroups take as
 // many vectors per thread as keeps them below the number the chip holds.

@@ -987,10 +987,10 @@ void step_bwd_fast(
             db[c] = dbias[pl.gc + c];
             dr[c] = dscale[pl.gc + c];
         }
-        if (LN) {
-            load_cells<CPT>(ln.dgamma + pl.gc, dgam);
-            load_cells<CPT>(ln.dbeta + pl.gc, dbet);
-        }
+    }
+    if (LN && ln.accumulate && pl.slot == 0) {
+        load_cells<CPT>(ln.dgamma + pl.gc, dgam);
+        load_cells<CPT>(ln.dbeta + pl.gc, dbet);
     }
 
     const int s0 = chunk * chunk_len, s1 = min(B, s0 + chunk_len);
@@ -1785,7 +1785,7 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
     // parameter gradients) as soon as the blocks alone give every CU a workgroup
     const bool whole = nblk >= device_cus();
     Plan p = make_plan(a, NSLOT, per_cu * device_cus(), whole);
-    const bool new_params = (a.flags & GRIDNET_OVERWRITE_PARAMS) != 0;
+    const bool new_params = (a.flags & (GRIDNET_OVERWRITE_PARAMS | GRIDNET_OVERWRITE_STEP_PARAMS)) != 0;
     // A split batch: every chunk gets a copy of the gradient arrays in the scratch; with less
     // room than chunks the batch is split less (down to not at all).
     const long slab_floats = kStepSlabPlanes * cells;
@@ -1797,6 +1797,7 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
     const int param_mode = split || new_params ? kParamStore : kParamAddExclusive;
     float *slab = (float *)a.slabs;
     LnFold ln = a.ln;
+    ln.accumulate = !split && !(a.flags & GRIDNET_OVERWRITE_PARAMS);
     if (split && LN) {
         ln.dgamma = slab + 29 * cells;
         ln.dbeta = slab + 30 * cells;
@@ -1825,7 +1826,7 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
             t.dst[4] = a.ln.dbeta;  t.end[4] = 31 * cells;
             t.count = 5;
         }
-        tail = plan_tail_job(slab, p.nchunk, slab_floats, t, new_params ? 0 : 1, by_rows ? cross_rows_threads(a) : 256);
+        tail = plan_tail_job(slab, p.nchunk, slab_floats, t, plan_accumulate_mask(a.flags), by_rows ? cross_rows_threads(a) : 256);
     }
     // same blocks, same batch chunks; the parameter gradients are complete, dx is not yet
     constexpr int XSLOT = BS == 8 ? kCrossSlots8 : kCrossSlots4;

@@ -20,6 +20,7 @@ FUSED_RESIDUAL, FUSED_WALK_REVERSE = 1, 2  # gridnet_hip_fused_forward_flags
 OVERWRITE_PARAMS = 1
 OVERWRITE_DX = 2
 OVERWRITE = 3
+OVERWRITE_STEP_PARAMS = 4  # fused and chain backward: all but dgamma, dbeta
 STATIC_SCRATCH_BYTES = 40 << 20  # GRIDNET_STATIC_SCRATCH_BYTES
 
 EXPORTS = (

@@ -111,10 +111,7 @@ class BodyRunner:
         if backward:
             self.ga = torch.empty(shape, device=dev, dtype=dtype)
             self.gb = torch.empty(shape, device=dev, dtype=dtype)
-            # one gradient set per parameter set.  The entry points either overwrite all parameter
-            # gradients of a call or accumulate into all of them, the LayerNorm's (shared by the
-            # steps) included: with separate parameters the last step's call overwrites, the
-            # others accumulate into buffers that backward() zero-fills first
+            # one gradient set per parameter set
             n_sets = outer if self.separate else 1
             self.dw_all = torch.empty((n_sets,) + tuple(weight.shape), device=dev, dtype=dtype)
             self.db_all = torch.empty((n_sets,) + tuple(bias.shape), device=dev, dtype=dtype)
@@ -191,11 +188,12 @@ class BodyRunner:
             return list(self.dw_all), list(self.db_all), list(self.dr_all)
         return self.dw_all[0], self.db_all[0], self.dr_all[0]
 
-    def _zero_separate_grads(self):
-        if self.separate and self.outer > 1:
-            self.dw_all[:-1].zero_()
-            self.db_all[:-1].zero_()
-            self.dr_all[:-1].zero_()
+    def _param_flags(self, j):
+        """The last step's call, the backward's first, writes every parameter gradient; the others add
+        to them, or, with parameters of their own, to the LayerNorm's only."""
+        if j == self.outer - 1:
+            return _n.OVERWRITE_PARAMS
+        return _n.OVERWRITE_STEP_PARAMS if self.separate else 0
 
     def _mark(self, name, phase):
         if self.on_launch is not None:
@@ -320,7 +318,7 @@ class BodyRunner:
                 *self._grads(j), self.dgamma.data_ptr(),
                 self.dbeta.data_ptr(), dn[j % 2].data_ptr(), self.sums[j].data_ptr(),
                 self.B, self.M, self.N, self.K, self.inner, self.bs, self.act,
-                _n.OVERWRITE_PARAMS if given else 0, self.fb_ws.data_ptr(), self.fb_ws_bytes, stream))
+                self._param_flags(j), self.fb_ws.data_ptr(), self.fb_ws_bytes, stream))
             self._mark("step_bwd", 1)
         # the LayerNorm in front of the first step: dx0 = G_1 + LayerNorm'(dn_0), with its dgamma, dbeta
         self._mark("ln_bwd", 0)
@@ -403,7 +401,7 @@ class BodyRunner:
                     self.halo[j % 2].data_ptr() if j else None,
                     *self._grads(j), self.dgamma.data_ptr(), self.dbeta.data_ptr(), dst.data_ptr(),
                     self.sums[j - 1].data_ptr() if j else None, self.B, self.M, self.N, self.K,
-                    self.inner, self.bs, self.act, _n.OVERWRITE_PARAMS if j == last else 0,
+                    self.inner, self.bs, self.act, self._param_flags(j),
                     self.fb_ws.data_ptr(), self.fb_ws_bytes, stream))
                 self._mark("step_bwd", 1)
                 g = dst
@@ -415,7 +413,7 @@ class BodyRunner:
                 self.stats[j].data_ptr(), self.sums[j].data_ptr(), *self._grads(j), self.dgamma.data_ptr(),
                 self.dbeta.data_ptr(), dst.data_ptr(), self.sums[j - 1].data_ptr() if j else None,
                 self.B, self.M, self.N, self.K, self.inner, self.bs, self.act,
-                _n.OVERWRITE_PARAMS if j == last else 0, self.fb_ws.data_ptr(), self.fb_ws_bytes,
+                self._param_flags(j), self.fb_ws.data_ptr(), self.fb_ws_bytes,
                 stream))
             self._mark("step_bwd", 1)
             g = dst
@@ -443,7 +441,6 @@ class BodyRunner:
         """Backward of the last ``forward``.  Returns (dweight, dbias, dscale, dgamma, dbeta, dx0);
         parameter gradients are summed over the outer steps (shared parameters)."""
         assert self.has_backward
-        self._zero_separate_grads()
         if self.outer_residual:
             return self._residual_backward(grad_out)
         if self.fused:
@@ -466,7 +463,8 @@ class BodyRunner:
                 self.dt, *self._params(j),
                 (self.h[j] if j else self.x0).data_ptr(), self.ga.data_ptr(), *self._grads(j),
                 self.gb.data_ptr(), self.B, self.M, self.N, self.K, self.inner,
-                self.bs, self.eps, self.normalize, self.act, flags | _n.OVERWRITE_DX,
+                self.bs, self.eps, self.normalize, self.act,
+                _n.OVERWRITE if self.separate else flags | _n.OVERWRITE_DX,
                 self.bw_ws.data_ptr(), self.bw_ws_bytes, stream))
             self._mark("step_bwd", 1)
             g = self.gb

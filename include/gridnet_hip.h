@@ -60,7 +60,10 @@ enum gridnet_flags {
      * initialised: it is fully written. */
     GRIDNET_OVERWRITE_PARAMS = 1, /* dweight, dbias, dscale (LayerNorm: dgamma, dbeta) */
     GRIDNET_OVERWRITE_DX = 2,     /* dx (LayerNorm: dx is always fully written) */
-    GRIDNET_OVERWRITE = 3
+    GRIDNET_OVERWRITE = 3,
+    /* gridnet_hip_fused_backward[_residual], gridnet_hip_chain_backward: dweight, dbias, dscale are
+     * written, dgamma and dbeta accumulated (steps with parameters of their own around one LayerNorm) */
+    GRIDNET_OVERWRITE_STEP_PARAMS = 4
 };
 
 /* Library build id (monotonic integer) -- lets a binding check it loaded what it expects. */

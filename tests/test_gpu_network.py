@@ -322,3 +322,52 @@ def test_two_streams_in_flight_do_not_disturb_each_other():
             # no atomics anywhere (64 blocks < CUs: the batch is split over workgroups, each chunk
             # has its own copy of the gradient arrays): bit for bit the same
             assert torch.equal(got, want), f"stream {i} output {j}"
+
+
+@pytest.mark.parametrize("shape,bs,batch,inner,kw", [
+    ((16, 16, 16), 8, 6, 2, {}),                  # the batch of a block in several chunks
+    ((16, 16, 24), 4, 5, 1, {}),                  # one inner iteration: by rows
+    ((56, 64, 64), 8, 2, 2, {}),                  # a workgroup per block
+    ((56, 64, 64), 8, 2, 1, {}),
+    ((56, 64, 64), 8, 2, 1, {"outer_residual": True}),
+    ((56, 64, 64), 8, 2, 2, {"outer_residual": True}),
+    ((56, 64, 64), 8, 2, 2, {"chain": True}),
+    ((16, 16, 16), 8, 6, 2, {"chain": True}),
+])
+def test_gradients_of_separate_parameters_are_written(shape, bs, batch, inner, kw):
+    """dweight, dbias and dscale of every step are written whatever their buffers held; dgamma and
+    dbeta, shared by the steps, are summed."""
+    from gridnet_amd.runner import BodyRunner
+    from oracle.fast import gridnet_step_fast
+
+    g = torch.Generator().manual_seed(21)
+    rn = lambda *s: torch.randn(*s, generator=g)
+    outer = 3
+    sets = [[0.19 * rn(27, *shape) for _ in range(outer)], [0.1 * rn(*shape) for _ in range(outer)],
+            [1 + 0.1 * rn(*shape) for _ in range(outer)]]
+    gamma, beta = 1 + 0.2 * rn(*shape), 0.2 * rn(*shape)
+    x, gy = rn(batch, *shape), rn(batch, *shape)
+    dev = "cuda:0"
+    run = BodyRunner(*[[t.to(dev) for t in s] for s in sets], gamma.to(dev), beta.to(dev), batch, inner, outer, bs,
+                     "silu", fused=True, **kw)
+    for buf in (run.dw_all, run.db_all, run.dr_all, run.dgamma, run.dbeta):
+        buf.fill_(float("nan"))
+    run.forward(x.to(dev))
+    dws, dbs, drs, dgamma, dbeta, dx = run.backward(gy.to(dev))
+    leaves = [[t.clone().requires_grad_(True) for t in s] for s in sets]
+    norm = [gamma.clone().requires_grad_(True), beta.clone().requires_grad_(True)]
+    h = x0 = x.clone().requires_grad_(True)
+    for j in range(outer):
+        step = lambda t: gridnet_step_fast(*(s[j] for s in leaves), t, inner, bs, 1e-5, False, "silu")
+        ln = lambda t: torch.nn.functional.layer_norm(t, shape, *norm)
+        if kw.get("outer_residual"):
+            n = ln(h)
+            h = h + (step(n) - n)
+        else:
+            h = ln(step(h))
+    h.backward(gy)
+    for j in range(outer):
+        for what, got, want in (("dweight", dws, leaves[0]), ("dbias", dbs, leaves[1]), ("dscale", drs, leaves[2])):
+            assert_close(got[j], want[j].grad, rtol=2e-4, atol=2e-5, what=f"{what}[{j}]")
+    for what, got, want in (("dgamma", dgamma, norm[0]), ("dbeta", dbeta, norm[1]), ("dx", dx, x0)):
+        assert_close(got, want.grad, rtol=2e-4, atol=2e-5, what=what)

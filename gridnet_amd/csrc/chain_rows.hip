@@ -13,7 +13,7 @@
 //   * The weight gradients come from the same stencil over delta: x[c] delta[c + off_t] is the gradient
 //     of the neighbour's weight 26 - t, and no other cell contributes to it.
 //   * Where the batch is split over workgroups every chunk keeps ONE copy of the gradient arrays for the
-//     whole chain, each step adding to what the step before left; the copies are added up once.
+//     whole chain, each step adding its sums to what the step before left; the copies are added up once.
 // (The pairs per wave behind the LayerNorms' per-sample numbers are merged by small kernels between the
 // steps, 4.7 us each.  Merged by the workgroups that need them, one wave an element ahead, they cost
 // the kernels 11 us forward and 24 us backward: everybody waits for that wave at the barrier.)
@@ -366,16 +366,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     };
     load_planes(a.weight, v);
-    if (a.accumulate) {
-        load_planes(dweight, nv);
-    } else {
+    // a step's sums start from zero, also where there is something to add them to (see the end)
 #pragma unroll
-        for (int k = 0; k < SETS; ++k)
+    for (int k = 0; k < SETS; ++k)
 #pragma unroll
-            for (int t = 0; t < 27; ++t)
+        for (int t = 0; t < 27; ++t)
 #pragma unroll
-                for (int c = 0; c < CPT; ++c) nv[k][t / 3][t % 3][c] = 0.f;
-    }
+            for (int c = 0; c < CPT; ++c) nv[k][t / 3][t % 3][c] = 0.f;
     float gam[CPT], bet[CPT], rv[CPT] = {}, db[SETS][CPT], dr[CPT] = {}, dgam[CPT], dbet[CPT];
     load_cells<CPT>(a.gamma + p.grow, gam);
     load_cells<CPT>(a.beta + p.grow, bet);
@@ -385,13 +382,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         dgam[c] = dbet[c] = 0.f;
 #pragma unroll
         for (int k = 0; k < SETS; ++k) db[k][c] = 0.f;
-    }
-    if (a.accumulate) {
-#pragma unroll
-        for (int k = 0; k < SETS; ++k) load_cells<CPT>(a.dbias + slab + k * cells + p.grow, db[k]);
-        if (SETS == 1) load_cells<CPT>(a.dscale + slab + p.grow, dr);
-        load_cells<CPT>(a.dgamma + slab + p.grow, dgam);
-        load_cells<CPT>(a.dbeta + slab + p.grow, dbet);
     }
 
     // ---- the rows around the tube that this thread moves: number r and, the first four rows, 16 + r ----
@@ -432,7 +422,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int k = 0; k < SETS; ++k) {
                 shift_in(v[k][pq][cc], cc);
-                shift_in(nv[k][pq][cc], cc);
 #pragma unroll
                 for (int c = 0; c < CPT; ++c) v[k][pq][cc][c] *= keep;
                 if (cc == 0 && p.first) v[k][pq][cc][0] = 0.f;
@@ -570,6 +559,27 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (s0 < s1) store_at<CPT>(a.dx + (long)(s1 - 1) * cells, own_off, out);
 
     // ---- parameter gradients: the shifts of the set-up back again, aligned stores of whole rows ----
+    // What the arrays hold is added HERE, once, to the finished sums of this step.  Accumulators that
+    // started from it would take every product of the chain into one running fp32 sum, most of them small
+    // beside it: 64 elements x 64 steps at 32^3, batch 256, left dbias 8e-7 to 5e-6 off the sum in 64 bits, this
+    // way 1e-7 to 5e-7, for 6.69 and 6.60 ms per training step (plain), 9.20 and 9.28 (gated).  The weights are
+    // done with: their registers take the old values, requested in one stretch.
+    float old_db[SETS][CPT] = {}, old_dr[CPT] = {}, old_dgam[CPT] = {}, old_dbet[CPT] = {};
+    if (a.accumulate) {
+        load_planes(dweight, v);
+#pragma unroll
+        for (int k = 0; k < SETS; ++k) load_cells<CPT>(a.dbias + slab + k * cells + p.grow, old_db[k]);
+        if (SETS == 1) load_cells<CPT>(a.dscale + slab + p.grow, old_dr);
+        load_cells<CPT>(a.dgamma + slab + p.grow, old_dgam);
+        load_cells<CPT>(a.dbeta + slab + p.grow, old_dbet);
+    } else {
+#pragma unroll
+        for (int k = 0; k < SETS; ++k)
+#pragma unroll
+            for (int t = 0; t < 27; ++t)
+#pragma unroll
+                for (int c = 0; c < CPT; ++c) v[k][t / 3][t % 3][c] = 0.f;
+    }
 #pragma unroll
     for (int pq = 0; pq < 9; ++pq) {
         const int gi = p.p0 + p.ci + pq / 3 - 1, gj = p.q0 + p.cj + pq % 3 - 1;
@@ -595,10 +605,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 }
                 const int t = pq * 3 + cc;
                 float *to = dweight + (long)((26 - t) * SETS + k) * cells + base;
-                if (row_ok && a.accumulate && ((cc == 0 && p.last) || (cc == 2 && p.first))) {
-                    // the weight that reads outside the grid keeps what its gradient holds
-                    if (CPT == 2) to[cc == 0 ? 0 : CPT - 1] = piece[cc == 0 ? 0 : CPT - 1];
-                } else if (row_ok) {
+                if (row_ok) {
+#pragma unroll
+                    for (int c = 0; c < CPT; ++c) piece[c] += v[k][pq][cc][c];
                     store_cells<CPT>(to, piece);
                 } else if (!a.accumulate) {  // the own weight of tap t reads outside the grid: no gradient
 #pragma unroll
@@ -607,8 +616,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 }
             }
     }
+    auto add = [](float (&to)[CPT], const float (&more)[CPT]) {
 #pragma unroll
-    for (int k = 0; k < SETS; ++k) store_cells<CPT>(a.dbias + slab + k * cells + p.grow, db[k]);
+        for (int c = 0; c < CPT; ++c) to[c] += more[c];
+    };
+    add(dr, old_dr);
+    add(dgam, old_dgam);
+    add(dbet, old_dbet);
+#pragma unroll
+    for (int k = 0; k < SETS; ++k) {
+        add(db[k], old_db[k]);
+        store_cells<CPT>(a.dbias + slab + k * cells + p.grow, db[k]);
+    }
     if (SETS == 1) store_cells<CPT>(a.dscale + slab + p.grow, dr);
     store_cells<CPT>(a.dgamma + slab + p.grow, dgam);
     store_cells<CPT>(a.dbeta + slab + p.grow, dbet);

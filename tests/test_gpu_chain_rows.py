@@ -104,3 +104,120 @@ def test_gated_body(shape, bs, batch, outer):
     once = net.bias.grad.clone()
     y.backward(gy.to(DEV))  # the graph was kept
     assert torch.equal(net.bias.grad, 2 * once)
+
+
+@pytest.mark.parametrize("gated", [False, True], ids=["plain", "gated"])
+def test_old_contents_are_added_once_to_the_finished_sum(gated):
+    """A running sum that starts from the old contents rounds once per element; added to the finished
+    sum they cost one rounding, so the result is exactly fp32(old + sum).  (Batch 5 is not split.)"""
+    from gridnet_amd import native as n
+
+    shape, batch = (8, 8, 32), 5
+    gamma, beta, x, gy = (t.to(DEV) for t in inputs(shape, batch))
+    w, b, r = (t.to(DEV) for t in make_params(shape, seed=4))
+    if gated:
+        w, b = torch.stack([w, w.flip(0)], 1), torch.stack([b, r])
+    saved = torch.empty(3 if gated else 1, *x.shape, device=DEV)
+    y_raw, out, dx, stats = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x), torch.empty(batch, 2, device=DEV)
+    scale = None if gated else r.data_ptr()
+    sizes = (batch, *shape, int(gated), 1)
+    ws = n.workspace(max(n.lib.gridnet_hip_rows_chain_workspace_bytes(*sizes, d) for d in (0, 1)), DEV)
+    n.check(n.lib.gridnet_hip_rows_chain_forward(
+        w.data_ptr(), b.data_ptr(), scale, gamma.data_ptr(), beta.data_ptr(), x.data_ptr(), y_raw.data_ptr(),
+        stats.data_ptr(), saved.data_ptr(), out.data_ptr(), batch, *shape, 1, int(gated), 1e-5,
+        n.activation_id("tanh"), ws.data_ptr(), ws.numel(), n.current_stream(x)))
+
+    def gradients(flags, into):
+        dw, db, dr, dg, dbt = (t.data_ptr() for t in into)
+        n.check(n.lib.gridnet_hip_rows_chain_backward(
+            w.data_ptr(), scale, gamma.data_ptr(), beta.data_ptr(), x.data_ptr(), y_raw.data_ptr(), stats.data_ptr(),
+            saved.data_ptr(), gy.data_ptr(), dw, db, None if gated else dr, dg, dbt, dx.data_ptr(), batch, *shape, 1,
+            int(gated), n.activation_id("tanh"), flags, ws.data_ptr(), ws.numel(), n.current_stream(x)))
+        return into
+
+    like = (w, b, r, gamma, beta)
+    alone = gradients(n.OVERWRITE_PARAMS, [torch.zeros_like(t) for t in like])
+    old = [torch.randn(t.shape, generator=torch.Generator().manual_seed(9)).to(DEV) for t in like]
+    got = gradients(0, [t.clone() for t in old])
+    for name, a, o, g in zip(("dweight", "dbias", "dscale", "dgamma", "dbeta"), got, old, alone):
+        assert torch.equal(a, o + g), name
+
+
+def test_a_chain_adds_each_steps_sum_once():
+    """dbeta of two steps where the second one's gradient is over 1e3 times the first one's: the first step's
+    terms, sequentially summed, are added to the second's in ONE rounding, half an ulp of the result;
+    term by term they would cost one each, fifteen of them.  (256 tubes: the batch is not split.)"""
+    from gridnet_amd.runner import BodyRunner
+    from oracle.network import network_forward_backward
+
+    shape, batch = (64, 64, 16), 15
+    gamma, beta, x, gy = inputs(shape, batch)
+    w, b, r = make_params(shape, seed=4)
+    params = [1e-6 * w, b, 1e5 * r, gamma, beta]  # the raw output varies by the biases, 1e4 times the input
+    run = BodyRunner(*(t.to(DEV) for t in params), batch, 1, 2, 8, "silu", fused=True, forward_all=False)
+    assert run.rows
+    run.forward(x.to(DEV))
+    got = run.backward(gy.to(DEV))[4].cpu()
+    want = network_forward_backward([t.double() for t in params], x.double(), gy.double(), inner_iterations=1,
+                                    outer_iterations=2, block_size=8, activation="silu")[5]
+    last = torch.zeros(shape)
+    for g in gy:  # the kernel's own order
+        last = last + g
+    first = want - gy.double().sum(0)
+    assert first.abs().max() < 1e-2
+    total = last.double() + first
+    # one rounding, and what fp32 leaves on the first step's gradient
+    bound = 2.0 ** -24 * total.abs() + 2e-4 * first.abs() + 1e-9
+    off = (got.double() - total).abs()
+    assert (off <= bound).all(), f"{int((off > bound).sum())} of {off.numel()}, worst {(off / bound).max():.1f} bounds"
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_gated_chain_at_the_scripts_defaults_is_as_exact_as_torch(seed):
+    """32^3, batch 256, 64 steps, the gradient from the last layer only: against the same chain in fp64
+    by torch's operators, this one and torch's own in fp32.  How well such a chain is conditioned
+    depends on its parameters (over seeds both are between 2e-7 and 1e-2 off in the gradients), so what
+    is held is the ratio: two evaluations in fp32, each a random share of the same bound, are seldom four
+    times apart in norm.  1e-7: the rounding of the result itself, 6e-8 at most, on either side."""
+    import torch.nn.functional as F
+
+    from gridnet_amd import GatedGridnet, GridLayerNorm
+    from gridnet_amd.network import gated_body
+    from oracle.gated import gated_step_fast
+
+    shape, batch, outer = (32, 32, 32), 256, 64
+    print(f"gated chain against fp64, seed {seed}", flush=True)
+    rnd = torch.Generator(device=DEV).manual_seed(seed)
+
+    def normal(*size, mean=0.0, std=1.0):
+        return torch.randn(*size, generator=rnd, device=DEV) * std + mean
+
+    params = [normal(27, 2, *shape, std=27 ** -0.5), normal(2, *shape, std=0.1), normal(*shape, mean=1.0, std=0.1),
+              normal(*shape, std=0.1)]
+    x = normal(*shape)[None].repeat(batch, 1, 1, 1)
+    x[..., 0] = torch.rand(batch, *shape[:2], generator=rnd, device=DEV)
+    gy = torch.zeros_like(x)
+    gy[..., -1] = normal(batch, *shape[:2], std=1e-4)
+
+    def by_torch(dtype):
+        leaves = [t.to(dtype).requires_grad_(True) for t in (x, *params)]
+        h = leaves[0]
+        for _ in range(outer):
+            h = F.layer_norm(gated_step_fast(leaves[1], leaves[2], h, 1, 8, "tanh"), shape, leaves[3], leaves[4])
+        h.backward(gy.to(dtype))
+        return [h.detach().double(), *[t.grad.double() for t in leaves]]
+
+    net = GatedGridnet(shape, 1, 8, device=DEV, activation="tanh")
+    norm = GridLayerNorm(shape, device=DEV)
+    with torch.no_grad():
+        for p, t in zip((net.weight, net.bias, norm.weight, norm.bias), params):
+            p.copy_(t)
+    leaf = x.clone().requires_grad_(True)
+    y = gated_body(leaf, net, norm, outer)
+    y.backward(gy)
+    got = [y.detach(), leaf.grad, net.weight.grad, net.bias.grad, norm.weight.grad, norm.bias.grad]
+    exact = by_torch(torch.float64)
+    for name, a, t, e in zip(("y", "dx0", "dweight", "dbias", "dgamma", "dbeta"), got, by_torch(torch.float32), exact):
+        ours, theirs = (((v.double() - e).norm() / e.norm()).item() for v in (a, t))
+        print(f"  {name}: {ours:.2e} off, torch {theirs:.2e}", flush=True)
+        assert ours <= 4 * theirs + 1e-7, name

@@ -6,7 +6,9 @@
 //
 // The functions here take only calls that are in order.  Anything else (a shape, dtype or device
 // that does not fit, an empty batch, host tensors, an unknown activation) makes them return None:
-// the Python operator is then called with the same arguments and raises, or handles it.
+// the Python operator is then called with the same arguments and raises, or handles it.  So does whatever
+// torch does to an autograd.Function and these functions would go round: forward-mode derivatives,
+// function transforms, tracing, dispatch modes, tensor subclasses (see tensor_arg and only_eager).
 //
 // The gradient buffers are handed to the library uninitialised with its overwrite flags; the Python
 // operators' zero fills (four kernels per backward) have nothing to add to.
@@ -15,6 +17,7 @@
 // pybind11's argument casters and torch::autograd::Function's boxed state cost more than the rest.
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -206,12 +209,28 @@ struct WithoutGil {
     ~WithoutGil() { PyEval_RestoreThread(state); }
 };
 
-const Tensor *tensor_arg(PyObject *o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+// Nothing but eager execution and autograd would see this call: no dispatch mode, functorch transform or
+// tracer on this thread.
+bool only_eager() {
+    constexpr c10::DispatchKeySet usual({c10::DispatchKey::BackendSelect, c10::DispatchKey::ADInplaceOrView});
+    return (c10::impl::tls_local_dispatch_key_set().included_ - usual).empty();
+}
+
+// An ordinary device tensor (or Parameter): no subclass, no wrapper of a transform, no lazy negation, and no
+// tangent of forward-mode differentiation, which these operators have no rule for.
+const Tensor *tensor_arg(PyObject *o) {
+    constexpr c10::DispatchKeySet usual({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA,
+                                         c10::DispatchKey::AutocastCUDA, c10::DispatchKey::ADInplaceOrView});
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const Tensor &t = THPVariable_Unpack(o);
+    if (!t.defined() || (t.key_set().raw_repr() & ~usual.raw_repr()) || t._fw_grad(0).defined()) return nullptr;
+    return &t;
+}
 
 // (weight, bias, residual_scale, init_activations, inner, block_size, eps, normalize, activation)
 PyObject *step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 9) Py_RETURN_NONE;
+    if (nargs != 9 || !only_eager()) Py_RETURN_NONE;
     const Tensor *w = tensor_arg(args[0]), *b = tensor_arg(args[1]), *r = tensor_arg(args[2]), *x = tensor_arg(args[3]);
     if (!w || !b || !r || !x || !usable_input(*x) || !goes_with(*w, *x) || !goes_with(*b, *x) || !goes_with(*r, *x) ||
         !shaped(*w, {27}, *x) || !shaped(*b, {}, *x) || !shaped(*r, {}, *x))
@@ -256,7 +275,7 @@ PyObject *step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 // (weight, bias, init_activations, inner, block_size, activation)
 PyObject *gated_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 6) Py_RETURN_NONE;
+    if (nargs != 6 || !only_eager()) Py_RETURN_NONE;
     const Tensor *w = tensor_arg(args[0]), *b = tensor_arg(args[1]), *x = tensor_arg(args[2]);
     if (!w || !b || !x || !usable_input(*x) || !goes_with(*w, *x) || !goes_with(*b, *x) || !shaped(*w, {27, 2}, *x) ||
         !shaped(*b, {2}, *x))
@@ -298,7 +317,7 @@ PyObject *gated_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 // (x, weight, bias, eps)
 PyObject *layer_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 4) Py_RETURN_NONE;
+    if (nargs != 4 || !only_eager()) Py_RETURN_NONE;
     const Tensor *x = tensor_arg(args[0]), *ga = tensor_arg(args[1]), *be = tensor_arg(args[2]);
     if (!x || !ga || !be || !usable_input(*x) || !goes_with(*ga, *x) || !goes_with(*be, *x) || !shaped(*ga, {}, *x) ||
         !shaped(*be, {}, *x))

@@ -82,6 +82,25 @@ def test_host_only_entry_points():
     assert rc == 4 and "workspace" in native.last_error()
 
 
+def test_native_operators_decline_tensors_without_data():
+    """Fake device tensors have no memory behind them: the native operators leave them to the Python ones."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from gridnet_amd import native
+
+    with FakeTensorMode():
+        w, p, x = (torch.empty(*s, 8, 8, 8, device="cuda") for s in ((27,), (), (2,)))
+        gw, gp = torch.empty(27, 2, 8, 8, 8, device="cuda"), torch.empty(2, 8, 8, 8, device="cuda")
+
+        def calls():
+            return (native.ops.step(w, p, p, x, 1, 8, 1e-5, False, "silu"),
+                    native.ops.gated_step(gw, gp, x, 1, 8, "tanh"), native.ops.layer_norm(x, p, p, 1e-5))
+
+        assert calls() == (None, None, None)
+    assert calls() == (None, None, None)  # nor outside the mode
+
+
 def test_shim_has_the_reference_call_surface():
     """Positional signatures of src/gridnet_cuda.cpp:61-72, 91-106, 133-141, 160-171."""
     import gridnet_cuda

@@ -173,18 +173,17 @@ struct GatedNode : public Node {
 };
 
 struct NormNode : public Node {
-    SavedVariable x, gamma;
-    Tensor mean, rstd;
+    SavedVariable x, gamma, mean, rstd;
     std::string name() const override { return "GridLayerNormBackward"; }
     void release_variables() override {
         x.reset_data();
         gamma.reset_data();
-        mean.reset();
-        rstd.reset();
+        mean.reset_data();
+        rstd.reset_data();
     }
     variable_list apply(variable_list &&grads) override {
         if (!grads[0].defined()) return variable_list(3);
-        const Tensor xs = x.unpack(), ga = gamma.unpack();
+        const Tensor xs = x.unpack(), ga = gamma.unpack(), m = mean.unpack(), r = rstd.unpack();
         c10::DeviceGuard guard(xs.device());
         const Tensor g = grads[0].contiguous();
         Tensor dx = fresh(xs), dgamma = fresh(ga), dbeta = fresh(ga);
@@ -192,7 +191,7 @@ struct NormNode : public Node {
         const long n = ga.numel();
         const size_t bytes = lib.layernorm_workspace_bytes(dt, B, n);
         const Tensor ws = workspace(bytes, xs);
-        check(lib.layernorm_backward(dt, g.data_ptr(), xs.data_ptr(), ga.data_ptr(), mean.data_ptr(), rstd.data_ptr(),
+        check(lib.layernorm_backward(dt, g.data_ptr(), xs.data_ptr(), ga.data_ptr(), m.data_ptr(), r.data_ptr(),
                                      dx.data_ptr(), dgamma.data_ptr(), dbeta.data_ptr(), B, n, GRIDNET_OVERWRITE_PARAMS,
                                      ws.data_ptr(), bytes, stream_of(xs)));
         return {dx, dgamma, dbeta};
@@ -347,8 +346,8 @@ PyObject *layer_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
         node->set_next_edges(torch::autograd::collect_next_edges(*x, *ga, *be));
         node->x = SavedVariable(*x, false);
         node->gamma = SavedVariable(*ga, false);
-        node->mean = mean;
-        node->rstd = rstd;
+        node->mean = SavedVariable(mean, false);
+        node->rstd = SavedVariable(rstd, false);
         torch::autograd::set_history(y, node);
     }
     return THPVariable_Wrap(std::move(y));

@@ -124,3 +124,24 @@ def test_tracing_and_subclasses_see_the_operator(which):
         traced = torch.jit.trace(lambda t: native(*tensors[:k], t, *tensors[k + 1:], *rest), tensors[k], check_trace=False)
         other = 2 * tensors[k] + 1
         assert torch.equal(traced(other), python(*tensors[:k], other, *tensors[k + 1:], *rest))
+
+
+@pytest.mark.parametrize("which", [0, 1, 2], ids=["step", "gated", "norm"])
+def test_saved_tensor_hooks_see_everything_that_is_kept(which):
+    native, python, tensors, rest = operators()[which]
+    results = []
+    for f in (native, python):
+        kept = []
+
+        def pack(t):
+            kept.append(tuple(t.shape))
+            return t.cpu()
+
+        leaves = [t.clone().requires_grad_(True) for t in tensors]
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(DEV)):
+            y = f(*leaves, *rest)
+        y.backward(torch.ones_like(y))
+        results.append((kept, [t.grad for t in leaves]))
+    assert results[0][0] == results[1][0]
+    for got, want in zip(results[0][1], results[1][1]):
+        assert torch.equal(got, want)

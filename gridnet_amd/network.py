@@ -139,27 +139,45 @@ class GatedBodyOp(torch.autograd.Function):
         return (*grads, None, None, None)
 
 
-def _bare(module):
-    """No hook would miss a call that goes round ``module.forward``."""
-    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
-                module._backward_pre_hooks)
+_HOOKS = ("forward", "forward_pre", "backward", "backward_pre")
+
+
+def _as_defined(module, cls):
+    """Nothing is passed by where ``module.forward`` is not called: ``cls`` itself and no subclass, no
+    ``forward`` of the instance's own, not compiled, and no hook, its own or for all modules."""
+    hooks = [getattr(module, f"_{kind}_hooks", None) for kind in _HOOKS]
+    hooks += [getattr(nn.modules.module, f"_global_{kind}_hooks") for kind in _HOOKS]
+    return (type(module) is cls and "forward" not in vars(module) and not any(hooks) and
+            getattr(module, "_compiled_call_impl", None) is None)
+
+
+def _rows_cover(h, network, norm, outer_iterations):
+    """Whether :class:`GatedBodyOp` computes what the modules, called one after the other, would."""
+    from . import GatedGridnet
+    from . import native as _n
+    from .layernorm import GridLayerNorm
+
+    if not (_as_defined(network, GatedGridnet) and _as_defined(norm, GridLayerNorm)):
+        return False
+    params = (network.weight, network.bias, norm.weight, norm.bias)
+    if outer_iterations < 1 or not (h.is_cuda and h.is_contiguous() and h.dim() == 4 and h.shape[0]):
+        return False
+    shape = tuple(h.shape[1:])
+    if not all(isinstance(t, torch.Tensor) and t.is_contiguous() and t.dtype == h.dtype == torch.float32 and
+               t.device == h.device for t in params):
+        return False
+    return (tuple(t.shape for t in params) == ((27, 2, *shape), (2, *shape), shape, shape) and
+            network.block_size in (4, 8) and not any(n % network.block_size for n in shape) and
+            bool(_n.lib.gridnet_hip_rows_chain_supported(_n.F32, *shape, network.inner_iterations, 0, 1)))
 
 
 def gated_body(h, network, norm, outer_iterations: int):
     """``outer_iterations`` x (``network``, ``norm``) on ``h``: a :class:`gridnet_amd.GatedGridnet` and a
     :class:`gridnet_amd.GridLayerNorm`, through :class:`GatedBodyOp` where that covers the problem and one
     after the other where it does not."""
-    from . import native as _n
-
-    params = (network.weight, network.bias, norm.weight, norm.bias)
-    shape = tuple(network.bias.shape[1:])
-    if (outer_iterations >= 1 and h.is_cuda and h.shape[0] > 0 and tuple(h.shape[1:]) == shape and
-            h.dtype == torch.float32 and _bare(network) and _bare(norm) and
-            network.block_size in (4, 8) and not any(n % network.block_size for n in shape) and
-            network.weight.shape == (27, 2, *shape) and norm.weight.shape == shape and norm.bias.shape == shape and
-            all(t.is_contiguous() and t.dtype == h.dtype and t.device == h.device for t in params) and
-            _n.lib.gridnet_hip_rows_chain_supported(_n.F32, *shape, network.inner_iterations, 0, 1)):
-        return GatedBodyOp.apply(h, *params, outer_iterations, network.activation, norm.eps)
+    if _rows_cover(h, network, norm, outer_iterations):
+        return GatedBodyOp.apply(h, network.weight, network.bias, norm.weight, norm.bias, outer_iterations,
+                                 network.activation, norm.eps)
     for _ in range(outer_iterations):
         h = norm(network(h))
     return h

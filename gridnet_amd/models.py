@@ -51,6 +51,7 @@ class MnistGridModel(nn.Module):
         if fused_body and gated:
             raise ValueError("the fused body covers the plain (not gated) network only")
         self.fused_body = fused_body
+        self.rows = None  # the gated loop as one node, see gated_body: None where there is room, False never
         self.outer_iters = outer_iters
         self.device = device
         self.init_in = nn.Parameter(torch.randn(32, 32, 32, device=device))
@@ -77,7 +78,7 @@ class MnistGridModel(nn.Module):
         if self.fused_body:
             return self.readout(fused_body(h, self.network, self.norm, self.outer_iters))
         if isinstance(self.network, GatedGridnet):
-            return self.readout(gated_body(h, self.network, self.norm, self.outer_iters))
+            return self.readout(gated_body(h, self.network, self.norm, self.outer_iters, self.rows))
         for _ in range(self.outer_iters):
             h = self.norm(self.network(h))
         return self.readout(h)

@@ -89,7 +89,8 @@ def fused_body(h, network, norm, outer_iterations: int, outer_residual: bool = F
 class GatedBodyOp(torch.autograd.Function):
     """The loop over a gated step with one inner iteration and its LayerNorm as one autograd node, on
     ``gridnet_hip_rows_chain_*``: a kernel per step and direction, the LayerNorm and the accumulation of
-    the shared parameters' gradients inside them."""
+    the shared parameters' gradients inside them.  It keeps four tensors per step for the backward where
+    the modules one after the other keep two (8.6 GB at 32^3, batch 256, 64 steps)."""
 
     @staticmethod
     def forward(ctx, x0, weight, bias, gamma, beta, outer_iterations, activation, eps):
@@ -171,11 +172,16 @@ def _rows_cover(h, network, norm, outer_iterations):
             bool(_n.lib.gridnet_hip_rows_chain_supported(_n.F32, *shape, network.inner_iterations, 0, 1)))
 
 
-def gated_body(h, network, norm, outer_iterations: int):
+def gated_body(h, network, norm, outer_iterations: int, rows=None):
     """``outer_iterations`` x (``network``, ``norm``) on ``h``: a :class:`gridnet_amd.GatedGridnet` and a
-    :class:`gridnet_amd.GridLayerNorm`, through :class:`GatedBodyOp` where that covers the problem and one
-    after the other where it does not."""
-    if _rows_cover(h, network, norm, outer_iterations):
+    :class:`gridnet_amd.GridLayerNorm`, through :class:`GatedBodyOp` where that covers the problem and, with
+    a backward to come, there is room for what it keeps (``rows=True``: without asking for room; ``False``:
+    never); one after the other where not."""
+    from .runner import room_for
+
+    if rows is not False and _rows_cover(h, network, norm, outer_iterations) and (
+            rows or not torch.is_grad_enabled() or
+            room_for(4 * outer_iterations * h.numel() * h.element_size(), h.device)):
         return GatedBodyOp.apply(h, network.weight, network.bias, norm.weight, norm.bias, outer_iterations,
                                  network.activation, norm.eps)
     for _ in range(outer_iterations):

@@ -33,8 +33,9 @@ forward of a chain with one parameter set is one launch too (``gridnet_hip_chain
 ``forward_all=False``: never).
 
 With one inner iteration per step, one parameter set and rows of 16, 32 or 64 cells a chain takes one kernel per
-step and direction (``gridnet_hip_rows_chain_*``; ``rows=False``: never); its forward keeps the
-pre-activations as well, one more tensor per step.
+step and direction (``gridnet_hip_rows_chain_*``).  Its forward keeps the pre-activations as well, one more
+tensor per step, so with a backward ``rows=None`` takes it where there is room for them (``room_for``);
+``True``: wherever the library supports it, ``False``: never.
 
 ``weight``, ``bias`` and ``scale`` may each be a list of ``outer`` tensors: one parameter set
 per outer step (the reference's ``--separate_params``, gridnet/scripts/train_imagenet.py:54-58).
@@ -48,6 +49,22 @@ per outer step (the reference's ``--separate_params``, gridnet/scripts/train_ima
 import torch
 
 from . import native as _n
+
+
+UNASKED = 1 / 128  # share of the device's memory, see room_for
+
+
+def room_for(nbytes: int, device) -> bool:
+    """Whether a chain may keep ``nbytes`` for its backward where a slower one would keep half of it: they
+    take at most half of the memory that is free, on the device or in torch's cache.  What the program
+    allocates until the backward has run then has as much again, and a batch that the slower chain leaves
+    room for is not refused.  Little (2.3 GB of 288) is taken without asking the driver."""
+    if nbytes <= UNASKED * torch.cuda.get_device_properties(device).total_memory:
+        return True
+    free = torch.cuda.mem_get_info(device)[0]
+    if 2 * nbytes > free and not torch.cuda.is_current_stream_capturing():  # a capture has a pool of its own
+        free += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    return 2 * nbytes <= free
 
 
 class BodyRunner:
@@ -91,7 +108,8 @@ class BodyRunner:
         self.rows = bool(
             fused and not outer_residual and not self.separate and rows is not False and
             not (backward and (chain or chain_all)) and
-            _n.lib.gridnet_hip_rows_chain_supported(self.dt, self.M, self.N, self.K, inner, self.normalize, 0))
+            _n.lib.gridnet_hip_rows_chain_supported(self.dt, self.M, self.N, self.K, inner, self.normalize, 0) and
+            (rows or not backward or room_for(2 * outer * batch * n * weight.element_size(), dev)))
         n_h, n_s = keep + 1, keep
         if fused and not outer_residual:
             whole = self.forward_all or self.rows  # keep the values between the steps themselves

@@ -92,3 +92,37 @@ def test_another_norm_and_a_strided_input():
     h = m.embed(x).transpose(1, 2)
     with pytest.raises(RuntimeError, match="must be contiguous"):
         gated_body(h, m.network, m.norm, 2)
+
+
+def test_without_room_the_shorter_history_is_kept(monkeypatch):
+    """The loop by whole rows keeps twice the tensors: where they would take more than half of what is
+    free, and where it is told not to, the modules (plain: the two-kernel chain) run, with the same results."""
+    from gridnet_amd import runner
+
+    m, x = model(), images()
+    want = m(x)
+    m.rows = False
+    assert "GatedBodyOpBackward" not in nodes(m(x))
+    m.rows = None
+    params = [torch.ones(n, 8, 8, 16, device=DEV).squeeze(0) / 9 for n in (27, 1, 1, 1, 1)]
+    acts = torch.randn(2, 8, 8, 16, generator=torch.Generator().manual_seed(2)).to(DEV)
+    plain = runner.BodyRunner(*params, 2, 1, 3, 8, "silu", fused=True)
+    assert plain.rows
+
+    monkeypatch.setattr(runner, "UNASKED", 0)
+    need = 4 * m.outer_iters * x.shape[0] * 32 ** 3 * 4
+    for free, fits in ((3 * need, True), (need, False)):
+        cached = torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (free - cached, 0))
+        y = m(x)
+        assert ("GatedBodyOpBackward" in nodes(y)) == fits
+        torch.testing.assert_close(y, want, rtol=1e-5, atol=1e-5)
+    with torch.no_grad():  # nothing is kept
+        assert torch.equal(m(x), want)
+    monkeypatch.setattr(runner, "room_for", lambda nbytes, device: False)
+    short = runner.BodyRunner(*params, 2, 1, 3, 8, "silu", fused=True)
+    assert not short.rows and runner.BodyRunner(*params, 2, 1, 3, 8, "silu", fused=True, rows=True).rows
+    assert runner.BodyRunner(*params, 2, 1, 3, 8, "silu", fused=True, backward=False).rows
+    torch.testing.assert_close(short.forward(acts), plain.forward(acts), rtol=1e-5, atol=1e-5)
+    for a, b in zip(short.backward(acts), plain.backward(acts)):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5)

@@ -112,7 +112,6 @@ struct ChainBwdArgs {
     float *out2;               // DEFER: halo_out [B, nblk, 488]; otherwise D [B, cells]
     float *x_part;             // DEFER: [B, nblk, 2] sums for the LayerNorm in front of this step
     int B, M, N, K, inner, nblk, nchunk, chunk_len, param_mode;
-    int norm_accumulate;       // dgamma and dbeta are added to what is there, whatever param_mode says
     long slab_stride;          // split batch: floats between the chunks' copies of the gradient arrays, else 0
     // ---- ALL: every step of the chain in one launch (see chain_bwd) ----
     // y_raw and y_stats then point at step 0's and the steps lie step_floats / 2 B floats apart;
@@ -412,20 +411,20 @@ void chain_bwd(const ChainBwdArgs a) {
     // delta windows: the halo stays zero for the whole kernel
     for (int idx = tid; idx < 2 * TL::WIN; idx += 256) dwin[idx] = 0.f;
     wait_global_loads();
-    if (a.param_mode == kParamAddExclusive) {
+    if (a.param_mode != kParamStore) {  // (one branch, as in step_bwd_fast)
         const long slab_off = slab_offset();
         // the accumulators start from what the gradient buffers hold and are stored at the end;
         // requested here, behind the set-up wait, the old values arrive during the first element
+        if (a.param_mode == kParamAddExclusive) {
 #pragma unroll
-        for (int t = 0; t < 27; ++t)
+            for (int t = 0; t < 27; ++t)
 #pragma unroll
-            for (int c = 0; c < CPT; ++c) nw[t][c] = (a.dweight + slab_off)[owner_of(t, c)];
-        load_cells<CPT>((a.dbias + slab_off) + pl.gc, db);
-        load_cells<CPT>((a.dscale + slab_off) + pl.gc, dr);
-    }
-    if (a.norm_accumulate) {
-        load_cells<CPT>((a.dgamma + slab_offset()) + pl.gc, dgam);
-        load_cells<CPT>((a.dbeta + slab_offset()) + pl.gc, dbet);
+                for (int c = 0; c < CPT; ++c) nw[t][c] = (a.dweight + slab_off)[owner_of(t, c)];
+            load_cells<CPT>((a.dbias + slab_off) + pl.gc, db);
+            load_cells<CPT>((a.dscale + slab_off) + pl.gc, dr);
+        }
+        load_cells<CPT>((a.dgamma + slab_off) + pl.gc, dgam);
+        load_cells<CPT>((a.dbeta + slab_off) + pl.gc, dbet);
     }
     auto acc_ref = [&](int k) -> float & { return reinterpret_cast<float *>(ctab)[(kTabAcc + k) * 256 + tid]; };
 #pragma unroll
@@ -924,7 +923,6 @@ template <int ACT, bool DEFER, bool WIDE> int launch_chain(const StepArgs &a, hi
     // a workgroup: plain stores for the parameter gradients, bitwise reproducible
     const bool whole = k.nblk >= plan_device_cus();
     plan_batch_chunks(a.B, k.nblk, 1, per_cu * plan_device_cus(), whole, k.nchunk, k.chunk_len);
-    const bool new_params = (a.flags & (GRIDNET_OVERWRITE_PARAMS | GRIDNET_OVERWRITE_STEP_PARAMS)) != 0;
     // A split batch: every chunk gets a copy of the gradient arrays in the scratch; with less
     // room than chunks the batch is split less (down to not at all).
     const long slab_floats = kStepSlabPlanes * cells;
@@ -934,8 +932,7 @@ template <int ACT, bool DEFER, bool WIDE> int launch_chain(const StepArgs &a, hi
             plan_batch_chunks(a.B, k.nblk, 1, (room < 2 ? 1 : room) * k.nblk, room < 2, k.nchunk, k.chunk_len);
     }
     const bool split = k.nchunk > 1;
-    k.param_mode = split || new_params ? kParamStore : kParamAddExclusive;
-    k.norm_accumulate = !split && !(a.flags & GRIDNET_OVERWRITE_PARAMS);
+    k.param_mode = plan_param_mode(split, a.flags);
     k.slab_stride = split ? slab_floats : 0;
     float *slab = (float *)a.slabs;
     k.weight = (const float *)a.weight; k.bias = (const float *)a.bias; k.scale = (const float *)a.scale;
@@ -1061,7 +1058,6 @@ template <int ACT, bool WIDE> int launch_chain_all(const ChainAll &c, hipStream_
     k.nchunk = 1;
     k.chunk_len = c.B;
     k.param_mode = (c.flags & GRIDNET_OVERWRITE_PARAMS) ? kParamStore : kParamAddExclusive;
-    k.norm_accumulate = k.param_mode == kParamAddExclusive;
     k.weight = c.weight; k.bias = c.bias; k.scale = c.scale; k.gamma = c.gamma; k.beta = c.beta;
     k.x0 = c.x0; k.y_raw = c.y_raw; k.y_stats = c.stats; k.sums = (float *)(ws + l.sums_at); k.dy = c.dy;
     k.dweight = c.dweight; k.dbias = c.dbias; k.dscale = c.dscale; k.dgamma = c.dgamma; k.dbeta = c.dbeta;

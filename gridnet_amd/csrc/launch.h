@@ -23,7 +23,7 @@ struct LnFold {
     const float *y_stats;       // [B,2]
     const float *y_sums;        // [B,2]: mean(g), mean(g * yhat) with g = gamma * incoming gradient
     float *dgamma, *dbeta;      // [M,N,K], summed over the batch
-    int accumulate;             // they are added to what is there, whatever dbias is (set by the launcher)
+    int accumulate;             // bwd_rows: they are added to what is there, whatever dbias is (set by the launcher)
     float *x_part;              // partial sums for the LayerNorm backward of x: [B, nblk, parts, 2]
     float *x_sums;              // [B,2] or null: where a backward that finishes the sums itself leaves them
                                 // (bwd_rows_leaves_sums); otherwise the caller finalizes x_part
@@ -80,7 +80,8 @@ constexpr int kGatedSlabPlanes = 56;
 enum ParamMode {
     kParamStore = 0,         // sole owner of the cells, output uninitialised: plain store
     kParamAddExclusive = 1,  // sole owner, output holds a prior sum: read-add-write
-    kParamAtomic = 2         // several workgroups (batch chunks) share the cells (generic kernels only)
+    kParamAtomic = 2,        // several workgroups (batch chunks) share the cells (generic kernels only)
+    kParamAddNorms = 3       // sole owner: dgamma and dbeta are added to what is there, the rest is stored
 };
 
 // The caller's gradient arrays and where each ends within one copy of them (see plan.h)

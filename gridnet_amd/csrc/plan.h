@@ -156,6 +156,12 @@ int plan_accumulate_mask(int flags) {
     return (flags & GRIDNET_OVERWRITE_STEP_PARAMS) ? 8 | 16 : ~0;
 }
 
+// The same for a backward that is not split (a split one stores into its copies).
+int plan_param_mode(bool split, int flags) {
+    if (split || (flags & GRIDNET_OVERWRITE_PARAMS)) return kParamStore;
+    return (flags & GRIDNET_OVERWRITE_STEP_PARAMS) ? kParamAddNorms : kParamAddExclusive;
+}
+
 // `nthreads`: threads per workgroup of the kernel that will run the job.  Its workgroups take as
 // many vectors per thread as keeps them below the number the chip holds.
 TailJob plan_tail_job(const float *slabs, int ncopies, long stride, const SlabTargets &t, int accumulate,

@@ -48,8 +48,8 @@ def build_torch_ops(out: str, verbose: bool) -> None:
 
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     includes = [*include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", *(f"-I{p}" for p in includes),
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", *(a for p in includes for a in ("-isystem", p)),
            os.path.join(CSRC, TORCH_OPS_SOURCE), "-o", out, *(f"-L{p}" for p in library_paths()),
            "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ldl"]
     if verbose:

@@ -100,7 +100,10 @@ using namespace gridnet;
 
 extern "C" {
 
-int gridnet_hip_version(void) { return 8; }  // 2: fused body; 3: residual forward and backward; 4: gated backward takes a workspace; 5: backward on static scratch; 6: chain backward, gradient copies for split batches; 7: whole chain in one launch; 8: fused forward with flags
+// 2: fused body; 3: residual forward and backward; 4: gated backward takes a workspace; 5: backward on static
+// scratch; 6: chain backward, gradient copies for split batches; 7: whole chain in one launch; 8: fused
+// forward with flags; 9: forward of a chain in one launch, chains by whole rows, GRIDNET_OVERWRITE_STEP_PARAMS
+int gridnet_hip_version(void) { return GRIDNET_HIP_VERSION; }
 
 const char *gridnet_hip_last_error(void) { return error_buffer(); }
 

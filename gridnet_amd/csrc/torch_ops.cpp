@@ -42,6 +42,7 @@ using torch::autograd::variable_list;
 // The library is bound by path and not by linking: the same file that the ctypes binding loaded
 // (the caller may have pointed it at another build), and so the same error buffer.
 struct Library {
+    decltype(&gridnet_hip_version) version;
     decltype(&gridnet_hip_last_error) last_error;
     decltype(&gridnet_hip_forward) forward;
     decltype(&gridnet_hip_backward_workspace_bytes) backward_workspace_bytes;
@@ -226,10 +227,14 @@ const Tensor *tensor_arg(PyObject *o) {
     return &t;
 }
 
+// Another number of arguments is no call to decline but another build than the Python files'.
+constexpr char kArguments[] = "%s takes %d arguments, got %zd (a stale _torch_ops.so?)";
+
 // (weight, bias, residual_scale, init_activations, inner, block_size, eps, normalize, activation)
 PyObject *step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 9 || !only_eager()) Py_RETURN_NONE;
+    if (nargs != 9) return PyErr_Format(PyExc_TypeError, kArguments, "step", 9, nargs);
+    if (!only_eager()) Py_RETURN_NONE;
     const Tensor *w = tensor_arg(args[0]), *b = tensor_arg(args[1]), *r = tensor_arg(args[2]), *x = tensor_arg(args[3]);
     if (!w || !b || !r || !x || !usable_input(*x) || !goes_with(*w, *x) || !goes_with(*b, *x) || !goes_with(*r, *x) ||
         !shaped(*w, {27}, *x) || !shaped(*b, {}, *x) || !shaped(*r, {}, *x))
@@ -274,7 +279,8 @@ PyObject *step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 // (weight, bias, init_activations, inner, block_size, activation)
 PyObject *gated_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 6 || !only_eager()) Py_RETURN_NONE;
+    if (nargs != 6) return PyErr_Format(PyExc_TypeError, kArguments, "gated_step", 6, nargs);
+    if (!only_eager()) Py_RETURN_NONE;
     const Tensor *w = tensor_arg(args[0]), *b = tensor_arg(args[1]), *x = tensor_arg(args[2]);
     if (!w || !b || !x || !usable_input(*x) || !goes_with(*w, *x) || !goes_with(*b, *x) || !shaped(*w, {27, 2}, *x) ||
         !shaped(*b, {2}, *x))
@@ -316,7 +322,8 @@ PyObject *gated_step(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
 // (x, weight, bias, eps)
 PyObject *layer_norm(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    if (nargs != 4 || !only_eager()) Py_RETURN_NONE;
+    if (nargs != 4) return PyErr_Format(PyExc_TypeError, kArguments, "layer_norm", 4, nargs);
+    if (!only_eager()) Py_RETURN_NONE;
     const Tensor *x = tensor_arg(args[0]), *ga = tensor_arg(args[1]), *be = tensor_arg(args[2]);
     if (!x || !ga || !be || !usable_input(*x) || !goes_with(*ga, *x) || !goes_with(*be, *x) || !shaped(*ga, {}, *x) ||
         !shaped(*be, {}, *x))
@@ -368,6 +375,10 @@ PyObject *bind(PyObject *, PyObject *path) {
     if (!h) return PyErr_Format(PyExc_ImportError, "cannot load %s: %s", file, dlerror());
 #define GRIDNET_FIND(member) \
     if (!find(h, "gridnet_hip_" #member, lib.member)) return nullptr
+    GRIDNET_FIND(version);
+    if (lib.version() != GRIDNET_HIP_VERSION)  // built against another header than the library
+        return PyErr_Format(PyExc_ImportError, "%s has version %d of the C ABI, _torch_ops.so was built for %d", file,
+                            lib.version(), GRIDNET_HIP_VERSION);
     GRIDNET_FIND(last_error);
     GRIDNET_FIND(forward);
     GRIDNET_FIND(backward_workspace_bytes);

@@ -67,6 +67,7 @@ enum gridnet_flags {
 };
 
 /* Library build id (monotonic integer) -- lets a binding check it loaded what it expects. */
+#define GRIDNET_HIP_VERSION 9
 int gridnet_hip_version(void);
 
 /* Thread-local message of the last non-zero status returned on this thread ("" if none). */

@@ -101,6 +101,24 @@ def test_native_operators_decline_tensors_without_data():
     assert calls() == (None, None, None)  # nor outside the mode
 
 
+def test_native_operators_and_library_of_different_builds_do_not_go_together(tmp_path):
+    import subprocess
+
+    from gridnet_amd import native
+
+    for op in (native.ops.step, native.ops.gated_step, native.ops.layer_norm):
+        with pytest.raises(TypeError, match="stale"):
+            op(1, 2)
+    other = tmp_path / "other.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-x", "c", "-", "-o", str(other)], check=True,
+                   input=b"int gridnet_hip_version(void) { return 8; }")
+    with pytest.raises(ImportError, match="version 8 of the C ABI"):
+        try:
+            native.ops.bind(str(other))
+        finally:
+            native.ops.bind(native.LIB_PATH)
+
+
 def test_shim_has_the_reference_call_surface():
     """Positional signatures of src/gridnet_cuda.cpp:61-72, 91-106, 133-141, 160-171."""
     import gridnet_cuda

@@ -651,7 +651,7 @@ int gridnet_hip_chain_forward_all(int dtype, const void *weight, const void *bia
     c.y_all = (float *)y_raw; c.stats = (float *)stats; c.out = (float *)out;
     c.B = B; c.M = M; c.N = N; c.K = K; c.inner = inner; c.outer = outer; c.activation = activation;
     c.eps = ln_eps;
-    c.workspace = workspace; c.workspace_bytes = workspace_bytes;
+    c.workspace = workspace;
     c.spin_limit = chain_spin_limit;
     const size_t need = chain_fwd_workspace(c);
     if (!workspace || workspace_bytes < need)
@@ -778,7 +778,7 @@ int gridnet_hip_chain_backward_all(int dtype, const void *weight, const void *bi
     c.dgamma = (float *)dgamma; c.dbeta = (float *)dbeta; c.dx = (float *)dx;
     c.B = B; c.M = M; c.N = N; c.K = K; c.inner = inner; c.outer = outer;
     c.activation = activation; c.flags = flags;
-    c.workspace = workspace; c.workspace_bytes = workspace_bytes;
+    c.workspace = workspace;
     c.spin_limit = chain_spin_limit;
     const size_t need = chain_all_workspace(c);
     if (!workspace || workspace_bytes < need)

@@ -649,25 +649,13 @@ template <typename K> int workgroups_per_cu(K kern, int threads, size_t lds) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)kern, threads, lds) != hipSuccess || n < 1) n = 1;
     return n;
 }
-template <typename K> int allow_lds(K kern, size_t lds) {
-    if (lds > 64 * 1024 &&
-        hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(GRIDNET_ERR_LAUNCH, "chain_rows: cannot enable %zu bytes of LDS", lds);
-    }
-    return GRIDNET_OK;
-}
-
 template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &c, hipStream_t st) {
     auto kern = rows_fwd<ACT, SETS, SAVE, K>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
     const int ntube = tubes_of(c), nt = fwd_threads(c), pairs = fwd_pairs(c);
     const size_t lds = 4 * (size_t)kWinRows * c.K * sizeof(float);
     static int per_cu = 0;  // per instantiation
-    if (per_cu == 0) {
-        if (int rc = allow_lds(kern, lds)) return rc;
-        per_cu = workgroups_per_cu(kern, nt, lds);
-    }
+    if (per_cu == 0) per_cu = workgroups_per_cu(kern, nt, lds);
     RowsFwdArgs a{};
     a.nchunk = plan_row_chunks(c.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, a.chunk_len);
     a.weight = c.weight; a.bias = c.bias; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
@@ -799,12 +787,15 @@ template <int SETS, bool SAVE> int forward_act(const RowsChain &c, hipStream_t s
 }
 // The gated backward works on saved factors: no activation in it.
 template <int SETS> int backward_act(const RowsChain &c, hipStream_t st) {
-    if constexpr (SETS == 2) return backward_rows<GRIDNET_ACT_RELU, SETS>(c, st);
-    switch (c.activation) {
-        case GRIDNET_ACT_RELU: return backward_rows<GRIDNET_ACT_RELU, SETS>(c, st);
-        case GRIDNET_ACT_LEAKY_RELU: return backward_rows<GRIDNET_ACT_LEAKY_RELU, SETS>(c, st);
-        case GRIDNET_ACT_SILU: return backward_rows<GRIDNET_ACT_SILU, SETS>(c, st);
-        case GRIDNET_ACT_TANH: return backward_rows<GRIDNET_ACT_TANH, SETS>(c, st);
+    if constexpr (SETS == 2) {
+        return backward_rows<GRIDNET_ACT_RELU, SETS>(c, st);
+    } else {
+        switch (c.activation) {
+            case GRIDNET_ACT_RELU: return backward_rows<GRIDNET_ACT_RELU, SETS>(c, st);
+            case GRIDNET_ACT_LEAKY_RELU: return backward_rows<GRIDNET_ACT_LEAKY_RELU, SETS>(c, st);
+            case GRIDNET_ACT_SILU: return backward_rows<GRIDNET_ACT_SILU, SETS>(c, st);
+            case GRIDNET_ACT_TANH: return backward_rows<GRIDNET_ACT_TANH, SETS>(c, st);
+        }
     }
     return fail(GRIDNET_ERR_ACTIVATION, "unknown activation function: id %d", c.activation);
 }

@@ -207,7 +207,6 @@ struct ChainAll {
     float *dweight, *dbias, *dscale, *dgamma, *dbeta, *dx;
     int B, M, N, K, inner, outer, activation, flags;
     void *workspace;
-    size_t workspace_bytes;
     int spin_limit;  // polls before a wait gives up; negative: ready words are never set (tests of the give-up path)
 };
 bool chain_all_supports(int B, int M, int N, int K, int inner, int outer);
@@ -225,7 +224,6 @@ struct ChainFwd {
     int B, M, N, K, inner, outer, activation;
     double eps;
     void *workspace;
-    size_t workspace_bytes;
     int spin_limit;  // as in ChainAll
 };
 bool chain_fwd_supports(int B, int M, int N, int K, int inner, int outer);

@@ -34,7 +34,7 @@ def assert_close(actual, expected, rtol=RTOL, atol=ATOL, what=""):
     expected = expected.detach().cpu().double()
     err = (actual - expected).abs()
     bound = atol + rtol * expected.abs()
-    bad = err > bound
+    bad = ~(err <= bound)  # a NaN is no match
     if bad.any():
         idx = torch.nonzero(bad)[0].tolist()
         worst = (err - bound).max().item()

@@ -103,11 +103,12 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
 }
 
 // 1 / sqrt(v) by the hardware's estimate and two Newton steps: a relative error below 1e-12 in a quarter
-// of the instructions of a square root and a division.
+// of the instructions of a square root and a division.  0 for infinity, as those give: a variance beyond
+// fp32 (squares of 1e20) leaves a sample's LayerNorm at beta, where the Newton steps would make it NaN.
 __device__ __forceinline__ double rsqrt_newton(double v) {
-    double r = __builtin_amdgcn_rsq(v);
-    r = r * fma(-0.5 * v * r, r, 1.5);
-    return r * fma(-0.5 * v * r, r, 1.5);
+    const double r0 = __builtin_amdgcn_rsq(v);
+    const double r = r0 * fma(-0.5 * v * r0, r0, 1.5);
+    return r0 == 0.0 ? 0.0 : r * fma(-0.5 * v * r, r, 1.5);
 }
 
 // The value of `v` in the lane before / after the caller's in the wave (DPP wave shifts: no LDS

@@ -13,13 +13,13 @@ DEV = "cuda:0"
 NAMES = ("y", "dweight", "dbias", "dscale", "dgamma", "dbeta", "dx0")
 
 
-def run_chain(shape, batch, inner, outer, activation, backward=True, **kw):
+def run_chain(shape, batch, inner, outer, activation, backward=True, x_scale=1.0, **kw):
     from gridnet_amd.runner import BodyRunner
 
     print(f"chain_fwd {shape} B={batch} inner={inner} outer={outer} {activation} {kw}", flush=True)
     g = torch.Generator().manual_seed(5)
     params = [*make_params(shape, seed=4), 1 + 0.2 * torch.randn(shape, generator=g), 0.2 * torch.randn(shape, generator=g)]
-    x, gy = make_acts(batch, shape, seed=6), make_acts(batch, shape, seed=7)
+    x, gy = x_scale * make_acts(batch, shape, seed=6), make_acts(batch, shape, seed=7)
     run = BodyRunner(*(t.to(DEV) for t in params), batch, inner, outer, 8, activation, fused=True, backward=backward, **kw)
     got = [run.forward(x.to(DEV)).clone()]
     if backward:
@@ -72,3 +72,14 @@ def test_the_largest_batch_and_one_more():
         assert run.forward_all == (b == batch)
         want = run_chain((16, 16, 16), b, 1, 5, "silu", backward=False, forward_all=False)[-1]
         assert_close(got[0], want[0], rtol=1e-5, atol=1e-5, what=f"batch {b}")
+
+
+@pytest.mark.parametrize("inner", [1, 2])
+def test_a_variance_beyond_fp32(inner):
+    """The squares of the raw values overflow: the LayerNorm leaves its beta, here as launch by launch."""
+    args = ((8, 16, 16), 2, inner, 3, "tanh")
+    got = run_chain(*args, backward=False, x_scale=1e25)
+    want = run_chain(*args, backward=False, x_scale=1e25, forward_all=False)
+    assert got[0].forward_all and not want[0].forward_all
+    assert torch.isfinite(want[-1][0]).all()
+    assert_close(got[-1][0], want[-1][0], rtol=1e-5, atol=1e-5)

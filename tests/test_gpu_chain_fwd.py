@@ -83,3 +83,29 @@ def test_a_variance_beyond_fp32(inner):
     assert got[0].forward_all and not want[0].forward_all
     assert torch.isfinite(want[-1][0]).all()
     assert_close(got[-1][0], want[-1][0], rtol=1e-5, atol=1e-5)
+
+
+def test_two_streams_in_flight():
+    """Two chains that together have more workgroups than the chip holds, launched alternately on two
+    streams: the cooperative launches wait for each other, or the waits inside run out and the chain is
+    repaired, but both end and are right."""
+    from gridnet_amd import native as n
+
+    batch, outer = 1, 6
+    while n.lib.gridnet_hip_chain_forward_all_supported(0, batch + 1, 32, 32, 32, 1, outer, 8, 0):
+        batch += 1
+    runs = []
+    for activation in ("silu", "tanh"):
+        run, _, x, _, got = run_chain((32, 32, 32), batch, 1, outer, activation, backward=False)
+        assert run.forward_all
+        runs.append((run, x.to(DEV), got[0], torch.cuda.Stream(device=DEV)))
+    for _, _, _, stream in runs:
+        stream.wait_stream(torch.cuda.current_stream())
+    results = []
+    for _ in range(4):
+        for k, (run, x, want, stream) in enumerate(runs):
+            with torch.cuda.stream(stream):
+                results.append((run.forward(x).clone(), want))
+    torch.cuda.synchronize()
+    for got, want in results:
+        assert_close(got, want, rtol=1e-5, atol=1e-5)

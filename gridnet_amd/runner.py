@@ -15,9 +15,10 @@ backward of a chain can go through ``gridnet_hip_chain_backward``: the backward 
 crosses a block boundary from step to step instead of finishing every dx (one kernel per step
 instead of two).  Same results to rounding.  ``chain=None`` (the default) takes it where the
 two-kernel backward would deal its cross-block part by block face (rows of more than 128 cells) or
-by rows that leave lanes idle (72 to 120 cells; 80 x 80 x 72, batch 32, 421 against 463 us per
-step); where that part goes by whole rows the two kernels are the faster pair
-(64^3 grid, batch 32, 12 steps: 3.12 against 3.19 ms per training step).  ``True``: wherever the
+by rows that leave lanes idle (72 to 120 cells: over 35 random grids, batch 3 to 50, two to eight inner
+iterations, it is 4 to 10 % faster on most up to 104 cells and within 3 % either way above); where that part
+goes by whole rows the two kernels are the faster pair (40 to 64 cells: by up to 8 %, 3 % slower at the worst;
+64^3 grid, batch 32, 12 steps: 3.12 against 3.19 ms per training step).  ``True``: wherever the
 library supports it; ``False``: never (nor the one launch below).
 
 Where the whole grid fits the GPU at once (every block a resident workgroup: a 64^3 grid on an

@@ -25,8 +25,8 @@
 // status word is raised; then it does the chain again, one workgroup per element and no waits
 // between workgroups.  The caller need not look at the status and nothing synchronises.
 //
-// All of it is latency: one 32^3 sample, one inner iteration, 2.9 us a step, of which the arithmetic is
-// 0.4; 64 steps with the MNIST model around them 826 -> 240 us.
+// All of it is latency: one 32^3 sample, one inner iteration, 3.4 us a step, of which the arithmetic is
+// 0.4; 64 steps with the MNIST model around them 824 -> 258 us.
 
 #include "common.h"
 #include "fast_tiles.h"
@@ -369,9 +369,9 @@ bool chain_fwd_supports(int B, int M, int N, int K, int inner, int outer) {
         per_cu = n;
     }
     if (per_cu < 1) return false;
-    // As many as fit: at two and three workgroups per CU a step still takes 6.9 us where the two kernels
-    // of a step, their launches included, take 10.7 (32^3, batch 8, one inner iteration; batch 1: 4.4
-    // against 9.4 us; 64^3, batch 1: 9.1 against 10.4).
+    // As many as fit.  Launches included, a step of 64 against the kernel and the merge of a step launch by
+    // launch (rows_fwd): 32^3, one inner iteration, batch 1, 3.8 against 6.7 us, batch 8 (two workgroups per
+    // CU), 5.8 against 10.1; 64^3, batch 1, 7.6 against 10.2; four inner iterations (step_fwd_split), batch 8, 7.3 against 14.5.
     return (long)M * N * K / 512 * B <= (long)per_cu * plan_device_cus();
 }
 

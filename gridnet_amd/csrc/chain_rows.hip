@@ -17,8 +17,9 @@
 // (The pairs per wave behind the LayerNorms' per-sample numbers are merged by small kernels between the
 // steps, 4.7 us each.  Merged by the workgroups that need them, one wave an element ahead, they cost
 // the kernels 11 us forward and 24 us backward: everybody waits for that wave at the barrier.)
-// 32^3, batch 256, silu, per step: forward 27.5 + 4.6 us (the merging kernel), backward 58 + 29 us
-// with fwd_rows, bwd_rows and cross_rows.
+// 32^3, batch 256, silu, per step: forward 27.6 + 4.7 us (the merging kernel), backward 66.8 + 4.8, at 4.3 TB/s
+// either way where a copy reaches 4.6 (fwd_rows, bwd_rows and cross_rows with their small kernels: 28.1 + 4.4,
+// 59.3 + 8.0 + 23.4).  Gated, tanh: 54.7 + 4.7 and 85.3 + 4.6 (op by op the whole training step took 21.3 ms, 9.3 now).
 
 #include "common.h"
 #include "fast_tiles.h"

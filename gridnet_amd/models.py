@@ -43,6 +43,9 @@ class Readout(nn.Module):
 class MnistGridModel(nn.Module):
     """28x28 images written into the ``[..., 0]`` face of a learned 32^3 initial grid."""
 
+    # the gated loop as one node, see gated_body: None where there is room, False never (not in the reference)
+    rows = None
+
     def __init__(self, inner_iters: int, outer_iters: int, init_scale: float,
                  residual_scale: float, activation: str, gated: bool, remember_bias: float,
                  device, fused_body: bool = False):
@@ -51,7 +54,6 @@ class MnistGridModel(nn.Module):
         if fused_body and gated:
             raise ValueError("the fused body covers the plain (not gated) network only")
         self.fused_body = fused_body
-        self.rows = None  # the gated loop as one node, see gated_body: None where there is room, False never
         self.outer_iters = outer_iters
         self.device = device
         self.init_in = nn.Parameter(torch.randn(32, 32, 32, device=device))

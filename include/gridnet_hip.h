@@ -400,7 +400,7 @@ int gridnet_hip_rows_chain_backward(const void *weight, const void *scale, const
                                     int activation, int flags, void *workspace, size_t workspace_bytes,
                                     void *stream);
 /* How often a wait inside the one-launch chain kernels polls before it gives up (default 200000,
- * about a second).  A negative value makes the kernels never signal completion to each other, so
+ * some tenths of a second).  A negative value makes the kernels never signal completion to each other, so
  * that every wait runs out after -limit polls: the give-up path, for tests.  Returns the old value. */
 int gridnet_hip_chain_set_spin_limit(int limit);
 

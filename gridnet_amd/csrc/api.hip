@@ -328,7 +328,8 @@ static int check_fused(const StepArgs &a, bool backward) {
 static size_t fused_forward_workspace(const StepArgs &a) {
     const size_t nblk = (size_t)(a.M / a.block_size) * (a.N / a.block_size) * (a.K / a.block_size);
     size_t pairs = nblk * step_fast_forward_parts(a.block_size);
-    if (fwd_rows_supports(a) && (size_t)fwd_rows_pairs(a) > pairs) pairs = (size_t)fwd_rows_pairs(a);
+    // not by fwd_rows_supports, whose answer depends on the batch: a workspace of the largest batch serves all
+    if (fwd_rows_covers(a) && (size_t)fwd_rows_pairs(a) > pairs) pairs = (size_t)fwd_rows_pairs(a);
     return (size_t)a.B * pairs * 2 * sizeof(float);
 }
 

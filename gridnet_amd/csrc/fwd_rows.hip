@@ -265,10 +265,11 @@ bool fills_chip(const StepArgs &a) {
 
 }  // namespace
 
-bool fwd_rows_supports(const StepArgs &a) {
+bool fwd_rows_covers(const StepArgs &a) {
     return a.dtype == GRIDNET_F32 && a.inner == 1 && !a.normalize && (a.block_size == 4 || a.block_size == 8) &&
-           k_ok(a.K) && a.M % 4 == 0 && a.N % 4 == 0 && fills_chip(a);
+           k_ok(a.K) && a.M % 4 == 0 && a.N % 4 == 0;
 }
+bool fwd_rows_supports(const StepArgs &a) { return fwd_rows_covers(a) && fills_chip(a); }
 
 // (mean, M2) pairs per sample that it leaves in a.ln.y_part: one per wave, over its live lanes' cells
 int fwd_rows_pairs(const StepArgs &a) { return (a.M * a.N / 16) * (16 * row_lanes(a.K, 4) / 64); }

@@ -157,6 +157,7 @@ int step_fast_cross_pairs(const StepArgs &a);     // the same for step_cross_lau
 // fwd_rows.hip: the forward of a step with ONE inner iteration, dealt by whole K-rows (fp32, normalize
 // off, K up to 128; the folded LayerNorm and the residual form as a.ln says)
 bool fwd_rows_supports(const StepArgs &a);
+bool fwd_rows_covers(const StepArgs &a);  // by its shape, whatever the batch: what a workspace is sized for
 int fwd_rows_pairs(const StepArgs &a);  // (mean, M2) pairs per sample in a.ln.y_part ...
 int fwd_rows_pair_count(const StepArgs &a);  // ... and the cells behind each
 int fwd_rows_launch(const StepArgs &a, hipStream_t st);

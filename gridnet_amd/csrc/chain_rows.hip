@@ -21,6 +21,8 @@
 // either way where a copy reaches 4.6 (fwd_rows, bwd_rows and cross_rows with their small kernels: 28.1 + 4.4,
 // 59.3 + 8.0 + 23.4).  Gated, tanh: 54.7 + 4.7 and 85.3 + 4.6 (op by op the whole training step took 21.3 ms, 9.3 now).
 
+#include <algorithm>
+
 #include "common.h"
 #include "fast_tiles.h"
 #include "launch.h"
@@ -687,6 +689,12 @@ int bwd_chunks(const RowsChain &c, int per_cu, int &chunk_len) {
     return n * ntube >= cus ? n : plan_row_chunks(c.B, ntube, cus, kRowsMinWalk, chunk_len);
 }
 constexpr int kBwdMostPerCu = 4;
+// no fewer than bwd_chunks gives, here or at any smaller batch: what the workspace is sized for
+int bwd_most_chunks(const RowsChain &c) {
+    const int fill = plan_device_cus() / tubes_of(c);
+    const int walks = std::min(kBwdMostPerCu * plan_device_cus() / tubes_of(c), c.B / 8);
+    return std::max({walks, std::min(fill, c.B / kRowsMinWalk), 1});
+}
 int grad_planes(const RowsChain &c) { return c.gated ? 58 : 31; }
 
 template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStream_t st) {
@@ -816,8 +824,7 @@ size_t rows_chain_workspace(const RowsChain &c, bool backward) {
         if (!c.keep) n += 2 * (size_t)c.B * cells_of(c) * sizeof(float);
         return n;
     }
-    int chunk_len;
-    const int chunks = bwd_chunks(c, kBwdMostPerCu, chunk_len);
+    const int chunks = bwd_most_chunks(c);
     return part_bytes(c.B, bwd_pairs(c)) + align_up((size_t)2 * c.B * sizeof(float)) +
            align_up(layernorm_workspace(GRIDNET_F32, c.B, cells_of(c))) + align_up((size_t)c.B * cells_of(c) * sizeof(float)) +
            (chunks > 1 ? (size_t)chunks * grad_planes(c) * cells_of(c) * sizeof(float) : 0);

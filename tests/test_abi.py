@@ -119,18 +119,22 @@ def test_native_operators_and_library_of_different_builds_do_not_go_together(tmp
             native.ops.bind(native.LIB_PATH)
 
 
-def test_a_fused_workspace_of_the_largest_batch_serves_the_smaller_ones():
-    """The kernels are chosen by the batch too; what a call needs must not be more at a smaller one.
-    (The backward's figure holds room to split the batch beside what it cannot do without: a smaller
+def test_a_workspace_of_the_largest_batch_serves_the_smaller_ones():
+    """Kernels and chunks are chosen by the batch too; what a call needs must not be more at a smaller one.
+    (The fused backward's figure holds room to split the batch beside what it cannot do without: a smaller
     workspace is accepted there.)"""
     from gridnet_amd import native
 
     for m in (8, 40, 48, 64):
-        for k in (8, 24, 40, 56, 72, 80, 96, 104, 128):
+        for k in (8, 16, 24, 32, 40, 56, 64, 72, 80, 96, 104, 128):
             for bs in (4, 8):
                 for inner in (1, 2):
                     need = [native.lib.gridnet_hip_fused_workspace_bytes(b, m, 48, k, inner, bs, 0) for b in range(1, 66)]
                     assert need == sorted(need), (m, k, bs, inner)
+            for gated, backward in ((0, 0), (0, 1), (1, 0), (1, 1)):
+                need = [native.lib.gridnet_hip_rows_chain_workspace_bytes(b, m, 48, k, gated, 1, backward)
+                        for b in range(1, 300)]
+                assert need == sorted(need), (m, k, gated, backward)
 
 
 def test_shim_has_the_reference_call_surface():

@@ -107,9 +107,14 @@ def gpu_run(wl, steps, warmup, fused, graph_replay=True, chain_all=None, chain=N
         assert p0 == 0 and p1 == 1
         spans.setdefault(name, []).append(e0.elapsed_time(e1) * 1e-3)
     kernel_s = {k: sum(v) / len(v) for k, v in spans.items()}
-    # entry points that take all outer steps in one call
-    whole = {name for name, flags in (("step_fwd", ("forward_all", "rows")), ("step_bwd", ("chain_all", "rows")))
-             if any(getattr(run, f, False) for f in flags)}
+    # entry points that take all outer steps in one call, and how
+    whole = {}
+    if getattr(run, "rows", False):
+        whole = dict.fromkeys(("step_fwd", "step_bwd"), "whole chain in one call, a kernel per step and direction")
+    if getattr(run, "forward_all", False):
+        whole["step_fwd"] = "forward of the chain in one launch"
+    if getattr(run, "chain_all", False):
+        whole["step_bwd"] = "backward of the chain in one launch"
     return wall, graph_s, kernel_s, whole
 
 
@@ -353,8 +358,7 @@ def main():
         "data": "synthetic",
         "config": {"workload": wl.name, "activation": wl.activation, "normalize": wl.normalize,
                    "pass": "fwd+bwd" if wl.backward else "fwd",
-                   "path": ("fused step+LayerNorm entry points" + (", backward of the chain in one launch"
-                                                                   if dominant in whole else ""))
+                   "path": "fused step+LayerNorm entry points" + (", " + whole[dominant] if dominant in whole else "")
                            if fused else "step and LayerNorm calls"},
         "timing": {"headline": "eager wall clock over the timed steps, synchronised on both sides",
                    "eager_ms_per_step": wall * 1e3,

@@ -29,7 +29,7 @@ weights and gradient accumulators from step to step and signal each other throug
 waits are bounded; ``chain_all_status()`` (which synchronises) tells whether one ran out, in which
 case ``backward`` must be repeated with ``chain_all`` off -- ``backward_checked`` does both.
 
-Where blocks and batch are few enough to be resident at once (a 32^3 grid at up to 16 samples) the
+Where blocks and batch are few enough to be resident at once (a 32^3 grid at up to 8 samples) the
 forward of a chain with one parameter set is one launch too (``gridnet_hip_chain_forward_all``;
 ``forward_all=False``: never).
 

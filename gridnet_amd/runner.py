@@ -57,14 +57,19 @@ UNASKED = 1 / 128  # share of the device's memory, see room_for
 
 def room_for(nbytes: int, device) -> bool:
     """Whether a chain may keep ``nbytes`` for its backward where a slower one would keep half of it: they
-    take at most half of the memory that is free, on the device or in torch's cache.  What the program
-    allocates until the backward has run then has as much again, and a batch that the slower chain leaves
-    room for is not refused.  Little (2.3 GB of 288) is taken without asking the driver."""
-    if nbytes <= UNASKED * torch.cuda.get_device_properties(device).total_memory:
+    take at most half of the memory that is free, on the device or in torch's cache, and within the share
+    of it that the process may use.  What the program allocates until the backward has run then has as
+    much again, and a batch that the slower chain leaves room for is not refused.  Little (2.3 GB of 288) is
+    taken without asking the driver."""
+    share = torch.cuda.get_per_process_memory_fraction(device)
+    limit = share * torch.cuda.get_device_properties(device).total_memory
+    if nbytes <= UNASKED * limit:
         return True
     free = torch.cuda.mem_get_info(device)[0]
     if 2 * nbytes > free and not torch.cuda.is_current_stream_capturing():  # a capture has a pool of its own
         free += torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    if share < 1:
+        free = min(free, limit - torch.cuda.memory_allocated(device))
     return 2 * nbytes <= free
 
 

@@ -117,6 +117,12 @@ def test_without_room_the_shorter_history_is_kept(monkeypatch):
         y = m(x)
         assert ("GatedBodyOpBackward" in nodes(y)) == fits
         torch.testing.assert_close(y, want, rtol=1e-5, atol=1e-5)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (1 << 60, 0))
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    for more, fits in ((3 * need, True), (need, False)):  # within what the process may use
+        share = (torch.cuda.memory_allocated() + more) / total
+        monkeypatch.setattr(torch.cuda, "get_per_process_memory_fraction", lambda device: share)
+        assert ("GatedBodyOpBackward" in nodes(m(x))) == fits
     with torch.no_grad():  # nothing is kept
         assert torch.equal(m(x), want)
     monkeypatch.setattr(runner, "room_for", lambda nbytes, device: False)

@@ -128,8 +128,7 @@ int gridnet_hip_forward(int dtype, const void *weight, const void *bias, const v
     if (int rc = check_step(a, false)) return rc;
     if (B == 0) return GRIDNET_OK;
     hipStream_t st = (hipStream_t)stream;
-    if (step_fast_supports(a, false)) return step_forward_fast(a, st);
-    return step_forward_generic(a, st);
+    return dtype == GRIDNET_F64 ? step_forward_f64(a, st) : step_forward_fast(a, st);
 }
 
 // What lies behind the first `used` bytes of a workspace (rounded up to 256) is room for the
@@ -151,6 +150,8 @@ size_t gridnet_hip_backward_workspace_bytes(int dtype, int B, int M, int N, int 
     a.dtype = dtype; a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner;
     a.block_size = block_size; a.normalize = normalize != 0; a.activation = GRIDNET_ACT_RELU;
     if (B <= 0 || M <= 0 || N <= 0 || K <= 0) return 0;
+    // (a caller that hands over less, or nothing, is served by the kernel that needs none)
+    if (step_f64_supports(a)) return step_f64_workspace(a) + step_f64_slab_bytes(a);
     if (!step_fast_supports(a, true)) return 0;
     const size_t slabs = step_fast_slab_bytes(a);
     return slabs ? (step_fast_backward_workspace(a) + 255) / 256 * 256 + slabs : step_fast_backward_workspace(a);
@@ -169,6 +170,11 @@ static int backward_step(int dtype, const void *weight, const void *bias, const 
     if (int rc = check_step(a, true)) return rc;
     if (B == 0) return GRIDNET_OK;
     hipStream_t st = (hipStream_t)stream;
+    if (!static_scratch && step_f64_supports(a) && workspace && workspace_bytes >= step_f64_workspace(a)) {
+        a.workspace = workspace; a.workspace_bytes = workspace_bytes;
+        give_slabs(a, workspace, workspace_bytes, step_f64_workspace(a));
+        return step_backward_f64(a, st);
+    }
     if (!step_fast_supports(a, true)) return step_backward_generic(a, st);  // needs no scratch
     const size_t need = step_fast_backward_workspace(a);
     if (static_scratch) {

@@ -136,8 +136,14 @@ struct LayerNormArgs {
 };
 
 // step_generic.hip
-int step_forward_generic(const StepArgs &a, hipStream_t st);
 int step_backward_generic(const StepArgs &a, hipStream_t st);
+
+// step_f64.hip: the fp64 forward, and the backward with scratch
+int step_forward_f64(const StepArgs &a, hipStream_t st);
+bool step_f64_supports(const StepArgs &a);
+size_t step_f64_workspace(const StepArgs &a);   // what it cannot do without
+size_t step_f64_slab_bytes(const StepArgs &a);  // room for the gradient copies of a split batch
+int step_backward_f64(const StepArgs &a, hipStream_t st);
 
 // step_fast.hip: fp32, block sizes 4 and 8, normalize on or off (off only with the folded LayerNorm)
 bool step_fast_supports(const StepArgs &a, bool backward);

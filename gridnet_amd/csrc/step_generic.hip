@@ -1,7 +1,6 @@
-// Generic block-local update kernels: one thread per cell, any dtype (fp32/fp64), any
-// activation, optional per-window normalisation, up to 32 inner iterations in backward.
-// This is the coverage path (fp64, and fp32 problems the tuned kernels decline); the tuned fp32
-// kernels are separate (step_fast.hip).
+// Generic backward of a block-local update: one thread per cell, any dtype (fp32/fp64), any
+// activation, optional per-window normalisation, up to 32 inner iterations, no scratch.
+// This is the coverage path (what the tuned kernels of step_fast.hip, fp32, and step_f64.hip decline).
 //
 // Work decomposition: one workgroup owns one spatial block (bs^3 threads) and walks a chunk
 // of batch elements with the block's 27 weights, bias and scale held in registers, so the
@@ -72,50 +71,6 @@ __device__ __forceinline__ T pre_activation(const T *win, const T (&w)[27], T bi
                 u += w[a * 9 + b * 3 + c] * v;
             }
     return u;
-}
-
-template <typename T, int BS, int ACT, bool NORM>
-__global__ __launch_bounds__(BS *BS *BS) void step_fwd_generic(
-    const T *__restrict__ weight, const T *__restrict__ bias, const T *__restrict__ scale,
-    const T *__restrict__ x, T *__restrict__ y, int B, int M, int N, int K, int inner, T eps,
-    int nblk, int nchunk, int chunk_len) {
-    using G = Geo<BS>;
-    __shared__ T win[G::W];
-    __shared__ T red[8];
-
-    const int tid = threadIdx.x;
-    int blk, chunk;
-    if (!split_block_id(blockIdx.x, nblk, nchunk, blk, chunk)) return;  // grid padding
-    const int kb = K / BS, nb = N / BS;
-    const int p0 = (blk / (kb * nb)) * BS, q0 = ((blk / kb) % nb) * BS, r0 = (blk % kb) * BS;
-    const int ci = tid / (BS * BS), cj = (tid / BS) % BS, ck = tid % BS;
-    const long cells = (long)M * N * K;
-    const long gc = ((long)(p0 + ci) * N + (q0 + cj)) * K + (r0 + ck);
-    const int base = (ci * G::S + cj) * G::S + ck;           // window index of tap (0,0,0)
-    const int centre = base + (G::S + 1) * G::S + 1;         // window index of the cell itself
-
-    T w[27];
-#pragma unroll
-    for (int t = 0; t < 27; ++t) w[t] = weight[t * cells + gc];
-    const T bv = bias[gc], rv = scale[gc];
-
-    const int s_end = min(B, (chunk + 1) * chunk_len);
-    for (int s = chunk * chunk_len; s < s_end; ++s) {
-        load_window<T, BS>(win, x + s * cells, p0, q0, r0, M, N, K, tid);
-        __syncthreads();
-        T cur = win[centre];
-        for (int it = 0; it < inner; ++it) {
-            T mean = T(0), sd = T(0), inv = T(1);
-            if (NORM) window_stats<T, BS>(win, red, tid, eps, mean, sd, inv);
-            const T u = pre_activation<T, BS, NORM>(win, w, bv, base, mean, inv);
-            cur += rv * Act<ACT, T>::f(u);
-            __syncthreads();  // everyone has read the old state
-            win[centre] = cur;
-            __syncthreads();
-        }
-        y[s * cells + gc] = cur;
-        __syncthreads();  // window is reloaded next
-    }
 }
 
 // LDS of the backward kernel: three windows, the table of per-tap products and the reduction
@@ -290,19 +245,6 @@ template <typename T> __global__ void fill_zero_kernel(T *p, long n) {
     for (; i < n; i += stride) p[i] = T(0);
 }
 
-template <typename T, int BS, int ACT>
-int launch_fwd_norm(const StepArgs &a, int nblk, int nchunk, int chunk_len, hipStream_t st) {
-    dim3 grid(padded_grid(nblk, nchunk)), block(Geo<BS>::NT);
-    auto args = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, block, 0, st, (const T *)a.weight, (const T *)a.bias,
-                           (const T *)a.scale, (const T *)a.x, (T *)a.y, a.B, a.M, a.N, a.K,
-                           a.inner, (T)a.eps, nblk, nchunk, chunk_len);
-    };
-    if (a.normalize) args(step_fwd_generic<T, BS, ACT, true>);
-    else args(step_fwd_generic<T, BS, ACT, false>);
-    return check_launch("step_fwd_generic");
-}
-
 template <typename T, int BS, int ACT, bool NORM>
 int launch_bwd_kernel(const StepArgs &a, int nblk, int nchunk, int chunk_len, int param_mode,
                       hipStream_t st) {
@@ -333,13 +275,11 @@ int launch_bwd_norm(const StepArgs &a, int nblk, int nchunk, int chunk_len, int 
     return launch_bwd_kernel<T, BS, ACT, false>(a, nblk, nchunk, chunk_len, param_mode, st);
 }
 
-template <typename T, int BS, bool BWD>
+template <typename T, int BS>
 int dispatch_act(const StepArgs &a, int nblk, int nchunk, int chunk_len, int param_mode,
                  hipStream_t st) {
-#define GRIDNET_CASE(ID)                                                                     \
-    case ID:                                                                                 \
-        if (BWD) return launch_bwd_norm<T, BS, ID>(a, nblk, nchunk, chunk_len, param_mode, st); \
-        return launch_fwd_norm<T, BS, ID>(a, nblk, nchunk, chunk_len, st);
+#define GRIDNET_CASE(ID) \
+    case ID: return launch_bwd_norm<T, BS, ID>(a, nblk, nchunk, chunk_len, param_mode, st);
     switch (a.activation) {
         GRIDNET_CASE(GRIDNET_ACT_RELU)
         GRIDNET_CASE(GRIDNET_ACT_LEAKY_RELU)
@@ -368,45 +308,33 @@ template <typename T> int fill_zero(T *p, long n, hipStream_t st) {
     return check_launch("fill_zero");
 }
 
-template <typename T> int run_generic(const StepArgs &a, bool bwd, hipStream_t st) {
+template <typename T> int run_generic(const StepArgs &a, hipStream_t st) {
     const int bs = a.block_size;
     const int nblk = (a.M / bs) * (a.N / bs) * (a.K / bs);
     int nchunk = pick_chunks(nblk, a.B);
     const int chunk_len = (a.B + nchunk - 1) / nchunk;
     nchunk = (a.B + chunk_len - 1) / chunk_len;
     int param_mode = kParamAtomic;
-    if (bwd) {
-        const long cells = (long)a.M * a.N * a.K;
-        const bool new_params = (a.flags & GRIDNET_OVERWRITE_PARAMS) != 0;
-        if (a.flags & GRIDNET_OVERWRITE_DX) {  // dx is built with atomics: start from zero
-            if (int rc = fill_zero((T *)a.dx, (long)a.B * cells, st)) return rc;
-        }
-        if (nchunk == 1) {
-            param_mode = new_params ? kParamStore : kParamAddExclusive;
-        } else if (new_params) {
-            if (int rc = fill_zero((T *)a.dweight, 27 * cells, st)) return rc;
-            if (int rc = fill_zero((T *)a.dbias, cells, st)) return rc;
-            if (int rc = fill_zero((T *)a.dscale, cells, st)) return rc;
-        }
+    const long cells = (long)a.M * a.N * a.K;
+    const bool new_params = (a.flags & GRIDNET_OVERWRITE_PARAMS) != 0;
+    if (a.flags & GRIDNET_OVERWRITE_DX) {  // dx is built with atomics: start from zero
+        if (int rc = fill_zero((T *)a.dx, (long)a.B * cells, st)) return rc;
     }
-    if (bs == 8) {
-        return bwd ? dispatch_act<T, 8, true>(a, nblk, nchunk, chunk_len, param_mode, st)
-                   : dispatch_act<T, 8, false>(a, nblk, nchunk, chunk_len, param_mode, st);
+    if (nchunk == 1) {
+        param_mode = new_params ? kParamStore : kParamAddExclusive;
+    } else if (new_params) {
+        if (int rc = fill_zero((T *)a.dweight, 27 * cells, st)) return rc;
+        if (int rc = fill_zero((T *)a.dbias, cells, st)) return rc;
+        if (int rc = fill_zero((T *)a.dscale, cells, st)) return rc;
     }
-    return bwd ? dispatch_act<T, 4, true>(a, nblk, nchunk, chunk_len, param_mode, st)
-               : dispatch_act<T, 4, false>(a, nblk, nchunk, chunk_len, param_mode, st);
+    return bs == 8 ? dispatch_act<T, 8>(a, nblk, nchunk, chunk_len, param_mode, st)
+                   : dispatch_act<T, 4>(a, nblk, nchunk, chunk_len, param_mode, st);
 }
 
 }  // namespace
 
-int step_forward_generic(const StepArgs &a, hipStream_t st) {
-    return a.dtype == GRIDNET_F64 ? run_generic<double>(a, false, st)
-                                  : run_generic<float>(a, false, st);
-}
-
 int step_backward_generic(const StepArgs &a, hipStream_t st) {
-    return a.dtype == GRIDNET_F64 ? run_generic<double>(a, true, st)
-                                  : run_generic<float>(a, true, st);
+    return a.dtype == GRIDNET_F64 ? run_generic<double>(a, st) : run_generic<float>(a, st);
 }
 
 }  // namespace gridnet

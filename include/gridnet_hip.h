@@ -95,7 +95,7 @@ int gridnet_hip_forward(int dtype, const void *weight, const void *bias, const v
  * share in its own copy with plain stores and the copies are added in chunk order (no atomics,
  * the same bits on every run).  A caller may hand over less, down to B*M*N*K elements (plus two
  * floats per block and batch element with normalize): the batch is then split less, or not at
- * all; the results agree to rounding.
+ * all; the results agree to rounding.  In fp64 it may hand over nothing: a slower kernel needs none.
  */
 size_t gridnet_hip_backward_workspace_bytes(int dtype, int B, int M, int N, int K, int inner,
                                             int block_size, int normalize);

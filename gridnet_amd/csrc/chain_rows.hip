@@ -14,12 +14,13 @@
 //     of the neighbour's weight 26 - t, and no other cell contributes to it.
 //   * Where the batch is split over workgroups every chunk keeps ONE copy of the gradient arrays for the
 //     whole chain, each step adding its sums to what the step before left; the copies are added up once.
-// (The pairs per wave behind the LayerNorms' per-sample numbers are merged by small kernels between the
-// steps, 4.7 us each.  Merged by the workgroups that need them, one wave an element ahead, they cost
-// the kernels 11 us forward and 24 us backward: everybody waits for that wave at the barrier.)
-// 32^3, batch 256, silu, per step: forward 27.6 + 4.7 us (the merging kernel), backward 66.8 + 4.8, at 4.3 TB/s
-// either way where a copy reaches 4.6 (fwd_rows, bwd_rows and cross_rows with their small kernels: 28.1 + 4.4,
-// 59.3 + 8.0 + 23.4).  Gated, tanh: 54.7 + 4.7 and 85.3 + 4.6 (op by op the whole training step took 21.3 ms, 9.3 now).
+//   * The pairs per wave behind the LayerNorms' per-sample numbers are merged by the workgroups of the next
+//     step while their weights are on their way (merge_lanes says where; a small kernel between the steps
+//     elsewhere, 4.7 us each).  Merged inside the walk, by one wave an element ahead, they cost the kernels
+//     11 us forward and 24 us backward: everybody waits for that wave at the barrier.
+// 32^3, batch 256, silu, per step: forward 28.3 us, backward 68.3, at 4.3 TB/s either way where a copy
+// reaches 4.6 (with the merging kernels 30.4 and 69.0; fwd_rows, bwd_rows and cross_rows with theirs: 28.1 + 4.4,
+// 59.3 + 8.0 + 23.4).  Gated, tanh: 55.5 and 86.6 (op by op the whole training step took 21.3 ms, 9.2 now).
 
 #include <algorithm>
 
@@ -99,28 +100,67 @@ __device__ __forceinline__ float2 load_pair_ahead(const float *pairs, int sample
     return make_float2(v[0], v[1]);
 }
 
+// The pairs per wave that the launch before left, [B][pairs][2], merged by the workgroup that walks the
+// samples s0 ... s0 + len: `lanes` threads (a power of two) to a sample, in double, a fixed order.  `finish`
+// gets the three sums of sample s0 + e: of the first numbers, the second, and the squares of the first.
+// AHEAD pieces of two pairs are requested at a time.
+template <int AHEAD, typename Finish>
+__device__ __forceinline__ void merge_pairs(const float *part, int pairs, int lanes, int s0, int len, Finish finish) {
+    const int q = threadIdx.x & (lanes - 1), shift = 31 - __builtin_clz(lanes), half = pairs / 2;
+    for (int e = (int)threadIdx.x >> shift; e < len; e += (int)blockDim.x >> shift) {
+        const float4 *from = reinterpret_cast<const float4 *>(part + 2L * (s0 + e) * pairs);
+        double a = 0.0, b = 0.0, c = 0.0;
+        for (int i0 = q; i0 < half; i0 += lanes * AHEAD) {
+            float4 v[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) v[k] = from[min(i0 + k * lanes, half - 1)];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                const bool in = i0 + k * lanes < half;
+                const double x = in ? v[k].x : 0.f, y = in ? v[k].y : 0.f, z = in ? v[k].z : 0.f, w = in ? v[k].w : 0.f;
+                a += x + z;
+                b += y + w;
+                c = fma(x, x, fma(z, z, c));
+            }
+        }
+        for (int m = 1; m < lanes; m *= 2) {
+            a += __shfl_xor(a, m);
+            b += __shfl_xor(b, m);
+            c += __shfl_xor(c, m);
+        }
+        if (q == 0) finish(e, a, b, c);
+    }
+}
+
 struct RowsFwdArgs {
     const float *weight, *bias, *scale, *gamma, *beta, *x;
     const float *x_stats;   // the LayerNorm in front of the step (null: x is used as it is)
+    const float *x_part;    // MERGE: the pairs that its statistics come from instead, merged by `lanes` threads each,
+    float *stats_out;       // and left here for the backward (or null)
+    int lanes;
+    double eps;
     float *y, *y_part;
     float *saved;           // plain: [B,cells]; gated: [3][B,cells]; or null
     int B, M, N, ntube, nchunk, chunk_len;
 };
 
+// MERGE: the statistics of x from the pairs of the step before.  A kernel without it has none of that code: with
+// a test instead, the gated forward took 57 -> 59 us where the pairs are merged elsewhere.
 // PLAIN: four cells and 108 weights per thread; GATED: two cells and 2 x 54.  Everything else as
 // fwd_rows.hip: six by six rows in LDS, two stages, one barrier per batch element.
-template <int ACT, int SETS, bool SAVE, int K>
+template <int ACT, int SETS, bool SAVE, int K, bool MERGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(SETS == 1 ? 3 : 2, 3)))
 void rows_fwd(RowsFwdArgs a) {
     constexpr int CPT = 4 / SETS, RPT = 3;
-    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][36][K], gamma rows, beta rows
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][36][K], gamma rows, beta rows, statistics
     int tube, chunk;
     if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
     const int tid = threadIdx.x, M = a.M, N = a.N, nw = blockDim.x / 64, wave = tid / 64;
     const RowPlace<CPT, K> p(tid, tube, N);
     const long cells = (long)M * N * K;
-    const bool ln_in = a.x_stats != nullptr;
+    const bool ln_in = MERGE || a.x_stats != nullptr;
     const int s0 = chunk * a.chunk_len, s1 = min(a.B, s0 + a.chunk_len);
+    float2 *stat = reinterpret_cast<float2 *>(lds + 4 * kWinRows * K);  // of the samples s0 ... s1, with MERGE
 
     float w[SETS][9][3][CPT], bv[SETS][CPT], rv[CPT];
 #pragma unroll
@@ -134,6 +174,15 @@ void rows_fwd(RowsFwdArgs a) {
 #pragma unroll
     for (int k = 0; k < SETS; ++k) load_cells<CPT>(a.bias + k * cells + p.grow, bv[k]);
     if (SETS == 1) load_cells<CPT>(a.scale + p.grow, rv);
+    if constexpr (MERGE) {  // while the parameters are on their way
+        const double n = (double)a.ntube * nw, count = cells / n;
+        merge_pairs<4>(a.x_part, a.ntube * nw, a.lanes, s0, s1 - s0, [&](int e, double m, double q, double mm) {
+            const double mean = m / n, var = (q + count * (mm - n * mean * mean)) / (n * count);
+            const float2 v = make_float2((float)mean, (float)(1.0 / sqrt((var > 0.0 ? var : 0.0) + a.eps)));
+            stat[e] = v;
+            if (tube == 0 && a.stats_out) reinterpret_cast<float2 *>(a.stats_out)[s0 + e] = v;
+        });
+    }
     const float keep_first = p.first ? 0.f : 1.f, keep_last = p.last ? 0.f : 1.f;
 #pragma unroll
     for (int k = 0; k < SETS; ++k)
@@ -169,12 +218,14 @@ void rows_fwd(RowsFwdArgs a) {
     const bool has_last = p.r + 16 * (RPT - 1) < kWinRows;
     const int own_row = (p.ci + 1) * kSide + p.cj + 1;
     wait_global_loads();
+    if (MERGE) lds_barrier();  // the statistics are there
 
     float xbuf[RPT][CPT];
     float2 next_stat = make_float2(0.f, 1.f);
     auto fetch = [&](int s) {
         const float *x = a.x + (long)s * cells;
-        if (ln_in) next_stat = load_pair_ahead(a.x_stats, s);
+        if (MERGE) next_stat = stat[s - s0];
+        else if (ln_in) next_stat = load_pair_ahead(a.x_stats, s);
 #pragma unroll
         for (int e = 0; e < RPT; ++e) load_at<CPT>(x, 4u * (unsigned)goff[e], xbuf[e]);
     };
@@ -313,7 +364,9 @@ struct RowsBwdArgs {
     const float *weight, *scale, *gamma, *beta;
     const float *dy;                // gradient with respect to LayerNorm(y)
     const float *y, *y_stats;
-    const float *y_sums;            // the LayerNorm backward's two sums per sample
+    float *y_sums;                  // the LayerNorm backward's two sums per sample
+    const float *y_part;            // MERGE: the pairs that they come from, merged here by `lanes` threads each
+    int lanes;
     const float *saved;
     const float *x, *x_stats;       // the step's input: raw, and the statistics of the LayerNorm on it (null: as it is)
     float *dx, *x_part;             // x_part: pairs for the LayerNorm on x, or null
@@ -325,7 +378,7 @@ struct RowsBwdArgs {
 
 // PLAIN: two cells per thread, GATED: one; 54 mirrored weights and 54 gradient accumulators for each set
 // and two cells.  A thread moves its own row and one or two of the 20 rows around the tube.
-template <int ACT, int SETS, int K>
+template <int ACT, int SETS, int K, bool MERGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_bwd(RowsBwdArgs a) {
     constexpr int CPT = 2 / SETS;
     extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K], then gamma and (plain) scale of the rows
@@ -369,6 +422,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     };
     load_planes(a.weight, v);
+    if constexpr (MERGE)  // while the weights are on their way
+        merge_pairs<8>(a.y_part, a.ntube * nw, a.lanes, s0, s1 - s0, [&](int e, double t1, double t2, double) {
+            reinterpret_cast<float2 *>(a.y_sums)[s0 + e] = make_float2((float)(t1 / (double)cells), (float)(t2 / (double)cells));
+        });
     // a step's sums start from zero, also where there is something to add them to (see the end)
 #pragma unroll
     for (int k = 0; k < SETS; ++k)
@@ -416,6 +473,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     store_cells<CPT>(gam_rows + own_at, gam);
     if (SETS == 1) store_cells<CPT>(scale_rows + own_at, rv);
     wait_global_loads();
+    if (MERGE) lds_barrier();  // the sums are there, also for the loads below: every wave has waited for its stores
 #pragma unroll
     for (int pq = 0; pq < 9; ++pq) {
         const int gi = p.p0 + p.ci + pq / 3 - 1, gj = p.q0 + p.cj + pq % 3 - 1;
@@ -652,29 +710,49 @@ template <typename K> int workgroups_per_cu(K kern, int threads, size_t lds) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)kern, threads, lds) != hipSuccess || n < 1) n = 1;
     return n;
 }
+// Threads to a sample where the workgroups of a step merge the pairs of the step before, beside the fetch of
+// their weights; 0: a kernel of its own does (4.7 us and a launch).  Every workgroup of a chunk merges the
+// same pairs, so it pays as long as they are few per thread.  Forward / backward of a step with the kernel and
+// without: 32^3, batch 16, 10.5 -> 8.7 / 17.1 -> 15.8 us; batch 64, 15.9 -> 13.7 / 31.9 -> 30.7; batch 256 (22 and 32
+// pairs per thread) 30.4 -> 28.3 / 69.0 -> 68.3; 64^3, batch 32 (44 pairs) 30.7 -> 32.1 / 74.0 -> 74.6.  Gated, 32^3,
+// batch 32, 17.1 -> 15.4 / 26.3 -> 25.3; batch 256, 57.0 -> 55.5 forward.
+constexpr int kMergeMostSamples = 64, kMergeMostPairs = 32;  // per workgroup; per thread
+int merge_lanes(int threads, int chunk_len, int pairs) {
+    if (pairs % 2 || chunk_len > kMergeMostSamples) return 0;
+    int lanes = 1;
+    while (2 * lanes * chunk_len <= threads && 4 * lanes <= pairs && lanes < kWave) lanes *= 2;
+    return (long)chunk_len * pairs <= kMergeMostPairs * (long)threads ? lanes : 0;
+}
+
 template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &c, hipStream_t st) {
-    auto kern = rows_fwd<ACT, SETS, SAVE, K>;
+    const auto kern = rows_fwd<ACT, SETS, SAVE, K, false>, merging = rows_fwd<ACT, SETS, SAVE, K, true>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
     const int ntube = tubes_of(c), nt = fwd_threads(c), pairs = fwd_pairs(c);
-    const size_t lds = 4 * (size_t)kWinRows * c.K * sizeof(float);
+    const size_t lds = 4 * (size_t)kWinRows * c.K * sizeof(float) + kMergeMostSamples * sizeof(float2);
     static int per_cu = 0;  // per instantiation
     if (per_cu == 0) per_cu = workgroups_per_cu(kern, nt, lds);
     RowsFwdArgs a{};
     a.nchunk = plan_row_chunks(c.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, a.chunk_len);
+    a.lanes = merge_lanes(nt, a.chunk_len, pairs);
+    a.eps = c.eps;
     a.weight = c.weight; a.bias = c.bias; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
     a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
     // workspace: the pairs; and, where nothing is kept, statistics and two raw tensors
     char *ws = (char *)c.workspace;
-    a.y_part = (float *)ws;
-    ws += part_bytes(c.B, pairs);
+    float *parts[2] = {(float *)ws, (float *)(ws + part_bytes(c.B, pairs))};
+    ws += 2 * part_bytes(c.B, pairs);
     float *own_stats = (float *)ws, *own_y = (float *)(ws + align_up((size_t)2 * c.B * sizeof(float)));
     for (int j = 0; j < c.outer; ++j) {
         float *stats = c.stats ? c.stats + (long)j * 2 * c.B : own_stats;
         a.x = j ? a.y : c.x0;
+        a.x_part = a.y_part;
+        a.stats_out = c.stats ? stats - 2 * c.B : nullptr;
+        a.y_part = parts[j & 1];
         a.y = c.y_raw ? c.y_raw + j * tensor : own_y + (j & 1) * tensor;
         a.saved = SAVE ? c.saved + (long)j * (SETS == 1 ? 1 : 3) * tensor : nullptr;
-        hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, a.nchunk)), dim3(nt), lds, st, a);
+        hipLaunchKernelGGL(j && a.lanes ? merging : kern, dim3(padded_grid(ntube, a.nchunk)), dim3(nt), lds, st, a);
         if (int rc = check_launch("rows_fwd")) return rc;
+        if (a.lanes && j + 1 < c.outer) continue;
         if (int rc = layernorm_finalize_stats(a.y_part, pairs, (int)(cells / pairs), stats, c.B, c.eps, st)) return rc;
         a.x_stats = stats;
     }
@@ -698,7 +776,7 @@ int bwd_most_chunks(const RowsChain &c) {
 int grad_planes(const RowsChain &c) { return c.gated ? 58 : 31; }
 
 template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStream_t st) {
-    auto kern = rows_bwd<ACT, SETS, K>;
+    const auto kern = rows_bwd<ACT, SETS, K, false>, merging = rows_bwd<ACT, SETS, K, true>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
     const int ntube = tubes_of(c), nt = bwd_threads(c), pairs = bwd_pairs(c);
     const size_t lds = (2 * SETS + 1 + (SETS == 1)) * (size_t)kWinRows * K * sizeof(float);
@@ -709,12 +787,13 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
     }
     RowsBwdArgs a{};
     a.nchunk = bwd_chunks(c, per_cu, a.chunk_len);
+    a.lanes = merge_lanes(nt, a.chunk_len, pairs);
     a.weight = c.weight; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
     a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
     // workspace: the pairs, the sums, scratch of the last LayerNorm's sums, a second dx, the copies
     char *ws = (char *)c.workspace;
-    float *part = (float *)ws;
-    ws += part_bytes(c.B, pairs);
+    float *parts[2] = {(float *)ws, (float *)(ws + part_bytes(c.B, pairs))};
+    ws += 2 * part_bytes(c.B, pairs);
     float *sums = (float *)ws;
     ws += align_up((size_t)2 * c.B * sizeof(float));
     float *scratch = (float *)ws;
@@ -760,14 +839,15 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
         a.saved = c.saved + j * (SETS == 1 ? 1 : 3) * tensor;
         a.x = j ? c.y_raw + (j - 1) * tensor : c.x0;
         a.x_stats = j ? c.stats + (j - 1) * 2 * c.B : nullptr;
-        a.x_part = j ? part : nullptr;
+        a.y_part = parts[(j + 1) & 1];
+        a.x_part = j ? parts[j & 1] : nullptr;
         a.dx = j & 1 ? other_dx : c.dx;
         a.accumulate = j < last || (!split && add);
-        hipLaunchKernelGGL(kern, dim3(padded_grid(ntube, a.nchunk)), dim3(nt), lds, st, a);
+        hipLaunchKernelGGL(j < last && a.lanes ? merging : kern, dim3(padded_grid(ntube, a.nchunk)), dim3(nt), lds, st, a);
         if (int rc = check_launch("rows_bwd")) return rc;
         a.dy = a.dx;
-        if (j)
-            if (int rc = layernorm_finalize_sums(part, pairs, cells, sums, c.B, st)) return rc;
+        if (j && !a.lanes)
+            if (int rc = layernorm_finalize_sums(parts[j & 1], pairs, cells, sums, c.B, st)) return rc;
     }
     if (!split) return GRIDNET_OK;
     return plan_launch_tail_job(plan_tail_job(slabs, a.nchunk, slab_floats, t, add ? ~0 : 0, 256), st);
@@ -820,12 +900,12 @@ bool rows_chain_supports(int M, int N, int K, bool gated) {
 
 size_t rows_chain_workspace(const RowsChain &c, bool backward) {
     if (!backward) {
-        size_t n = part_bytes(c.B, fwd_pairs(c)) + align_up((size_t)2 * c.B * sizeof(float));
+        size_t n = 2 * part_bytes(c.B, fwd_pairs(c)) + align_up((size_t)2 * c.B * sizeof(float));
         if (!c.keep) n += 2 * (size_t)c.B * cells_of(c) * sizeof(float);
         return n;
     }
     const int chunks = bwd_most_chunks(c);
-    return part_bytes(c.B, bwd_pairs(c)) + align_up((size_t)2 * c.B * sizeof(float)) +
+    return 2 * part_bytes(c.B, bwd_pairs(c)) + align_up((size_t)2 * c.B * sizeof(float)) +
            align_up(layernorm_workspace(GRIDNET_F32, c.B, cells_of(c))) + align_up((size_t)c.B * cells_of(c) * sizeof(float)) +
            (chunks > 1 ? (size_t)chunks * grad_planes(c) * cells_of(c) * sizeof(float) : 0);
 }

@@ -221,3 +221,37 @@ def test_gated_chain_at_the_scripts_defaults_is_as_exact_as_torch(seed):
         ours, theirs = (((v.double() - e).norm() / e.norm()).item() for v in (a, t))
         print(f"  {name}: {ours:.2e} off, torch {theirs:.2e}", flush=True)
         assert ours <= 4 * theirs + 1e-7, name
+
+
+# pairs of the merge: an odd number (a kernel of its own), two, more than a request's worth per thread, several
+# threads to a sample and one; chunks that end early; too many samples per workgroup
+@pytest.mark.parametrize("shape,batch", [((12, 12, 16), 5), ((4, 8, 16), 7), ((16, 16, 32), 37), ((32, 32, 32), 70),
+                                         ((8, 8, 32), 300), ((16, 32, 64), 11), ((4, 4, 32), 5000)], ids=str)
+def test_statistics_merged_by_the_next_step(shape, batch):
+    """Statistics and backward sums of every step, against sums over the tensors themselves in double (fp32
+    pairs over 256 values: 2^-24 times a few)."""
+    from gridnet_amd.runner import BodyRunner
+
+    print(f"merged statistics {shape} B={batch}", flush=True)
+    gamma, beta, x, gy = inputs(shape, batch)
+    run = BodyRunner(*(t.to(DEV) for t in (*make_params(shape, seed=4), gamma, beta)), batch, 1, 3, 4, "silu", fused=True,
+                     forward_all=False, rows=True)
+    y = run.forward(x.to(DEV)).clone()
+    raw = run.s_all.double().flatten(2)
+    mean, var = raw.mean(2), raw.var(2, unbiased=False)
+    assert_close(run.stats[..., 0], mean, rtol=1e-6, atol=1e-6, what="mean")
+    assert_close(run.stats[..., 1], (var + run.ln_eps).rsqrt(), rtol=1e-6, atol=0, what="rstd")
+    last = (run.s_all[2] - run.stats[2, :, 0].view(-1, 1, 1, 1)) * run.stats[2, :, 1].view(-1, 1, 1, 1)
+    assert_close(y, (last * run.gamma + run.beta).double(), rtol=1e-6, atol=1e-6, what="y")
+    dx = run.backward(gy.to(DEV))[-1].clone()
+    assert torch.equal(run.backward(gy.to(DEV))[-1], dx)
+    # the first step's input gradient from the second's: backward once more in one step of its own
+    step = BodyRunner(*(t.to(DEV) for t in (*make_params(shape, seed=4), gamma, beta)), batch, 1, 1, 4, "silu", fused=True,
+                      forward_all=False, rows=True)
+    h, grad = [x.to(DEV)], gy.to(DEV)
+    for _ in range(2):
+        h.append(step.forward(h[-1]).clone())
+    for j in (2, 1, 0):  # every step's LayerNorm sums by the kernel for the last one
+        step.forward(h[j])
+        grad = step.backward(grad)[-1].clone()
+    assert_close(dx, grad.double(), rtol=1e-5, atol=1e-5, what="dx")

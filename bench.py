@@ -111,6 +111,8 @@ def gpu_run(wl, steps, warmup, fused, graph_replay=True, chain_all=None, chain=N
     whole = {}
     if getattr(run, "rows", False):
         whole = dict.fromkeys(("step_fwd", "step_bwd"), "whole chain in one call, a kernel per step and direction")
+    if getattr(run, "merges", False):
+        whole["step_fwd"] = "whole chain in one call, a kernel per step"
     if getattr(run, "forward_all", False):
         whole["step_fwd"] = "forward of the chain in one launch"
     if getattr(run, "chain_all", False):

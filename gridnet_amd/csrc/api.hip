@@ -102,7 +102,7 @@ extern "C" {
 
 // 2: fused body; 3: residual forward and backward; 4: gated backward takes a workspace; 5: backward on static
 // scratch; 6: chain backward, gradient copies for split batches; 7: whole chain in one launch; 8: fused
-// forward with flags; 9: forward of a chain in one launch, chains by whole rows, GRIDNET_OVERWRITE_STEP_PARAMS
+// forward with flags; 9: forward of a chain in one launch, chains by whole rows, GRIDNET_OVERWRITE_STEP_PARAMS; 10: fused forward of a chain
 int gridnet_hip_version(void) { return GRIDNET_HIP_VERSION; }
 
 const char *gridnet_hip_last_error(void) { return error_buffer(); }
@@ -416,6 +416,69 @@ int gridnet_hip_fused_forward_flags(int dtype, const void *weight, const void *b
     return fused_forward(dtype, weight, bias, scale, gamma, beta, x, x_stats, y, y_stats, B, M, N, K, inner,
                          block_size, ln_eps, activation, workspace, workspace_bytes, stream,
                          (flags & GRIDNET_FUSED_RESIDUAL) ? 1 : 0, (flags & GRIDNET_FUSED_WALK_REVERSE) ? 1 : 0);
+}
+
+static StepArgs fused_chain_args(int B, int M, int N, int K, int inner, int block_size) {
+    StepArgs a{};
+    a.dtype = GRIDNET_F32; a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner; a.block_size = block_size;
+    a.activation = GRIDNET_ACT_RELU;
+    a.ln.gamma = (const float *)&a;  // only whether there is one matters
+    return a;
+}
+
+int gridnet_hip_fused_forward_chain_merges(int dtype, int B, int M, int N, int K, int inner, int block_size) {
+    if (dtype != GRIDNET_F32 || block_size != 8 || B <= 0 || M <= 0 || N <= 0 || K <= 0 || M % 8 || N % 8 || K % 8 ||
+        inner < 1 || (long)M * N * K * 27 >= (1L << 31))
+        return 0;
+    return step_fast_merge_lanes(fused_chain_args(B, M, N, K, inner, block_size)) > 0;
+}
+
+size_t gridnet_hip_fused_forward_chain_workspace_bytes(int B, int M, int N, int K, int inner, int block_size) {
+    if (B <= 0 || M <= 0 || N <= 0 || K <= 0 || (block_size != 4 && block_size != 8)) return 0;
+    return 2 * ((fused_forward_workspace(fused_chain_args(B, M, N, K, inner, block_size)) + 255) / 256 * 256);
+}
+
+int gridnet_hip_fused_forward_chain(int dtype, const void *const *weight, const void *const *bias,
+                                    const void *const *scale, const void *gamma, const void *beta, const void *x0,
+                                    void *const *y_raw, void *const *y_stats, int B, int M, int N, int K, int inner,
+                                    int outer, int block_size, double ln_eps, int activation, void *workspace,
+                                    size_t workspace_bytes, void *stream) {
+    if (outer < 1) return fail(GRIDNET_ERR_ARGUMENT, "outer must be at least 1, got %d", outer);
+    if (!weight || !bias || !scale || !y_raw || !y_stats) return fail(GRIDNET_ERR_ARGUMENT, "null pointer");
+    StepArgs a{};
+    a.dtype = dtype; a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner; a.block_size = block_size;
+    a.activation = activation;
+    for (int j = 0; j < outer; ++j) {  // everything is looked at before anything is launched
+        a.weight = weight[j]; a.bias = bias[j]; a.scale = scale[j]; a.x = j ? y_raw[j - 1] : x0; a.y = y_raw[j];
+        if (int rc = check_fused(a, false)) return rc;
+        if (B > 0 && (!gamma || !beta || !y_stats[j])) return fail(GRIDNET_ERR_ARGUMENT, "null pointer");
+    }
+    if (B == 0) return GRIDNET_OK;
+    const size_t need = gridnet_hip_fused_forward_chain_workspace_bytes(B, M, N, K, inner, block_size);
+    if (!workspace || workspace_bytes < need)
+        return fail(GRIDNET_ERR_WORKSPACE, "fused forward chain needs %zu bytes of workspace, got %zu", need,
+                    workspace ? workspace_bytes : (size_t)0);
+    hipStream_t st = (hipStream_t)stream;
+    float *parts[2] = {(float *)workspace, (float *)((char *)workspace + need / 2)};
+    a.ln.gamma = (const float *)gamma;
+    a.ln.beta = (const float *)beta;
+    a.ln.merge_lanes = step_fast_merge_lanes(a);
+    a.ln.x_eps = ln_eps;
+    for (int j = 0; j < outer; ++j) {
+        a.weight = weight[j]; a.bias = bias[j]; a.scale = scale[j]; a.x = j ? y_raw[j - 1] : x0; a.y = y_raw[j];
+        const bool merge = j && a.ln.merge_lanes;
+        a.ln.x_pairs = merge ? parts[(j - 1) & 1] : nullptr;
+        a.ln.x_stats_out = merge ? (float *)y_stats[j - 1] : nullptr;
+        a.ln.x_stats = j && !merge ? (const float *)y_stats[j - 1] : nullptr;
+        a.ln.y_part = parts[j & 1];
+        a.ln.walk_reverse = j & 1;
+        if (int rc = step_forward_fast(a, st)) return rc;
+        if (a.ln.merge_lanes && j + 1 < outer) continue;
+        if (int rc = layernorm_finalize_stats(parts[j & 1], step_fast_forward_pairs(a), step_fast_forward_pair_count(a),
+                                              (float *)y_stats[j], B, ln_eps, st))
+            return rc;
+    }
+    return GRIDNET_OK;
 }
 
 int gridnet_hip_fused_forward_residual(int dtype, const void *weight, const void *bias,

@@ -15,7 +15,7 @@
 //   * Where the batch is split over workgroups every chunk keeps ONE copy of the gradient arrays for the
 //     whole chain, each step adding its sums to what the step before left; the copies are added up once.
 //   * The pairs per wave behind the LayerNorms' per-sample numbers are merged by the workgroups of the next
-//     step while their weights are on their way (merge_lanes says where; a small kernel between the steps
+//     step while their weights are on their way (plan_merge_lanes says where; a small kernel between the steps
 //     elsewhere, 4.7 us each).  Merged inside the walk, by one wave an element ahead, they cost the kernels
 //     11 us forward and 24 us backward: everybody waits for that wave at the barrier.
 // 32^3, batch 256, silu, per step: forward 28.3 us, backward 68.3, at 4.3 TB/s either way where a copy
@@ -100,38 +100,6 @@ __device__ __forceinline__ float2 load_pair_ahead(const float *pairs, int sample
     return make_float2(v[0], v[1]);
 }
 
-// The pairs per wave that the launch before left, [B][pairs][2], merged by the workgroup that walks the
-// samples s0 ... s0 + len: `lanes` threads (a power of two) to a sample, in double, a fixed order.  `finish`
-// gets the three sums of sample s0 + e: of the first numbers, the second, and the squares of the first.
-// AHEAD pieces of two pairs are requested at a time.
-template <int AHEAD, typename Finish>
-__device__ __forceinline__ void merge_pairs(const float *part, int pairs, int lanes, int s0, int len, Finish finish) {
-    const int q = threadIdx.x & (lanes - 1), shift = 31 - __builtin_clz(lanes), half = pairs / 2;
-    for (int e = (int)threadIdx.x >> shift; e < len; e += (int)blockDim.x >> shift) {
-        const float4 *from = reinterpret_cast<const float4 *>(part + 2L * (s0 + e) * pairs);
-        double a = 0.0, b = 0.0, c = 0.0;
-        for (int i0 = q; i0 < half; i0 += lanes * AHEAD) {
-            float4 v[AHEAD];
-#pragma unroll
-            for (int k = 0; k < AHEAD; ++k) v[k] = from[min(i0 + k * lanes, half - 1)];
-#pragma unroll
-            for (int k = 0; k < AHEAD; ++k) {
-                const bool in = i0 + k * lanes < half;
-                const double x = in ? v[k].x : 0.f, y = in ? v[k].y : 0.f, z = in ? v[k].z : 0.f, w = in ? v[k].w : 0.f;
-                a += x + z;
-                b += y + w;
-                c = fma(x, x, fma(z, z, c));
-            }
-        }
-        for (int m = 1; m < lanes; m *= 2) {
-            a += __shfl_xor(a, m);
-            b += __shfl_xor(b, m);
-            c += __shfl_xor(c, m);
-        }
-        if (q == 0) finish(e, a, b, c);
-    }
-}
-
 struct RowsFwdArgs {
     const float *weight, *bias, *scale, *gamma, *beta, *x;
     const float *x_stats;   // the LayerNorm in front of the step (null: x is used as it is)
@@ -177,8 +145,7 @@ void rows_fwd(RowsFwdArgs a) {
     if constexpr (MERGE) {  // while the parameters are on their way
         const double n = (double)a.ntube * nw, count = cells / n;
         merge_pairs<4>(a.x_part, a.ntube * nw, a.lanes, s0, s1 - s0, [&](int e, double m, double q, double mm) {
-            const double mean = m / n, var = (q + count * (mm - n * mean * mean)) / (n * count);
-            const float2 v = make_float2((float)mean, (float)(1.0 / sqrt((var > 0.0 ? var : 0.0) + a.eps)));
+            const float2 v = merged_statistics(m, q, mm, n, count, a.eps);
             stat[e] = v;
             if (tube == 0 && a.stats_out) reinterpret_cast<float2 *>(a.stats_out)[s0 + e] = v;
         });
@@ -710,20 +677,6 @@ template <typename K> int workgroups_per_cu(K kern, int threads, size_t lds) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)kern, threads, lds) != hipSuccess || n < 1) n = 1;
     return n;
 }
-// Threads to a sample where the workgroups of a step merge the pairs of the step before, beside the fetch of
-// their weights; 0: a kernel of its own does (4.7 us and a launch).  Every workgroup of a chunk merges the
-// same pairs, so it pays as long as they are few per thread.  Forward / backward of a step with the kernel and
-// without: 32^3, batch 16, 10.5 -> 8.7 / 17.1 -> 15.8 us; batch 64, 15.9 -> 13.7 / 31.9 -> 30.7; batch 256 (22 and 32
-// pairs per thread) 30.4 -> 28.3 / 69.0 -> 68.3; 64^3, batch 32 (44 pairs) 30.7 -> 32.1 / 74.0 -> 74.6.  Gated, 32^3,
-// batch 32, 17.1 -> 15.4 / 26.3 -> 25.3; batch 256, 57.0 -> 55.5 forward.
-constexpr int kMergeMostSamples = 64, kMergeMostPairs = 32;  // per workgroup; per thread
-int merge_lanes(int threads, int chunk_len, int pairs) {
-    if (pairs % 2 || chunk_len > kMergeMostSamples) return 0;
-    int lanes = 1;
-    while (2 * lanes * chunk_len <= threads && 4 * lanes <= pairs && lanes < kWave) lanes *= 2;
-    return (long)chunk_len * pairs <= kMergeMostPairs * (long)threads ? lanes : 0;
-}
-
 template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &c, hipStream_t st) {
     const auto kern = rows_fwd<ACT, SETS, SAVE, K, false>, merging = rows_fwd<ACT, SETS, SAVE, K, true>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
@@ -733,7 +686,7 @@ template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &
     if (per_cu == 0) per_cu = workgroups_per_cu(kern, nt, lds);
     RowsFwdArgs a{};
     a.nchunk = plan_row_chunks(c.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, a.chunk_len);
-    a.lanes = merge_lanes(nt, a.chunk_len, pairs);
+    a.lanes = plan_merge_lanes(nt, a.chunk_len, pairs);
     a.eps = c.eps;
     a.weight = c.weight; a.bias = c.bias; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
     a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
@@ -787,7 +740,7 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
     }
     RowsBwdArgs a{};
     a.nchunk = bwd_chunks(c, per_cu, a.chunk_len);
-    a.lanes = merge_lanes(nt, a.chunk_len, pairs);
+    a.lanes = plan_merge_lanes(nt, a.chunk_len, pairs);
     a.weight = c.weight; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
     a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
     // workspace: the pairs, the sums, scratch of the last LayerNorm's sums, a second dx, the copies

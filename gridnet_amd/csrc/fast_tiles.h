@@ -173,6 +173,44 @@ __device__ __forceinline__ float load_ahead(const float *p, int i) {
     return p[i + zero];
 }
 
+// The pairs per wave that the launch before left, [B][pairs][2], merged by the workgroup that walks the
+// samples s0 ... s0 + len: `lanes` threads (a power of two) to a sample, in double, a fixed order.  `finish`
+// gets the three sums of sample s0 + e: of the first numbers, the second, and the squares of the first.
+// AHEAD pieces of two pairs are requested at a time.
+template <int AHEAD, typename Finish>
+__device__ __forceinline__ void merge_pairs(const float *part, int pairs, int lanes, int s0, int len, Finish finish) {
+    const int q = threadIdx.x & (lanes - 1), shift = 31 - __builtin_clz(lanes), half = pairs / 2;
+    for (int e = (int)threadIdx.x >> shift; e < len; e += (int)blockDim.x >> shift) {
+        const float4 *from = reinterpret_cast<const float4 *>(part + 2L * (s0 + e) * pairs);
+        double a = 0.0, b = 0.0, c = 0.0;
+        for (int i0 = q; i0 < half; i0 += lanes * AHEAD) {
+            float4 v[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) v[k] = from[min(i0 + k * lanes, half - 1)];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                const bool in = i0 + k * lanes < half;
+                const double x = in ? v[k].x : 0.f, y = in ? v[k].y : 0.f, z = in ? v[k].z : 0.f, w = in ? v[k].w : 0.f;
+                a += x + z;
+                b += y + w;
+                c = fma(x, x, fma(z, z, c));
+            }
+        }
+        for (int m = 1; m < lanes; m *= 2) {
+            a += __shfl_xor(a, m);
+            b += __shfl_xor(b, m);
+            c += __shfl_xor(c, m);
+        }
+        if (q == 0) finish(e, a, b, c);
+    }
+}
+// (mean, rstd) from those sums of (mean_i, M2_i) pairs, `n` of them over `count` cells each: as the kernel
+// that does it alone (layernorm.hip)
+__device__ __forceinline__ float2 merged_statistics(double m, double q, double mm, double n, double count, double eps) {
+    const double mean = m / n, var = (q + count * (mm - n * mean * mean)) / (n * count);
+    return make_float2((float)mean, (float)(1.0 / sqrt((var > 0.0 ? var : 0.0) + eps)));
+}
+
 // Wait for every global load issued so far (s_waitcnt vmcnt(0) only).  Placed once after the
 // per-workgroup parameter loads: with those known complete, the waits the compiler inserts
 // inside the batch loop no longer cover the prefetch of the next batch element as well.

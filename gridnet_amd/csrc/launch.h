@@ -50,6 +50,12 @@ struct LnFold {
     // whose steps alternate finds what the step before touched last (its output, the parameter
     // planes it fetched last) still in the last-level cache when its working set exceeds that cache.
     int walk_reverse;
+    // forward, instead of x_stats: the pairs that the forward of the step before left as its y_part, merged by the
+    // workgroups of this one (step_fast_merge_lanes) and left in x_stats_out
+    const float *x_pairs;
+    float *x_stats_out;  // [B,2]
+    int merge_lanes;
+    double x_eps;
 };
 
 struct StepArgs {
@@ -154,6 +160,9 @@ int step_backward_fast(const StepArgs &a, hipStream_t st);
 // partial statistics per (block, batch element) that the kernels above write when asked to
 int step_fast_forward_parts(int block_size);   // (mean, M2) pairs per block at most, each over forward_part_count cells
 int step_fast_forward_part_count(int block_size);
+// threads to a sample with which the forward of a chain's step merges the pairs of the step before (LnFold::x_pairs);
+// 0: it does not, they go through layernorm_finalize_stats
+int step_fast_merge_lanes(const StepArgs &a);
 int step_fast_forward_pairs(const StepArgs &a);       // pairs per sample that the forward of `a` leaves ...
 int step_fast_forward_pair_count(const StepArgs &a);  // ... and the cells behind each
 int step_fast_backward_parts(int block_size);  // (sum g, sum g*xhat) pairs per (block, element), at most

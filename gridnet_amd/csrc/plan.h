@@ -74,6 +74,20 @@ int plan_row_chunks(int B, int ntube, int resident, int min_walk, int &chunk_len
     return (B + chunk_len - 1) / chunk_len;
 }
 
+// Threads to a sample where the workgroups of a step merge the pairs of the step before, beside the fetch of
+// their weights; 0: a kernel of its own does (4.7 us and a launch).  Every workgroup of a chunk merges the
+// same pairs, so it pays as long as they are few per thread.  Forward / backward of a step with the kernel and
+// without: 32^3, batch 16, 10.5 -> 8.7 / 17.1 -> 15.8 us; batch 64, 15.9 -> 13.7 / 31.9 -> 30.7; batch 256 (22 and 32
+// pairs per thread) 30.4 -> 28.3 / 69.0 -> 68.3; 64^3, batch 32 (44 pairs) 30.7 -> 32.1 / 74.0 -> 74.6.  Gated, 32^3,
+// batch 32, 17.1 -> 15.4 / 26.3 -> 25.3; batch 256, 57.0 -> 55.5 forward.
+constexpr int kMergeMostSamples = 64, kMergeMostPairs = 32;  // per workgroup; per thread
+int plan_merge_lanes(int threads, int chunk_len, int pairs) {
+    if (pairs % 2 || chunk_len > kMergeMostSamples) return 0;
+    int lanes = 1;
+    while (2 * lanes * chunk_len <= threads && 4 * lanes <= pairs && lanes < kWave) lanes *= 2;
+    return (long)chunk_len * pairs <= kMergeMostPairs * (long)threads ? lanes : 0;
+}
+
 __global__ void plan_fill_zero_f32(float *p, long n) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long stride = (long)gridDim.x * blockDim.x;

@@ -293,7 +293,16 @@ __device__ __forceinline__ float partner_lane(float v) {
 
 // LN, RES: the variants with the LayerNorm of the network body folded in, as in step_fwd_fast.
 // NORM: per-window normalisation, as in step_fwd_fast (running sums, unchanged stencil).
-template <int ACT, bool LN, bool RES = false, bool NORM = false>
+// The statistics of this workgroup's samples from the pairs of the step before, beside the fetch of its weights.
+__device__ __forceinline__ void merge_statistics(const LnFold &ln, int pairs, bool leave, int s0, int len, float2 *stat) {
+    merge_pairs<4>(ln.x_pairs, pairs, ln.merge_lanes, s0, len, [&](int e, double m, double q, double mm) {
+        stat[e] = merged_statistics(m, q, mm, pairs, 256.0, ln.x_eps);
+        if (leave) reinterpret_cast<float2 *>(ln.x_stats_out)[s0 + e] = stat[e];
+    });
+}
+
+// MERGE (with LN): x_stats from the pairs of the step before.
+template <int ACT, bool LN, bool RES = false, bool NORM = false, bool MERGE = false>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(NORM ? 2 : 3)))
 void step_fwd_split(
     const float *__restrict__ weight, const float *__restrict__ bias,
@@ -312,7 +321,8 @@ void step_fwd_split(
     float *back = lds + 4 * SW::COPY;  // RES (which comes with LN)
     float *sums_at_commit = lds + 2 * SW::COPY, *own_sums = sums_at_commit + 8;  // NORM: [2][4], [2][2][2]
     const int wave = threadIdx.x >> 6;
-    const bool ln_in = LN && ln.x_stats != nullptr;  // x is the raw output of the step before
+    __shared__ float2 stat[MERGE ? kMergeMostSamples : 1];
+    const bool ln_in = LN && (MERGE || ln.x_stats != nullptr);  // x is the raw output of the step before
 
     int blk, chunk;
     if (!split_block_id(ln.walk_reverse ? reversed_on_its_xcd(blockIdx.x, gridDim.x) : blockIdx.x, nblk, nchunk,
@@ -363,6 +373,7 @@ void step_fwd_split(
             rv[r] = second ? rt[3 - r] : rt[r];
         }
     }
+    if constexpr (MERGE) merge_statistics(ln, 2 * nblk, blk == 0, chunk * chunk_len, min(chunk_len, B - chunk * chunk_len), stat);
     float wsum[4];  // NORM: sum of the 27 weights of every owned cell
     if (NORM) {
 #pragma unroll
@@ -449,7 +460,10 @@ void step_fwd_split(
     float pre_mean = 0.f, pre_rstd = 1.f;  // LayerNorm statistics of the element in `pre`
     auto fetch_element = [&](int s) {
         fx.fetch(x + s * cells, pre);
-        if (ln_in) {
+        if (MERGE) {
+            pre_mean = stat[s - s0].x;
+            pre_rstd = stat[s - s0].y;
+        } else if (ln_in) {
             pre_mean = load_ahead(ln.x_stats, 2 * s);
             pre_rstd = load_ahead(ln.x_stats, 2 * s + 1);
         }
@@ -580,7 +594,7 @@ void step_fwd_split(
 // larger workgroups the 29 parameter planes of a block are fetched twice per launch instead of
 // three times (64^3 grid, batch 32).  Two waves per SIMD instead of three: the second element's
 // state and prefetch need the registers.
-template <int ACT>
+template <int ACT, bool MERGE>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
 void step_fwd_pair(
     const float *__restrict__ weight, const float *__restrict__ bias,
@@ -593,7 +607,8 @@ void step_fwd_pair(
     // per element two copies of the window; then gamma and beta laid out alike
     __shared__ __attribute__((aligned(16))) float lds[(2 * E + 2) * SW::COPY];
     float *gwin = lds + 2 * E * SW::COPY, *bwin = gwin + SW::COPY;
-    const bool ln_in = ln.x_stats != nullptr;  // x is the raw output of the step before
+    __shared__ float2 stat[MERGE ? kMergeMostSamples : 1];
+    const bool ln_in = MERGE || ln.x_stats != nullptr;  // x is the raw output of the step before
 
     int blk, chunk;
     if (!split_block_id(ln.walk_reverse ? reversed_on_its_xcd(blockIdx.x, gridDim.x) : blockIdx.x, nblk, nchunk,
@@ -639,6 +654,7 @@ void step_fwd_pair(
             rv[r] = second ? rt[3 - r] : rt[r];
         }
     }
+    if constexpr (MERGE) merge_statistics(ln, 2 * nblk, blk == 0, chunk * chunk_len, min(chunk_len, B - chunk * chunk_len), stat);
     auto commit = [&](float *to, int copies, const typename FX::Buf &v, bool fold, float mean, float rstd) {
 #pragma unroll
         for (int e = 0; e < FX::RPT; ++e)
@@ -689,8 +705,8 @@ void step_fwd_pair(
         for (int e = 0; e < E; ++e) {
             const int sc = min(s + e, s1 - 1);
             fx.fetch(x + sc * cells, pre[e]);
-            pre_mean[e] = ln_in ? load_ahead(ln.x_stats, 2 * sc) : 0.f;
-            pre_rstd[e] = ln_in ? load_ahead(ln.x_stats, 2 * sc + 1) : 1.f;
+            pre_mean[e] = MERGE ? stat[sc - s0].x : ln_in ? load_ahead(ln.x_stats, 2 * sc) : 0.f;
+            pre_rstd[e] = MERGE ? stat[sc - s0].y : ln_in ? load_ahead(ln.x_stats, 2 * sc + 1) : 1.f;
         }
     };
     if (s0 < s1) fetch_pair(s0);
@@ -1674,6 +1690,13 @@ Plan make_plan(const StepArgs &a, int nslot, int resident, bool whole_batch_per_
     return p;
 }
 
+// the statistics that a workgroup merges have kMergeMostSamples places in its LDS (an even number)
+void most_samples(int B, Plan &p) {
+    if (p.chunk_len <= kMergeMostSamples) return;
+    p.chunk_len = kMergeMostSamples;
+    p.nchunk = (B + p.chunk_len - 1) / p.chunk_len;
+}
+
 constexpr int kMinForwardWalk = 4;  // elements that a chunk made shorter to even the rounds still walks
 
 template <int BS, int CPT, int NSLOT, int ACT, bool LN, bool RES = false, bool NORM = false>
@@ -1696,9 +1719,9 @@ int launch_fwd_ln(const StepArgs &a, hipStream_t st) {
                        p.chunk_len, a.ln, (float)a.eps);
     return check_launch("step_fwd_fast");
 }
-template <int ACT, bool LN, bool RES = false, bool NORM = false>
+template <int ACT, bool LN, bool RES = false, bool NORM = false, bool MERGE = false>
 int launch_fwd_split(const StepArgs &a, hipStream_t st) {
-    auto kern = step_fwd_split<ACT, LN, RES, NORM>;
+    auto kern = step_fwd_split<ACT, LN, RES, NORM, MERGE>;
     static int per_cu = 0;
     if (per_cu == 0) {
         int n = 0;
@@ -1707,14 +1730,15 @@ int launch_fwd_split(const StepArgs &a, hipStream_t st) {
     }
     Plan p = make_plan(a, 1, per_cu * device_cus(), false);
     plan_even_rounds(a.B, p.nblk, 1, per_cu * device_cus(), kMinForwardWalk, p.nchunk, p.chunk_len);
+    if (MERGE) most_samples(a.B, p);
     hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(128), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
                        (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
                        p.chunk_len, a.ln, (float)a.eps);
     return check_launch("step_fwd_split");
 }
-template <int ACT> int launch_fwd_pair(const StepArgs &a, hipStream_t st) {
-    auto kern = step_fwd_pair<ACT>;
+template <int ACT, bool MERGE> int launch_fwd_pair(const StepArgs &a, hipStream_t st) {
+    auto kern = step_fwd_pair<ACT, MERGE>;
     static int per_cu = 0;
     if (per_cu == 0) {
         int n = 0;
@@ -1723,12 +1747,26 @@ template <int ACT> int launch_fwd_pair(const StepArgs &a, hipStream_t st) {
     }
     Plan p = make_plan(a, 2, per_cu * device_cus(), false);
     plan_even_rounds(a.B, p.nblk, 2, per_cu * device_cus(), kMinForwardWalk, p.nchunk, p.chunk_len);
+    if (MERGE) most_samples(a.B, p);
     hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(128), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
                        (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
                        p.chunk_len, a.ln);
     return check_launch("step_fwd_pair");
 }
+// The chain's forward on SMALL grids (fewer blocks than a sixth of the workgroups the chip
+// holds, so that a workgroup of step_fwd_split gets four batch elements or fewer for one fetch
+// of its 29 parameter planes): two elements per pass.  Measured with 3 waves per SIMD for
+// step_fwd_split: 32^3 grid, batch 64: 0.279 -> 0.238 ms per 8-step chain; on larger grids the
+// lower occupancy of the pair kernel costs more than it brings (64^3 / batch 32: 66 -> 69 us
+// per step, 128^3 / batch 8: 2.61 -> 3.00 ms per 16-step chain).
+bool walks_pairs(const StepArgs &a) {
+    if (a.block_size != 8 || !a.ln.gamma || a.ln.residual || a.B < 2 || a.inner < 1) return false;
+    const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
+    const int chunks = 6 * device_cus() / nblk;  // what step_fwd_split's plan would use
+    return chunks >= 1 && (a.B + chunks - 1) / chunks <= 4;
+}
+
 template <int BS, int CPT, int NSLOT, int ACT> int launch_fwd(const StepArgs &a, hipStream_t st) {
     if (a.normalize) {
         if (BS == 8) return launch_fwd_split<ACT, false, false, true>(a, st);
@@ -1738,17 +1776,9 @@ template <int BS, int CPT, int NSLOT, int ACT> int launch_fwd(const StepArgs &a,
         if (BS == 8) return launch_fwd_split<ACT, true, true>(a, st);
         return launch_fwd_ln<BS, CPT, NSLOT, ACT, true, true>(a, st);
     }
-    // The chain's forward on SMALL grids (fewer blocks than a sixth of the workgroups the chip
-    // holds, so that a workgroup of step_fwd_split gets four batch elements or fewer for one fetch
-    // of its 29 parameter planes): two elements per pass.  Measured with 3 waves per SIMD for
-    // step_fwd_split: 32^3 grid, batch 64: 0.279 -> 0.238 ms per 8-step chain; on larger grids the
-    // lower occupancy of the pair kernel costs more than it brings (64^3 / batch 32: 66 -> 69 us
-    // per step, 128^3 / batch 8: 2.61 -> 3.00 ms per 16-step chain).
-    if (BS == 8 && a.ln.gamma && a.B >= 2 && a.inner >= 1) {
-        const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
-        const int chunks = 6 * device_cus() / nblk;  // what step_fwd_split's plan would use
-        if (chunks >= 1 && (a.B + chunks - 1) / chunks <= 4) return launch_fwd_pair<ACT>(a, st);
-    }
+    if (BS == 8 && walks_pairs(a))
+        return a.ln.x_pairs ? launch_fwd_pair<ACT, true>(a, st) : launch_fwd_pair<ACT, false>(a, st);
+    if (BS == 8 && a.ln.gamma && a.ln.x_pairs) return launch_fwd_split<ACT, true, false, false, true>(a, st);
     if (BS == 8) return a.ln.gamma ? launch_fwd_split<ACT, true>(a, st) : launch_fwd_split<ACT, false>(a, st);
     if (a.ln.gamma) return launch_fwd_ln<BS, CPT, NSLOT, ACT, true>(a, st);
     return launch_fwd_ln<BS, CPT, NSLOT, ACT, false>(a, st);
@@ -1927,6 +1957,13 @@ int step_fast_forward_pairs(const StepArgs &a) {
 }
 int step_fast_forward_pair_count(const StepArgs &a) {
     return fwd_rows_supports(a) ? fwd_rows_pair_count(a) : step_fast_forward_part_count(a.block_size);
+}
+int step_fast_merge_lanes(const StepArgs &a) {
+    if (a.block_size != 8 || a.ln.residual || a.normalize || fwd_rows_supports(a)) return 0;
+    // the chunks are those of the launches above: six or, in pairs of elements, four workgroups per CU
+    const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8), nslot = walks_pairs(a) ? 2 : 1;
+    Plan p = make_plan(a, nslot, (nslot == 2 ? 4 : 6) * device_cus(), false);
+    return plan_merge_lanes(128, p.chunk_len, 2 * nblk);
 }
 int step_fast_backward_parts(int block_size) { return block_size == 8 ? 2 : 1; }
 int step_fast_backward_pairs(const StepArgs &a) {

@@ -39,6 +39,9 @@ EXPORTS = (
     "gridnet_hip_layernorm_forward",
     "gridnet_hip_layernorm_backward",
     "gridnet_hip_fused_workspace_bytes",
+    "gridnet_hip_fused_forward_chain_merges",
+    "gridnet_hip_fused_forward_chain_workspace_bytes",
+    "gridnet_hip_fused_forward_chain",
     "gridnet_hip_fused_forward",
     "gridnet_hip_fused_forward_residual",
     "gridnet_hip_fused_forward_flags",
@@ -105,6 +108,12 @@ def _load():
     lib.gridnet_hip_layernorm_backward.argtypes = [i, p, p, p, p, p, p, p, p, i, l, i, p, z, p]
     lib.gridnet_hip_fused_workspace_bytes.restype = z
     lib.gridnet_hip_fused_workspace_bytes.argtypes = [i, i, i, i, i, i, i]
+    lib.gridnet_hip_fused_forward_chain_merges.restype = i
+    lib.gridnet_hip_fused_forward_chain_merges.argtypes = [i] * 7
+    lib.gridnet_hip_fused_forward_chain_workspace_bytes.restype = z
+    lib.gridnet_hip_fused_forward_chain_workspace_bytes.argtypes = [i] * 6
+    lib.gridnet_hip_fused_forward_chain.restype = i
+    lib.gridnet_hip_fused_forward_chain.argtypes = [i] + [ctypes.POINTER(p)] * 3 + [p] * 3 + [ctypes.POINTER(p)] * 2 + [i] * 7 + [d, i, p, z, p]
     lib.gridnet_hip_fused_forward.restype = i
     lib.gridnet_hip_fused_forward.argtypes = [i, p, p, p, p, p, p, p, p, p, i, i, i, i, i, i, d, i,
                                               p, z, p]
@@ -195,6 +204,11 @@ def check_input(t: torch.Tensor, name: str) -> None:
         raise RuntimeError(f"{name} must be a CUDA tensor")
     if not t.is_contiguous():
         raise RuntimeError(f"{name} must be contiguous")
+
+
+def pointers(tensors):
+    """Their device addresses, as an array in host memory."""
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
 
 
 def current_stream(t: torch.Tensor) -> int:

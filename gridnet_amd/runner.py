@@ -29,6 +29,9 @@ weights and gradient accumulators from step to step and signal each other throug
 waits are bounded; ``chain_all_status()`` (which synchronises) tells whether one ran out, in which
 case ``backward`` must be repeated with ``chain_all`` off -- ``backward_checked`` does both.
 
+On grids of few blocks (32^3; larger ones with few samples) the launch-by-launch forward goes through
+``gridnet_hip_fused_forward_chain``, whose steps finish the LayerNorm statistics of the step before.
+
 Where blocks and batch are few enough to be resident at once (a 32^3 grid at up to 8 samples) the
 forward of a chain with one parameter set is one launch too (``gridnet_hip_chain_forward_all``;
 ``forward_all=False``: never).
@@ -116,6 +119,9 @@ class BodyRunner:
             not (backward and (chain or chain_all)) and
             _n.lib.gridnet_hip_rows_chain_supported(self.dt, self.M, self.N, self.K, inner, self.normalize, 0) and
             (rows or not backward or room_for(2 * outer * batch * n * weight.element_size(), dev)))
+        self.merges = bool(
+            fused and not outer_residual and not self.forward_all and not self.rows and outer > 1 and
+            _n.lib.gridnet_hip_fused_forward_chain_merges(self.dt, batch, self.M, self.N, self.K, inner, block_size))
         n_h, n_s = keep + 1, keep
         if fused and not outer_residual:
             whole = self.forward_all or self.rows  # keep the values between the steps themselves
@@ -158,6 +164,9 @@ class BodyRunner:
             elif self.rows:
                 self.fw_ws_bytes = _n.lib.gridnet_hip_rows_chain_workspace_bytes(
                     batch, self.M, self.N, self.K, 0, int(backward), 0)
+            elif self.merges:
+                self.fw_ws_bytes = _n.lib.gridnet_hip_fused_forward_chain_workspace_bytes(
+                    batch, self.M, self.N, self.K, inner, block_size)
             else:
                 self.fw_ws_bytes = _n.lib.gridnet_hip_fused_workspace_bytes(
                     batch, self.M, self.N, self.K, inner, block_size, 0)
@@ -262,6 +271,17 @@ class BodyRunner:
                 self.fw_ws.data_ptr(), self.fw_ws_bytes, stream))
             self._mark("step_fwd", 1)
             return self.h[0]
+        if self.merges:
+            ys = [self.s[j] if keep else (self.s[0], self.h[1])[j % 2] for j in range(self.outer)]
+            stats = [self.stats[j if keep else j % 2] for j in range(self.outer)]
+            self._mark("step_fwd", 0)
+            _n.check(_n.lib.gridnet_hip_fused_forward_chain(
+                self.dt, *(_n.pointers(t) for t in (self.ws, self.bs_, self.rs)), self.gamma.data_ptr(),
+                self.beta.data_ptr(), x0.data_ptr(), _n.pointers(ys), _n.pointers(stats), self.B, self.M, self.N,
+                self.K, self.inner, self.outer, self.bs, self.ln_eps, self.act, self.fw_ws.data_ptr(),
+                self.fw_ws_bytes, stream))
+            self._mark("step_fwd", 1)
+            return self._last_norm(ys[-1], stats[-1], stream)
         x, x_stats = x0, None
         for j in range(self.outer):
             # forward only: nothing is kept, two raw buffers and two statistics rows alternate
@@ -280,6 +300,9 @@ class BodyRunner:
                 self.fw_ws.data_ptr(), self.fw_ws_bytes, stream))
             self._mark("step_fwd", 1)
             x, x_stats = y, y_stats
+        return self._last_norm(x, x_stats, stream)
+
+    def _last_norm(self, x, x_stats, stream):
         out = self.h[0]
         self._mark("ln_fwd", 0)
         _n.check(_n.lib.gridnet_hip_layernorm_apply(

@@ -67,7 +67,7 @@ enum gridnet_flags {
 };
 
 /* Library build id (monotonic integer) -- lets a binding check it loaded what it expects. */
-#define GRIDNET_HIP_VERSION 9
+#define GRIDNET_HIP_VERSION 10
 int gridnet_hip_version(void);
 
 /* Thread-local message of the last non-zero status returned on this thread ("" if none). */
@@ -224,6 +224,20 @@ int gridnet_hip_fused_forward_flags(int dtype, const void *weight, const void *b
                                     const void *x_stats, void *y, void *y_stats, int B, int M, int N,
                                     int K, int inner, int block_size, double ln_eps, int activation,
                                     int flags, void *workspace, size_t workspace_bytes, void *stream);
+
+/* A chain of `outer` such steps, each on the output of the one before: step j with weight[j], bias[j], scale[j]
+ * (arrays in host memory, of device pointers; a chain with one parameter set repeats it) leaves y_raw[j] and
+ * y_stats[j].  Buffers may repeat from step to step as long as neighbouring steps have different ones.  On grids
+ * of few blocks the workgroups of a step finish the statistics of the step before beside the fetch of their
+ * parameters, and the launch between any two steps is saved: gridnet_hip_fused_forward_chain_merges() tells;
+ * elsewhere it is gridnet_hip_fused_forward_flags() `outer` times, every other step in reverse. */
+int gridnet_hip_fused_forward_chain_merges(int dtype, int B, int M, int N, int K, int inner, int block_size);
+size_t gridnet_hip_fused_forward_chain_workspace_bytes(int B, int M, int N, int K, int inner, int block_size);
+int gridnet_hip_fused_forward_chain(int dtype, const void *const *weight, const void *const *bias,
+                                    const void *const *scale, const void *gamma, const void *beta, const void *x0,
+                                    void *const *y_raw, void *const *y_stats, int B, int M, int N, int K, int inner,
+                                    int outer, int block_size, double ln_eps, int activation, void *workspace,
+                                    size_t workspace_bytes, void *stream);
 
 /* The reference's outer_residual form of one outer step, forward
  * (gridnet/scripts/train_imagenet.py:81-83: n = norm(h); h = h + (net(n) - n)):

@@ -599,7 +599,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
 void step_fwd_pair(
     const float *__restrict__ weight, const float *__restrict__ bias,
     const float *__restrict__ scale, const float *__restrict__ x, float *__restrict__ y, int B, int M,
-    int N, int K, int inner, int nblk, int nchunk, int chunk_len, LnFold ln) {
+    int N, int K, int inner, int nblk, int nchunk, int together, int chunk_len, LnFold ln) {
     using TL = Tile<8, 4>;
     using SW = SplitWin;
     using FX = Fetch<TL>;
@@ -611,8 +611,7 @@ void step_fwd_pair(
     const bool ln_in = MERGE || ln.x_stats != nullptr;  // x is the raw output of the step before
 
     int blk, chunk;
-    if (!split_block_id(ln.walk_reverse ? reversed_on_its_xcd(blockIdx.x, gridDim.x) : blockIdx.x, nblk, nchunk,
-                        blk, chunk))
+    if (!split_block_id(blockIdx.x, nblk, nchunk, together, ln.walk_reverse, blk, chunk))
         return;  // grid padding
     const Place<TL, 4, 1> pl(threadIdx.x, blk, N, K);
     const FX fx(pl.lane, pl.p0, pl.q0, pl.r0, M, N, K);
@@ -1748,9 +1747,10 @@ template <int ACT, bool MERGE> int launch_fwd_pair(const StepArgs &a, hipStream_
     Plan p = make_plan(a, 2, per_cu * device_cus(), false);
     plan_even_rounds(a.B, p.nblk, 2, per_cu * device_cus(), kMinForwardWalk, p.nchunk, p.chunk_len);
     if (MERGE) most_samples(a.B, p);
-    hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(128), 0, st,
+    const int together = cu_share(p.nblk, p.nchunk, per_cu);
+    hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk, together)), dim3(128), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
-                       (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
+                       (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk, together,
                        p.chunk_len, a.ln);
     return check_launch("step_fwd_pair");
 }

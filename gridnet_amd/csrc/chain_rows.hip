@@ -109,7 +109,7 @@ struct RowsFwdArgs {
     double eps;
     float *y, *y_part;
     float *saved;           // plain: [B,cells]; gated: [3][B,cells]; or null
-    int B, M, N, ntube, nchunk, chunk_len;
+    int B, M, N, ntube, nchunk, chunk_len, together;
 };
 
 // MERGE: the statistics of x from the pairs of the step before.  A kernel without it has none of that code: with
@@ -122,7 +122,7 @@ void rows_fwd(RowsFwdArgs a) {
     constexpr int CPT = 4 / SETS, RPT = 3;
     extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][36][K], gamma rows, beta rows, statistics
     int tube, chunk;
-    if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
+    if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, a.together, false, tube, chunk)) return;  // grid padding
     const int tid = threadIdx.x, M = a.M, N = a.N, nw = blockDim.x / 64, wave = tid / 64;
     const RowPlace<CPT, K> p(tid, tube, N);
     const long cells = (long)M * N * K;
@@ -340,7 +340,7 @@ struct RowsBwdArgs {
     float *dweight, *dbias, *dscale, *dgamma, *dbeta;
     long slab_stride;               // a copy of the gradient arrays per batch chunk (0: the arrays themselves)
     int accumulate;                 // on top of what the gradient arrays hold
-    int B, M, N, ntube, nchunk, chunk_len;
+    int B, M, N, ntube, nchunk, chunk_len, together;
 };
 
 // PLAIN: two cells per thread, GATED: one; 54 mirrored weights and 54 gradient accumulators for each set
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int CPT = 2 / SETS;
     extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K], then gamma and (plain) scale of the rows
     int tube, chunk;
-    if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, tube, chunk)) return;  // grid padding
+    if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, a.together, false, tube, chunk)) return;  // grid padding
     const int tid = threadIdx.x, M = a.M, N = a.N, nw = blockDim.x / 64, wave = tid / 64;
     const RowPlace<CPT, K> p(tid, tube, N);
     const long cells = (long)M * N * K, tensor = (long)a.B * cells;
@@ -677,6 +677,10 @@ template <typename K> int workgroups_per_cu(K kern, int threads, size_t lds) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)kern, threads, lds) != hipSuccess || n < 1) n = 1;
     return n;
 }
+// The chunks of a tube on one CU.  Per step, forward / backward: 32^3, batch 256, 29.1 -> 28.2 / 68.7 -> 67.0 us; batch
+// 64, 13.4 -> 13.1 / 29.9 -> 29.4.  Not with rows of 64 cells: 64^3, batch 32, forward 30.8 -> 32.5.
+template <int K> int rows_together(int ntube, int nchunk, int per_cu) { return K < 64 ? cu_share(ntube, nchunk, per_cu) : 0; }
+
 template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &c, hipStream_t st) {
     const auto kern = rows_fwd<ACT, SETS, SAVE, K, false>, merging = rows_fwd<ACT, SETS, SAVE, K, true>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
@@ -687,6 +691,7 @@ template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &
     RowsFwdArgs a{};
     a.nchunk = plan_row_chunks(c.B, ntube, per_cu * plan_device_cus(), kRowsMinWalk, a.chunk_len);
     a.lanes = plan_merge_lanes(nt, a.chunk_len, pairs);
+    a.together = rows_together<K>(ntube, a.nchunk, per_cu);
     a.eps = c.eps;
     a.weight = c.weight; a.bias = c.bias; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
     a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
@@ -741,6 +746,7 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
     RowsBwdArgs a{};
     a.nchunk = bwd_chunks(c, per_cu, a.chunk_len);
     a.lanes = plan_merge_lanes(nt, a.chunk_len, pairs);
+    a.together = rows_together<K>(ntube, a.nchunk, per_cu);
     a.weight = c.weight; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
     a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;
     // workspace: the pairs, the sums, scratch of the last LayerNorm's sums, a second dx, the copies

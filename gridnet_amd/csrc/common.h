@@ -239,26 +239,28 @@ __device__ __forceinline__ bool split_block_id(int wg, int nblk, int nchunk, int
     return slot / nchunk < per_xcd && blk < nblk;
 }
 
-// The same with the workgroups that share parameters on one CU: the chunks of a block, which fetch the same
-// planes.  An XCD deals its workgroups to its CUs in turn (seen in HW_ID on this part), so number s of an XCD meets
-// s + 32, s + 64, ... on its CU as long as the CUs fill up for the first time; `together` of them do (cu_share).
-// Nothing but the time depends on it.  For the kernel with many chunks per block (step_fwd_pair: 32^3, batch 64,
-// 27.9 -> 26.5 us per step); where a CU's workgroups would be neighbouring blocks instead the order above is the
-// better one (step_fwd_split, 128^3, batch 8, one chunk: 159 -> 180 us; 64^3, batch 32, three: 1 % longer).
+// The same with the chunks of a block, which fetch the same parameters, on one CU: what one of them has asked for
+// the others find in the L1.  An XCD deals its workgroups to its CUs in turn (seen in HW_ID on this part), so number
+// s of an XCD meets s + 32, s + 64, ... on its CU as long as the CUs fill up for the first time; up to `together`
+// of them do (cu_share; 0: numbered as above).  Nothing but the time depends on it.  Only where a CU holds no more
+// workgroups than a block has chunks: with neighbouring blocks on a CU the order above is the better one
+// (step_fwd_split, 128^3, batch 8, one chunk, six workgroups per CU: 159 -> 180 us; 64^3, batch 32, three: 1 % longer).
+// With it: step_fwd_pair, 32^3, batch 64, 27.9 -> 26.5 us; a step forward + backward with normalize, 40 x 48 x 56, batch
+// 13, 127 -> 118; chains by whole rows, 32^3, batch 256, 29.1 -> 28.2 and 68.7 -> 67.0.
 constexpr int kCusPerXcd = 32;
 __host__ __device__ __forceinline__ int cu_share(int nblk, int nchunk, int resident_per_cu) {
-    const int slots = ((nblk + kXcds - 1) / kXcds) * nchunk, share = (slots + kCusPerXcd - 1) / kCusPerXcd;
-    return share < resident_per_cu ? share : resident_per_cu;
-}
-__host__ __device__ __forceinline__ int padded_grid(int nblk, int nchunk, int together) {
-    const int slots = ((nblk + kXcds - 1) / kXcds) * nchunk, first = kCusPerXcd * together;
-    return kXcds * (slots > first ? slots : first);
+    const int slots = ((nblk + kXcds - 1) / kXcds) * nchunk, most = (slots + kCusPerXcd - 1) / kCusPerXcd;
+    const int share = most < resident_per_cu ? most : resident_per_cu;
+    return share > 1 && nchunk >= share ? share : 0;
 }
 __device__ __forceinline__ bool split_block_id(int wg, int nblk, int nchunk, int together, bool reverse, int &blk,
                                                int &chunk) {
-    const int slot = wg / kXcds, first = kCusPerXcd * together, slots = ((nblk + kXcds - 1) / kXcds) * nchunk;
-    const int at = slot < first ? slot % kCusPerXcd * together + slot / kCusPerXcd : slot;
-    if (at >= slots) return false;
+    const int slots = ((nblk + kXcds - 1) / kXcds) * nchunk, first = min(slots, kCusPerXcd * together);
+    int at = wg / kXcds;
+    if (at < first) {  // CU c takes first / 32 numbers in a row, the first CUs one more
+        const int cu = at % kCusPerXcd, each = first / kCusPerXcd, more = first % kCusPerXcd;
+        at = cu * each + min(cu, more) + at / kCusPerXcd;
+    }
     return split_block_id(wg % kXcds + kXcds * (reverse ? slots - 1 - at : at), nblk, nchunk, blk, chunk);
 }
 

@@ -307,7 +307,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(NORM ? 2 : 
 void step_fwd_split(
     const float *__restrict__ weight, const float *__restrict__ bias,
     const float *__restrict__ scale, const float *__restrict__ x, float *__restrict__ y, int B, int M,
-    int N, int K, int inner, int nblk, int nchunk, int chunk_len, LnFold ln, float norm_eps) {
+    int N, int K, int inner, int nblk, int nchunk, int together, int chunk_len, LnFold ln, float norm_eps) {
     using TL = Tile<8, 4>;
     using SW = SplitWin;
     using FX = Fetch<TL>;
@@ -325,8 +325,7 @@ void step_fwd_split(
     const bool ln_in = LN && (MERGE || ln.x_stats != nullptr);  // x is the raw output of the step before
 
     int blk, chunk;
-    if (!split_block_id(ln.walk_reverse ? reversed_on_its_xcd(blockIdx.x, gridDim.x) : blockIdx.x, nblk, nchunk,
-                        blk, chunk))
+    if (!split_block_id(blockIdx.x, nblk, nchunk, together, ln.walk_reverse, blk, chunk))
         return;  // grid padding
     const Place<TL, 4, 1> pl(threadIdx.x, blk, N, K);
     const FX fx(pl.lane, pl.p0, pl.q0, pl.r0, M, N, K);
@@ -853,7 +852,7 @@ void step_bwd_fast(
     const float *__restrict__ scale, const float *__restrict__ x, const float *__restrict__ dy,
     float *__restrict__ dweight, float *__restrict__ dbias, float *__restrict__ dscale,
     float *__restrict__ dx, float *__restrict__ dsum_out, int B, int M, int N, int K, int inner,
-    int nblk, int nchunk, int chunk_len, int param_mode, int dx_accumulate, LnFold ln,
+    int nblk, int nchunk, int together, int chunk_len, int param_mode, int dx_accumulate, LnFold ln,
     float norm_eps, float *__restrict__ qr_out, long slab_stride) {
     using TL = Tile<BS, CPT>;
     static_assert(!(NORM && (LN || RES)), "the folded LayerNorm comes without normalisation");
@@ -866,7 +865,7 @@ void step_bwd_fast(
     const bool ln_in = LN && ln.x_stats != nullptr;
 
     int blk, chunk;
-    if (!split_block_id(blockIdx.x, nblk, nchunk, blk, chunk)) return;  // grid padding
+    if (!split_block_id(blockIdx.x, nblk, nchunk, together, false, blk, chunk)) return;  // grid padding
     if (slab_stride) {
         // the batch of this block is split over workgroups: every chunk commits into a copy of
         // the gradient arrays of its own (plain stores; the copies are added up afterwards)
@@ -1733,6 +1732,7 @@ int launch_fwd_split(const StepArgs &a, hipStream_t st) {
     hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(128), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
                        (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
+                       cu_share(p.nblk, p.nchunk, per_cu),
                        p.chunk_len, a.ln, (float)a.eps);
     return check_launch("step_fwd_split");
 }
@@ -1747,11 +1747,10 @@ template <int ACT, bool MERGE> int launch_fwd_pair(const StepArgs &a, hipStream_
     Plan p = make_plan(a, 2, per_cu * device_cus(), false);
     plan_even_rounds(a.B, p.nblk, 2, per_cu * device_cus(), kMinForwardWalk, p.nchunk, p.chunk_len);
     if (MERGE) most_samples(a.B, p);
-    const int together = cu_share(p.nblk, p.nchunk, per_cu);
-    hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk, together)), dim3(128), 0, st,
+    hipLaunchKernelGGL(kern, dim3(padded_grid(p.nblk, p.nchunk)), dim3(128), 0, st,
                        (const float *)a.weight, (const float *)a.bias, (const float *)a.scale,
-                       (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk, together,
-                       p.chunk_len, a.ln);
+                       (const float *)a.x, (float *)a.y, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
+                       cu_share(p.nblk, p.nchunk, per_cu), p.chunk_len, a.ln);
     return check_launch("step_fwd_pair");
 }
 // The chain's forward on SMALL grids (fewer blocks than a sixth of the workgroups the chip
@@ -1842,8 +1841,9 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
                        (const float *)a.x, (const float *)a.dy, split ? slab : (float *)a.dweight,
                        split ? slab + 27 * cells : (float *)a.dbias,
                        split ? slab + 28 * cells : (float *)a.dscale, (float *)a.dx,
-                       (float *)a.workspace, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk, p.chunk_len,
-                       param_mode, dx_accumulate, ln, (float)a.eps, qr, split ? slab_floats : 0L);
+                       (float *)a.workspace, a.B, a.M, a.N, a.K, a.inner, p.nblk, p.nchunk,
+                       cu_share(p.nblk, p.nchunk, per_cu), p.chunk_len, param_mode, dx_accumulate,
+                       ln, (float)a.eps, qr, split ? slab_floats : 0L);
     if (int rc = check_launch("step_bwd_fast")) return rc;
     const bool by_rows = cross_rows_supports(a);
     TailJob tail{};

@@ -109,7 +109,8 @@ struct RowsFwdArgs {
     double eps;
     float *y, *y_part;
     float *saved;           // plain: [B,cells]; gated: [3][B,cells]; or null
-    int B, M, N, ntube, nchunk, chunk_len, together;
+    int B, M, N, ntube, nchunk, chunk_len;
+    CuShare together;
 };
 
 // MERGE: the statistics of x from the pairs of the step before.  A kernel without it has none of that code: with
@@ -340,7 +341,8 @@ struct RowsBwdArgs {
     float *dweight, *dbias, *dscale, *dgamma, *dbeta;
     long slab_stride;               // a copy of the gradient arrays per batch chunk (0: the arrays themselves)
     int accumulate;                 // on top of what the gradient arrays hold
-    int B, M, N, ntube, nchunk, chunk_len, together;
+    int B, M, N, ntube, nchunk, chunk_len;
+    CuShare together;
 };
 
 // PLAIN: two cells per thread, GATED: one; 54 mirrored weights and 54 gradient accumulators for each set
@@ -679,7 +681,9 @@ template <typename K> int workgroups_per_cu(K kern, int threads, size_t lds) {
 }
 // The chunks of a tube on one CU.  Per step, forward / backward: 32^3, batch 256, 29.1 -> 28.2 / 68.7 -> 67.0 us; batch
 // 64, 13.4 -> 13.1 / 29.9 -> 29.4.  Not with rows of 64 cells: 64^3, batch 32, forward 30.8 -> 32.5.
-template <int K> int rows_together(int ntube, int nchunk, int per_cu) { return K < 64 ? cu_share(ntube, nchunk, per_cu) : 0; }
+template <int K> CuShare rows_together(int ntube, int nchunk, int per_cu) {
+    return K < 64 ? cu_share(ntube, nchunk, per_cu) : CuShare{};
+}
 
 template <int ACT, int SETS, bool SAVE, int K> int run_forward(const RowsChain &c, hipStream_t st) {
     const auto kern = rows_fwd<ACT, SETS, SAVE, K, false>, merging = rows_fwd<ACT, SETS, SAVE, K, true>;

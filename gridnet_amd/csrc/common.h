@@ -239,29 +239,44 @@ __device__ __forceinline__ bool split_block_id(int wg, int nblk, int nchunk, int
     return slot / nchunk < per_xcd && blk < nblk;
 }
 
-// The same with the chunks of a block, which fetch the same parameters, on one CU: what one of them has asked for
-// the others find in the L1.  An XCD deals its workgroups to its CUs in turn (seen in HW_ID on this part), so number
-// s of an XCD meets s + 32, s + 64, ... on its CU as long as the CUs fill up for the first time; up to `together`
-// of them do (cu_share; 0: numbered as above).  Nothing but the time depends on it.  Only where a CU holds no more
-// workgroups than a block has chunks: with neighbouring blocks on a CU the order above is the better one
-// (step_fwd_split, 128^3, batch 8, one chunk, six workgroups per CU: 159 -> 180 us; 64^3, batch 32, three: 1 % longer).
-// With it: step_fwd_pair, 32^3, batch 64, 27.9 -> 26.5 us; a step forward + backward with normalize, 40 x 48 x 56, batch
-// 13, 127 -> 118; chains by whole rows, 32^3, batch 256, 29.1 -> 28.2 and 68.7 -> 67.0.
+// The same with workgroups that fetch the same on one CU: what one of them has asked for the others find in its
+// L1.  An XCD deals its workgroups to its CUs in turn (seen in HW_ID on this part), so number s of an XCD meets
+// s + 32, s + 64, ... on its CU as long as the CUs fill up for the first time.  In rounds of 32 * `together` numbers a
+// CU takes neighbours in number; of a round that the grid or the room on the CUs cuts short the first CUs take one
+// more.  Nothing but the time depends on it.  Not for chunks AND neighbouring blocks on a CU at once, nor for more
+// than two neighbours (step_fwd_split, 128^3, batch 8, six on a CU: 159 -> 180 us).
 constexpr int kCusPerXcd = 32;
-__host__ __device__ __forceinline__ int cu_share(int nblk, int nchunk, int resident_per_cu) {
-    const int slots = ((nblk + kXcds - 1) / kXcds) * nchunk, most = (slots + kCusPerXcd - 1) / kCusPerXcd;
-    const int share = most < resident_per_cu ? most : resident_per_cu;
-    return share > 1 && nchunk >= share ? share : 0;
+struct CuShare {
+    int together;    // neighbours on a CU in a whole round
+    int full, first; // numbers of an XCD in whole rounds, and in all that are dealt so
+    int each, more;  // of the round cut short: numbers per CU, CUs with one more
+};
+inline CuShare cu_rounds(int slots, int together, int resident_per_cu) {
+    const int most = (slots + kCusPerXcd - 1) / kCusPerXcd, held = most < resident_per_cu ? most : resident_per_cu;
+    if (together > held) together = held;
+    if (together < 2) return {};
+    const int size = kCusPerXcd * together, room = held / together * size, first = slots < room ? slots : room;
+    const int full = first / size * size;
+    return {together, full, first, (first - full) / kCusPerXcd, (first - full) % kCusPerXcd};
 }
-__device__ __forceinline__ bool split_block_id(int wg, int nblk, int nchunk, int together, bool reverse, int &blk,
+// The chunks of a block.  step_fwd_pair, 32^3, batch 64, 27.9 -> 26.5 us; step_fwd_split, 64^3, batch 32, 73.3 -> 72.2; a
+// step forward + backward with normalize, 40 x 48 x 56, batch 13, 127 -> 118; chains by whole rows, 32^3, batch 256,
+// 29.1 -> 28.2 and 68.7 -> 67.0.
+inline CuShare cu_share(int nblk, int nchunk, int resident_per_cu) {
+    return cu_rounds(((nblk + kXcds - 1) / kXcds) * nchunk, nchunk, resident_per_cu);
+}
+__device__ __forceinline__ bool split_block_id(int wg, int nblk, int nchunk, const CuShare &cu, bool reverse, int &blk,
                                                int &chunk) {
-    const int slots = ((nblk + kXcds - 1) / kXcds) * nchunk, first = min(slots, kCusPerXcd * together);
-    int at = wg / kXcds;
-    if (at < first) {  // CU c takes first / 32 numbers in a row, the first CUs one more
-        const int cu = at % kCusPerXcd, each = first / kCusPerXcd, more = first % kCusPerXcd;
-        at = cu * each + min(cu, more) + at / kCusPerXcd;
+    unsigned at = (unsigned)wg / kXcds;
+    if (at < (unsigned)cu.full) {
+        const unsigned size = kCusPerXcd * cu.together, in = at % size;
+        at = at - in + in % kCusPerXcd * cu.together + in / kCusPerXcd;
+    } else if (at < (unsigned)cu.first) {
+        const unsigned in = at - cu.full, c = in % kCusPerXcd;
+        at = cu.full + c * cu.each + min(c, (unsigned)cu.more) + in / kCusPerXcd;
     }
-    return split_block_id(wg % kXcds + kXcds * (reverse ? slots - 1 - at : at), nblk, nchunk, blk, chunk);
+    const int slots = ((nblk + kXcds - 1) / kXcds) * nchunk;
+    return split_block_id(wg % kXcds + kXcds * (reverse ? slots - 1 - (int)at : (int)at), nblk, nchunk, blk, chunk);
 }
 
 }  // namespace gridnet

@@ -307,7 +307,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(NORM ? 2 : 
 void step_fwd_split(
     const float *__restrict__ weight, const float *__restrict__ bias,
     const float *__restrict__ scale, const float *__restrict__ x, float *__restrict__ y, int B, int M,
-    int N, int K, int inner, int nblk, int nchunk, int together, int chunk_len, LnFold ln, float norm_eps) {
+    int N, int K, int inner, int nblk, int nchunk, CuShare together, int chunk_len, LnFold ln, float norm_eps) {
     using TL = Tile<8, 4>;
     using SW = SplitWin;
     using FX = Fetch<TL>;
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
 void step_fwd_pair(
     const float *__restrict__ weight, const float *__restrict__ bias,
     const float *__restrict__ scale, const float *__restrict__ x, float *__restrict__ y, int B, int M,
-    int N, int K, int inner, int nblk, int nchunk, int together, int chunk_len, LnFold ln) {
+    int N, int K, int inner, int nblk, int nchunk, CuShare together, int chunk_len, LnFold ln) {
     using TL = Tile<8, 4>;
     using SW = SplitWin;
     using FX = Fetch<TL>;
@@ -852,7 +852,7 @@ void step_bwd_fast(
     const float *__restrict__ scale, const float *__restrict__ x, const float *__restrict__ dy,
     float *__restrict__ dweight, float *__restrict__ dbias, float *__restrict__ dscale,
     float *__restrict__ dx, float *__restrict__ dsum_out, int B, int M, int N, int K, int inner,
-    int nblk, int nchunk, int together, int chunk_len, int param_mode, int dx_accumulate, LnFold ln,
+    int nblk, int nchunk, CuShare together, int chunk_len, int param_mode, int dx_accumulate, LnFold ln,
     float norm_eps, float *__restrict__ qr_out, long slab_stride) {
     using TL = Tile<BS, CPT>;
     static_assert(!(NORM && (LN || RES)), "the folded LayerNorm comes without normalisation");

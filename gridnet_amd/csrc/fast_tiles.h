@@ -135,6 +135,16 @@ template <int TPS> __device__ __forceinline__ float slot_wave_sum(float v) {
     return (r0 + r1) + (r2 + r3);
 }
 
+// (mean, M2 about that mean) of four rows of lanes, `row_cells` cells each, from the rows' pairs
+__device__ __forceinline__ void four_rows_moments(const float (&m)[4], const float (&q)[4], int row_cells, float &mean,
+                                                  float &m2) {
+    mean = 0.25f * ((m[0] + m[1]) + (m[2] + m[3]));
+    float dev = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) dev = fmaf(m[r] - mean, m[r] - mean, dev);
+    m2 = ((q[0] + q[1]) + (q[2] + q[3])) + row_cells * dev;
+}
+
 // (mean, M2 about that mean) of the cells that the lanes of a slot in this wave hold, from the
 // same pair per 16-lane row (each over `row_cells` cells): the rows' means are averaged and the
 // M2 combined with the exact pairwise formula, M2 = sum M2_r + row_cells sum (mean_r - mean)^2.
@@ -155,11 +165,7 @@ __device__ __forceinline__ void slot_wave_moments(float row_mean, float row_m2, 
         mean = 0.5f * (a + b);
         m2 = (upper ? q[2] + q[3] : q[0] + q[1]) + row_cells * ((a - mean) * (a - mean) + (b - mean) * (b - mean));
     } else {
-        mean = 0.25f * ((m[0] + m[1]) + (m[2] + m[3]));
-        float dev = 0.f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dev = fmaf(m[r] - mean, m[r] - mean, dev);
-        m2 = ((q[0] + q[1]) + (q[2] + q[3])) + row_cells * dev;
+        four_rows_moments(m, q, row_cells, mean, m2);
     }
 }
 

@@ -91,6 +91,26 @@ void step_fwd_fast(
     const long cells = (long)M * N * K;
     const bool ln_in = LN && ln.x_stats != nullptr;  // x is the raw output of the step before
 
+    const int s0 = chunk * chunk_len, s1 = min(B, s0 + chunk_len);
+    typename Fetch<TL>::Buf pre;
+    float pre_mean = 0.f, pre_rstd = 1.f;  // LayerNorm statistics of the element in `pre`
+    // NORM: the window is kept minus one of its own values (the block's first cell), see
+    // Fetch::commit_sums; `shift` belongs to the element being iterated, `pre_shift` to `pre`
+    float pre_shift = 0.f, shift = 0.f, done_shift = 0.f;
+    const int first_cell = (pl.p0 * N + pl.q0) * K + pl.r0;
+    auto fetch_element = [&](int s) {
+        fx.fetch(x + s * cells, pre);
+        if (ln_in) {
+            pre_mean = load_ahead(ln.x_stats, 2 * s);
+            pre_rstd = load_ahead(ln.x_stats, 2 * s + 1);
+        }
+        if (NORM) pre_shift = load_ahead(x + s * cells, first_cell);
+    };
+    // The first element in front of the weights, where its registers do not have to hold gamma and beta first:
+    // one trip to memory instead of two.
+    constexpr bool FIRST_AHEAD = BS == 8 && !LN;
+    if (FIRST_AHEAD && s0 + pl.slot < s1) fetch_element(s0 + pl.slot);
+
     float w[27][CPT], bv[CPT], rv[CPT];
 #pragma unroll
     for (int t = 0; t < 27; ++t) load_cells<CPT>(weight + t * cells + pl.gc, w[t]);
@@ -111,7 +131,6 @@ void step_fwd_fast(
             for (int t = 0; t < 27; ++t) wsum[c] += w[t][c];
         }
     }
-    typename Fetch<TL>::Buf pre;
     if (ln_in) {  // gamma and beta of the window, once per workgroup
         if (pl.slot == 0) {
             typename Fetch<TL>::Buf bet;
@@ -123,21 +142,7 @@ void step_fwd_fast(
     }
     wait_global_loads();
 
-    const int s0 = chunk * chunk_len, s1 = min(B, s0 + chunk_len);
-    float pre_mean = 0.f, pre_rstd = 1.f;  // LayerNorm statistics of the element in `pre`
-    // NORM: the window is kept minus one of its own values (the block's first cell), see
-    // Fetch::commit_sums; `shift` belongs to the element being iterated, `pre_shift` to `pre`
-    float pre_shift = 0.f, shift = 0.f, done_shift = 0.f;
-    const int first_cell = (pl.p0 * N + pl.q0) * K + pl.r0;
-    auto fetch_element = [&](int s) {
-        fx.fetch(x + s * cells, pre);
-        if (ln_in) {
-            pre_mean = load_ahead(ln.x_stats, 2 * s);
-            pre_rstd = load_ahead(ln.x_stats, 2 * s + 1);
-        }
-        if (NORM) pre_shift = load_ahead(x + s * cells, first_cell);
-    };
-    if (s0 + pl.slot < s1) fetch_element(s0 + pl.slot);
+    if (!FIRST_AHEAD && s0 + pl.slot < s1) fetch_element(s0 + pl.slot);
     // The result of an element is stored one element late, after the next window has been
     // committed: the wait for the prefetched window would otherwise also wait for a store that
     // was issued an instant earlier (loads and stores share one in-order counter).
@@ -395,6 +400,21 @@ void step_fwd_split(
     const int side00 = base + SW::CEN + pl.kt * SW::SS + pl.i * SW::SP + pl.j;
     const int own = cen00 + SW::PS + SW::RS;
 
+    // The first element is requested in front of the parameters, one trip to memory instead of two (normalize, 16^3,
+    // batch 1, two inner iterations, 6.3 -> 5.9 us; 32^3, batch 8, 13.9 -> 13.2); with the LayerNorm its registers hold
+    // gamma and beta first.
+    constexpr bool FIRST_AHEAD = !LN;
+    const int s0 = chunk * chunk_len, s1 = min(B, s0 + chunk_len);
+    typename FX::Buf pre;
+    // NORM: the window is kept minus one of its own values (the block's first cell), see
+    // Fetch::commit_sums; `pre_shift` belongs to `pre`, `shift` to the element being iterated
+    float pre_shift = 0.f, shift = 0.f, done_shift = 0.f;
+    const int first_cell = (pl.p0 * N + pl.q0) * K + pl.r0;
+    if (FIRST_AHEAD && s0 < s1) {
+        fx.fetch(x + s0 * cells, pre);
+        if (NORM) pre_shift = load_ahead(x + s0 * cells, first_cell);
+    }
+
     // Parameters in register order.  First half: w[t][r] is tap t of column r.  Second half:
     // register r is column 7-r and a step of one register is a step of -1 along K, so the tap
     // with K-offset cc sits at register offset 2-cc.
@@ -433,10 +453,6 @@ void step_fwd_split(
     // the producer is applied on the way: (v - mean) * rstd * gamma + beta, gamma and beta from
     // their own windows; entries outside the grid stay zero.
     float part[4];  // NORM: what the last commit added up
-    // NORM: the window is kept minus one of its own values (the block's first cell), see
-    // Fetch::commit_sums; `pre_shift` belongs to `pre`, `shift` to the element being iterated
-    float pre_shift = 0.f, shift = 0.f, done_shift = 0.f;
-    const int first_cell = (pl.p0 * N + pl.q0) * K + pl.r0;
     auto commit = [&](float *to, int copies, const typename FX::Buf &v, bool fold, float mean, float rstd,
                       float *give_back = nullptr) {
 #pragma unroll
@@ -487,7 +503,6 @@ void step_fwd_split(
                 }
             }
     };
-    typename FX::Buf pre;
     if (ln_in) {  // gamma and beta of the window, once per workgroup
         fx.fetch(ln.gamma, pre);
         commit(gwin, 1, pre, false, 0.f, 1.f);
@@ -502,7 +517,6 @@ void step_fwd_split(
         store_cells<4>(y + s * cells + pl.gc, out);
     };
 
-    const int s0 = chunk * chunk_len, s1 = min(B, s0 + chunk_len);
     float pre_mean = 0.f, pre_rstd = 1.f;  // LayerNorm statistics of the element in `pre`
     auto fetch_element = [&](int s) {
         fx.fetch(x + s * cells, pre);
@@ -515,7 +529,7 @@ void step_fwd_split(
         }
         if (NORM) pre_shift = load_ahead(x + s * cells, first_cell);
     };
-    if (s0 < s1) fetch_element(s0);
+    if (!FIRST_AHEAD && s0 < s1) fetch_element(s0);
     // The result of an element is stored one element late, after the next window has been
     // committed (see step_fwd_fast).
     float done[4];
@@ -991,6 +1005,41 @@ void step_bwd_fast(
     };
     auto always = [](int, int) { return true; };
 
+    const int s0 = chunk * chunk_len, s1 = min(B, s0 + chunk_len);
+    // what is requested one element ahead: the x window, the incoming gradient of the owned
+    // cells and, for LN, the raw output there and the per-sample numbers of both LayerNorms
+    typename Fetch<TL>::Buf pre;
+    float g[CPT], gnext[CPT], ynext[CPT], nx_mean = 0.f, nx_rstd = 1.f, ny[4] = {0.f, 1.f, 0.f, 0.f};
+    // RES: G'' of the owned cells (of the step after), G' as formed for the current element, and
+    // the latter again for the element whose results are stored one element late
+    float gprev[CPT], gin[CPT], gin_done[CPT];
+    const bool through_ln = LN && (!RES || ln.y_raw != nullptr);  // dy passes a LayerNorm on load
+    // NORM: the x window is kept minus one of its own values (the block's first cell), see
+    // Fetch::commit_sums; everything downstream only sees differences of window entries, except
+    // R, which is handed on for the unshifted x (R + shift * Q)
+    float pre_shift = 0.f, shift = 0.f;
+    const int first_cell = (pl.p0 * N + pl.q0) * K + pl.r0;
+    auto fetch_element = [&](int s) {
+        fx.fetch(x + s * cells, pre);
+        load_cells<CPT>(dy + s * cells + pl.gc, gnext);
+        if (RES && through_ln) load_cells<CPT>(ln.g_prev + s * cells + pl.gc, gprev);
+        if (through_ln) {
+            load_cells<CPT>(ln.y_raw + s * cells + pl.gc, ynext);
+            ny[0] = load_ahead(ln.y_stats, 2 * s);
+            ny[1] = load_ahead(ln.y_stats, 2 * s + 1);
+            ny[2] = load_ahead(ln.y_sums, 2 * s);
+            ny[3] = load_ahead(ln.y_sums, 2 * s + 1);
+        }
+        if (ln_in) {
+            nx_mean = load_ahead(ln.x_stats, 2 * s);
+            nx_rstd = load_ahead(ln.x_stats, 2 * s + 1);
+        }
+        if (NORM) pre_shift = load_ahead(x + s * cells, first_cell);
+    };
+    // the first element in front of the weights, where there is room: one trip to memory instead of two
+    constexpr bool FIRST_AHEAD = CPT == 1 && !LN;
+    if (FIRST_AHEAD && s0 + pl.slot < s1) fetch_element(s0 + pl.slot);
+
     // ---- once per workgroup: parameters and mirrored neighbour weights ----
     // w : this cell's weights (forward recompute)
     // v : V[t][c] = W[26-t, c + off_t], what the neighbour at c + off_t multiplies cell c by
@@ -1055,7 +1104,6 @@ void step_bwd_fast(
         store_cells<CPT>(wout_at, wout);
         store_cells<CPT>(d2acc_at, zero);
     }
-    typename Fetch<TL>::Buf pre;
     if (ln_in && pl.slot == 0) {  // gamma and beta of the window, once per workgroup
         typename Fetch<TL>::Buf bet;
         fx.fetch(ln.gamma, pre);
@@ -1089,36 +1137,6 @@ void step_bwd_fast(
         }
     }
 
-    const int s0 = chunk * chunk_len, s1 = min(B, s0 + chunk_len);
-    // what is requested one element ahead: the x window, the incoming gradient of the owned
-    // cells and, for LN, the raw output there and the per-sample numbers of both LayerNorms
-    float g[CPT], gnext[CPT], ynext[CPT], nx_mean = 0.f, nx_rstd = 1.f, ny[4] = {0.f, 1.f, 0.f, 0.f};
-    // RES: G'' of the owned cells (of the step after), G' as formed for the current element, and
-    // the latter again for the element whose results are stored one element late
-    float gprev[CPT], gin[CPT], gin_done[CPT];
-    const bool through_ln = LN && (!RES || ln.y_raw != nullptr);  // dy passes a LayerNorm on load
-    // NORM: the x window is kept minus one of its own values (the block's first cell), see
-    // Fetch::commit_sums; everything downstream only sees differences of window entries, except
-    // R, which is handed on for the unshifted x (R + shift * Q)
-    float pre_shift = 0.f, shift = 0.f;
-    const int first_cell = (pl.p0 * N + pl.q0) * K + pl.r0;
-    auto fetch_element = [&](int s) {
-        fx.fetch(x + s * cells, pre);
-        load_cells<CPT>(dy + s * cells + pl.gc, gnext);
-        if (RES && through_ln) load_cells<CPT>(ln.g_prev + s * cells + pl.gc, gprev);
-        if (through_ln) {
-            load_cells<CPT>(ln.y_raw + s * cells + pl.gc, ynext);
-            ny[0] = load_ahead(ln.y_stats, 2 * s);
-            ny[1] = load_ahead(ln.y_stats, 2 * s + 1);
-            ny[2] = load_ahead(ln.y_sums, 2 * s);
-            ny[3] = load_ahead(ln.y_sums, 2 * s + 1);
-        }
-        if (ln_in) {
-            nx_mean = load_ahead(ln.x_stats, 2 * s);
-            nx_rstd = load_ahead(ln.x_stats, 2 * s + 1);
-        }
-        if (NORM) pre_shift = load_ahead(x + s * cells, first_cell);
-    };
     // the element just fetched becomes the current one: its gradient (through the LayerNorm
     // backward for LN) and its window
     auto take_element = [&]() {
@@ -1149,7 +1167,7 @@ void step_bwd_fast(
     };
     if (ln_in) lds_barrier();  // gamma and beta windows
     if (s0 + pl.slot < s1) {
-        fetch_element(s0 + pl.slot);
+        if (!FIRST_AHEAD) fetch_element(s0 + pl.slot);
         take_element();
     }
     // Per element: commit its window, barrier, [stores of the PREVIOUS element], recompute,
@@ -1874,7 +1892,27 @@ bool walks_pairs(const StepArgs &a) {
     return chunks >= 1 && (a.B + chunks - 1) / chunks <= 4;
 }
 
+// Small grids: one cell per thread instead of two (backward) or one or two instead of four (forward), a block by eight
+// or four waves.  A launch that gives a CU few workgroups has one wave per SIMD, which waits out every LDS trip and every
+// dependent operation alone; with half the cells per thread there are two, each with half the work.  Counted in
+// (block, element) pairs per CU: a full chip is better off with fewer LDS accesses per operation.  Forward, backward's
+// first + second kernel, us, with normalize: 16^3, batch 1, two inner iterations, 5.9 -> 5.2, 16.9 + 4.2 -> 11.7 + 4.3; 32^3,
+// batch 2, ten, 12.1 -> 10.9, 32.3 + 6.7 -> 27.3 + 6.6; batch 8, four (two pairs per CU), 11.1 -> 10.8, 34.6 + 13.7 -> 30.8 + 10.0;
+// batch 16 (four), 14.6 -> 15.0, 42.9 + 12.6 -> 44.7 + 10.5; batch 64, 30.6 -> 35.0, 97.8 + 15.3 -> 130.8 + 13.9.  Without
+// normalize: 32^3, batch 2, 11.3 -> 8.4, 24.7 + 5.8 -> 18.5 + 5.7; batch 8, 9.4 -> 9.1, 29.9 + 10.6 -> 22.7 + 8.6; batch 16, 11.6 ->
+// 13.1, 34.2 + 12.7 -> 30.3 + 9.2; batch 64, 25.2 -> 27.5, 63.3 + 13.2 -> 72.3 + 12.2.  The backward not where a workgroup has
+// the whole batch of its block: 64^3, batch 1, with normalize 33.3 -> 36.8.
+constexpr int kFewPairsForward = 2, kFewPairsBackward = 4, kFewPairsBackwardNormalize = 3;  // per CU
+bool few_pairs(const StepArgs &a, int per_cu) {
+    return (long)(a.M / 8) * (a.N / 8) * (a.K / 8) * a.B <= (long)per_cu * device_cus();
+}
+
 template <int BS, int CPT, int NSLOT, int ACT> int launch_fwd(const StepArgs &a, hipStream_t st) {
+    if constexpr (BS == 8) {
+        // one cell per thread where the window needs no sums over eight waves (normalize, 32^3, batch 2: 12.8 us)
+        if (!a.ln.gamma && few_pairs(a, kFewPairsForward))
+            return a.normalize ? launch_fwd_ln<8, 2, 1, ACT, false, false, true>(a, st) : launch_fwd_ln<8, 1, 1, ACT, false>(a, st);
+    }
     if (a.normalize) {
         if (BS == 8) return launch_fwd_split<ACT, false, false, true>(a, st);
         return launch_fwd_ln<BS, CPT, NSLOT, ACT, false, false, true>(a, st);
@@ -1981,6 +2019,12 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
     return GRIDNET_OK;
 }
 template <int BS, int CPT, int NSLOT, int ACT> int launch_bwd(const StepArgs &a, hipStream_t st) {
+    if constexpr (BS == 8) {
+        const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
+        if (!a.ln.gamma && nblk < device_cus() && few_pairs(a, a.normalize ? kFewPairsBackwardNormalize : kFewPairsBackward) &&
+            bwd_lds_bytes<8, 1, 1>(a.inner, false, a.normalize) <= kMaxLds)
+            return a.normalize ? launch_bwd_ln<8, 1, 1, ACT, false, false, true>(a, st) : launch_bwd_ln<8, 1, 1, ACT, false>(a, st);
+    }
     if (a.normalize) return launch_bwd_ln<BS, CPT, NSLOT, ACT, false, false, true>(a, st);
     if (a.ln.gamma && a.ln.residual) return launch_bwd_ln<BS, CPT, NSLOT, ACT, true, true>(a, st);
     if (a.ln.gamma) return launch_bwd_ln<BS, CPT, NSLOT, ACT, true>(a, st);

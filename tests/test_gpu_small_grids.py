@@ -1,0 +1,36 @@
+"""The step's kernels for small grids (csrc/step_fast.hip, few_pairs: one or two cells per thread) and those that take over
+where a CU gets more (block, element) pairs, on both sides of the line, against the CPU oracle in fp64."""
+
+import pytest
+import torch
+
+from helpers import ATOL, RTOL, acts_clear_of_kink, assert_close, make_acts, make_params
+from test_gpu_step import oracle, run_op
+
+pytestmark = pytest.mark.gpu
+
+
+# (pairs on 256 CUs): one block; the forward's line at two pairs per CU, the backward's at three with normalize and four
+# without (65 is not split evenly); blocks that have a neighbour on one side only; ten inner iterations (at twenty the
+# gradients reach 3e3 and torch's own fp32 evaluation on the CPU lies 1.3 to 1.5 times outside the bar); 256 blocks,
+# whose workgroups have the whole batch in the backward
+@pytest.mark.parametrize("shape,batch,inner", [
+    ((8, 8, 8), 1, 1), ((8, 8, 8), 3, 4), ((16, 16, 16), 64, 2), ((16, 16, 16), 65, 2), ((24, 32, 40), 17, 2), ((24, 32, 40), 18, 2),
+    ((16, 16, 32), 48, 2), ((16, 16, 32), 64, 2), ((16, 16, 32), 65, 2), ((16, 8, 24), 2, 10), ((32, 64, 64), 1, 2),
+    ((32, 64, 64), 2, 2)], ids=str)
+@pytest.mark.parametrize("normalize", [False, True], ids=["plain", "normalize"])
+@pytest.mark.parametrize("activation", ["silu", "leaky_relu"])
+def test_step_on_both_sides_of_the_line(shape, batch, inner, normalize, activation):
+    print(f"small grid {shape} B={batch} inner={inner} normalize={normalize} {activation}", flush=True)
+    w, b, r = make_params(shape, seed=11)
+    if inner >= 8:
+        w, r = w * 0.5, r * 0.5
+    x = acts_clear_of_kink(w, b, r, batch, shape, inner, 8, 1e-5, normalize, activation, seed=12)
+    gy = make_acts(batch, shape, seed=13)
+    y, grads = run_op(w, b, r, x, gy, inner, 8, 1e-5, normalize, activation)
+    ey, egrads = oracle(w, b, r, x, gy, inner, 8, 1e-5, normalize, activation)
+    assert_close(y, ey, RTOL, ATOL, "y")
+    for name, g, e in zip(("dweight", "dbias", "dscale", "dx"), grads, egrads):
+        # An entry is a sum of batch x inner products; its rounding error goes with the size of those, 2e-7 of the rms of the
+        # array (fp32, any order), not with what is left of the sum: 50 of these where the rms is above one.
+        assert_close(g, e, RTOL, ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)

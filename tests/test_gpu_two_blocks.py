@@ -11,11 +11,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# the fewest workgroups of two blocks (one element each) and half a chunk more; blocks at both ends of a row; three
-# chunks, the last one short (a walk of 24 iterations) against 88; more blocks than the chip holds (16 against 136)
+# just too many elements for the kernels of small grids, one to a workgroup, and one more than the chunks; blocks at
+# both ends of a row; three chunks, the last one short (a walk of 24 iterations) against 88; more blocks than the chip
+# holds (16 against 136)
 @pytest.mark.parametrize("shape,two,one,inner,activation", [
-    *[((16, 16, 64), 16, 4, 2, a) for a in ("relu", "leaky_relu", "silu", "tanh")], ((16, 16, 64), 33, 4, 3, "silu"),
-    ((8, 24, 128), 11, 3, 3, "tanh"), ((64, 64, 64), 17, 64, 4, "silu"), ((128, 128, 128), 2, 17, 8, "leaky_relu")], ids=str)
+    *[((16, 16, 64), 17, 600, 2, a) for a in ("relu", "leaky_relu", "silu", "tanh")], ((16, 16, 64), 49, 600, 3, "silu"),
+    ((8, 24, 128), 11, 300, 3, "tanh"), ((64, 64, 64), 17, 64, 4, "silu"), ((128, 128, 128), 2, 17, 8, "leaky_relu")], ids=str)
 def test_step_is_the_one_of_single_blocks(shape, two, one, inner, activation):
     from gridnet_amd import gridnet_step
 

@@ -1900,7 +1900,9 @@ bool walks_pairs(const StepArgs &a) {
 // batch 2, ten, 12.1 -> 10.9, 32.3 + 6.7 -> 27.3 + 6.6; batch 8, four (two pairs per CU), 11.1 -> 10.8, 34.6 + 13.7 -> 30.8 + 10.0;
 // batch 16 (four), 14.6 -> 15.0, 42.9 + 12.6 -> 44.7 + 10.5; batch 64, 30.6 -> 35.0, 97.8 + 15.3 -> 130.8 + 13.9.  Without
 // normalize: 32^3, batch 2, 11.3 -> 8.4, 24.7 + 5.8 -> 18.5 + 5.7; batch 8, 9.4 -> 9.1, 29.9 + 10.6 -> 22.7 + 8.6; batch 16, 11.6 ->
-// 13.1, 34.2 + 12.7 -> 30.3 + 9.2; batch 64, 25.2 -> 27.5, 63.3 + 13.2 -> 72.3 + 12.2.  The backward not where a workgroup has
+// 13.1, 34.2 + 12.7 -> 30.3 + 9.2; batch 64, 25.2 -> 27.5, 63.3 + 13.2 -> 72.3 + 12.2.  Backward of a
+// step of a chain, both kernels: 16^3, batch 1, 26.8 -> 21.0; 48^3, batch 2, 44.3 -> 32.9; 32^3, batch 16, 49.5 -> 42.9; batch 32,
+// 58.3 -> 56.9.  The backward not where a workgroup has
 // the whole batch of its block: 64^3, batch 1, with normalize 33.3 -> 36.8.
 constexpr int kFewPairsForward = 2, kFewPairsBackward = 4, kFewPairsBackwardNormalize = 3;  // per CU
 bool few_pairs(const StepArgs &a, int per_cu) {
@@ -2021,9 +2023,12 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
 template <int BS, int CPT, int NSLOT, int ACT> int launch_bwd(const StepArgs &a, hipStream_t st) {
     if constexpr (BS == 8) {
         const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
-        if (!a.ln.gamma && nblk < device_cus() && few_pairs(a, a.normalize ? kFewPairsBackwardNormalize : kFewPairsBackward) &&
-            bwd_lds_bytes<8, 1, 1>(a.inner, false, a.normalize) <= kMaxLds)
-            return a.normalize ? launch_bwd_ln<8, 1, 1, ACT, false, false, true>(a, st) : launch_bwd_ln<8, 1, 1, ACT, false>(a, st);
+        if (nblk < device_cus() && few_pairs(a, a.normalize ? kFewPairsBackwardNormalize : kFewPairsBackward) &&
+            bwd_lds_bytes<8, 1, 1>(a.inner, a.ln.gamma != nullptr, a.normalize) <= kMaxLds) {
+            if (a.normalize) return launch_bwd_ln<8, 1, 1, ACT, false, false, true>(a, st);
+            if (a.ln.gamma && a.ln.residual) return launch_bwd_ln<8, 1, 1, ACT, true, true>(a, st);
+            return a.ln.gamma ? launch_bwd_ln<8, 1, 1, ACT, true>(a, st) : launch_bwd_ln<8, 1, 1, ACT, false>(a, st);
+        }
     }
     if (a.normalize) return launch_bwd_ln<BS, CPT, NSLOT, ACT, false, false, true>(a, st);
     if (a.ln.gamma && a.ln.residual) return launch_bwd_ln<BS, CPT, NSLOT, ACT, true, true>(a, st);

@@ -8,6 +8,7 @@ from helpers import ATOL, RTOL, acts_clear_of_kink, assert_close, make_acts, mak
 from test_gpu_step import oracle, run_op
 
 pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
 
 
 # (pairs on 256 CUs): one block; the forward's line at two pairs per CU, the backward's at three with normalize and four
@@ -34,3 +35,26 @@ def test_step_on_both_sides_of_the_line(shape, batch, inner, normalize, activati
         # An entry is a sum of batch x inner products; its rounding error goes with the size of those, 2e-7 of the rms of the
         # array (fp32, any order), not with what is left of the sum: 50 of these where the rms is above one.
         assert_close(g, e, RTOL, ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)
+
+
+# the backward of a chain at the last batch of the small kernels, against one sample more that receives no gradient
+@pytest.mark.parametrize("shape,batch,inner", [((16, 16, 32), 64, 2), ((32, 32, 32), 16, 3), ((24, 32, 40), 17, 2)], ids=str)
+@pytest.mark.parametrize("residual", [False, True], ids=["chain", "residual"])
+def test_chain_on_both_sides_of_the_line(shape, batch, inner, residual):
+    from gridnet_amd.runner import BodyRunner
+
+    print(f"small grid, chain {shape} B={batch} inner={inner} residual={residual}", flush=True)
+    g = torch.Generator().manual_seed(3)
+    params = [t.to(DEV) for t in (*make_params(shape, seed=11), *((a + 0.2 * torch.randn(shape, generator=g)) for a in (1, 0)))]
+    x, gy = (make_acts(batch + 1, shape, seed=s).to(DEV) for s in (12, 13))
+    gy[batch] = 0
+    got = []
+    for n in (batch, batch + 1):
+        run = BodyRunner(*params, n, inner, 2, 8, "silu", fused=True, outer_residual=residual)
+        run.forward(x[:n])
+        got.append([t.clone() for t in run.backward(gy[:n])])
+    for name, a, e in zip(("dweight", "dbias", "dscale", "dgamma", "dbeta", "dx"), *got):
+        e = e[:batch] if name == "dx" else e
+        assert torch.isfinite(a).all()
+        # both sides round; the bound of above, twice
+        assert_close(a, e, 2 * RTOL, 2 * ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)

@@ -18,8 +18,8 @@
 //     step while their weights are on their way (plan_merge_lanes says where; a small kernel between the steps
 //     elsewhere, 4.7 us each).  Merged inside the walk, by one wave an element ahead, they cost the kernels
 //     11 us forward and 24 us backward: everybody waits for that wave at the barrier.
-// 32^3, batch 256, silu, per step: forward 28.3 us, backward 68.3, at 4.3 TB/s either way where a copy
-// reaches 4.6 (with the merging kernels 30.4 and 69.0; fwd_rows, bwd_rows and cross_rows with theirs: 28.1 + 4.4,
+// 32^3, batch 256, silu, per step: forward 28.2 us, backward 67.0, at 4.3 TB/s either way where a copy
+// reaches 4.6 (with the merging kernels, the chunks of a tube on several CUs, 30.4 and 69.0; fwd_rows, bwd_rows and cross_rows with theirs: 28.1 + 4.4,
 // 59.3 + 8.0 + 23.4).  Gated, tanh: 55.5 and 86.6 (op by op the whole training step took 21.3 ms, 9.2 now).
 
 #include <algorithm>

@@ -108,7 +108,7 @@ void step_fwd_fast(
     };
     // The first element in front of the weights, where its registers do not have to hold gamma and beta first:
     // one trip to memory instead of two.
-    constexpr bool FIRST_AHEAD = BS == 8 && !LN;
+    constexpr bool FIRST_AHEAD = (BS == 8 || CPT == 1) && !LN;
     if (FIRST_AHEAD && s0 + pl.slot < s1) fetch_element(s0 + pl.slot);
 
     float w[27][CPT], bv[CPT], rv[CPT];
@@ -1909,7 +1909,22 @@ bool few_pairs(const StepArgs &a, int per_cu) {
     return (long)(a.M / 8) * (a.N / 8) * (a.K / 8) * a.B <= (long)per_cu * device_cus();
 }
 
+// 4^3 blocks, forward: four slots to a workgroup each fetch the weights, and idle where there is less than an element for
+// each.  Where the walk is short (shorter on grids that the launch fills with workgroups only just) or the blocks are few,
+// one slot of one cell per thread, a wave of its own.  Plain, us: 16^3, batch 1, two inner iterations, 5.6 -> 4.0; four: 32^3,
+// batch 1, 8.0 -> 5.6, batch 2, 8.1 -> 6.9; 48^3, batch 2, 17.3 -> 12.4; 64^3, batch 1, 33.4 -> 14.1, batch 4, 35.4 -> 26.9; 96^3, batch
+// 4, 103 -> 58; 128^3, batch 1, 220 -> 95; but 32^3, batch 4, 8.6 -> 9.4; 48^3, batch 4, 18.1 -> 19.6; 64^3, batch 32, 82 -> 122.
+constexpr int kFewPairsForSlots = 6, kShortWalkForSlots = 8, kManyBlocksForSlots = 8;
+bool few_for_slots(const StepArgs &a) {
+    const long nblk = (long)(a.M / 4) * (a.N / 4) * (a.K / 4), cus = device_cus();
+    return (long)a.B * a.inner <= (nblk > kManyBlocksForSlots * cus ? 2 : 1) * kShortWalkForSlots ||
+           nblk * a.B <= kFewPairsForSlots * cus;
+}
+
 template <int BS, int CPT, int NSLOT, int ACT> int launch_fwd(const StepArgs &a, hipStream_t st) {
+    if constexpr (BS == 4 && CPT > 1) {
+        if (few_for_slots(a)) return launch_fwd<4, 1, 1, ACT>(a, st);
+    }
     if constexpr (BS == 8) {
         // one cell per thread where the window needs no sums over eight waves (normalize, 32^3, batch 2: 12.8 us)
         if (!a.ln.gamma && few_pairs(a, kFewPairsForward))
@@ -2020,20 +2035,50 @@ int launch_bwd_ln(const StepArgs &a, hipStream_t st) {
     if (int rc = check_launch("step_bwd_cross")) return rc;
     return GRIDNET_OK;
 }
-template <int BS, int CPT, int NSLOT, int ACT> int launch_bwd(const StepArgs &a, hipStream_t st) {
-    if constexpr (BS == 8) {
-        const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
-        if (nblk < device_cus() && few_pairs(a, a.normalize ? kFewPairsBackwardNormalize : kFewPairsBackward) &&
-            bwd_lds_bytes<8, 1, 1>(a.inner, a.ln.gamma != nullptr, a.normalize) <= kMaxLds) {
-            if (a.normalize) return launch_bwd_ln<8, 1, 1, ACT, false, false, true>(a, st);
-            if (a.ln.gamma && a.ln.residual) return launch_bwd_ln<8, 1, 1, ACT, true, true>(a, st);
-            return a.ln.gamma ? launch_bwd_ln<8, 1, 1, ACT, true>(a, st) : launch_bwd_ln<8, 1, 1, ACT, false>(a, st);
-        }
-    }
+template <int BS, int CPT, int NSLOT, int ACT> int launch_bwd_as(const StepArgs &a, hipStream_t st) {
     if (a.normalize) return launch_bwd_ln<BS, CPT, NSLOT, ACT, false, false, true>(a, st);
     if (a.ln.gamma && a.ln.residual) return launch_bwd_ln<BS, CPT, NSLOT, ACT, true, true>(a, st);
     if (a.ln.gamma) return launch_bwd_ln<BS, CPT, NSLOT, ACT, true>(a, st);
     return launch_bwd_ln<BS, CPT, NSLOT, ACT, false>(a, st);
+}
+// 4^3 blocks, backward: a slot is half a wave (two cells per thread) or a wave (one), and where a workgroup has the whole
+// batch of its block the slots are all the waves a CU gets: two slots, a wave, on the 512 blocks of 32^3 are two waves per
+// CU.  So as many slots as fill the chip (two waves per SIMD), and one cell per thread where the batch is too short for
+// that.  First kernel, us, plain / with normalize, four inner iterations, two slots -> : eight: 32^3, batch 64, 149 -> 63 / 253 ->
+// 99; four: 40^3, batch 32, 90 -> 63 / 150 -> 95; but 48^3 (1728 blocks), batch 32, 98 -> 116 / 162 -> 178.  One cell, four slots: 16^3,
+// batch 64, 35 -> 21 / 39 -> 27; 32^3, batch 8, 29 -> 20 / 44 -> 27 (eight slots of two: 25 / 34); but 24^3, batch 64, 43 -> 46 / 58 ->
+// 60.  One cell, one slot: 16^3, batch 1, two iterations, 13.6 -> 6.9 / 17.5 -> 9.0; 64^3, batch 1, 51 -> 31 / 60 -> 36, batch 4, 63 -> 55 /
+// 80 -> 70; 96^3, batch 4, 183 -> 147 / 249 -> 175; but 64^3, batch 8, 80 -> 83 / 113 -> 113, batch 32, 197 -> 279 / 315 -> 388.
+constexpr int kFewPairsBackward4 = 16, kShortWalkBackward4 = 16;
+template <int ACT> int launch_bwd_slots(const StepArgs &a, hipStream_t st) {
+    const int nblk = (a.M / 4) * (a.N / 4) * (a.K / 4), cus = device_cus();
+    const bool ln = a.ln.gamma != nullptr;
+    auto fit = [&](size_t lds, int workgroups) { return lds * workgroups <= kMaxLds; };
+    const bool eight = nblk >= cus && nblk <= 2 * cus && fit(bwd_lds_bytes<4, 2, 8>(a.inner, ln, a.normalize), 2);
+    const bool four = nblk >= cus && nblk <= 4 * cus && fit(bwd_lds_bytes<4, 2, 4>(a.inner, ln, a.normalize), 4);
+    const bool few = nblk < cus ? (long)nblk * a.B <= (long)kFewPairsBackward4 * cus
+                     : nblk <= 2 * cus ? a.B < 32
+                     : nblk <= 4 * cus ? a.B <= 4
+                                       : a.B == 1 || (long)a.B * a.inner <= kShortWalkBackward4;
+    if (few && nblk <= 2 * cus && a.B >= 4 && fit(bwd_lds_bytes<4, 1, 4>(a.inner, ln, a.normalize), 2))
+        return launch_bwd_as<4, 1, 4, ACT>(a, st);
+    if (few && (a.B < 4 || nblk > 2 * cus) && fit(bwd_lds_bytes<4, 1, 1>(a.inner, ln, a.normalize), 4))
+        return launch_bwd_as<4, 1, 1, ACT>(a, st);
+    if (eight) return launch_bwd_as<4, 2, 8, ACT>(a, st);
+    if (four) return launch_bwd_as<4, 2, 4, ACT>(a, st);
+    return launch_bwd_as<4, 2, 2, ACT>(a, st);
+}
+template <int BS, int CPT, int NSLOT, int ACT> int launch_bwd(const StepArgs &a, hipStream_t st) {
+    if constexpr (BS == 4) {
+        static_assert(CPT == 2 && NSLOT == 2, "the shape that step_fast_supports asks for");
+        return launch_bwd_slots<ACT>(a, st);
+    } else {
+        const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
+        if (nblk < device_cus() && few_pairs(a, a.normalize ? kFewPairsBackwardNormalize : kFewPairsBackward) &&
+            bwd_lds_bytes<8, 1, 1>(a.inner, a.ln.gamma != nullptr, a.normalize) <= kMaxLds)
+            return launch_bwd_as<8, 1, 1, ACT>(a, st);
+        return launch_bwd_as<8, CPT, NSLOT, ACT>(a, st);
+    }
 }
 
 // ---- the tuned shapes ---------------------------------------------------------------------

@@ -587,9 +587,12 @@ template <int BS, bool BWD, bool NORM> int dispatch_f64(const StepArgs &a, hipSt
 // 78 / 50 and 91 / 75; 48^3 in 4^3 blocks (1728 of them): 56 / 62 and 86 / 114; 40^3, batch 1: 21 / 22 and 33 / 33,
 // 4^3 blocks 19 / 22 and 26 / 26.  Up to 2^17 cells: gridnet_hip_backward has asked callers with larger fp64
 // grids for no scratch.  No iteration at all, and histories beyond LDS (more than 15 iterations of 8^3 blocks), stay there too.
+// Size queries come here with arguments that nothing has looked at: what the sums below cannot take is refused first.
 bool step_f64_supports(const StepArgs &a) {
-    return a.dtype == GRIDNET_F64 && a.inner >= 1 && a.B >= 2 && blocks_of(a) < 1024 &&
-           (long)a.M * a.N * a.K <= 1L << 17 &&
+    if (a.dtype != GRIDNET_F64 || (a.block_size != 4 && a.block_size != 8) || a.inner < 1 || a.inner > kMaxBackwardIters)
+        return false;
+    return a.B >= 2 && a.M <= 1 << 17 && a.N <= 1 << 17 && (long)a.M * a.N <= 1L << 17 &&
+           (long)a.M * a.N * a.K <= 1L << 17 && blocks_of(a) < 1024 &&
            (a.block_size == 8 ? bwd_f64_lds<8>(a.inner) : bwd_f64_lds<4>(a.inner)) <= kF64MaxLds;
 }
 size_t step_f64_workspace(const StepArgs &a) { return dsum_bytes(a) + halo_bytes(a); }

@@ -5,6 +5,8 @@ import ctypes
 import inspect
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -82,6 +84,27 @@ def test_host_only_entry_points():
     assert rc == 4 and "workspace" in native.last_error()
 
 
+@pytest.mark.parametrize("block_size", [0, -1, -8, 3, 5, 16])
+def test_size_queries_of_block_sizes_that_are_refused(block_size):
+    """Callers ask for the size before the call that checks the arguments: the answer is 0, in every
+    precision.  In a process of its own, for what must not happen there is that it dies."""
+    queries = [f"gridnet_hip_backward_workspace_bytes({dt}, 4, 16, 16, 16, {inner}, {block_size}, {norm})"
+               for dt in (0, 1, 2) for inner in (1, 2, 2000000) for norm in (0, 1)]
+    queries += [f"gridnet_hip_backward_gated_workspace_bytes({dt}, 4, 16, 16, 16, 2, {block_size})" for dt in (0, 1)]
+    queries += [f"gridnet_hip_fused_workspace_bytes(4, 16, 16, 16, 2, {block_size}, {b})" for b in (0, 1)]
+    queries += [f"gridnet_hip_fused_forward_chain_workspace_bytes(4, 16, 16, 16, 2, {block_size})",
+                f"gridnet_hip_chain_all_workspace_bytes(4, 16, 16, 16, 2, 4, {block_size})"]
+    assert answers(queries) == [0] * len(queries)
+
+
+def answers(queries):
+    code = f"from gridnet_amd.native import lib\nfor q in {queries!r}: print(eval('lib.' + q), flush=True)"
+    run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    got = [int(v) for v in run.stdout.split()]
+    assert run.returncode == 0, f"status {run.returncode} at {queries[len(got)]}: {run.stderr}"
+    return got
+
+
 def test_native_operators_decline_tensors_without_data():
     """Fake device tensors have no memory behind them: the native operators leave them to the Python ones."""
     import torch
@@ -102,8 +125,6 @@ def test_native_operators_decline_tensors_without_data():
 
 
 def test_native_operators_and_library_of_different_builds_do_not_go_together(tmp_path):
-    import subprocess
-
     from gridnet_amd import native
 
     for op in (native.ops.step, native.ops.gated_step, native.ops.layer_norm):

@@ -144,12 +144,18 @@ static void give_slabs(StepArgs &a, void *workspace, size_t workspace_bytes, siz
     }
 }
 
+// Whether there are blocks at all.  The size queries below answer 0 otherwise: they are asked before the call
+// that checks its arguments, and the plans behind them divide by the number of blocks.
+static bool has_blocks(int B, int M, int N, int K, int block_size) {
+    return B > 0 && (block_size == 4 || block_size == 8) && M >= block_size && N >= block_size && K >= block_size;
+}
+
 size_t gridnet_hip_backward_workspace_bytes(int dtype, int B, int M, int N, int K, int inner,
                                             int block_size, int normalize) {
     StepArgs a{};
     a.dtype = dtype; a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner;
     a.block_size = block_size; a.normalize = normalize != 0; a.activation = GRIDNET_ACT_RELU;
-    if (B <= 0 || M <= 0 || N <= 0 || K <= 0) return 0;
+    if (!has_blocks(B, M, N, K, block_size)) return 0;
     // (a caller that hands over less, or nothing, is served by the kernel that needs none)
     if (step_f64_supports(a)) return step_f64_workspace(a) + step_f64_slab_bytes(a);
     if (!step_fast_supports(a, true)) return 0;
@@ -240,7 +246,7 @@ size_t gridnet_hip_backward_gated_workspace_bytes(int dtype, int B, int M, int N
     StepArgs a{};
     a.dtype = dtype; a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner;
     a.block_size = block_size; a.activation = GRIDNET_ACT_RELU;
-    if (B <= 0 || M <= 0 || N <= 0 || K <= 0) return 0;
+    if (!has_blocks(B, M, N, K, block_size)) return 0;
     if (!gated_fast_supports(a, true)) return 0;
     const size_t slabs = gated_fast_slab_bytes(a);
     return slabs ? (gated_fast_backward_workspace(a) + 255) / 256 * 256 + slabs : gated_fast_backward_workspace(a);
@@ -361,7 +367,7 @@ size_t gridnet_hip_fused_workspace_bytes(int B, int M, int N, int K, int inner, 
     StepArgs a{};
     a.dtype = GRIDNET_F32; a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner;
     a.block_size = block_size; a.activation = GRIDNET_ACT_RELU;
-    if (B <= 0 || M <= 0 || N <= 0 || K <= 0 || (block_size != 4 && block_size != 8)) return 0;
+    if (!has_blocks(B, M, N, K, block_size)) return 0;
     if (!backward) return fused_forward_workspace(a);
     const size_t need = fused_backward_dsum(a) + fused_backward_parts(a), slabs = step_fast_slab_bytes(a);
     return slabs ? (need + 255) / 256 * 256 + slabs : need;
@@ -434,7 +440,7 @@ int gridnet_hip_fused_forward_chain_merges(int dtype, int B, int M, int N, int K
 }
 
 size_t gridnet_hip_fused_forward_chain_workspace_bytes(int B, int M, int N, int K, int inner, int block_size) {
-    if (B <= 0 || M <= 0 || N <= 0 || K <= 0 || (block_size != 4 && block_size != 8)) return 0;
+    if (!has_blocks(B, M, N, K, block_size)) return 0;
     return 2 * ((fused_forward_workspace(fused_chain_args(B, M, N, K, inner, block_size)) + 255) / 256 * 256);
 }
 

@@ -97,6 +97,21 @@ def test_size_queries_of_block_sizes_that_are_refused(block_size):
     assert answers(queries) == [0] * len(queries)
 
 
+@pytest.mark.parametrize("side,block_size", [(1, 4), (3, 4), (1, 8), (4, 8), (7, 8)])
+def test_size_queries_of_grids_without_a_block(side, block_size):
+    grid = f"{side}, {side}, {side}"
+    queries = [f"gridnet_hip_backward_workspace_bytes({dt}, 4, {grid}, {inner}, {block_size}, {norm})"
+               for dt in (0, 1) for inner in (1, 2) for norm in (0, 1)]
+    queries += [f"gridnet_hip_backward_gated_workspace_bytes(0, 4, {grid}, 2, {block_size})"]
+    queries += [f"gridnet_hip_fused_workspace_bytes(4, {grid}, {inner}, {block_size}, {b})" for inner in (1, 2) for b in (0, 1)]
+    queries += [f"gridnet_hip_fused_forward_chain_workspace_bytes(4, {grid}, 2, {block_size})",
+                f"gridnet_hip_fused_forward_chain_merges(0, 4, {grid}, 2, {block_size})",
+                f"gridnet_hip_chain_forward_all_supported(0, 4, {grid}, 2, 4, {block_size}, 0)",
+                f"gridnet_hip_chain_all_supported(0, 4, {grid}, 2, 4, {block_size}, 0)",
+                f"gridnet_hip_chain_all_workspace_bytes(4, {grid}, 2, 4, {block_size})"]
+    assert answers(queries) == [0] * len(queries)
+
+
 def answers(queries):
     code = f"from gridnet_amd.native import lib\nfor q in {queries!r}: print(eval('lib.' + q), flush=True)"
     run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)

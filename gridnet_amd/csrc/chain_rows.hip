@@ -332,8 +332,8 @@ struct RowsBwdArgs {
     const float *weight, *scale, *gamma, *beta;
     const float *dy;                // gradient with respect to LayerNorm(y)
     const float *y, *y_stats;
-    float *y_sums;                  // the LayerNorm backward's two sums per sample
-    const float *y_part;            // MERGE: the pairs that they come from, merged here by `lanes` threads each
+    const float *y_sums;            // the LayerNorm backward's two sums per sample,
+    const float *y_part;            // MERGE: or the pairs that they come from, merged here by `lanes` threads each
     int lanes;
     const float *saved;
     const float *x, *x_stats;       // the step's input: raw, and the statistics of the LayerNorm on it (null: as it is)
@@ -347,10 +347,14 @@ struct RowsBwdArgs {
 
 // PLAIN: two cells per thread, GATED: one; 54 mirrored weights and 54 gradient accumulators for each set
 // and two cells.  A thread moves its own row and one or two of the 20 rows around the tube.
+// MERGE: the merged sums go through LDS into SETS registers of every wave, which the loop takes them from with a
+// readlane.  (Read from LDS by every element they cost the step 4 us of 67.)  The plain update has one register to
+// spare for them, and merges for 32 samples at most: both sums of sample s0 + e in lanes 2 e and 2 e + 1.
+constexpr int bwd_merge_most(int sets) { return sets == 1 ? kWave / 2 : kWave; }
 template <int ACT, int SETS, int K, bool MERGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_bwd(RowsBwdArgs a) {
     constexpr int CPT = 2 / SETS;
-    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K], then gamma and (plain) scale of the rows
+    extern __shared__ __attribute__((aligned(16))) float lds[];  // [2][SETS][36][K], then gamma and (plain) scale of the rows; MERGE: the sums
     int tube, chunk;
     if (!split_block_id(blockIdx.x, a.ntube, a.nchunk, a.together, false, tube, chunk)) return;  // grid padding
     const int tid = threadIdx.x, M = a.M, N = a.N, nw = blockDim.x / 64, wave = tid / 64;
@@ -360,6 +364,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int s0 = chunk * a.chunk_len, s1 = min(a.B, s0 + a.chunk_len);
     const long slab = chunk * a.slab_stride;
     float *dweight = a.dweight + slab;
+    float *merged = lds + (2 * SETS + 1 + (SETS == 1)) * kWinRows * K;  // of the samples s0 ... s1
 
     // ---- mirrored weights W[26 - t, c + off_t] and the gradients of those weights ----
     // A tap's weights for the thread's cells lie along K, one cell off its own for dk = -1 / +1: aligned
@@ -393,7 +398,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     load_planes(a.weight, v);
     if constexpr (MERGE)  // while the weights are on their way
         merge_pairs<8>(a.y_part, a.ntube * nw, a.lanes, s0, s1 - s0, [&](int e, double t1, double t2, double) {
-            reinterpret_cast<float2 *>(a.y_sums)[s0 + e] = make_float2((float)(t1 / (double)cells), (float)(t2 / (double)cells));
+            reinterpret_cast<float2 *>(merged)[e] = make_float2((float)(t1 / (double)cells), (float)(t2 / (double)cells));
         });
     // a step's sums start from zero, also where there is something to add them to (see the end)
 #pragma unroll
@@ -442,7 +447,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     store_cells<CPT>(gam_rows + own_at, gam);
     if (SETS == 1) store_cells<CPT>(scale_rows + own_at, rv);
     wait_global_loads();
-    if (MERGE) lds_barrier();  // the sums are there, also for the loads below: every wave has waited for its stores
+    const int lane = tid & 63;
+    float sums[SETS] = {};
+    if (MERGE) {
+        lds_barrier();  // the sums are there
+#pragma unroll
+        for (int k = 0; k < SETS; ++k) sums[k] = merged[SETS * lane + k];  // behind the last sample: anything, not used
+    }
 #pragma unroll
     for (int pq = 0; pq < 9; ++pq) {
         const int gi = p.p0 + p.ci + pq / 3 - 1, gj = p.q0 + p.cj + pq % 3 - 1;
@@ -464,15 +475,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr int NF = SETS;
     struct Ahead {
         float dy[3][CPT], y[3][CPT], f[3][NF][CPT], gate[CPT], x[CPT];
-        float numbers;  // of the sample, by lane: statistics of y, the two sums, statistics of x
+        float numbers;  // of the sample, by lane: statistics of y, the two sums (not with MERGE), statistics of x
     };
     const unsigned own_off = 4u * (unsigned)p.grow;
     const unsigned off[3] = {own_off, 4u * (unsigned)hoff[0], 4u * (unsigned)hoff[1]};
-    const int lane = tid & 63;
+    // MERGE: statistics of y in lanes 0 and 1, of x in 4 and 5, from one base (both are parts of one array)
     const float *number = lane < 2 ? a.y_stats + lane : lane < 4 ? a.y_sums + (lane - 2) : lane < 6 && ln_in ? a.x_stats + (lane - 4) : a.y_stats;
+    const float *stats = ln_in ? a.x_stats : a.y_stats;
+    const unsigned stat_at = 4u * (lane & 1) + (lane < 4 ? (unsigned)((const char *)a.y_stats - (const char *)stats) : 0u);
     auto fetch = [&](int s, Ahead &n) {
         const long at = (long)s * cells;
-        n.numbers = number[2 * s];
+        if constexpr (MERGE) {
+            float v[1];
+            load_at<1>(stats + 2L * s, stat_at, v);
+            n.numbers = v[0];
+        } else {
+            n.numbers = number[2 * s];
+        }
         load_at<CPT>(a.x + at, own_off, n.x);
         if (SETS == 2) load_at<CPT>(a.saved + 2 * tensor + at, own_off, n.gate);
 #pragma unroll
@@ -486,7 +505,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     float out[CPT];
     auto element = [&](int s, float *stage, Ahead &n) {
         auto number_of = [&](int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(n.numbers), k)); };
-        const float ymean = number_of(0), yrstd = number_of(1), c1 = number_of(2), c2 = number_of(3);
+        auto sum_of = [&](int k) {
+            return __int_as_float(SETS == 1 ? __builtin_amdgcn_readlane(__float_as_int(sums[0]), 2 * (s - s0) + k)
+                                            : __builtin_amdgcn_readlane(__float_as_int(sums[k * (SETS - 1)]), s - s0));
+        };
+        const float ymean = number_of(0), yrstd = number_of(1);
+        const float c1 = MERGE ? sum_of(0) : number_of(2), c2 = MERGE ? sum_of(1) : number_of(3);
         const float xmean = number_of(4), xrstd = number_of(5);
         // through the LayerNorm's backward: the gradient with respect to the step's raw output
         auto raw_gradient = [&](float dy, float y, float gamma, float &yh) {
@@ -741,7 +765,7 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
     const auto kern = rows_bwd<ACT, SETS, K, false>, merging = rows_bwd<ACT, SETS, K, true>;
     const long cells = cells_of(c), tensor = (long)c.B * cells;
     const int ntube = tubes_of(c), nt = bwd_threads(c), pairs = bwd_pairs(c);
-    const size_t lds = (2 * SETS + 1 + (SETS == 1)) * (size_t)kWinRows * K * sizeof(float);
+    const size_t lds = (2 * SETS + 1 + (SETS == 1)) * (size_t)kWinRows * K * sizeof(float) + SETS * kWave * sizeof(float);
     static int per_cu = 0;  // per instantiation
     if (per_cu == 0) {
         const int n = workgroups_per_cu(kern, nt, lds);
@@ -749,7 +773,7 @@ template <int ACT, int SETS, int K> int run_backward(const RowsChain &c, hipStre
     }
     RowsBwdArgs a{};
     a.nchunk = bwd_chunks(c, per_cu, a.chunk_len);
-    a.lanes = plan_merge_lanes(nt, a.chunk_len, pairs);
+    a.lanes = a.chunk_len <= bwd_merge_most(SETS) ? plan_merge_lanes(nt, a.chunk_len, pairs) : 0;
     a.together = rows_together<K>(ntube, a.nchunk, per_cu);
     a.weight = c.weight; a.scale = c.scale; a.gamma = c.gamma; a.beta = c.beta;
     a.B = c.B; a.M = c.M; a.N = c.N; a.ntube = ntube;

@@ -225,8 +225,10 @@ def test_gated_chain_at_the_scripts_defaults_is_as_exact_as_torch(seed):
 
 # pairs of the merge: an odd number (a kernel of its own), two, more than a request's worth per thread, several
 # threads to a sample and one; chunks that end early; too many samples per workgroup
+# (chunks of 32 samples, the most that the plain backward merges for, and of 33)
 @pytest.mark.parametrize("shape,batch", [((12, 12, 16), 5), ((4, 8, 16), 7), ((16, 16, 32), 37), ((32, 32, 32), 70),
-                                         ((8, 8, 32), 300), ((16, 32, 64), 11), ((4, 4, 32), 5000)], ids=str)
+                                         ((8, 8, 32), 300), ((16, 32, 64), 11), ((4, 4, 32), 5000),
+                                         ((16, 16, 32), 1024), ((16, 16, 32), 1025)], ids=str)
 def test_statistics_merged_by_the_next_step(shape, batch):
     """Statistics and backward sums of every step, against sums over the tensors themselves in double (fp32
     pairs over 256 values: 2^-24 times a few)."""
@@ -255,3 +257,42 @@ def test_statistics_merged_by_the_next_step(shape, batch):
         step.forward(h[j])
         grad = step.backward(grad)[-1].clone()
     assert_close(dx, grad.double(), rtol=1e-5, atol=1e-5, what="dx")
+
+
+@pytest.mark.parametrize("gated", [False, True], ids=["plain", "gated"])
+def test_merged_sums_stay_in_the_workgroup(gated):
+    """What a workgroup merges it hands to its waves through its LDS.  In memory, where all workgroups of a step would
+    write the same words and read them back, the sums of the last step still stand after the backward."""
+    from gridnet_amd import native as n
+
+    shape, batch, outer = (16, 16, 32), 37, 3
+    gamma, beta, x, gy = (t.to(DEV) for t in inputs(shape, batch))
+    w, b, r = (t.to(DEV) for t in make_params(shape, seed=4))
+    if gated:
+        w, b = torch.stack([w, w.flip(0)], 1), torch.stack([b, r])
+    sets, act, stream = 1 + gated, n.activation_id("tanh"), n.current_stream(x)
+    saved = torch.empty(outer, 3 if gated else 1, *x.shape, device=DEV)
+    y_raw, stats = torch.empty(outer, *x.shape, device=DEV), torch.empty(outer, batch, 2, device=DEV)
+    out, dx = torch.empty_like(x), torch.empty_like(x)
+    grads = [torch.empty_like(t) for t in (w, b, r, gamma, beta)]
+    scale = None if gated else r.data_ptr()
+    ws = n.workspace(max(n.lib.gridnet_hip_rows_chain_workspace_bytes(batch, *shape, int(gated), 1, d) for d in (0, 1)), DEV)
+    n.check(n.lib.gridnet_hip_rows_chain_forward(
+        w.data_ptr(), b.data_ptr(), scale, gamma.data_ptr(), beta.data_ptr(), x.data_ptr(), y_raw.data_ptr(),
+        stats.data_ptr(), saved.data_ptr(), out.data_ptr(), batch, *shape, outer, int(gated), 1e-5, act,
+        ws.data_ptr(), ws.numel(), stream))
+    dw, db, dr, dg, dbt = (t.data_ptr() for t in grads)
+    n.check(n.lib.gridnet_hip_rows_chain_backward(
+        w.data_ptr(), scale, gamma.data_ptr(), beta.data_ptr(), x.data_ptr(), y_raw.data_ptr(), stats.data_ptr(),
+        saved.data_ptr(), gy.data_ptr(), dw, db, None if gated else dr, dg, dbt, dx.data_ptr(), batch, *shape, outer,
+        int(gated), act, n.OVERWRITE_PARAMS, ws.data_ptr(), ws.numel(), stream))
+    want = torch.empty(batch, 2, device=DEV)
+    scratch = n.workspace(n.lib.gridnet_hip_layernorm_workspace_bytes(0, batch, x[0].numel()), DEV)
+    n.check(n.lib.gridnet_hip_layernorm_backward_sums(
+        0, gy.data_ptr(), y_raw[-1].data_ptr(), stats[-1].data_ptr(), gamma.data_ptr(), want.data_ptr(), batch,
+        x[0].numel(), scratch.data_ptr(), scratch.numel(), stream))
+    # the workspace: two arrays of pairs, one for each wave and sample, and the sums behind them
+    pairs = shape[0] // 4 * (shape[1] // 4) * (16 * shape[2] * sets // 2 // 64)
+    at = -ws.data_ptr() % 256 + 2 * ((batch * pairs * 8 + 255) // 256 * 256)
+    assert torch.equal(ws[at:at + batch * 8].view(torch.float32).view(batch, 2), want)
+    assert torch.isfinite(dx).all()

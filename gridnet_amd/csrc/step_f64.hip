@@ -21,7 +21,8 @@
 // over the whole window; what the halo adds to either sum is delta[c] times a number per cell and element
 // (`wh`, `sh`: the cell's weights that read the halo, and those times what they read).  A halo entry gets
 // sum w D1 - x_h Q + R with D1 = sum_i inv_i delta_i, Q = sum_i C_i, R = sum_i (C_i mean_i - inv_i A_i / W),
-// the gradient of a weight that reads it x_h D1 - D2, D2 = sum_i mean_i inv_i delta_i.
+// the gradient of a weight that reads it x_h D1 - D2, D2 = sum_i mean_i inv_i delta_i; x and the means less the
+// window's shift (`shift_of`), or these differences would cancel.
 // No atomics anywhere: two runs give the same bits.
 //
 // What bounds it: latency, at one workgroup of eight waves per CU (216 to 256 registers).  24 x 32 x 32, batch
@@ -59,12 +60,14 @@ template <int BS> struct Cell {
     using G = Geo<BS>;
     int p0, q0, r0, i, j, k;  // block origin in the grid, place in the block
     int gc, base, centre;     // grid index, window positions of tap 0 and of the cell itself
+    int first;                // grid index of the block's first cell
     __device__ __forceinline__ Cell(int tid, int blk, int N, int K) {
         const int kb = K / BS, nb = N / BS;
         p0 = (blk / (kb * nb)) * BS, q0 = ((blk / kb) % nb) * BS, r0 = (blk % kb) * BS;
         const int b = tid / BS % BS, c = tid / (BS * BS);
         k = tid % BS, i = BS == 8 ? b : c, j = BS == 8 ? c : b;
         gc = ((p0 + i) * N + (q0 + j)) * K + (r0 + k);
+        first = (p0 * N + q0) * K + r0;
         base = i * G::PS + j * G::RS + k;
         centre = G::tap(base, 13);
     }
@@ -119,15 +122,27 @@ template <int BS> struct Edges {
                           ? (gi * N + gj) * K + gk : -1;
         }
     }
-    // the shell of sample `xs` into both window copies, and into `halo`
-    __device__ __forceinline__ void fill(const double *xs, double *win, double (&halo)[SH::kPerThread]) const {
+    // the shell of sample `xs`, less `shift`, into both window copies, and into `halo` (0 where there is no entry)
+    __device__ __forceinline__ void fill(const double *xs, double shift, double *win, double (&halo)[SH::kPerThread]) const {
 #pragma unroll
         for (int e = 0; e < SH::kPerThread; ++e) {
-            halo[e] = grid[e] >= 0 ? xs[grid[e]] : 0.0;
+            halo[e] = (grid[e] >= 0 ? xs[grid[e]] : 0.0) - (at[e] >= 0 ? shift : 0.0);
             if (at[e] >= 0) win[at[e]] = win[G::WIN + at[e]] = halo[e];
         }
     }
 };
+
+// What a normalised window is worked on without: its block's first cell.  The result does not depend on it, and
+// differences of neighbours are exact, where sums and differences of values with a large mean round at its scale.
+// Error of dweight over its norm, without -> with, 24^3, three iterations, x around 100: 4e-15 -> 2e-16, 1e4: 4e-13 ->
+// 2e-16, 1e6: 3e-11 -> 1e-14.  It costs the forward up to 5 %, the backward's kernels 1 to 2 and 0.3 us.
+// None where squares of it leave the range: that window's variance is infinite, as it is without.
+__device__ __forceinline__ double shift_of(double first) { return __builtin_fabs(first) < 1e150 ? first : 0.0; }
+// (the same for the whole workgroup: in scalar registers)
+__device__ __forceinline__ double shift_of_block(const double *xs, int first) {
+    const double v = shift_of(xs[first]);
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)), __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
 
 // Sums over the workgroup, the same bits in every thread; `red` is this call's own (two calls in a row take
 // different ones), so one barrier is enough.
@@ -201,8 +216,9 @@ __global__ __launch_bounds__(BS *BS *BS) void step_fwd_f64(
     const int s_end = min(B, (chunk + 1) * chunk_len);
     for (int s = chunk * chunk_len; s < s_end; ++s) {
         const double *xs = x + s * cells;
-        double cur = xs[p.gc], halo[Shell<BS>::kPerThread];
-        edges.fill(xs, win, halo);  // the element before is done with the windows: its last pass wrote none
+        const double shift = NORM ? shift_of_block(xs, p.first) : 0.0;
+        double cur = NORM ? xs[p.gc] - shift : xs[p.gc], halo[Shell<BS>::kPerThread];
+        edges.fill(xs, shift, win, halo);  // the element before is done with the windows: its last pass wrote none
         win[p.centre] = cur;
         lds_barrier();
         for (int it = 0; it < inner; ++it) {
@@ -213,12 +229,14 @@ __global__ __launch_bounds__(BS *BS *BS) void step_fwd_f64(
             if (it + 1 < inner) win[((it + 1) & 1) * G::WIN + p.centre] = cur;
             lds_barrier();
         }
-        y[s * cells + p.gc] = cur;
+        y[s * cells + p.gc] = NORM ? cur + shift : cur;
     }
 }
 
+// (two waves per SIMD asked for: left alone the compiler takes a few registers more with normalize and 4^3 blocks, and
+// there is one; 40^3, batch 4, three iterations, 57 us instead of 47)
 template <int BS, int ACT, bool NORM>
-__global__ __launch_bounds__(BS *BS *BS) void step_bwd_f64(
+__global__ __launch_bounds__(BS *BS *BS, 2) void step_bwd_f64(
     const double *__restrict__ weight, const double *__restrict__ bias, const double *__restrict__ scale,
     const double *__restrict__ x, const double *__restrict__ dy, double *__restrict__ dweight,
     double *__restrict__ dbias, double *__restrict__ dscale, double *__restrict__ dx, double *__restrict__ dsum,
@@ -263,9 +281,10 @@ __global__ __launch_bounds__(BS *BS *BS) void step_bwd_f64(
     const int s_end = min(B, (chunk + 1) * chunk_len);
     for (int s = chunk * chunk_len; s < s_end; ++s) {
         const double *xs = x + s * cells;
-        double cur = xs[gc], g = dy[s * cells + gc], halo[SH::kPerThread];
+        const double shift = NORM ? shift_of_block(xs, p.first) : 0.0;
+        double cur = NORM ? xs[gc] - shift : xs[gc], g = dy[s * cells + gc], halo[SH::kPerThread];
         lds_barrier();  // the element before is done with the windows
-        edges.fill(xs, win, halo);
+        edges.fill(xs, shift, win, halo);
         win[centre] = cur;
         // The cell's own weights are fetched for every element and are gone on the way back: with them the
         // 81 doubles per thread do not fit beside the rest (24 to 72 registers spilled).
@@ -405,7 +424,7 @@ __global__ __launch_bounds__(BS *BS *BS) void step_bwd_f64(
 
 
 // What the cells of other blocks owe a cell: dx[c] += sum over the taps t that leave c's block of
-// W[26-t, c+off_t] D[c+off_t], and with normalisation R - x[c] Q of every block that has c in its halo.  A
+// W[26-t, c+off_t] D[c+off_t], and with normalisation R - x[c] Q, x less the shift, of every block that has c in its halo.  A
 // thread per cell and batch element, for the cells some tap of which leaves the block.  The workgroups behind
 // those add up the copies of the parameter gradients.  Four waves per SIMD for their sake: with the weights
 // in registers for several elements (two waves) the kernel took 13.2 us at 24 x 32 x 32, batch 6, now 8.3.
@@ -480,7 +499,8 @@ template <int BS, bool NORM> __global__ __launch_bounds__(256, 4) void step_cros
             }
             if (there) {
                 const double *qr = a.halo_part + ((long)s * a.nblk + ((long)b[0] * nb + b[1]) * kb + b[2]) * 2;
-                sum += qr[1] - x * qr[0];
+                const long first = (((long)b[0] * a.N + b[1]) * a.K + b[2]) * BS;  // of block b
+                sum += qr[1] - (x - shift_of(a.x[(long)s * cells + first])) * qr[0];
             }
         }
     }
@@ -584,7 +604,7 @@ template <int BS, bool BWD, bool NORM> int dispatch_f64(const StepArgs &a, hipSt
 // Where the scattering kernel would split the batch of a block, and add the parameter gradients by atomics:
 // batches of two and more, fewer than 1024 blocks.  Elsewhere its one launch less decides.  Backward there / here
 // (two inner iterations; three with normalize), 40^3, batch 4, 8^3 blocks: 82 / 47 and 106 / 69 us; 4^3 blocks:
-// 78 / 50 and 91 / 75; 48^3 in 4^3 blocks (1728 of them): 56 / 62 and 86 / 114; 40^3, batch 1: 21 / 22 and 33 / 33,
+// 78 / 50 and 91 / 67; 48^3 in 4^3 blocks (1728 of them): 56 / 62 and 86 / 114; 40^3, batch 1: 21 / 22 and 33 / 33,
 // 4^3 blocks 19 / 22 and 26 / 26.  Up to 2^17 cells: gridnet_hip_backward has asked callers with larger fp64
 // grids for no scratch.  No iteration at all, and histories beyond LDS (more than 15 iterations of 8^3 blocks), stay there too.
 // Size queries come here with arguments that nothing has looked at: what the sums below cannot take is refused first.

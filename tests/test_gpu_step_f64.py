@@ -77,3 +77,25 @@ def test_infinity_stays_where_its_taps_are():
     for name, g, e in zip(("dweight", "dbias", "dscale", "dx"), grads, want):
         assert torch.equal(torch.isfinite(g), torch.isfinite(e)), name
     assert not torch.isfinite(grads[0]).all()
+
+
+@pytest.mark.parametrize("shape,bs,inner,batch", [((24, 24, 24), 8, 3, 2), ((24, 24, 24), 8, 12, 3),
+                                                  ((12, 12, 12), 4, 3, 3), ((12, 12, 12), 4, 8, 2)])
+def test_a_window_far_from_zero_is_normalised_as_exactly(shape, bs, inner, batch):
+    """The middle block of three a side, whose window holds no zeros from outside the grid, does not depend on a
+    constant that every input has on top.  Here that is 2^20, on inputs of 30 bits behind the point, which it leaves
+    exact.  Worked on without it the gradients are those of inputs around zero, to the bound there; one rounding at its
+    scale is 1e-10.  (The output holds the constant: half an ulp of it.)"""
+    from test_gpu_step import run_op
+
+    w, b, r = make_params(shape, seed=13, dtype=torch.float64)
+    x = torch.round(make_acts(batch, shape, seed=14, dtype=torch.float64) * 2 ** 30) / 2 ** 30
+    middle = (..., *[slice(bs, 2 * bs)] * 3)
+    gy = torch.zeros_like(x)
+    gy[middle] = make_acts(batch, (bs, bs, bs), seed=15, dtype=torch.float64)
+    y, grads = run_op(w, b, r, x + 2.0 ** 20, gy, inner, bs, 1e-5, True, "tanh")
+    want_y, want = oracle(w, b, r, x, gy, inner, bs, 1e-5, True, "tanh")
+    assert_close(y[middle].cpu() - 2.0 ** 20, want_y[middle], 0, 2.0 ** -32, "y")
+    for name, g, e in zip(("dweight", "dbias", "dscale", "dx"), grads, want):
+        part = middle if name != "dx" else (...,)
+        assert_close(g[part], e[part], 1e-12, 1e-12, name)

@@ -40,6 +40,8 @@
 // when one workgroup owns the whole batch of its block, written with plain stores.  Results are
 // bitwise reproducible in that case.
 
+#include <algorithm>
+
 #include "common.h"
 #include "fast_tiles.h"
 #include "plan.h"
@@ -2049,7 +2051,13 @@ template <int BS, int CPT, int NSLOT, int ACT> int launch_bwd_as(const StepArgs 
 // batch 64, 35 -> 21 / 39 -> 27; 32^3, batch 8, 29 -> 20 / 44 -> 27 (eight slots of two: 25 / 34); but 24^3, batch 64, 43 -> 46 / 58 ->
 // 60.  One cell, one slot: 16^3, batch 1, two iterations, 13.6 -> 6.9 / 17.5 -> 9.0; 64^3, batch 1, 51 -> 31 / 60 -> 36, batch 4, 63 -> 55 /
 // 80 -> 70; 96^3, batch 4, 183 -> 147 / 249 -> 175; but 64^3, batch 8, 80 -> 83 / 113 -> 113, batch 32, 197 -> 279 / 315 -> 388.
-constexpr int kFewPairsBackward4 = 16, kShortWalkBackward4 = 16;
+// Batches of two and three with one slot, a workgroup and a copy of the gradients for each sample (step_fast_slab_bytes):
+// two slots of half a wave -> one that walks them -> one each, first kernel, four iterations: 16^3, batch 2, 14.4 -> 9.8 ->
+// 7.9 / 18.9 -> 14.5 -> 10.4; batch 3, 15.2 -> 10.4 -> 7.9 / 19.9 -> 14.9 -> 10.5; 24^3, batch 3, 17.1 -> 12.3 -> 10.8 / 22.4 ->
+// 17.7 -> 14.2; the copies cost the second kernel 0.3 us at most, 0.7 at 24^3, batch 2.  A step of a chain, both kernels:
+// 16^3, batch 2, 21.4 -> 16.0 -> 13.4; only 24^3, batch 3, with two iterations loses by it, 24.0 -> 18.6 -> 19.5.  With the
+// whole batch of a block in a workgroup: 32^3, batch 2, 16.1 -> 11.9 / 21.0 -> 16.8; batch 3, 20.2 -> 15.0 / 28.4 -> 21.8.
+constexpr int kFewPairsBackward4 = 16, kShortWalkBackward4 = 16, kOneSlotBackward4 = 3;
 template <int ACT> int launch_bwd_slots(const StepArgs &a, hipStream_t st) {
     const int nblk = (a.M / 4) * (a.N / 4) * (a.K / 4), cus = device_cus();
     const bool ln = a.ln.gamma != nullptr;
@@ -2060,9 +2068,9 @@ template <int ACT> int launch_bwd_slots(const StepArgs &a, hipStream_t st) {
                      : nblk <= 2 * cus ? a.B < 32
                      : nblk <= 4 * cus ? a.B <= 4
                                        : a.B == 1 || (long)a.B * a.inner <= kShortWalkBackward4;
-    if (few && nblk <= 2 * cus && a.B >= 4 && fit(bwd_lds_bytes<4, 1, 4>(a.inner, ln, a.normalize), 2))
+    if (few && nblk <= 2 * cus && a.B > kOneSlotBackward4 && fit(bwd_lds_bytes<4, 1, 4>(a.inner, ln, a.normalize), 2))
         return launch_bwd_as<4, 1, 4, ACT>(a, st);
-    if (few && (a.B < 4 || nblk > 2 * cus) && fit(bwd_lds_bytes<4, 1, 1>(a.inner, ln, a.normalize), 4))
+    if (few && (a.B <= kOneSlotBackward4 || nblk > 2 * cus) && fit(bwd_lds_bytes<4, 1, 1>(a.inner, ln, a.normalize), 4))
         return launch_bwd_as<4, 1, 1, ACT>(a, st);
     if (eight) return launch_bwd_as<4, 2, 8, ACT>(a, st);
     if (four) return launch_bwd_as<4, 2, 4, ACT>(a, st);
@@ -2201,12 +2209,12 @@ size_t step_fast_backward_workspace(const StepArgs &a) {
 size_t step_fast_slab_bytes(const StepArgs &a) {
     if (bwd_rows_supports(a)) return bwd_rows_slab_bytes(a);
     // the most chunks any plan of the backward kernels makes: resident workgroups (two per CU with
-    // 8^3 blocks, bounded by 16 with 4^3) over the blocks, and never more than the batch gives
+    // 8^3 blocks, bounded by 16 with 4^3) over the blocks, and never more than the batch gives: a chunk
+    // is a sample with 8^3 blocks, two with 4^3 but for the batches that launch_bwd_slots deals to one slot
     const long nblk = (long)(a.M / a.block_size) * (a.N / a.block_size) * (a.K / a.block_size);
     if (nblk >= device_cus()) return 0;  // one workgroup owns the whole batch of its block
-    const int nslot = a.block_size == 8 ? kBwdSlots8 : kBwdSlots4;
     long chunks = (long)(a.block_size == 8 ? 2 : 16) * device_cus() / nblk;
-    const long most = (a.B + nslot - 1) / nslot;
+    const long most = a.block_size == 8 ? a.B : std::max(std::min(a.B, kOneSlotBackward4), (a.B + kBwdSlots4 - 1) / kBwdSlots4);
     if (chunks > most) chunks = most;
     if (chunks < 2) return 0;
     return (size_t)chunks * kStepSlabPlanes * a.M * a.N * a.K * sizeof(float);

@@ -173,6 +173,21 @@ def test_a_workspace_of_the_largest_batch_serves_the_smaller_ones():
                 assert need == sorted(need), (m, k, gated, backward)
 
 
+def test_short_batches_of_small_blocks_have_room_to_be_split():
+    """4^3 blocks: batches of two and three are walked by a wave per sample, which takes a copy of the 31 gradient planes
+    for each; no smaller batch gets more room than a larger one."""
+    from gridnet_amd import native
+
+    for shape in ((8, 8, 8), (16, 16, 16), (16, 24, 32)):
+        cells, last = shape[0] * shape[1] * shape[2], 0
+        for batch in range(1, 40):
+            room = native.lib.gridnet_hip_backward_workspace_bytes(0, batch, *shape, 4, 4, 0) - 4 * batch * cells
+            if batch in (2, 3):
+                assert room >= batch * 31 * 4 * cells, (shape, batch)
+            assert room >= last, (shape, batch)
+            last = room
+
+
 def test_shim_has_the_reference_call_surface():
     """Positional signatures of src/gridnet_cuda.cpp:61-72, 91-106, 133-141, 160-171."""
     import gridnet_cuda

@@ -16,12 +16,13 @@ DEV = "cuda:0"
 # without (65 is not split evenly); blocks that have a neighbour on one side only; ten inner iterations (at twenty the
 # gradients reach 3e3 and torch's own fp32 evaluation on the CPU lies 1.3 to 1.5 times outside the bar); 256 blocks,
 # whose workgroups have the whole batch in the backward.  4^3 blocks (few_for_slots, launch_bwd_slots): one slot and four of
-# one cell per thread, two, four and eight of two, full and with elements missing
+# one cell per thread, two, four and eight of two, full and with elements missing; two and three samples, each a wave's
+# with a copy of the gradients of its own, and three that a wave walks
 @pytest.mark.parametrize("shape,batch,inner,bs", [(*c, 8) for c in [
     ((8, 8, 8), 1, 1), ((8, 8, 8), 3, 4), ((16, 16, 16), 64, 2), ((16, 16, 16), 65, 2), ((24, 32, 40), 17, 2), ((24, 32, 40), 18, 2),
     ((16, 16, 32), 48, 2), ((16, 16, 32), 64, 2), ((16, 16, 32), 65, 2), ((16, 8, 24), 2, 10), ((32, 64, 64), 1, 2),
     ((32, 64, 64), 2, 2)]] + [(*c, 4) for c in [
-    ((4, 4, 4), 1, 2), ((8, 4, 12), 3, 4), ((16, 16, 16), 4, 2), ((16, 16, 16), 32, 2), ((16, 16, 16), 64, 2), ((16, 16, 16), 65, 2),
+    ((4, 4, 4), 1, 2), ((8, 4, 12), 3, 4), ((16, 16, 16), 2, 10), ((24, 24, 20), 2, 2), ((24, 24, 20), 3, 4), ((16, 16, 16), 4, 2), ((16, 16, 16), 32, 2), ((16, 16, 16), 64, 2), ((16, 16, 16), 65, 2),
     ((32, 32, 16), 3, 2), ((32, 32, 16), 9, 2), ((32, 32, 16), 31, 2), ((32, 32, 16), 32, 2), ((32, 32, 16), 37, 2), ((32, 36, 36), 4, 2),
     ((32, 36, 36), 5, 2), ((32, 36, 36), 18, 2), ((48, 48, 36), 4, 4), ((48, 48, 36), 5, 4)]], ids=str)
 @pytest.mark.parametrize("normalize", [False, True], ids=["plain", "normalize"])

@@ -18,9 +18,9 @@
 //     step while their weights are on their way (plan_merge_lanes says where; a small kernel between the steps
 //     elsewhere, 4.7 us each).  Merged inside the walk, by one wave an element ahead, they cost the kernels
 //     11 us forward and 24 us backward: everybody waits for that wave at the barrier.
-// 32^3, batch 256, silu, per step: forward 28.2 us, backward 67.0, at 4.3 TB/s either way where a copy
-// reaches 4.6 (with the merging kernels, the chunks of a tube on several CUs, 30.4 and 69.0; fwd_rows, bwd_rows and cross_rows with theirs: 28.1 + 4.4,
-// 59.3 + 8.0 + 23.4).  Gated, tanh: 55.5 and 86.6 (op by op the whole training step took 21.3 ms, 9.2 now).
+// 32^3, batch 256, silu, per step: forward 27.5 us, backward 67.7, at 4.2 to 4.3 TB/s where a copy
+// reaches 4.6 (with the kernel that merges 29.1 + 68.4, and with the chunks of a tube on several CUs, 30.4 and 69.0; fwd_rows, bwd_rows and cross_rows with theirs: 28.1 + 4.4,
+// 59.3 + 8.0 + 23.4).  Gated, tanh: 55.7 and 85.8 + 4.9 (op by op the whole training step took 21.3 ms, 9.1 now).
 
 #include <algorithm>
 
@@ -349,7 +349,9 @@ struct RowsBwdArgs {
 // and two cells.  A thread moves its own row and one or two of the 20 rows around the tube.
 // MERGE: the merged sums go through LDS into SETS registers of every wave, which the loop takes them from with a
 // readlane.  (Read from LDS by every element they cost the step 4 us of 67.)  The plain update has one register to
-// spare for them, and merges for 32 samples at most: both sums of sample s0 + e in lanes 2 e and 2 e + 1.
+// spare for them, and merges for 32 samples at most: both sums of sample s0 + e in lanes 2 e and 2 e + 1.  Longer chunks,
+// of over a thousand samples on fewer than 64 tubes, leave it to the kernel between the steps (16 x 16 x 32, batch 2048, 121 ->
+// 123 us); the register filled again after 32 samples spilled three, and 32^3, batch 256, lost what it gains.
 constexpr int bwd_merge_most(int sets) { return sets == 1 ? kWave / 2 : kWave; }
 template <int ACT, int SETS, int K, bool MERGE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_bwd(RowsBwdArgs a) {

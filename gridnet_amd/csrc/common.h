@@ -170,7 +170,7 @@ __device__ __forceinline__ void finalize_sums_of_sample(const float *__restrict_
 // one-thread-per-cell fp32 kernels publish their 27 products in a table prod[27][bs^3] and every
 // window entry e sums the ones aimed at it: tap t from cell e - offset(t), where that cell exists.
 // ds_add_f64 keeps up, and an fp64 table would leave room for one workgroup per CU only (measured
-// 1.7x slower than the scatter), so fp64 keeps the atomics.
+// 1.7x slower than the scatter), so the scattering kernels keep the atomics in fp64 (step_f64.hip gathers without a table).
 template <typename T> constexpr bool kGatherTaps = sizeof(T) == 4;
 
 template <int BS> struct TapGather {

@@ -77,9 +77,9 @@ int plan_row_chunks(int B, int ntube, int resident, int min_walk, int &chunk_len
 // Threads to a sample where the workgroups of a step merge the pairs of the step before, beside the fetch of
 // their weights; 0: a kernel of its own does (4.7 us and a launch).  Every workgroup of a chunk merges the
 // same pairs, so it pays as long as they are few per thread.  Forward / backward of a step with the kernel and
-// without: 32^3, batch 16, 10.5 -> 8.7 / 17.1 -> 15.8 us; batch 64, 15.9 -> 13.7 / 31.9 -> 30.7; batch 256 (22 and 32
-// pairs per thread) 30.4 -> 28.3 / 69.0 -> 68.3; 64^3, batch 32 (44 pairs) 30.7 -> 32.1 / 74.0 -> 74.6.  Gated, 32^3,
-// batch 32, 17.1 -> 15.4 / 26.3 -> 25.3; batch 256, 57.0 -> 55.5 forward.
+// without: 32^3, batch 16, 11.1 -> 9.0 / 17.4 -> 16.1 us; batch 64, 15.5 -> 13.4 / 30.7 -> 29.9; batch 256 (22 and 32
+// pairs per thread) 31.0 -> 28.7 / 68.2 -> 67.3; 64^3, batch 32 (44 pairs) 30.7 -> 32.1 / 74.0 -> 74.6.  Gated, 32^3,
+// batch 32, 18.1 -> 16.1 / 26.2 -> 25.8; batch 256, 56.0 -> 54.7 forward.
 constexpr int kMergeMostSamples = 64, kMergeMostPairs = 32;  // per workgroup; per thread
 int plan_merge_lanes(int threads, int chunk_len, int pairs) {
     if (pairs % 2 || chunk_len > kMergeMostSamples) return 0;

@@ -225,10 +225,11 @@ def test_gated_chain_at_the_scripts_defaults_is_as_exact_as_torch(seed):
 
 # pairs of the merge: an odd number (a kernel of its own), two, more than a request's worth per thread, several
 # threads to a sample and one; chunks that end early; too many samples per workgroup
-# (chunks of 32 samples, the most that the plain backward merges for, and of 33)
+# (backward: chunks of 32 samples, the most that the plain kernel merges for, of 33, 64 and 65)
 @pytest.mark.parametrize("shape,batch", [((12, 12, 16), 5), ((4, 8, 16), 7), ((16, 16, 32), 37), ((32, 32, 32), 70),
                                          ((8, 8, 32), 300), ((16, 32, 64), 11), ((4, 4, 32), 5000),
-                                         ((16, 16, 32), 1024), ((16, 16, 32), 1025)], ids=str)
+                                         ((16, 16, 32), 1024), ((16, 16, 32), 1025), ((16, 16, 32), 2048),
+                                         ((16, 16, 32), 2049)], ids=str)
 def test_statistics_merged_by_the_next_step(shape, batch):
     """Statistics and backward sums of every step, against sums over the tensors themselves in double (fp32
     pairs over 256 values: 2^-24 times a few)."""

@@ -369,7 +369,9 @@ size_t gridnet_hip_fused_workspace_bytes(int B, int M, int N, int K, int inner, 
     a.block_size = block_size; a.activation = GRIDNET_ACT_RELU;
     if (!has_blocks(B, M, N, K, block_size)) return 0;
     if (!backward) return fused_forward_workspace(a);
-    const size_t need = fused_backward_dsum(a) + fused_backward_parts(a), slabs = step_fast_slab_bytes(a);
+    const size_t need = fused_backward_dsum(a) + fused_backward_parts(a);
+    a.ln.gamma = (const float *)&a;  // only whether there is one matters
+    const size_t slabs = step_fast_slab_bytes(a);
     return slabs ? (need + 255) / 256 * 256 + slabs : need;
 }
 

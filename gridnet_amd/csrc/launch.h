@@ -169,6 +169,13 @@ int step_fast_backward_parts(int block_size);  // (sum g, sum g*xhat) pairs per 
 int step_fast_backward_pairs(const StepArgs &a);  // pairs per sample that the backward of `a` leaves
 int step_fast_cross_pairs(const StepArgs &a);     // the same for step_cross_launch alone (behind chain_bwd)
 
+// step_quads.hip: a step of a chain with 4^3 blocks, four samples to a wave (what step_forward_fast and
+// step_backward_fast take it for)
+bool step_quads_supports(const StepArgs &a, bool backward);
+size_t step_quads_slab_bytes(const StepArgs &a);  // room for the gradient copies of its backward, 0 where it is not taken
+int step_quads_forward(const StepArgs &a, hipStream_t st);
+int step_quads_backward(const StepArgs &a, hipStream_t st);
+
 // fwd_rows.hip: the forward of a step with ONE inner iteration, dealt by whole K-rows (fp32, normalize
 // off, K up to 128; the folded LayerNorm and the residual form as a.ln says)
 bool fwd_rows_supports(const StepArgs &a);

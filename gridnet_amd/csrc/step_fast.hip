@@ -2214,20 +2214,23 @@ size_t step_fast_slab_bytes(const StepArgs &a) {
     // 8^3 blocks, bounded by 16 with 4^3) over the blocks, and never more than the batch gives: a chunk
     // is a sample with 8^3 blocks, two with 4^3 but for the batches that launch_bwd_slots deals to one slot
     const long nblk = (long)(a.M / a.block_size) * (a.N / a.block_size) * (a.K / a.block_size);
-    if (nblk >= device_cus()) return 0;  // one workgroup owns the whole batch of its block
+    const size_t quads = step_quads_slab_bytes(a);
+    if (nblk >= device_cus()) return quads;  // one workgroup owns the whole batch of its block
     long chunks = (long)(a.block_size == 8 ? 2 : 16) * device_cus() / nblk;
     const long most = a.block_size == 8 ? a.B : std::max(std::min(a.B, kOneSlotBackward4), (a.B + kBwdSlots4 - 1) / kBwdSlots4);
     if (chunks > most) chunks = most;
-    if (chunks < 2) return 0;
-    return (size_t)chunks * kStepSlabPlanes * a.M * a.N * a.K * sizeof(float);
+    if (chunks < 2) return quads;
+    return std::max(quads, (size_t)chunks * kStepSlabPlanes * a.M * a.N * a.K * sizeof(float));
 }
 
 int step_forward_fast(const StepArgs &a, hipStream_t st) {
     if (fwd_rows_supports(a)) return fwd_rows_launch(a, st);  // one inner iteration: a plain stencil, by whole rows
+    if (step_quads_supports(a, false)) return step_quads_forward(a, st);
     return dispatch<false>(a, st);
 }
 int step_backward_fast(const StepArgs &a, hipStream_t st) {
     if (bwd_rows_supports(a)) return bwd_rows_launch(a, st);  // one inner iteration: by whole rows
+    if (step_quads_supports(a, true)) return step_quads_backward(a, st);
     return dispatch<true>(a, st);
 }
 

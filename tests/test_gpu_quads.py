@@ -1,0 +1,41 @@
+"""4^3 blocks, four samples to a wave (csrc/step_quads.hip) at the edges of what it works on, against the CPU oracle in
+fp64: groups of samples and of blocks that are not full, the shortest and the longest history, batches in chunks."""
+
+import pytest
+import torch
+
+from helpers import ATOL, RTOL, assert_close, make_acts, make_params
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# forward: the rows' blocks in workgroups of four, three, two and one; one, two and more groups of samples, the last one of
+# every size; two to nine iterations.  The backward is this file's where the last column says so: a walk of 32 at least, groups
+# that are nearly full, more than half of the places of its waves taken
+@pytest.mark.parametrize("shape,batch,inner,quads", [
+    ((4, 4, 4), 4, 2, False), ((4, 8, 12), 5, 3, False), ((8, 8, 20), 7, 2, False), ((8, 4, 36), 6, 9, False),
+    ((32, 32, 32), 16, 8, True), ((32, 32, 32), 31, 7, True), ((16, 16, 16), 256, 4, True), ((32, 32, 36), 32, 2, True),
+    ((40, 44, 44), 16, 2, True), ((40, 44, 44), 4, 8, True), ((40, 44, 44), 16, 9, False), ((48, 48, 60), 16, 2, True)], ids=str)
+@pytest.mark.parametrize("residual", [False, True], ids=["chain", "residual"])
+@pytest.mark.parametrize("activation", ["silu", "tanh"])
+def test_chain_against_the_oracle(shape, batch, inner, quads, residual, activation):
+    from gridnet_amd.runner import BodyRunner
+    from oracle.network import network_forward_backward
+
+    print(f"quads, chain {shape} B={batch} inner={inner} residual={residual} {activation} backward here: {quads}", flush=True)
+    g = torch.Generator().manual_seed(3)
+    w, b, r = make_params(shape, seed=11)
+    if inner >= 7:
+        w, r = w * 0.5, r * 0.5
+    params = [w, b, r, *((a + 0.2 * torch.randn(shape, generator=g)) for a in (1, 0))]
+    x, gy = (make_acts(batch, shape, seed=s) for s in (12, 13))
+    run = BodyRunner(*(t.to(DEV) for t in params), batch, inner, 2, 4, activation, fused=True, outer_residual=residual)
+    got = [run.forward(x.to(DEV)).clone(), *(t.clone() for t in run.backward(gy.to(DEV)))]
+    for name, a, e in zip("y dweight dbias dscale dgamma dbeta dx".split(), [run.forward(x.to(DEV)), *run.backward(gy.to(DEV))], got):
+        assert torch.equal(a, e), f"{name}: two runs differ"
+    want = network_forward_backward([t.double() for t in params], x.double(), gy.double(), inner_iterations=inner,
+                                    outer_iterations=2, block_size=4, activation=activation, outer_residual=residual)
+    for name, a, e in zip("y dweight dbias dscale dgamma dbeta dx".split(), got, want):
+        # an entry of the gradients is a sum over the batch, and its error goes with its terms (2e-7 of the array's rms)
+        assert_close(a, e, RTOL, ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)

@@ -135,6 +135,28 @@ template <int TPS> __device__ __forceinline__ float slot_wave_sum(float v) {
     return (r0 + r1) + (r2 + r3);
 }
 
+// The same for ONE lane of the wave's share of the slot (has_sum), which is all that a sum for LDS needs: six dependent
+// operations for the whole wave instead of eleven.
+template <int TPS> __device__ __forceinline__ bool has_sum(int lane) {
+    return TPS > 64 ? (lane & 63) == 63 : (lane & (TPS - 1)) == 0;
+}
+template <int TPS> __device__ __forceinline__ float sum_for_one(float v) {
+    if constexpr (TPS <= 64) {
+        return slot_wave_sum<TPS>(v);
+    } else {
+#define GRIDNET_ADD_DPP(ctrl, rows) \
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, true))
+        GRIDNET_ADD_DPP(0x111, 0xf);  // row_shr:1, 2, 4, 8: lane 15 of a row of 16 has its sum
+        GRIDNET_ADD_DPP(0x112, 0xf);
+        GRIDNET_ADD_DPP(0x114, 0xf);
+        GRIDNET_ADD_DPP(0x118, 0xf);
+        GRIDNET_ADD_DPP(0x142, 0xa);  // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3
+        GRIDNET_ADD_DPP(0x143, 0xc);
+#undef GRIDNET_ADD_DPP
+        return v;
+    }
+}
+
 // (mean, M2 about that mean) of four rows of lanes, `row_cells` cells each, from the rows' pairs
 __device__ __forceinline__ void four_rows_moments(const float (&m)[4], const float (&q)[4], int row_cells, float &mean,
                                                   float &m2) {

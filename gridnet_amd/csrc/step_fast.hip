@@ -900,16 +900,16 @@ template <int BS, int CPT> __host__ __device__ constexpr int bwd_slot_floats(int
 }
 // NORM, per slot behind all of the above: (mean, std, 1/(std+eps), -) of the window before
 // every inner iteration, then the sums the waves of a slot exchange: 4 floats per wave taken
-// at commit, 2 x 2 per wave for the owned cells (alternating between iterations), 2 per wave in
-// the reverse sweep
+// at commit, 2 x 2 per wave for the owned cells and 2 x 2 in the reverse sweep (alternating
+// between iterations)
 template <int BS, int CPT> __host__ __device__ constexpr int bwd_norm_waves() {
     return Tile<BS, CPT>::TPS >= 64 ? Tile<BS, CPT>::TPS / 64 : 1;
 }
-// ... and three values per owned cell that live as long as the kernel but are touched once per
-// iteration or element (sum of the cell's weights, sum of those whose taps read the halo, D2
-// summed over the batch): in LDS, the register file has no room for them
+// ... and two values per owned cell that live as long as the kernel but are touched once per
+// iteration or element (sum of the cell's weights, D2 summed over the batch): in LDS, the
+// register file has no room for them
 template <int BS, int CPT> __host__ __device__ constexpr int bwd_norm_floats(int inner) {
-    return 4 * inner + 12 * bwd_norm_waves<BS, CPT>() + 3 * CPT * Tile<BS, CPT>::TPS;
+    return 4 * inner + 12 * bwd_norm_waves<BS, CPT>() + 2 * CPT * Tile<BS, CPT>::TPS;
 }
 // ... and at least the 27 weight planes of the block, which pass through LDS once at set-up
 template <int BS, int CPT, int NSLOT> size_t bwd_lds_bytes(int inner, bool ln = false, bool norm = false) {
@@ -927,11 +927,12 @@ template <int BS, int CPT, int NSLOT> size_t bwd_lds_bytes(int inner, bool ln = 
 // iteration i adds to window entry k is (N = (bs+2)^3 entries)
 //   inv_i (dn_i[k] - A_i / N) - (x_i[k] - mean_i) C_i,   A_i = sum_k dn_i[k],
 //   C_i = inv_i^2 / (N std_i) * sum_k dn_i[k] (x_i[k] - mean_i).
-// Both sums run over the whole window.  The owned cells' part comes from the gather of the
-// reverse sweep; the halo's part needs no halo entry of dn: summed over the halo,
-// dn_i = sum_c delta_i[c] * (sum of c's weights whose taps read the halo) and
-// dn_i x = sum_c delta_i[c] * (those weights times the halo values they read), and both
-// brackets are fixed for the element (the halo is frozen).  What the HALO entries receive over
+// Both sums run over the whole window, but need no entry of dn: a cell sends its weights times
+// delta_i, so with z_i = sum_t w_t n_i, the pre-activation without its bias,
+//   A_i = sum_c delta_i[c] * (sum of c's weights),   sum_k dn_i[k] (x_i[k] - mean_i) = sum_c delta_i[c] z_i[c] / inv_i,
+// known as soon as delta_i is: the sums travel with the delta window, behind the same barrier.  (Formed from the gathered dn and
+// the halo's share of them they took a second barrier per reverse iteration and a stencil over the halo per element.)
+// The history holds z_i and not the pre-activation, which would leave z_i the rounding error of the bias.  What the HALO entries receive over
 // all iterations is, for halo entry h,
 //   sum over (c, t) reading h of w_t[c] D1[c]  -  x_h Q + R,
 //   D1 = sum_i inv_i delta_i,  Q = sum_i C_i,  R = sum_i (mean_i C_i - inv_i A_i / N):
@@ -988,8 +989,7 @@ void step_bwd_fast(
     float *nstat = lds + NSLOT * slot_floats + pl.slot * norm_stride;
     float *ncommit = nstat + 4 * inner, *nown = ncommit + 4 * NW, *nrev = nown + 4 * NW;
     float *wsum_at = nrev + 4 * NW + pl.lane * CPT;  // this thread's: sum of a cell's weights
-    float *wout_at = wsum_at + CPT * TL::TPS;         // of those whose taps read the halo
-    float *d2acc_at = wout_at + CPT * TL::TPS;        // D2 summed over the batch elements
+    float *d2acc_at = wsum_at + CPT * TL::TPS;        // D2 summed over the batch elements
     const int wave_in_slot = TL::TPS >= 64 ? pl.lane / 64 : 0;
     constexpr float inv_count = 1.f / TL::NWIN;
 
@@ -1088,22 +1088,18 @@ void step_bwd_fast(
                                          : 0.f;
         lds_barrier();  // the windows reuse this memory
     }
-    // NORM: sum of a cell's 27 weights, and of those whose taps read the halo (only this thread
-    // ever touches its three LDS entries per cell: no barrier needed for them)
+    // NORM: sum of a cell's 27 weights (only this thread ever touches its two LDS entries per cell:
+    // no barrier needed for them)
     float zero[CPT];
     if (NORM) {
-        float wsum[CPT], wout[CPT];
+        float wsum[CPT];
 #pragma unroll
         for (int c = 0; c < CPT; ++c) {
-            wsum[c] = wout[c] = zero[c] = 0.f;
+            wsum[c] = zero[c] = 0.f;
 #pragma unroll
-            for (int t = 0; t < 27; ++t) {
-                wsum[c] += w[t][c];
-                wout[c] += in_block(t, c) ? 0.f : w[t][c];
-            }
+            for (int t = 0; t < 27; ++t) wsum[c] += w[t][c];
         }
         store_cells<CPT>(wsum_at, wsum);
-        store_cells<CPT>(wout_at, wout);
         store_cells<CPT>(d2acc_at, zero);
     }
     if (ln_in && pl.slot == 0) {  // gamma and beta of the window, once per workgroup
@@ -1161,8 +1157,8 @@ void step_bwd_fast(
             shift = pre_shift;
             fx.commit_sums(win, pre, shift, part);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) part[q] = slot_wave_sum<TL::TPS>(part[q]);
-            if ((pl.lane & 63 & (TL::TPS - 1)) == 0)
+            for (int q = 0; q < 4; ++q) part[q] = sum_for_one<TL::TPS>(part[q]);
+            if (has_sum<TL::TPS>(pl.lane))
                 *reinterpret_cast<float4 *>(ncommit + wave_in_slot * 4) =
                     make_float4(part[0], part[1], part[2], part[3]);
         } else fx.commit(win, pre);
@@ -1220,7 +1216,7 @@ void step_bwd_fast(
         // ---- forward recompute, remembering x_i and u_i of the owned cells ----
         for (int it = 0; it < inner; ++it) {
             if (active) {
-                float u[CPT];
+                float u[CPT], z[CPT];
                 if (NORM) {
                     if (it > 0) {
                         own1 = own2 = 0.f;
@@ -1238,13 +1234,17 @@ void step_bwd_fast(
                     float wsum[CPT];
                     load_cells<CPT>(wsum_at, wsum);
 #pragma unroll
-                    for (int c = 0; c < CPT; ++c) u[c] = fmaf(inv, fmaf(-mean, wsum[c], u[c]), bv[c]);
+                    for (int c = 0; c < CPT; ++c) {
+                        const float t = fmaf(-mean, wsum[c], u[c]);
+                        u[c] = fmaf(inv, t, bv[c]);
+                        z[c] = inv * t;
+                    }
                 } else {
                     stencil<TL, CPT, kBwdDepth>(win + (it & 1) * TL::WIN, pl.row00, w, bv, u);
                 }
                 float *h = hist + it * (TL::TPS * 2 * CPT);
                 store_cells<CPT>(h, cur);
-                store_cells<CPT>(h + TL::TPS * CPT, u);
+                store_cells<CPT>(h + TL::TPS * CPT, NORM ? z : u);
                 if (it + 1 < inner) {
                     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
@@ -1255,9 +1255,9 @@ void step_bwd_fast(
                         s2 = fmaf(cur[c], cur[c], s2);
                     }
                     if (NORM) {  // the owned cells' part of the next iteration's statistics
-                        s1 = slot_wave_sum<TL::TPS>(s1);
-                        s2 = slot_wave_sum<TL::TPS>(s2);
-                        if ((pl.lane & 63 & (TL::TPS - 1)) == 0)
+                        s1 = sum_for_one<TL::TPS>(s1);
+                        s2 = sum_for_one<TL::TPS>(s2);
+                        if (has_sum<TL::TPS>(pl.lane))
                             *reinterpret_cast<float2 *>(nown + (((it + 1) & 1) * NW + wave_in_slot) * 2) =
                                 make_float2(s1, s2);
                     }
@@ -1270,20 +1270,28 @@ void step_bwd_fast(
         }
 
         // ---- reverse sweep: delta window copy (it & 1) holds delta_it ----
-        // NORM: dsum is D1, d2 is D2; x_i of the owned cells as the stencil saw it (xn); delta of
-        // the iteration; the halo brackets (wout is fixed, sout belongs to the element); Q and R
-        float dsum[CPT], xi[CPT], xn[CPT], d2[CPT], dlt[CPT], sout[CPT], q_sum = 0.f, r_sum = 0.f;
+        // NORM: dsum is D1, d2 is D2; x_i of the owned cells as the stencil saw it (xn); the sums of the iteration; Q and R
+        float dsum[CPT], xi[CPT], xn[CPT], d2[CPT], pa = 0.f, pz = 0.f, q_sum = 0.f, r_sum = 0.f;
 #pragma unroll
-        for (int c = 0; c < CPT; ++c) dsum[c] = d2[c] = sout[c] = 0.f;
+        for (int c = 0; c < CPT; ++c) dsum[c] = d2[c] = 0.f;
         for (int it = inner - 1; it >= 0; --it) {
             if (active) {
                 const float *h = hist + it * (TL::TPS * 2 * CPT);
-                float u[CPT];
+                float u[CPT], z[CPT], wsum[CPT];
                 load_cells<CPT>(h, xi);
                 load_cells<CPT>(h + TL::TPS * CPT, u);
-                if (NORM && it < inner - 1) {
-                    const float4 st4 = *reinterpret_cast<const float4 *>(nstat + 4 * it);
-                    mean = st4.x; sd = st4.y; inv = st4.z;
+                if (NORM) {
+                    load_cells<CPT>(wsum_at, wsum);
+#pragma unroll
+                    for (int c = 0; c < CPT; ++c) {
+                        z[c] = u[c];
+                        u[c] += bv[c];
+                    }
+                    if (it < inner - 1) {
+                        const float4 st4 = *reinterpret_cast<const float4 *>(nstat + 4 * it);
+                        mean = st4.x; sd = st4.y; inv = st4.z;
+                    }
+                    pa = pz = 0.f;
                 }
 #pragma unroll
                 for (int c = 0; c < CPT; ++c) {
@@ -1293,7 +1301,8 @@ void step_bwd_fast(
                     dr[c] = fmaf(f, g[c], dr[c]);
                     db[c] += delta;
                     if (NORM) {
-                        dlt[c] = delta;
+                        pa = fmaf(delta, wsum[c], pa);
+                        pz = fmaf(delta, z[c], pz);
                         dsum[c] = fmaf(inv, delta, dsum[c]);
                         d2[c] = fmaf(mean * inv, delta, d2[c]);
                         xn[c] = (xi[c] - mean) * inv;
@@ -1302,6 +1311,12 @@ void step_bwd_fast(
                         xn[c] = xi[c];
                     }
                     dwin[(it & 1) * TL::WIN + pl.own + c] = delta;
+                }
+                if (NORM) {
+                    pa = NW > 1 ? sum_for_one<TL::TPS>(pa) : slot_wave_sum<TL::TPS>(pa);
+                    pz = NW > 1 ? sum_for_one<TL::TPS>(pz) : slot_wave_sum<TL::TPS>(pz);
+                    if (NW > 1 && has_sum<TL::TPS>(pl.lane))
+                        *reinterpret_cast<float2 *>(nrev + ((it & 1) * NW + wave_in_slot) * 2) = make_float2(pa, pz);
                 }
             }
             if (it == 0) {
@@ -1320,11 +1335,6 @@ void step_bwd_fast(
                     });
             }
             slot_barrier<TL::TPS>();
-            if (NORM && active && it == inner - 1) {
-                // once per element: what the owned cells' taps into the halo see there (the
-                // halo window holds zeros in the block's cells, so the other taps add nothing)
-                stencil<TL, CPT, kBwdDepth>(xhalo, pl.row00, w, zero, sout);
-            }
             float dn[CPT];  // NORM: gradient with respect to the normalised value of the owned cells
 #pragma unroll
             for (int c = 0; c < CPT; ++c) dn[c] = 0.f;
@@ -1341,43 +1351,22 @@ void step_bwd_fast(
                         }
                 });
             }
-            if (NORM) {
-                // A = sum dn and sum dn * x over the whole window, the halo through its brackets
-                float pa = 0.f, pb = 0.f;
-                if (active) {
-                    float wout[CPT];
-                    load_cells<CPT>(wout_at, wout);
-#pragma unroll
-                    for (int c = 0; c < CPT; ++c) {
-                        pa += fmaf(dlt[c], wout[c], dn[c]);
-                        pb += fmaf(dlt[c], sout[c], dn[c] * xi[c]);
-                    }
-                    pa = slot_wave_sum<TL::TPS>(pa);
-                    pb = slot_wave_sum<TL::TPS>(pb);
-                }
+            if (NORM && active) {
                 if (NW > 1) {
-                    if (active && (pl.lane & 63) == 0)
-                        *reinterpret_cast<float2 *>(nrev + wave_in_slot * 2) = make_float2(pa, pb);
-                    lds_barrier();
-                    if (active) {
-                        pa = pb = 0.f;
+                    pa = pz = 0.f;
 #pragma unroll
-                        for (int q = 0; q < NW; ++q) {
-                            const float2 p2 = *reinterpret_cast<const float2 *>(nrev + q * 2);
-                            pa += p2.x; pb += p2.y;
-                        }
+                    for (int q = 0; q < NW; ++q) {  // fixed order: every thread gets the same sums
+                        const float2 p2 = *reinterpret_cast<const float2 *>(nrev + ((it & 1) * NW + q) * 2);
+                        pa += p2.x; pz += p2.y;
                     }
                 }
-                if (active) {
-                    const float a_mean = pa * inv_count;
-                    const float proj = fmaf(-mean, pa, pb);  // sum dn (x - mean)
-                    const float coef = proj * inv * inv * inv_count / fmaxf(sd, 1e-30f);
+                const float a_mean = pa * inv_count;
+                const float coef = pz * inv * inv_count / fmaxf(sd, 1e-30f);
 #pragma unroll
-                    for (int c = 0; c < CPT; ++c)
-                        g[c] += fmaf(inv, dn[c] - a_mean, -(xi[c] - mean) * coef);
-                    q_sum += coef;
-                    r_sum += fmaf(mean, coef, -inv * a_mean);
-                }
+                for (int c = 0; c < CPT; ++c)
+                    g[c] += fmaf(inv, dn[c] - a_mean, -(xi[c] - mean) * coef);
+                q_sum += coef;
+                r_sum += fmaf(mean, coef, -inv * a_mean);
             }
         }
 

@@ -25,8 +25,9 @@
 // status word is raised; then it does the chain again, one workgroup per element and no waits
 // between workgroups.  The caller need not look at the status and nothing synchronises.
 //
-// All of it is latency: one 32^3 sample, one inner iteration, 3.4 us a step, of which the arithmetic is
-// 0.4; 64 steps with the MNIST model around them 824 -> 258 us.
+// All of it is latency: one 32^3 sample, one inner iteration, 2.5 us a step, of which the arithmetic is
+// 0.4 (3.6 with the taps behind the statistics, see chain_fwd); 64 steps with the MNIST model around them
+// 824 -> 213 us.
 
 #include "common.h"
 #include "fast_tiles.h"
@@ -101,17 +102,23 @@ __device__ __forceinline__ void load_weights(const float *weight, int cells, int
         for (int c = 0; c < 3; ++c) w[3 * r + c] = weight[(long)(3 * r + 1 + (c - 1) * dir) * cells + cell];
 }
 
+// sum + the 27 taps on a window
+template <typename T>
+__device__ __forceinline__ T taps(const float *win, int at, int dir, const float (&w)[27], T sum) {
+    const float *row = win + at, *from[3] = {row - dir, row, row + dir};
+#pragma unroll
+    for (int t = 0; t < 27; ++t)
+        sum = fma((T)w[t], (T)from[t % 3][(t / 9 - 1) * kSide * kSide + (t / 3 % 3 - 1) * kSide], sum);
+    return sum;
+}
+
 // All inner iterations of one block: x in, x out; the shell is in both window copies and x in the
 // first.
 template <int ACT>
 __device__ __forceinline__ float advance(float (*win)[kWindow], int at, int dir, const float (&w)[27], float bias,
                                          float scale, float x, int inner, float &last_u) {
     for (int it = 0; it < inner; ++it) {
-        const float *row = win[it & 1] + at, *from[3] = {row - dir, row, row + dir};
-        float u = bias;
-#pragma unroll
-        for (int t = 0; t < 27; ++t)
-            u = fmaf(w[t], from[t % 3][(t / 9 - 1) * kSide * kSide + (t / 3 % 3 - 1) * kSide], u);
+        const float u = taps(win[it & 1], at, dir, w, bias);
         x = fmaf(scale, Act<ACT, float>::f(u), x);
         last_u = u;
         if (it + 1 < inner) {
@@ -164,76 +171,124 @@ struct GroupSums {
     }
 };
 
-template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd(ChainFwdArgs a) {
+// The wave that merges the statistics of step j - 1: every block's words, in the same order everywhere.
+// `early`: its first words as they were before the taps, or null.
+struct Words { unsigned long long of[kAhead]; };
+__device__ __forceinline__ Words request_words(const ChainFwdArgs &a, const unsigned long long *from, int i0) {
+    Words w;  // together: one trip to memory
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) w.of[k] = ld_agent(from + min(i0 + 64 * k, kGroups * a.nblk - 1));
+    return w;
+}
+__device__ __forceinline__ void merge_words(const ChainFwdArgs &a, const unsigned long long *from, const Words *early, int j, int s,
+                                            bool first, int &budget, float *norm) {
+    const int lane = threadIdx.x & 63, nwords = kGroups * a.nblk;
+    GroupSums sums;
+    for (int i0 = lane; i0 < nwords; i0 += 64 * kAhead) {
+        Words got = early && i0 == lane ? *early : request_words(a, from, i0);
+        unsigned long long (&word)[kAhead] = got.of;
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            while (word[k] == ~0ull && budget > 0) {
+                if (--budget == 0) st_agent(a.status, 1u);
+                __builtin_amdgcn_s_sleep(1);
+                word[k] = ld_agent(from + min(i0 + 64 * k, nwords - 1));
+            }
+            if (i0 + 64 * k < nwords) sums.add(word[k]);
+        }
+    }
+    sums.over_wave();
+    float mean, rstd;
+    sums.finish(1.0 / nwords, a.eps, mean, rstd);
+    if (lane == 0) {
+        norm[0] = mean;
+        norm[1] = rstd;
+        if (first && a.stats) {
+            a.stats[((long)(j - 1) * a.B + s) * 2] = mean;
+            a.stats[((long)(j - 1) * a.B + s) * 2 + 1] = rstd;
+        }
+    }
+}
+
+// The statistics of a step are there half a microsecond after its cells (a reduction, another trip to memory, the merge), so
+// the taps of the next step do not wait for them: with c any number near the block's values,
+//   sum_t w_t LN(y_t) = rstd (S - (mean - c) G) + H,   S = sum_t w_t gamma_t (y_t - c), G = sum_t w_t gamma_t, H = sum_t w_t beta_t,
+// S from the raw cells as they come in, G and H once per launch.  c is the mean of 32 of the block's values: S and
+// (mean - c) G then are of the size of the normalised sum, and the result is as exact as that (errors against 64 bits over eleven
+// kinds of chain, six seeds each: 1.00 times those of normalising first).  Per step of 64: 32^3, batch 1, 3.6 -> 2.5 us, batch 8,
+// 5.8 -> 3.9; 64^3, batch 1, 7.5 -> 6.8.  With one inner iteration only: the backward of more recomputes the step from its normalised
+// input, and the forward keeps to its operations.  (A wave of its own for the statistics, nine to a workgroup: two workgroups no
+// longer fit a CU, although the occupancy query says that they do.)
+template <int ACT, bool ONE> __global__ __launch_bounds__(kCfThreads) __attribute__((amdgpu_waves_per_eu(4))) void chain_fwd(ChainFwdArgs a) {
     __shared__ float win[2][kWindow];
     __shared__ __attribute__((aligned(16))) float values[kCfThreads];
     __shared__ float norm[2];
-    const int dir = k_direction(threadIdx.x, a.inner);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid / 64;
+    const int dir = ONE ? 1 : k_direction(tid, a.inner);
     const int blk = blockIdx.x % a.nblk, s = blockIdx.x / a.nblk;
     const int cells = a.M * a.N * a.K;
+    const long slot_cells = (long)a.B * cells, slot_parts = (long)kGroups * a.B * a.nblk;
+    int budget = a.spin_limit < 0 ? -a.spin_limit : a.spin_limit;
+    unsigned long long *parts = a.parts + (long)kGroups * s * a.nblk;
     const CellPlace p(tid, blk, a.M, a.N, a.K);
     const bool has = p.edge >= 0;
-    const long slot_cells = (long)a.B * cells, slot_parts = (long)kGroups * a.B * a.nblk;
-
     float w[27];
     load_weights(a.weight, cells, p.cell, dir, w);
     const float bias = a.bias[p.cell], scale = a.scale[p.cell], gam = a.gamma[p.cell], bet = a.beta[p.cell];
     const float egam = has ? a.gamma[p.edge] : 0.f, ebet = has ? a.beta[p.edge] : 0.f;
     float own = a.x0[(long)s * cells + p.cell];  // this cell's raw value
-    float edge = has ? a.x0[(long)s * cells + p.edge] : 0.f;
-    const double inv_groups = 1.0 / (kGroups * a.nblk);
-    int budget = a.spin_limit < 0 ? -a.spin_limit : a.spin_limit;
+    const float edge = has ? a.x0[(long)s * cells + p.edge] : 0.f;
     float *ring = a.ring + (long)s * cells;
-    unsigned long long *parts = a.parts + (long)kGroups * s * a.nblk;
 
+    float sum_gamma = 0.f, bias_beta = 0.f;
+    if (ONE) {
+        win[0][p.at] = gam;
+        win[1][p.at] = bet;
+        if (p.edge_at >= 0) {
+            win[0][p.edge_at] = egam;
+            win[1][p.edge_at] = ebet;
+        }
+        lds_barrier();
+        sum_gamma = (float)taps(win[0], p.at, dir, w, 0.0);
+        bias_beta = (float)taps(win[1], p.at, dir, w, (double)bias);
+        lds_barrier();
+    }
     for (int j = 0; j <= a.outer; ++j) {
-        float x = own, e = edge;
+        float x = own, e = edge, u, centre = 0.f;
+        // what step j - 1 left: the shell's cells, and the statistics of the element
+        const unsigned long long *words = parts + ((j - 1) & (kRing - 1)) * slot_parts;
+        Words early;
         if (j > 0) {
-            // what step j - 1 left: the shell's cells, and the statistics of the element
             const float *from = ring + ((j - 1) & (kRing - 1)) * slot_cells;
-            const unsigned long long *pf = parts + ((j - 1) & (kRing - 1)) * slot_parts;
-            const bool want = has && j < a.outer;
-            float v = want ? ld_agent(from + p.edge) : 0.f;
-            if (wave == 0) {
-                GroupSums sums;
-                const int nwords = kGroups * a.nblk;
-                for (int i0 = lane; i0 < nwords; i0 += 64 * kAhead) {
-                    unsigned long long word[kAhead];  // requested together: one trip to memory
-#pragma unroll
-                    for (int k = 0; k < kAhead; ++k) word[k] = ld_agent(pf + min(i0 + 64 * k, nwords - 1));
-#pragma unroll
-                    for (int k = 0; k < kAhead; ++k) {
-                        while (word[k] == ~0ull && budget > 0) {
-                            if (--budget == 0) st_agent(a.status, 1u);
-                            __builtin_amdgcn_s_sleep(1);
-                            word[k] = ld_agent(pf + min(i0 + 64 * k, nwords - 1));
-                        }
-                        if (i0 + 64 * k < nwords) sums.add(word[k]);
-                    }
-                }
-                sums.over_wave();
-                float mean, rstd;
-                sums.finish(inv_groups, a.eps, mean, rstd);
-                if (lane == 0) {
-                    norm[0] = mean;
-                    norm[1] = rstd;
-                    if (blk == 0 && a.stats) {
-                        a.stats[((long)(j - 1) * a.B + s) * 2] = mean;
-                        a.stats[((long)(j - 1) * a.B + s) * 2 + 1] = rstd;
-                    }
-                }
+            const bool want = j < a.outer && has;
+            e = want ? ld_agent(from + p.edge) : 0.f;
+            if (ONE) {
+                const float2 c = *reinterpret_cast<const float2 *>(values + 32 * (tid & 15) + (6 * tid & 30));
+                centre = row16_sum(fmaf(1.f / 32, c.x, 1.f / 32 * c.y));  // the same in every lane
+                x = (own - centre) * gam;
+            } else if (wave == 0) {
+                merge_words(a, words, nullptr, j, s, blk == 0, budget, norm);
             }
-            while (want && __float_as_uint(v) == kEmpty && budget > 0) {
+            while (want && __float_as_uint(e) == kEmpty && budget > 0) {
                 if (--budget == 0) st_agent(a.status, 1u);
                 __builtin_amdgcn_s_sleep(1);
-                v = ld_agent(from + p.edge);
+                e = ld_agent(from + p.edge);
             }
-            wait_global_loads();  // and the stores before: the slot emptied a step ago is empty
+            if (ONE) e = has ? (e - centre) * egam : 0.f;
+        }
+        if (ONE) {
+            win[0][p.at] = x;
+            if (p.edge_at >= 0) win[0][p.edge_at] = e;
             lds_barrier();
+            if (j > 0 && wave == 0) early = request_words(a, words, lane);
+            u = taps(win[0], p.at, dir, w, j > 0 ? 0.f : bias);
+            if (j > 0 && wave == 0) merge_words(a, words, &early, j, s, blk == 0, budget, norm);
+        }
+        if (j > 0) {
+            wait_global_loads();  // and the stores before: the slot emptied a step ago is empty
+            lds_barrier();        // the statistics
             const float mean = norm[0], rstd = norm[1];
             x = fmaf((own - mean) * rstd, gam, bet);
-            e = want ? fmaf((v - mean) * rstd, egam, ebet) : 0.f;
             if (j == a.outer) {
                 a.out[(long)s * cells + p.cell] = x;
                 break;
@@ -242,12 +297,18 @@ template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd(Chain
                 st_agent(ring + ((j - 2) & (kRing - 1)) * slot_cells + p.cell, __uint_as_float(kEmpty));
                 if (tid < kGroups) st_agent(parts + ((j - 2) & (kRing - 1)) * slot_parts + kGroups * blk + tid, ~0ull);
             }
+            // a variance beyond fp32 leaves nothing but beta
+            if (ONE) u = rstd == 0.f ? bias_beta : fmaf(rstd, fmaf(centre - mean, sum_gamma, u), bias_beta);
+            else e = has ? fmaf((e - mean) * rstd, egam, ebet) : 0.f;
         }
-        win[0][p.at] = x;
-        if (p.edge_at >= 0) win[0][p.edge_at] = win[1][p.edge_at] = e;
-        lds_barrier();
-        float u;
-        own = advance<ACT>(win, p.at, dir, w, bias, scale, x, a.inner, u);
+        if (ONE) {
+            own = fmaf(scale, Act<ACT, float>::f(u), x);
+        } else {
+            win[0][p.at] = x;
+            if (p.edge_at >= 0) win[0][p.edge_at] = win[1][p.edge_at] = e;
+            lds_barrier();
+            own = advance<ACT>(win, p.at, dir, w, bias, scale, x, a.inner, u);
+        }
         st_agent(ring + (j & (kRing - 1)) * slot_cells + p.cell, own);
         values[tid] = own;
         lds_barrier();
@@ -345,8 +406,8 @@ template <int ACT> int launch_chain_fwd(const ChainFwd &c, hipStream_t st) {
     const long blocks = (vecs + 1023) / 1024;
     hipLaunchKernelGGL(chain_fwd_clear, dim3((unsigned)(blocks > 2048 ? 2048 : blocks)), dim3(256), 0, st, (uint4 *)ws, vecs);
     void *args[] = {&a};
-    const hipError_t e = hipLaunchCooperativeKernel((const void *)chain_fwd<ACT>, dim3((unsigned)(a.nblk * c.B)),
-                                                    dim3(kCfThreads), args, 0, st);
+    const hipError_t e = hipLaunchCooperativeKernel(c.inner == 1 ? (const void *)chain_fwd<ACT, true> : (const void *)chain_fwd<ACT, false>,
+                                                    dim3((unsigned)(a.nblk * c.B)), dim3(kCfThreads), args, 0, st);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return fail(GRIDNET_ERR_LAUNCH, "chain_fwd: cooperative launch failed: %s", hipGetErrorString(e));
@@ -363,15 +424,15 @@ bool chain_fwd_supports(int B, int M, int N, int K, int inner, int outer) {
     static int per_cu = 0;
     if (per_cu == 0) {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)chain_fwd<GRIDNET_ACT_TANH>, kCfThreads, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)chain_fwd<GRIDNET_ACT_TANH, true>, kCfThreads, 0) !=
                 hipSuccess || n < 1)
             n = -1;
         per_cu = n;
     }
     if (per_cu < 1) return false;
     // As many as fit.  Launches included, a step of 64 against the kernel and the merge of a step launch by
-    // launch (rows_fwd): 32^3, one inner iteration, batch 1, 3.8 against 6.7 us, batch 8 (two workgroups per
-    // CU), 5.8 against 10.1; 64^3, batch 1, 7.6 against 10.2; four inner iterations (step_fwd_split), batch 8, 7.3 against 14.5.
+    // launch (rows_fwd): 32^3, one inner iteration, batch 1, 2.5 against 6.7 us, batch 8 (two workgroups per
+    // CU), 3.9 against 10.1; 64^3, batch 1, 6.8 against 10.2; four inner iterations (step_fwd_split), batch 8, 7.3 against 14.5.
     return (long)M * N * K / 512 * B <= (long)per_cu * plan_device_cus();
 }
 

@@ -45,6 +45,31 @@ def test_against_oracle(shape, batch, inner, outer, activation):
     assert torch.equal(again[0], got[0])
 
 
+@pytest.mark.parametrize("offset", [0.0, 50.0])
+@pytest.mark.parametrize("shape,batch,outer", [((8, 8, 8), 1, 2), ((16, 8, 40), 3, 6), ((32, 32, 32), 2, 3)], ids=str)
+def test_values_far_from_zero(shape, batch, outer, offset):
+    """One inner iteration takes its taps from the raw values less a number near them and puts the
+    statistics in afterwards: no less exact than a step launch by launch, which normalises first."""
+    from gridnet_amd.runner import BodyRunner
+    from oracle.network import network_forward
+
+    print(f"chain_fwd {shape} B={batch} outer={outer} offset {offset}", flush=True)
+    g = torch.Generator().manual_seed(8)
+    params = [*make_params(shape, seed=4), 1 + 0.2 * torch.randn(shape, generator=g),
+              offset + 0.2 * torch.randn(shape, generator=g)]
+    x = offset + make_acts(batch, shape, seed=6)
+    want = network_forward(*(t.double() for t in params), x.double(), inner_iterations=1, outer_iterations=outer,
+                           block_size=8, activation="tanh")
+    error = {}
+    for all_ in (True, False):
+        run = BodyRunner(*(t.to(DEV) for t in params), batch, 1, outer, 8, "tanh", fused=True, backward=False,
+                         forward_all=all_)
+        assert run.forward_all == all_
+        error[all_] = (run.forward(x.to(DEV)).cpu().double() - want).square().mean().sqrt().item()
+    # both are sums of some thousand roundings of the same size
+    assert error[True] <= 1.5 * error[False] + 1e-7 * (1 + offset), error
+
+
 def test_a_wait_that_runs_out_is_repaired():
     from gridnet_amd import native as n
 

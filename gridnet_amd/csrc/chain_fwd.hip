@@ -92,8 +92,8 @@ struct CellPlace {
 };
 
 // Cells in the second half of a block's rows take the three taps along k from high to low, as in the
-// kernels for 8^3 blocks (those for one inner iteration do not), so that a chain has the same bits
-// here and there: their weights are kept mirrored.
+// kernels for 8^3 blocks (those for one inner iteration do not): their weights are kept mirrored.  Those kernels take
+// the taps beyond the rows' ends first of all; a chain's last bits differ by that.
 __device__ __forceinline__ int k_direction(int tid, int inner) { return inner > 1 && (tid & 4) ? -1 : 1; }
 __device__ __forceinline__ void load_weights(const float *weight, int cells, int cell, int dir, float (&w)[27]) {
 #pragma unroll

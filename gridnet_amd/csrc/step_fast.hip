@@ -280,12 +280,18 @@ void step_fwd_fast(
 //   * centre: the 8 block columns of every window row as 8 floats, the second four REVERSED
 //     (columns 0 1 2 3 7 6 5 4).  A thread owns four cells of a row, holds them in the order
 //     they are stored, and reads or writes them as one aligned, conflict-free 128-bit access;
-//   * side: the two halo columns of every row, dense, one 32-bit read per row.
+//   * side: the two halo columns of every row, dense: the end entry of a thread's row.  It does not change with the
+//     iterations, so the nine of them are summed up once per element, in front of the other taps (once in memory, too).
 // The sixth value of a row, the cell next to the thread's four on the inner side, is the last
 // register of the lane that owns the other half of the row (lane ^ 1): one DPP operand, no LDS.
 // With the second half reversed both lanes of a pair see the same picture -- [side entry, own
 // four cells outward-in, partner's cell] -- so the code is uniform; the lanes of the second
 // half hold their weights mirrored along K to match.
+// An iteration is 116 vector instructions, 103 of them multiply-adds, eight reads (the thread's own row is in its
+// registers) and a write.  It was 138, 18 reads and a write, with the end entries in every iteration and the sixth values by
+// moves; per step, four inner iterations: 64^3, batch 32, 66.0 -> 62.6 us (eight: 93.3 -> 85.8); 128^3, batch 8, 151.5 -> 133.5; in
+// pairs, 32^3, batch 64, 24.0 -> 21.6.  At 64^3 an iteration is 6 us, which is what its instructions take at four clocks each;
+// the rest of a step, 40 us, is the fetch of the planes and the tensors, 20 us at the rate of a copy.
 struct SplitWin {
     static constexpr int S = 10, RS = 8, PS = S * RS;  // centre rows and planes (floats)
     static constexpr int CEN = S * PS;
@@ -293,9 +299,21 @@ struct SplitWin {
     static constexpr int COPY = CEN + 2 * SS;          // floats per window copy
 };
 
-// value of `v` in the lane that owns the other half of the row (lanes 2m and 2m+1 swap)
-__device__ __forceinline__ float partner_lane(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+// u += the taps of one row but for its end entry: q holds the thread's four cells, the sixth value is a DPP operand of
+// its multiply-add (the compiler makes a move of it, one of seventeen instructions here).  A DPP operand must not be a
+// vector ALU result of the two instructions before: two products that take none stand in front.
+__device__ __forceinline__ void row_taps(const float (&w0)[4], const float (&w1)[4], const float (&w2)[4],
+                                         const float (&q)[4], float (&u)[4]) {
+#pragma unroll
+    for (int r = 1; r < 4; ++r) u[r] = fmaf(w0[r], q[r - 1], u[r]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = fmaf(w1[r], q[r], u[r]);
+    u[0] = fmaf(w2[0], q[1], u[0]);
+    asm("v_fmac_f32 %0, %3, %6\n\t"
+        "v_fmac_f32 %1, %4, %7\n\t"
+        "v_fmac_f32_dpp %2, %7, %5 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+        : "+v"(u[1]), "+v"(u[2]), "+v"(u[3])
+        : "v"(w2[1]), "v"(w2[2]), "v"(w2[3]), "v"(q[2]), "v"(q[3]));
 }
 
 // The statistics of this workgroup's samples from the pairs of the step before, beside the fetch of its weights.
@@ -498,11 +516,10 @@ void step_fwd_split(
                     part[2] += halo_row ? 0.f : s1;
                     part[3] += halo_row ? 0.f : s2;
                 }
-                for (int copy = 0; copy < copies; ++copy) {
+                for (int copy = 0; copy < copies; ++copy)
                     *reinterpret_cast<float4 *>(to + copy * SW::COPY + cen_at[e]) =
                         make_float4(c[0], c[1], c[2], c[3]);
-                    to[copy * SW::COPY + side_at[e]] = end;
-                }
+                to[side_at[e]] = end;  // read once, from the first copy
             }
     };
     if (ln_in) {  // gamma and beta of the window, once per workgroup
@@ -568,6 +585,9 @@ void step_fwd_split(
             const float4 b4 = *reinterpret_cast<const float4 *>(sums_at_commit + 4);
             halo1 = a4.x + b4.x; halo2 = a4.y + b4.y; own1 = a4.z + b4.z; own2 = a4.w + b4.w;
         }
+        float first = NORM ? 0.f : bv[0];  // what the end entries add: the same for every iteration
+#pragma unroll
+        for (int ab = 0; ab < 9; ++ab) first = fmaf(w[ab * 3][0], lds[side00 + ab / 3 * SW::SP + ab % 3], first);
         for (int it = 0; it < inner; ++it) {
             const float *from = lds + (it & 1) * SW::COPY;
             float u[4];
@@ -583,22 +603,20 @@ void step_fwd_split(
                 ninv = 1.f / (sqrtf(var) + norm_eps);
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) u[r] = NORM ? 0.f : bv[r];
+            for (int r = 0; r < 4; ++r) u[r] = r == 0 ? first : NORM ? 0.f : bv[r];
 #pragma unroll
             for (int a = 0; a < 3; ++a)
 #pragma unroll
                 for (int b = 0; b < 3; ++b) {
-                    const float4 q =
-                        *reinterpret_cast<const float4 *>(from + cen00 + a * SW::PS + b * SW::RS);
-                    float v[6];
-                    v[0] = from[side00 + a * SW::SP + b];
-                    v[1] = q.x; v[2] = q.y; v[3] = q.z; v[4] = q.w;
-                    v[5] = partner_lane(q.w);
+                    float q[4];
+                    if (a == 1 && b == 1) {
 #pragma unroll
-                    for (int cc = 0; cc < 3; ++cc)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            u[r] = fmaf(w[a * 9 + b * 3 + cc][r], v[r + cc], u[r]);
+                        for (int r = 0; r < 4; ++r) q[r] = cur[r];
+                    } else {
+                        load_cells<4>(from + cen00 + a * SW::PS + b * SW::RS, q);
+                    }
+                    const int t = a * 9 + b * 3;
+                    row_taps(w[t], w[t + 1], w[t + 2], q, u);
                 }
             if (NORM) {
 #pragma unroll
@@ -664,8 +682,7 @@ void step_fwd_split(
 // ---- forward, 8^3 blocks, the chain's variant: two batch elements per pass -------------------
 // step_fwd_split<ACT, LN = true> with every thread advancing TWO batch elements side by side:
 // the same 108 weights in registers feed both, the two elements' dependent FMA chains and LDS
-// round trips interleave (neither the LDS nor the vector ALU is saturated by one element per
-// wave: what limits step_fwd_split is latency), a barrier serves two elements, and with fewer,
+// round trips interleave (what limits step_fwd_split beside the vector ALU is latency), a barrier serves two elements, and with fewer,
 // larger workgroups the 29 parameter planes of a block are fetched twice per launch instead of
 // three times (64^3 grid, batch 32).  Two waves per SIMD instead of three: the second element's
 // state and prefetch need the registers.
@@ -755,11 +772,10 @@ void step_fwd_pair(
                 if (!(fx.ok[e] && fx.edge_ok[e])) end = 0.f;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) c[r] = fx.ok[e] ? c[r] : 0.f;
-                for (int copy = 0; copy < copies; ++copy) {
+                for (int copy = 0; copy < copies; ++copy)
                     *reinterpret_cast<float4 *>(to + copy * SW::COPY + cen_at[e]) =
                         make_float4(c[0], c[1], c[2], c[3]);
-                    to[copy * SW::COPY + side_at[e]] = end;
-                }
+                to[side_at[e]] = end;  // read once, from the first copy
             }
     };
     typename FX::Buf pre[E];
@@ -814,30 +830,35 @@ void step_fwd_pair(
             const float4 q = *reinterpret_cast<const float4 *>(lds + e * 2 * SW::COPY + own);
             cur[e][0] = q.x; cur[e][1] = q.y; cur[e][2] = q.z; cur[e][3] = q.w;
         }
+        float first[E];  // bias and what the end entries add
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            first[e] = bv[0];
+#pragma unroll
+            for (int ab = 0; ab < 9; ++ab)
+                first[e] = fmaf(w[ab * 3][0], lds[e * 2 * SW::COPY + side00 + ab / 3 * SW::SP + ab % 3], first[e]);
+        }
         for (int it = 0; it < inner; ++it) {
             float u[E][4];
 #pragma unroll
             for (int e = 0; e < E; ++e)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) u[e][r] = bv[r];
+                for (int r = 0; r < 4; ++r) u[e][r] = r == 0 ? first[e] : bv[r];
 #pragma unroll
             for (int a = 0; a < 3; ++a)
 #pragma unroll
                 for (int b = 0; b < 3; ++b) {
 #pragma unroll
                     for (int e = 0; e < E; ++e) {
-                        const float *from = lds + (e * 2 + (it & 1)) * SW::COPY;
-                        const float4 q =
-                            *reinterpret_cast<const float4 *>(from + cen00 + a * SW::PS + b * SW::RS);
-                        float v[6];
-                        v[0] = from[side00 + a * SW::SP + b];
-                        v[1] = q.x; v[2] = q.y; v[3] = q.z; v[4] = q.w;
-                        v[5] = partner_lane(q.w);
+                        float q[4];
+                        if (a == 1 && b == 1) {
 #pragma unroll
-                        for (int cc = 0; cc < 3; ++cc)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r)
-                                u[e][r] = fmaf(w[a * 9 + b * 3 + cc][r], v[r + cc], u[e][r]);
+                            for (int r = 0; r < 4; ++r) q[r] = cur[e][r];
+                        } else {
+                            load_cells<4>(lds + (e * 2 + (it & 1)) * SW::COPY + cen00 + a * SW::PS + b * SW::RS, q);
+                        }
+                        const int t = a * 9 + b * 3;
+                        row_taps(w[t], w[t + 1], w[t + 2], q, u[e]);
                     }
                 }
 #pragma unroll
@@ -1870,17 +1891,23 @@ template <int ACT, bool MERGE> int launch_fwd_pair(const StepArgs &a, hipStream_
     if (p.nblk >= kTwoBlocksFewestInPairs && two_blocks(a, p, resident)) return launch(step_fwd_pair<ACT, MERGE, 2>, 2);
     return launch(kern, 1);
 }
-// The chain's forward on SMALL grids (fewer blocks than a sixth of the workgroups the chip
-// holds, so that a workgroup of step_fwd_split gets four batch elements or fewer for one fetch
-// of its 29 parameter planes): two elements per pass.  Measured with 3 waves per SIMD for
-// step_fwd_split: 32^3 grid, batch 64: 0.279 -> 0.238 ms per 8-step chain; on larger grids the
-// lower occupancy of the pair kernel costs more than it brings (64^3 / batch 32: 66 -> 69 us
-// per step, 128^3 / batch 8: 2.61 -> 3.00 ms per 16-step chain).
+// Where the chain's forward takes two elements per pass.  On SMALL grids (fewer blocks than a sixth of the workgroups the
+// chip holds), because a workgroup of step_fwd_split gets four elements or fewer there for one fetch of its 29 parameter
+// planes: 32^3, batch 64, four inner iterations, 25.0 -> 21.6 us per step.  And where its four workgroups to a CU are a
+// single full round, no CU walks more elements than with the six of step_fwd_split, and the walk is short enough that the
+// fetch counts: 32^3, batch 256, 55.7 -> 53.3; 40^3, batch 64, eight, 51.9 -> 47.2; 64^3, batch 16, 39.2 -> 36.8, batch 32, 62.6 ->
+// 60.9, batch 64, eight, 154.5 -> 148.7; 80^3, batch 32, 113.2 -> 104.7.  With fewer waves than that the third wave per SIMD
+// is worth more (56^3, batch 64, 84.8 against 93.3; 64 x 64 x 96, batch 48, 114.8 and 130.3), with several rounds too (96^3, batch 16,
+// 105 and 114; 128^3, batch 8, 134 and 144), and on long walks neither is ahead (64^3, batch 128, 193 and 195).
 bool walks_pairs(const StepArgs &a) {
     if (a.block_size != 8 || !a.ln.gamma || a.ln.residual || a.B < 2 || a.inner < 1) return false;
-    const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8);
-    const int chunks = 6 * device_cus() / nblk;  // what step_fwd_split's plan would use
-    return chunks >= 1 && (a.B + chunks - 1) / chunks <= 4;
+    const int nblk = (a.M / 8) * (a.N / 8) * (a.K / 8), cus = device_cus();
+    if (nblk > 6 * cus) return false;
+    const Plan ones = make_plan(a, 1, 6 * cus, false), twos = make_plan(a, 2, 4 * cus, false);
+    if (ones.chunk_len <= 4) return true;
+    const auto busiest_cu = [&](const Plan &p) { return (long)(p.nblk * p.nchunk + cus - 1) / cus * p.chunk_len; };
+    const int groups = twos.nblk * twos.nchunk;
+    return groups <= 4 * cus && 8 * groups >= 7 * 4 * cus && twos.chunk_len <= 32 && busiest_cu(twos) <= busiest_cu(ones);
 }
 
 // Small grids: one cell per thread instead of two (backward) or one or two instead of four (forward), a block by eight

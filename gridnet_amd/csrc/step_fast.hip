@@ -73,10 +73,10 @@ void step_fwd_fast(
     const float *__restrict__ scale, const float *__restrict__ x, float *__restrict__ y, int B, int M,
     int N, int K, int inner, int nblk, int nchunk, int chunk_len, LnFold ln, float norm_eps) {
     using TL = Tile<BS, CPT>;
-    constexpr int GROUPS = TL::TPS / 16;  // 16-lane groups of a slot
+    constexpr int GROUP = TL::TPS >= 64 ? 64 : 16, GROUPS = TL::TPS / GROUP;  // lanes that sum up together: waves, rows in smaller slots
     constexpr int NORM_FLOATS = NORM ? NSLOT * GROUPS * (4 + 2 * 2) : 0;
     // per slot two copies of the window; then, for the folded LayerNorm, the packed gamma/beta;
-    // then, for NORM, per slot and 16-lane group the sums taken at commit and, twice (alternating
+    // then, for NORM, per slot and group of lanes the sums taken at commit and, twice (alternating
     // between inner iterations), the sums of the owned cells
     __shared__ __attribute__((aligned(16))) float
         lds[NSLOT * 2 * TL::WIN + (LN ? Fetch<TL>::AFFINE : 0) + NORM_FLOATS];
@@ -122,7 +122,7 @@ void step_fwd_fast(
     float wsum[CPT], zero[CPT];
     float *sums_at_commit = lds + NSLOT * 2 * TL::WIN + (LN ? Fetch<TL>::AFFINE : 0) + pl.slot * GROUPS * 8;
     float *own_sums = sums_at_commit + GROUPS * 4;  // [2][GROUPS][2]
-    const int group = pl.lane / 16;
+    const int group = pl.lane / GROUP;
     constexpr float inv_count = 1.f / (TL::S * TL::S * TL::S);
     if (NORM) {
 #pragma unroll
@@ -159,11 +159,8 @@ void step_fwd_fast(
                 float part[4];
                 shift = pre_shift;
                 fx.commit_sums(win, pre, shift, part);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) part[q] = row16_sum(part[q]);
-                if ((pl.lane & 15) == 0)
-                    *reinterpret_cast<float4 *>(sums_at_commit + group * 4) =
-                        make_float4(part[0], part[1], part[2], part[3]);
+                leave_sums<GROUP>(sums_at_commit + group * 4, pl.lane, part[0], part[1]);
+                leave_sums<GROUP>(sums_at_commit + group * 4 + 2, pl.lane, part[2], part[3]);
             } else fx.commit(win, pre);
         }
         slot_barrier<TL::TPS>();
@@ -223,13 +220,8 @@ void step_fwd_fast(
                     s1 += cur[c];
                     s2 = fmaf(cur[c], cur[c], s2);
                 }
-                if (NORM && it + 1 < inner) {  // the owned cells' part of the next statistics
-                    s1 = row16_sum(s1);
-                    s2 = row16_sum(s2);
-                    if ((pl.lane & 15) == 0)
-                        *reinterpret_cast<float2 *>(own_sums + (((it + 1) & 1) * GROUPS + group) * 2) =
-                            make_float2(s1, s2);
-                }
+                if (NORM && it + 1 < inner)  // the owned cells' part of the next statistics
+                    leave_sums<GROUP>(own_sums + (((it + 1) & 1) * GROUPS + group) * 2, pl.lane, s1, s2);
             }
             slot_barrier<TL::TPS>();
         }
@@ -562,11 +554,8 @@ void step_fwd_split(
         commit(lds, 2, pre, ln_in, pre_mean, pre_rstd, RES ? back + ((s - s0) & 1) * SW::CEN : nullptr);
         if (NORM) {
             shift = pre_shift;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) part[q] = slot_wave_sum<64>(part[q]);
-            if ((threadIdx.x & 63) == 0)
-                *reinterpret_cast<float4 *>(sums_at_commit + wave * 4) =
-                    make_float4(part[0], part[1], part[2], part[3]);
+            leave_sums<64>(sums_at_commit + wave * 4, threadIdx.x, part[0], part[1]);
+            leave_sums<64>(sums_at_commit + wave * 4 + 2, threadIdx.x, part[2], part[3]);
         }
         lds_barrier();
         if (done_s >= 0) {
@@ -626,13 +615,9 @@ void step_fwd_split(
             for (int r = 0; r < 4; ++r) cur[r] = fmaf(rv[r], Act<ACT, float>::f(u[r]), cur[r]);
             *reinterpret_cast<float4 *>(lds + ((it + 1) & 1) * SW::COPY + own) =
                 make_float4(cur[0], cur[1], cur[2], cur[3]);
-            if (NORM && it + 1 < inner) {  // the owned cells' part of the next statistics
-                const float s1 = slot_wave_sum<64>((cur[0] + cur[1]) + (cur[2] + cur[3]));
-                const float s2 = slot_wave_sum<64>(
-                    fmaf(cur[0], cur[0], fmaf(cur[1], cur[1], fmaf(cur[2], cur[2], cur[3] * cur[3]))));
-                if ((threadIdx.x & 63) == 0)
-                    *reinterpret_cast<float2 *>(own_sums + ((it + 1) & 1) * 4 + wave * 2) = make_float2(s1, s2);
-            }
+            if (NORM && it + 1 < inner)  // the owned cells' part of the next statistics
+                leave_sums<64>(own_sums + ((it + 1) & 1) * 4 + wave * 2, threadIdx.x, (cur[0] + cur[1]) + (cur[2] + cur[3]),
+                               fmaf(cur[0], cur[0], fmaf(cur[1], cur[1], fmaf(cur[2], cur[2], cur[3] * cur[3]))));
             lds_barrier();
         }
         if (RES) {  // x + (result - n): the difference x - n was left at commit, in register order
@@ -1011,7 +996,8 @@ void step_bwd_fast(
     float *ncommit = nstat + 4 * inner, *nown = ncommit + 4 * NW, *nrev = nown + 4 * NW;
     float *wsum_at = nrev + 4 * NW + pl.lane * CPT;  // this thread's: sum of a cell's weights
     float *d2acc_at = wsum_at + CPT * TL::TPS;        // D2 summed over the batch elements
-    const int wave_in_slot = TL::TPS >= 64 ? pl.lane / 64 : 0;
+    constexpr int GROUP = TL::TPS >= 64 ? 64 : 32;  // lanes that sum up together
+    const int wave_in_slot = pl.lane / GROUP;
     constexpr float inv_count = 1.f / TL::NWIN;
 
     // nw[t][c] belongs to the weight of the neighbour at c + off_t where that lies in this block,
@@ -1177,11 +1163,8 @@ void step_bwd_fast(
             float part[4];
             shift = pre_shift;
             fx.commit_sums(win, pre, shift, part);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) part[q] = sum_for_one<TL::TPS>(part[q]);
-            if (has_sum<TL::TPS>(pl.lane))
-                *reinterpret_cast<float4 *>(ncommit + wave_in_slot * 4) =
-                    make_float4(part[0], part[1], part[2], part[3]);
+            leave_sums<GROUP>(ncommit + wave_in_slot * 4, pl.lane, part[0], part[1]);
+            leave_sums<GROUP>(ncommit + wave_in_slot * 4 + 2, pl.lane, part[2], part[3]);
         } else fx.commit(win, pre);
     };
     if (ln_in) lds_barrier();  // gamma and beta windows
@@ -1275,13 +1258,8 @@ void step_bwd_fast(
                         s1 += cur[c];
                         s2 = fmaf(cur[c], cur[c], s2);
                     }
-                    if (NORM) {  // the owned cells' part of the next iteration's statistics
-                        s1 = sum_for_one<TL::TPS>(s1);
-                        s2 = sum_for_one<TL::TPS>(s2);
-                        if (has_sum<TL::TPS>(pl.lane))
-                            *reinterpret_cast<float2 *>(nown + (((it + 1) & 1) * NW + wave_in_slot) * 2) =
-                                make_float2(s1, s2);
-                    }
+                    if (NORM)  // the owned cells' part of the next iteration's statistics
+                        leave_sums<GROUP>(nown + (((it + 1) & 1) * NW + wave_in_slot) * 2, pl.lane, s1, s2);
                 } else {  // x_inner itself is never needed: that copy becomes the halo window
 #pragma unroll
                     for (int c = 0; c < CPT; ++c) win[((it + 1) & 1) * TL::WIN + pl.own + c] = 0.f;
@@ -1334,10 +1312,12 @@ void step_bwd_fast(
                     dwin[(it & 1) * TL::WIN + pl.own + c] = delta;
                 }
                 if (NORM) {
-                    pa = NW > 1 ? sum_for_one<TL::TPS>(pa) : slot_wave_sum<TL::TPS>(pa);
-                    pz = NW > 1 ? sum_for_one<TL::TPS>(pz) : slot_wave_sum<TL::TPS>(pz);
-                    if (NW > 1 && has_sum<TL::TPS>(pl.lane))
-                        *reinterpret_cast<float2 *>(nrev + ((it & 1) * NW + wave_in_slot) * 2) = make_float2(pa, pz);
+                    if (NW > 1) {
+                        leave_sums<GROUP>(nrev + ((it & 1) * NW + wave_in_slot) * 2, pl.lane, pa, pz);
+                    } else {
+                        pa = slot_wave_sum<TL::TPS>(pa);
+                        pz = slot_wave_sum<TL::TPS>(pz);
+                    }
                 }
             }
             if (it == 0) {

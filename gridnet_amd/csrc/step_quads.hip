@@ -47,21 +47,25 @@ constexpr int kGroup = 4;           // samples to a wave
 constexpr int kWaves = 4;           // to a workgroup: neighbouring blocks of a K-row, the same samples
 constexpr int kThreads = kWaves * kWave;
 constexpr int kWinRows = 36;        // rows of a window, 6 x 6
-// Floats of a wave's LDS.  Rows by sample, [36][4 samples][4 cells]; the four floats between planes spread the
-// 4-byte writes by cell over all banks.  The entries beyond the rows' ends, [36][2][4 samples].
-constexpr int kPlane = 6 * 16 + 4, kRows = 6 * kPlane, kSides = kWinRows * 8, kWindow = kRows + kSides;
+// Floats of a wave's LDS.  Rows by sample, [36][4 samples][4 cells]; the floats between planes spread the backward's
+// 4-byte writes by cell, or the forward's 16-byte writes, over all banks.  The entries beyond the rows' ends, [36][2][4 samples].
+constexpr int kPlaneBackward = 6 * 16 + 4, kPlaneForward = 6 * 16 + 16, kSides = kWinRows * 8;
+constexpr int rows_floats(int plane) { return 6 * plane; }
+constexpr int window_floats(int plane) { return rows_floats(plane) + kSides; }
+// the four waves' windows: 16 floats past a multiple of 64, so that the pieces of a row, one for each wave, go to different banks
+constexpr int kForwardFloats = window_floats(kPlaneForward) + 16;
 // gamma and beta of the workgroup's rows and of the entries beyond their ends
 constexpr int kAffineRows = kWinRows * kWaves * 8, kAffine = kAffineRows + kWinRows * 4;
 // Deltas by cell, [row][4 cells][4 samples], zeros around the block: row (i, j) is number 5 (i + 1) + j + 1, the row behind
 // a plane's last is the one in front of the next plane's first.
 constexpr int kDeltaPlane = 5 * 16, kDeltas = 6 * kDeltaPlane + 16;
-constexpr int kExchange = 27 * 64;  // the weights, once at set-up
+constexpr int kExchange = 27 * 64 + 16;  // the weights, once at set-up
 // history: u of all iterations but the last, x of those between (the first and the last stay in registers)
 __host__ __device__ constexpr int history_floats(int inner) {
     return 256 * ((inner > 1 ? inner - 1 : 0) + (inner > 2 ? inner - 2 : 0));
 }
 __host__ __device__ constexpr int backward_floats(int inner) {
-    const int run = kWindow + kDeltas + history_floats(inner);
+    const int run = window_floats(kPlaneBackward) + kDeltas + 40 + history_floats(inner);  // 16 past a multiple of 64, too
     return run > kExchange ? run : kExchange;
 }
 
@@ -119,23 +123,28 @@ struct QuadWork {
     }
 };
 
-// Where a lane sits in its wave's block.
-struct QuadPlace {
-    int lane, row, k;        // lane = 4 * row + k; k is the cell or the sample
+// Where a lane sits in its wave's block.  The LDS serves a 16-byte read sixteen lanes at a time: lanes 0-3, 12-15, 20-23
+// and 24-27 together, then the others of the lower half wave, and so on.  Those are given the four rows of a plane, which lie side by
+// side.  With row = lane / 4 they came from two planes, and every read took eight cycles instead of four (counted): the LDS was
+// busy for 70 % of the forward and 61 % of the backward, four tenths of it with conflicts.  Now 48 and 40 %; a step of 64^3, batch
+// 128, eight iterations, forward 324 -> 312 us by events, backward 1 % less: the vector ALU and its clock bind it, not the LDS.
+template <int PLANE> struct QuadPlace {
+    int lane, row, k;        // k is the cell or the sample
     int i, j;                // of the row in the block
     int own;                 // cell (row, k) in the grid
     int rows00, cell;        // LDS: window row (i, j) by sample k; cell (row, k) of the first sample
     int sides00;             // LDS: the end of window row (i, j) on the side of cell k, first sample
     __device__ __forceinline__ QuadPlace(const QuadWork &work, int N, int K) {
         lane = threadIdx.x & (kWave - 1);
-        row = lane >> 2;
+        const int quad = lane >> 2;
         k = lane & 3;
-        i = row >> 2;
-        j = row & 3;
+        i = quad >> 3 << 1 | (__popc(quad & 7) & 1);
+        j = quad >> 1 & 3;
+        row = 4 * i + j;
         own = ((work.p0 + i) * N + work.q0 + j) * K + work.r0 + 4 * min(work.wave, work.blocks - 1) + k;
-        rows00 = i * kPlane + j * 16 + 4 * k;
-        cell = (i + 1) * kPlane + (j + 1) * 16 + k;
-        sides00 = kRows + (i * 6 + j) * 8 + (k >> 1) * 4;
+        rows00 = i * PLANE + j * 16 + 4 * k;
+        cell = (i + 1) * PLANE + (j + 1) * 16 + k;
+        sides00 = rows_floats(PLANE) + (i * 6 + j) * 8 + (k >> 1) * 4;
     }
     __device__ __forceinline__ bool has(int a, int c) const {  // the block has row (i + a - 1, j + c - 1)
         return (unsigned)(i + a - 1) < 4u && (unsigned)(j + c - 1) < 4u;
@@ -195,11 +204,11 @@ struct QuadFetch {
     // Into the windows, `stride` floats apart: a row's four cells to their block, its first and last to the blocks beside it.
     // LN: normalised on the way, with the statistics of the thread's sample.  The LDS places are worked out here, from a thread
     // number that the compiler cannot see through: it would keep them in registers that the loops have no room for.
-    // An end goes to [row][side][sample], or for BY_ROW, the forward, [row][sample][side].
-    template <bool LN, bool BY_ROW = false>
+    // An end goes to [row][side][sample], in the forward to [row][sample][side].
+    template <bool LN, int PLANE>
     __device__ __forceinline__ void commit(float *windows, int stride, const Buf &v, const float *affine, float mean,
                                            float rstd) const {
-        constexpr int SIDE = BY_ROW ? 1 : 4, SAMPLE = BY_ROW ? 2 : 1;
+        constexpr int SIDE = PLANE == kPlaneForward ? 1 : 4, SAMPLE = PLANE == kPlaneForward ? 2 : 1;
         const int t = opaque(threadIdx.x), m = t & 3, s = t >> 2 & 3;
         float *win = windows + m * stride;
 #pragma unroll
@@ -216,8 +225,8 @@ struct QuadFetch {
                 }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) val[q] = where & 1 ? val[q] : 0.f;
-                *reinterpret_cast<quad *>(win + r * 16 + r / 6 * 4 + s * 4) = val;
-                float *sides = win + kRows + r * 8 + s * SAMPLE;
+                *reinterpret_cast<quad *>(win + r * 16 + r / 6 * (PLANE - 96) + s * 4) = val;
+                float *sides = win + rows_floats(PLANE) + r * 8 + s * SAMPLE;
                 if (m > 0 && m < blocks) sides[SIDE - stride] = val[0];
                 if (m < kWaves - 1) sides[stride] = val[3];
             }
@@ -233,12 +242,11 @@ struct QuadFetch {
                     val = fmaf((val - mean) * rstd, gb.x, gb.y);
                 }
                 const int r = e * 32 + (t >> 4) * 2 + (t >> 1 & 1);
-                windows[(side ? blocks - 1 : 0) * stride + kRows + r * 8 + side * SIDE + s * SAMPLE] = where & 1 ? val : 0.f;
+                windows[(side ? blocks - 1 : 0) * stride + rows_floats(PLANE) + r * 8 + side * SIDE + s * SAMPLE] = where & 1 ? val : 0.f;
             }
         }
     }
 };
-static_assert(kPlane == 6 * 16 + 4, "commit places row r at 16 r + 4 (r / 6)");
 
 // A cell's 27 weights as the bands of its row: W[n][h] what entry h of neighbour row n is multiplied with (zero where it
 // is no neighbour), S[n] the same for the entry beyond the row's end that the cell reads (cells 0 and 3).
@@ -259,7 +267,7 @@ struct Bands {
 };
 
 // bias and what the entries beyond the rows' ends add, by cell: the same for every iteration
-__device__ __forceinline__ quad side_sums(const float *win, const QuadPlace &pl, const Bands &w, float bias) {
+__device__ __forceinline__ quad side_sums(const float *win, const QuadPlace<kPlaneBackward> &pl, const Bands &w, float bias) {
     quad u = {bias, bias, bias, bias};
 #pragma unroll
     for (int n = 0; n < 9; ++n) {
@@ -273,9 +281,9 @@ __device__ __forceinline__ quad side_sums(const float *win, const QuadPlace &pl,
 
 // u += the 27 taps but for the rows' ends, by cell, DEPTH rows requested ahead of the arithmetic.
 template <int DEPTH>
-__device__ __forceinline__ quad band_sums(const float *win, const QuadPlace &pl, const float (&w)[9][4], quad u) {
+__device__ __forceinline__ quad band_sums(const float *win, const QuadPlace<kPlaneBackward> &pl, const float (&w)[9][4], quad u) {
     quad v[DEPTH];
-    const auto row = [&](int n) { return load_quad(win + pl.rows00 + n / 3 * kPlane + n % 3 * 16); };
+    const auto row = [&](int n) { return load_quad(win + pl.rows00 + n / 3 * kPlaneBackward + n % 3 * 16); };
 #pragma unroll
     for (int n = 0; n < DEPTH; ++n) v[n] = row(n);
 #pragma unroll
@@ -295,14 +303,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
 void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias, const float *__restrict__ scale,
                const float *__restrict__ x, float *__restrict__ y, int B, int M, int N, int K, int inner, int nblk,
                int nchunk, int chunk_len, LnFold ln) {
+    constexpr int PLANE = kPlaneForward, WINDOW = kForwardFloats;
     constexpr int SIDE_WEIGHTS = 16 * 18;  // [row][neighbour row][side]
-    __shared__ __attribute__((aligned(16))) float lds[kWaves * (kWindow + SIDE_WEIGHTS) + kAffine];
+    __shared__ __attribute__((aligned(16))) float lds[kWaves * (WINDOW + SIDE_WEIGHTS) + kAffine];
     QuadWork work;
     if (!work.find(ln.walk_reverse ? reversed_on_its_xcd(blockIdx.x, gridDim.x) : blockIdx.x, M, N, K, nchunk, chunk_len, B))
         return;
-    const QuadPlace pl(work, N, K);
+    const QuadPlace<PLANE> pl(work, N, K);
     const QuadFetch fx(work, M, N, K);
-    float *win = lds + work.wave * kWindow, *affine = lds + kWaves * kWindow;
+    float *win = lds + work.wave * WINDOW, *affine = lds + kWaves * WINDOW;
     float *ends = affine + kAffine + work.wave * SIDE_WEIGHTS + pl.row * 18;
     const long cells = (long)M * N * K;
     const bool ln_in = ln.x_stats != nullptr;
@@ -345,20 +354,20 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
     };
     for (int s = work.first; s < work.end; s += kGroup) {
         lds_barrier();  // gamma and beta; the windows are free
-        if (ln_in) fx.template commit<true, true>(lds, kWindow, pre, affine, mean, rstd);
-        else fx.template commit<false, true>(lds, kWindow, pre, affine, mean, rstd);
+        if (ln_in) fx.template commit<true, PLANE>(lds, WINDOW, pre, affine, mean, rstd);
+        else fx.template commit<false, PLANE>(lds, WINDOW, pre, affine, mean, rstd);
         if (RES) raw = raw_next;
         lds_barrier();
         if (work.active) store_group();
         if (s + kGroup < work.end) fetch_group(s + kGroup);
         if (!work.active) continue;
-        float *own = win + pl.rows00 + kPlane + 16;
+        float *own = win + pl.rows00 + PLANE + 16;
         cur = load_quad(own);
         const quad base = cur;
         quad u0 = bv;
 #pragma unroll
         for (int n = 0; n < 9; ++n) {  // the entries beyond the row's ends: the same for every iteration
-            const float2 v = *reinterpret_cast<const float2 *>(win + kRows + (pl.i * 6 + pl.j) * 8 + 2 * pl.k + (n / 3 * 6 + n % 3) * 8);
+            const float2 v = *reinterpret_cast<const float2 *>(win + rows_floats(PLANE) + (pl.i * 6 + pl.j) * 8 + 2 * pl.k + (n / 3 * 6 + n % 3) * 8);
             const float2 e = *reinterpret_cast<const float2 *>(ends + 2 * n);
             u0[0] = fmaf(e.x, v.x, u0[0]);
             u0[3] = fmaf(e.y, v.y, u0[3]);
@@ -366,7 +375,7 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
         for (int it = 0; it < inner; ++it) {
             constexpr int DEPTH = 5;
             quad u = u0, v[DEPTH];
-            const auto row = [&](int n) { return load_quad(win + pl.rows00 + n / 3 * kPlane + n % 3 * 16); };
+            const auto row = [&](int n) { return load_quad(win + pl.rows00 + n / 3 * PLANE + n % 3 * 16); };
 #pragma unroll
             for (int n = 0; n < DEPTH; ++n) v[n] = row(n);
 #pragma unroll
@@ -438,11 +447,12 @@ void quads_bwd(const float *__restrict__ weight, const float *__restrict__ bias,
         ln.dgamma += off;
         ln.dbeta += off;
     }
-    const QuadPlace pl(work, N, K);
+    constexpr int PLANE = kPlaneBackward;
+    const QuadPlace<PLANE> pl(work, N, K);
     const QuadFetch fx(work, M, N, K);
     const int stride = backward_floats(inner);
     float *affine = lds, *windows = lds + kAffine, *win = windows + work.wave * stride;
-    float *deltas = win + kWindow, *hist_u = deltas + kDeltas, *hist_x = hist_u + 256 * (inner - 1);
+    float *deltas = win + window_floats(PLANE), *hist_u = deltas + kDeltas, *hist_x = hist_u + 256 * (inner - 1);
     const long cells = (long)M * N * K;
     const bool ln_in = ln.x_stats != nullptr;
     const bool through_ln = !RES || ln.y_raw != nullptr;
@@ -452,7 +462,7 @@ void quads_bwd(const float *__restrict__ weight, const float *__restrict__ bias,
     float v[9][4];
     {   // the neighbours' weights, exchanged through LDS
 #pragma unroll
-        for (int t = 0; t < 27; ++t) win[t * kWave + pl.lane] = weight[t * cells + pl.own];
+        for (int t = 0; t < 27; ++t) win[t * kWave + pl.row * 4 + pl.k] = weight[t * cells + pl.own];
         wave_order();
 #pragma unroll
         for (int n = 0; n < 9; ++n)
@@ -538,8 +548,8 @@ void quads_bwd(const float *__restrict__ weight, const float *__restrict__ bias,
             g[q] = v;
         });
         if (RES) gin = g;
-        if (ln_in) fx.template commit<true>(windows, stride, pre, affine, x_mean, x_rstd);
-        else fx.template commit<false>(windows, stride, pre, affine, x_mean, x_rstd);
+        if (ln_in) fx.template commit<true, PLANE>(windows, stride, pre, affine, x_mean, x_rstd);
+        else fx.template commit<false, PLANE>(windows, stride, pre, affine, x_mean, x_rstd);
     };
     fetch_group(work.first);
     // What leaves is stored one group late, behind the wait for the windows: loads and stores share one in-order counter.
@@ -599,7 +609,7 @@ void quads_bwd(const float *__restrict__ weight, const float *__restrict__ bias,
             // a sum of its own, added to g once: its terms are rounded at their size and not at that of g
             quad sum = {0.f, 0.f, 0.f, 0.f}, by_sample[kDepthPairs], by_cell[kDepthPairs];
             const auto request = [&](int n) {
-                by_sample[n % kDepthPairs] = load_quad(win + pl.rows00 + n / 3 * kPlane + n % 3 * 16);
+                by_sample[n % kDepthPairs] = load_quad(win + pl.rows00 + n / 3 * PLANE + n % 3 * 16);
                 by_cell[n % kDepthPairs] = load_quad(deltas00 + n / 3 * kDeltaPlane + n % 3 * 16);
             };
 #pragma unroll
@@ -623,12 +633,12 @@ void quads_bwd(const float *__restrict__ weight, const float *__restrict__ bias,
         }
         db += (dsum[0] + dsum[1]) + (dsum[2] + dsum[3]);
         // the weights that read the halo: the window without the block
-        *reinterpret_cast<quad *>(win + pl.rows00 + kPlane + 16) = quad{0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<quad *>(win + pl.rows00 + PLANE + 16) = quad{0.f, 0.f, 0.f, 0.f};
         wave_order();
 #pragma unroll
         for (int n = 0; n < 9; ++n) {
             if (n != 4) {
-                const float *row = win + pl.cell + (n / 3 - 1) * kPlane + (n % 3 - 1) * 16;
+                const float *row = win + pl.cell + (n / 3 - 1) * PLANE + (n % 3 - 1) * 16;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) nw[n] = mfma(dsum[q], row[4 * q], nw[n]);
             }

@@ -18,8 +18,8 @@
 // zeros.  They run on the vector ALU's multipliers, not beside them (8 cycles each, to which a multiply-add of another wave
 // adds its own), so an iteration's 108 there and back cost what the 324 multiply-adds they stand for do; what they save is half of
 // the LDS traffic, half of the other instructions and all of the registers that step_bwd_fast spills in its loops.  The same step:
-// 1053 -> 830 us.  What bounds it: the vector ALU, busy three quarters of the time at two waves per SIMD, and a clock of 2.0 to
-// 2.2 GHz under these instructions.
+// 1053 -> 830 us (860 to 950 on other boxes).  What bounds it: the vector ALU, by counters 44 % of the time in matrix and 18 % in
+// other instructions; two waves per SIMD do not fill the waits between dependent matrix instructions; and a clock of 2.0 to 2.2 GHz.
 //
 // A wave's registers come in two layouts there:
 //   by cell:   lane (row, k), one register per sample -- what the matrix instruction leaves when the window is its

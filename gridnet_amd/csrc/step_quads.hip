@@ -26,9 +26,12 @@
 //              first operand; bias, scale and the small gradients are one register each;
 //   by sample: lane (row, sample), one register per cell of the row -- its first operand, read from LDS.
 //
-// Inside a chain only: the zeros of the band multiply values of the same sample, and an infinity or a NaN there spreads
-// to the row's other cells.  The LayerNorm behind every step of a chain spreads it over the whole sample anyway; a step on
-// its own keeps it to the cells that read it.
+// In front of a LayerNorm only: the backward's zeros of the band, and of rows that are not the block's, multiply values of the same
+// sample, and an infinity or a NaN there spreads to cells that do not read it.  A LayerNorm behind the step spreads what the output or
+// its gradient hold of that kind over the whole sample anyway; a step on its own and the last one of the residual loop, which is
+// handed its gradient as it is, keep it within the taps' reach and go to step_bwd_fast.  What is left is a gradient that overflows
+// inside the sweep (or meets an infinite weight whose cell's activation is saturated): the gradients of this step's own parameters then
+// are NaN in more of the block's cells than that; those of all earlier steps are for the whole sample either way.
 
 #include <type_traits>
 
@@ -455,6 +458,8 @@ void quads_bwd(const float *__restrict__ weight, const float *__restrict__ bias,
     float *deltas = win + window_floats(PLANE), *hist_u = deltas + kDeltas, *hist_x = hist_u + 256 * (inner - 1);
     const long cells = (long)M * N * K;
     const bool ln_in = ln.x_stats != nullptr;
+    // always true, and not known to be: the residual form spills 8 registers more where these loads and what is made of them
+    // are not in blocks of their own
     const bool through_ln = !RES || ln.y_raw != nullptr;
 
     Bands w;
@@ -802,6 +807,7 @@ static bool covers(const StepArgs &a) {
 bool step_quads_supports(const StepArgs &a, bool backward) {
     if (!covers(a)) return false;
     if (!backward) return true;
+    if (!a.ln.y_raw) return false;  // no LayerNorm behind the step
     int nchunk, chunk_len;
     return a.inner <= kMostIterations && cross_rows_supports(a) &&
            plan_backward(a, plan_slab_capacity(a.slabs, a.slab_bytes, kStepSlabPlanes * (long)a.M * a.N * a.K), nchunk, chunk_len);

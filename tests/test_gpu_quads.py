@@ -39,3 +39,31 @@ def test_chain_against_the_oracle(shape, batch, inner, quads, residual, activati
     for name, a, e in zip("y dweight dbias dscale dgamma dbeta dx".split(), got, want):
         # an entry of the gradients is a sum over the batch, and its error goes with its terms (2e-7 of the array's rms)
         assert_close(a, e, RTOL, ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)
+
+
+def test_an_infinite_gradient_stays_within_the_taps_reach():
+    """The last step of the residual loop has no LayerNorm behind it that would spread a non-finite gradient over its sample."""
+    from gridnet_amd.runner import BodyRunner
+    from oracle.network import network_forward_backward
+
+    shape, batch, inner, at = (32, 32, 36), 32, 2, (9, 13, 16)  # the first cell of a row of its block
+    print(f"quads, residual {shape} B={batch} inner={inner}, an infinite gradient", flush=True)
+    g = torch.Generator().manual_seed(3)
+    params = [*make_params(shape, seed=11), *((a + 0.2 * torch.randn(shape, generator=g)) for a in (1, 0))]
+    x, gy = (make_acts(batch, shape, seed=s) for s in (12, 13))
+    run = BodyRunner(*(t.to(DEV) for t in params), batch, inner, 1, 4, "tanh", fused=True, outer_residual=True)
+    run.forward(x.to(DEV))
+    bad = gy.clone()
+    bad[5][at] = float("inf")
+    got = [t.clone().cpu() for t in run.backward(bad.to(DEV))]
+    want = network_forward_backward([t.double() for t in params], x.double(), gy.double(), inner_iterations=inner,
+                                    outer_iterations=1, block_size=4, activation="tanh", outer_residual=True)[1:]
+    away = torch.stack(torch.meshgrid(*(torch.arange(n) for n in shape), indexing="ij")).sub(torch.tensor(at).view(3, 1, 1, 1))
+    away = away.abs().amax(0)
+    # an iteration of the reverse sweep carries it one cell further, the first one none; gradients of weights are worked
+    # out where the weight's tap reads from
+    for name, a, e, reach in zip("dweight dbias dscale dgamma dbeta".split(), got, want, (2, 1, 1, 2, 2)):
+        a, e = a[..., away > reach], e[..., away > reach]
+        assert_close(a, e, RTOL, ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)
+    others = [s for s in range(batch) if s != 5]
+    assert_close(got[5][others], want[5][others], what="dx")

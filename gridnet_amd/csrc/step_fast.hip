@@ -933,12 +933,14 @@ template <int BS, int CPT, int NSLOT> size_t bwd_lds_bytes(int inner, bool ln = 
 // iteration i adds to window entry k is (N = (bs+2)^3 entries)
 //   inv_i (dn_i[k] - A_i / N) - (x_i[k] - mean_i) C_i,   A_i = sum_k dn_i[k],
 //   C_i = inv_i^2 / (N std_i) * sum_k dn_i[k] (x_i[k] - mean_i).
-// Both sums run over the whole window, but need no entry of dn: a cell sends its weights times
-// delta_i, so with z_i = sum_t w_t n_i, the pre-activation without its bias,
-//   A_i = sum_c delta_i[c] * (sum of c's weights),   sum_k dn_i[k] (x_i[k] - mean_i) = sum_c delta_i[c] z_i[c] / inv_i,
+// Both sums run over the whole window, but need no entry of dn: a cell sends its weights times delta_i, so with
+// t_i = sum_t w_t (x_i - mean_i), of which the pre-activation is b + inv_i t_i,
+//   A_i = sum_c delta_i[c] * (sum of c's weights),   sum_k dn_i[k] (x_i[k] - mean_i) = sum_c delta_i[c] t_i[c],
 // known as soon as delta_i is: the sums travel with the delta window, behind the same barrier.  (Formed from the gathered dn and
 // the halo's share of them they took a second barrier per reverse iteration and a stencil over the halo per element.)
-// The history holds z_i and not the pre-activation, which would leave z_i the rounding error of the bias.  What the HALO entries receive over
+// The history holds t_i: from the pre-activation it would come with the rounding error of the bias.  The sweep forms the
+// pre-activation of it as the recompute does, in one multiply-add: value and derivative of an activation with a kink are
+// those of one side of it.  What the HALO entries receive over
 // all iterations is, for halo entry h,
 //   sum over (c, t) reading h of w_t[c] D1[c]  -  x_h Q + R,
 //   D1 = sum_i inv_i delta_i,  Q = sum_i C_i,  R = sum_i (mean_i C_i - inv_i A_i / N):
@@ -1220,7 +1222,7 @@ void step_bwd_fast(
         // ---- forward recompute, remembering x_i and u_i of the owned cells ----
         for (int it = 0; it < inner; ++it) {
             if (active) {
-                float u[CPT], z[CPT];
+                float u[CPT], t[CPT];
                 if (NORM) {
                     if (it > 0) {
                         own1 = own2 = 0.f;
@@ -1239,16 +1241,15 @@ void step_bwd_fast(
                     load_cells<CPT>(wsum_at, wsum);
 #pragma unroll
                     for (int c = 0; c < CPT; ++c) {
-                        const float t = fmaf(-mean, wsum[c], u[c]);
-                        u[c] = fmaf(inv, t, bv[c]);
-                        z[c] = inv * t;
+                        t[c] = fmaf(-mean, wsum[c], u[c]);
+                        u[c] = fmaf(inv, t[c], bv[c]);
                     }
                 } else {
                     stencil<TL, CPT, kBwdDepth>(win + (it & 1) * TL::WIN, pl.row00, w, bv, u);
                 }
                 float *h = hist + it * (TL::TPS * 2 * CPT);
                 store_cells<CPT>(h, cur);
-                store_cells<CPT>(h + TL::TPS * CPT, NORM ? z : u);
+                store_cells<CPT>(h + TL::TPS * CPT, NORM ? t : u);
                 if (it + 1 < inner) {
                     float s1 = 0.f, s2 = 0.f;
 #pragma unroll
@@ -1270,27 +1271,27 @@ void step_bwd_fast(
 
         // ---- reverse sweep: delta window copy (it & 1) holds delta_it ----
         // NORM: dsum is D1, d2 is D2; x_i of the owned cells as the stencil saw it (xn); the sums of the iteration; Q and R
-        float dsum[CPT], xi[CPT], xn[CPT], d2[CPT], pa = 0.f, pz = 0.f, q_sum = 0.f, r_sum = 0.f;
+        float dsum[CPT], xi[CPT], xn[CPT], d2[CPT], pa = 0.f, pt = 0.f, q_sum = 0.f, r_sum = 0.f;
 #pragma unroll
         for (int c = 0; c < CPT; ++c) dsum[c] = d2[c] = 0.f;
         for (int it = inner - 1; it >= 0; --it) {
             if (active) {
                 const float *h = hist + it * (TL::TPS * 2 * CPT);
-                float u[CPT], z[CPT], wsum[CPT];
+                float u[CPT], t[CPT], wsum[CPT];
                 load_cells<CPT>(h, xi);
                 load_cells<CPT>(h + TL::TPS * CPT, u);
                 if (NORM) {
                     load_cells<CPT>(wsum_at, wsum);
-#pragma unroll
-                    for (int c = 0; c < CPT; ++c) {
-                        z[c] = u[c];
-                        u[c] += bv[c];
-                    }
                     if (it < inner - 1) {
                         const float4 st4 = *reinterpret_cast<const float4 *>(nstat + 4 * it);
                         mean = st4.x; sd = st4.y; inv = st4.z;
                     }
-                    pa = pz = 0.f;
+#pragma unroll
+                    for (int c = 0; c < CPT; ++c) {
+                        t[c] = u[c];
+                        u[c] = fmaf(inv, t[c], bv[c]);
+                    }
+                    pa = pt = 0.f;
                 }
 #pragma unroll
                 for (int c = 0; c < CPT; ++c) {
@@ -1301,7 +1302,7 @@ void step_bwd_fast(
                     db[c] += delta;
                     if (NORM) {
                         pa = fmaf(delta, wsum[c], pa);
-                        pz = fmaf(delta, z[c], pz);
+                        pt = fmaf(delta, t[c], pt);
                         dsum[c] = fmaf(inv, delta, dsum[c]);
                         d2[c] = fmaf(mean * inv, delta, d2[c]);
                         xn[c] = (xi[c] - mean) * inv;
@@ -1313,10 +1314,10 @@ void step_bwd_fast(
                 }
                 if (NORM) {
                     if (NW > 1) {
-                        leave_sums<GROUP>(nrev + ((it & 1) * NW + wave_in_slot) * 2, pl.lane, pa, pz);
+                        leave_sums<GROUP>(nrev + ((it & 1) * NW + wave_in_slot) * 2, pl.lane, pa, pt);
                     } else {
                         pa = slot_wave_sum<TL::TPS>(pa);
-                        pz = slot_wave_sum<TL::TPS>(pz);
+                        pt = slot_wave_sum<TL::TPS>(pt);
                     }
                 }
             }
@@ -1354,15 +1355,15 @@ void step_bwd_fast(
             }
             if (NORM && active) {
                 if (NW > 1) {
-                    pa = pz = 0.f;
+                    pa = pt = 0.f;
 #pragma unroll
                     for (int q = 0; q < NW; ++q) {  // fixed order: every thread gets the same sums
                         const float2 p2 = *reinterpret_cast<const float2 *>(nrev + ((it & 1) * NW + q) * 2);
-                        pa += p2.x; pz += p2.y;
+                        pa += p2.x; pt += p2.y;
                     }
                 }
                 const float a_mean = pa * inv_count;
-                const float coef = pz * inv * inv_count / fmaxf(sd, 1e-30f);
+                const float coef = pt * inv * inv * inv_count / fmaxf(sd, 1e-30f);
 #pragma unroll
                 for (int c = 0; c < CPT; ++c)
                     g[c] += fmaf(inv, dn[c] - a_mean, -(xi[c] - mean) * coef);

@@ -23,7 +23,8 @@
 // has polled `spin_limit` times in all it raises the status word and waits no more, and the kernel
 // ends on whatever it read.  chain_fwd_repair, always launched behind it, returns at once unless the
 // status word is raised; then it does the chain again, one workgroup per element and no waits
-// between workgroups.  The caller need not look at the status and nothing synchronises.
+// between workgroups, operation by operation as chain_fwd does it: the same bits, whichever of the two they are from.  The caller
+// need not look at the status and nothing synchronises.
 //
 // All of it is latency: one 32^3 sample, one inner iteration, 2.5 us a step, of which the arithmetic is
 // 0.4 (3.6 with the taps behind the statistics, see chain_fwd); 64 steps with the MNIST model around them
@@ -110,6 +111,30 @@ __device__ __forceinline__ T taps(const float *win, int at, int dir, const float
     for (int t = 0; t < 27; ++t)
         sum = fma((T)w[t], (T)from[t % 3][(t / 9 - 1) * kSide * kSide + (t / 3 % 3 - 1) * kSide], sum);
     return sum;
+}
+
+// sum_t w_t gamma_t, and sum_t w_t beta_t + bias: see chain_fwd.  The windows are free again when it returns.
+__device__ __forceinline__ void affine_sums(float (*win)[kWindow], const CellPlace &p, const float (&w)[27], float bias, float gam,
+                                            float bet, float egam, float ebet, float &sum_gamma, float &bias_beta) {
+    win[0][p.at] = gam;
+    win[1][p.at] = bet;
+    if (p.edge_at >= 0) {
+        win[0][p.edge_at] = egam;
+        win[1][p.edge_at] = ebet;
+    }
+    lds_barrier();
+    sum_gamma = (float)taps(win[0], p.at, 1, w, 0.0);
+    bias_beta = (float)taps(win[1], p.at, 1, w, (double)bias);
+    lds_barrier();
+}
+// The mean of 32 of a block's values, the same in every lane.
+__device__ __forceinline__ float centre_of(const float *values, int tid) {
+    const float2 c = *reinterpret_cast<const float2 *>(values + 32 * (tid & 15) + (6 * tid & 30));
+    return row16_sum(fmaf(1.f / 32, c.x, 1.f / 32 * c.y));
+}
+// The pre-activation from the taps on (y - centre) gamma; a variance beyond fp32 leaves nothing but beta.
+__device__ __forceinline__ float with_statistics(float taps, float centre, float mean, float rstd, float sum_gamma, float bias_beta) {
+    return rstd == 0.f ? bias_beta : fmaf(rstd, fmaf(centre - mean, sum_gamma, taps), bias_beta);
 }
 
 // All inner iterations of one block: x in, x out; the shell is in both window copies and x in the
@@ -241,18 +266,7 @@ template <int ACT, bool ONE> __global__ __launch_bounds__(kCfThreads) __attribut
     float *ring = a.ring + (long)s * cells;
 
     float sum_gamma = 0.f, bias_beta = 0.f;
-    if (ONE) {
-        win[0][p.at] = gam;
-        win[1][p.at] = bet;
-        if (p.edge_at >= 0) {
-            win[0][p.edge_at] = egam;
-            win[1][p.edge_at] = ebet;
-        }
-        lds_barrier();
-        sum_gamma = (float)taps(win[0], p.at, dir, w, 0.0);
-        bias_beta = (float)taps(win[1], p.at, dir, w, (double)bias);
-        lds_barrier();
-    }
+    if (ONE) affine_sums(win, p, w, bias, gam, bet, egam, ebet, sum_gamma, bias_beta);
     for (int j = 0; j <= a.outer; ++j) {
         float x = own, e = edge, u, centre = 0.f;
         // what step j - 1 left: the shell's cells, and the statistics of the element
@@ -263,8 +277,7 @@ template <int ACT, bool ONE> __global__ __launch_bounds__(kCfThreads) __attribut
             const bool want = j < a.outer && has;
             e = want ? ld_agent(from + p.edge) : 0.f;
             if (ONE) {
-                const float2 c = *reinterpret_cast<const float2 *>(values + 32 * (tid & 15) + (6 * tid & 30));
-                centre = row16_sum(fmaf(1.f / 32, c.x, 1.f / 32 * c.y));  // the same in every lane
+                centre = centre_of(values, tid);
                 x = (own - centre) * gam;
             } else if (wave == 0) {
                 merge_words(a, words, nullptr, j, s, blk == 0, budget, norm);
@@ -297,8 +310,7 @@ template <int ACT, bool ONE> __global__ __launch_bounds__(kCfThreads) __attribut
                 st_agent(ring + ((j - 2) & (kRing - 1)) * slot_cells + p.cell, __uint_as_float(kEmpty));
                 if (tid < kGroups) st_agent(parts + ((j - 2) & (kRing - 1)) * slot_parts + kGroups * blk + tid, ~0ull);
             }
-            // a variance beyond fp32 leaves nothing but beta
-            if (ONE) u = rstd == 0.f ? bias_beta : fmaf(rstd, fmaf(centre - mean, sum_gamma, u), bias_beta);
+            if (ONE) u = with_statistics(u, centre, mean, rstd, sum_gamma, bias_beta);
             else e = has ? fmaf((e - mean) * rstd, egam, ebet) : 0.f;
         }
         if (ONE) {
@@ -323,36 +335,54 @@ template <int ACT, bool ONE> __global__ __launch_bounds__(kCfThreads) __attribut
 }
 
 // The same chain by one workgroup per element, for the case that a wait of chain_fwd ran out.  The
-// blocks of a step one after the other, raw values from one ring slot to the next.
-template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd_repair(ChainFwdArgs a) {
+// blocks of a step one after the other, raw values from one ring slot to the next; the statistics' words pass through
+// memory to be merged in chain_fwd's order.
+template <int ACT, bool ONE> __global__ __launch_bounds__(kCfThreads) void chain_fwd_repair(ChainFwdArgs a) {
     if (*a.status == 0) return;
     __shared__ float win[2][kWindow];
     __shared__ __attribute__((aligned(16))) float values[kCfThreads];
-    __shared__ unsigned long long words[kGroups];
-    const int tid = threadIdx.x, s = blockIdx.x, dir = k_direction(tid, a.inner);
+    __shared__ float norm[2];
+    const int tid = threadIdx.x, s = blockIdx.x, dir = ONE ? 1 : k_direction(tid, a.inner);
     const int cells = a.M * a.N * a.K;
     const long slot_cells = (long)a.B * cells, mine = (long)s * cells;
-    const double inv_groups = 1.0 / (kGroups * a.nblk);
+    unsigned long long *words = a.parts + (long)kGroups * s * a.nblk;
     float mean = 0.f, rstd = 1.f;
     for (int j = 0; j < a.outer; ++j) {
         const float *from = j ? a.ring + ((j - 1) & 1) * slot_cells + mine : a.x0 + mine;
         float *to = a.ring + (j & 1) * slot_cells + mine;
-        GroupSums sums;
         for (int blk = 0; blk < a.nblk; ++blk) {
             const CellPlace p(tid, blk, a.M, a.N, a.K);
+            const bool has = p.edge >= 0;
             float w[27];
             load_weights(a.weight, cells, p.cell, dir, w);
-            float x = from[p.cell], e = p.edge >= 0 ? from[p.edge] : 0.f;
-            if (j) {
-                x = fmaf((x - mean) * rstd, a.gamma[p.cell], a.beta[p.cell]);
-                e = p.edge >= 0 ? fmaf((e - mean) * rstd, a.gamma[p.edge], a.beta[p.edge]) : 0.f;
+            const float bias = a.bias[p.cell], scale = a.scale[p.cell], gam = a.gamma[p.cell], bet = a.beta[p.cell];
+            const float egam = has ? a.gamma[p.edge] : 0.f, ebet = has ? a.beta[p.edge] : 0.f;
+            const float own = from[p.cell], edge = has ? from[p.edge] : 0.f;
+            float x = own, e = edge, u, y, centre = 0.f, sum_gamma = 0.f, bias_beta = 0.f;
+            __syncthreads();  // the block before is done with the window and the values
+            if (ONE && j) {
+                values[tid] = own;
+                affine_sums(win, p, w, bias, gam, bet, egam, ebet, sum_gamma, bias_beta);
+                centre = centre_of(values, tid);
+                x = (own - centre) * gam;
+                e = has ? (edge - centre) * egam : 0.f;
+            } else if (j) {
+                x = fmaf((own - mean) * rstd, gam, bet);
+                e = has ? fmaf((edge - mean) * rstd, egam, ebet) : 0.f;
             }
-            __syncthreads();  // the block before is done with the window
             win[0][p.at] = x;
             if (p.edge_at >= 0) win[0][p.edge_at] = win[1][p.edge_at] = e;
             __syncthreads();
-            float u;
-            const float y = advance<ACT>(win, p.at, dir, w, a.bias[p.cell], a.scale[p.cell], x, a.inner, u);
+            if (ONE) {
+                u = taps(win[0], p.at, dir, w, j ? 0.f : bias);
+                if (j) {
+                    x = fmaf((own - mean) * rstd, gam, bet);
+                    u = with_statistics(u, centre, mean, rstd, sum_gamma, bias_beta);
+                }
+                y = fmaf(scale, Act<ACT, float>::f(u), x);
+            } else {
+                y = advance<ACT>(win, p.at, dir, w, bias, scale, x, a.inner, u);
+            }
             to[p.cell] = y;
             if (a.y_all) a.y_all[(long)j * slot_cells + mine + p.cell] = y;
             if (a.saved) a.saved[(long)j * slot_cells + mine + p.cell] = u;
@@ -360,17 +390,15 @@ template <int ACT> __global__ __launch_bounds__(kCfThreads) void chain_fwd_repai
             __syncthreads();
             if (tid / 64 < kGroups) {
                 const unsigned long long word = group_moments(values, tid);
-                if ((tid & 63) == 0) words[tid / 64] = word;
+                if ((tid & 63) == 0) st_agent(words + kGroups * blk + tid / 64, word);
             }
-            __syncthreads();
-            for (int g = 0; g < kGroups; ++g) sums.add(words[g]);
         }
-        sums.finish(inv_groups, a.eps, mean, rstd);
-        if (tid == 0 && a.stats) {
-            a.stats[((long)j * a.B + s) * 2] = mean;
-            a.stats[((long)j * a.B + s) * 2 + 1] = rstd;
-        }
-        __syncthreads();  // the step's values are there for every thread
+        __syncthreads();  // the step's values and words are there for every thread
+        int budget = 0;   // no waits
+        if (tid < 64) merge_words(a, words, nullptr, j + 1, s, true, budget, norm);
+        __syncthreads();
+        mean = norm[0];
+        rstd = norm[1];
     }
     const float *last = a.ring + ((a.outer - 1) & 1) * slot_cells + mine;
     for (int c = tid; c < cells; c += kCfThreads)
@@ -406,13 +434,14 @@ template <int ACT> int launch_chain_fwd(const ChainFwd &c, hipStream_t st) {
     const long blocks = (vecs + 1023) / 1024;
     hipLaunchKernelGGL(chain_fwd_clear, dim3((unsigned)(blocks > 2048 ? 2048 : blocks)), dim3(256), 0, st, (uint4 *)ws, vecs);
     void *args[] = {&a};
-    const hipError_t e = hipLaunchCooperativeKernel(c.inner == 1 ? (const void *)chain_fwd<ACT, true> : (const void *)chain_fwd<ACT, false>,
-                                                    dim3((unsigned)(a.nblk * c.B)), dim3(kCfThreads), args, 0, st);
+    const auto chain = c.inner == 1 ? chain_fwd<ACT, true> : chain_fwd<ACT, false>;
+    const auto repair = c.inner == 1 ? chain_fwd_repair<ACT, true> : chain_fwd_repair<ACT, false>;
+    const hipError_t e = hipLaunchCooperativeKernel((const void *)chain, dim3((unsigned)(a.nblk * c.B)), dim3(kCfThreads), args, 0, st);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return fail(GRIDNET_ERR_LAUNCH, "chain_fwd: cooperative launch failed: %s", hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(chain_fwd_repair<ACT>, dim3((unsigned)c.B), dim3(kCfThreads), 0, st, a);
+    hipLaunchKernelGGL(repair, dim3((unsigned)c.B), dim3(kCfThreads), 0, st, a);
     return check_launch("chain_fwd");
 }
 

@@ -85,6 +85,25 @@ def test_a_wait_that_runs_out_is_repaired():
         assert_close(a, e, rtol=1e-5, atol=1e-5, what=name)
 
 
+@pytest.mark.parametrize("shape", [(16, 8, 24), (8, 16, 16)], ids=str)  # with rows of 16 the pre-activations are kept, too
+@pytest.mark.parametrize("inner,activation", [(1, "silu"), (2, "silu"), (1, "leaky_relu")])
+def test_a_repaired_chain_has_the_same_bits(shape, inner, activation):
+    from gridnet_amd import native as n
+
+    args = (shape, 3, inner, 5, activation)
+    run, *_, want = run_chain(*args)
+    kept = [run.s_all, run.stats, *([run.saved] if run.rows else [])]
+    assert run.forward_all and run.rows == (shape[2] == 16 and inner == 1)
+    old = n.lib.gridnet_hip_chain_set_spin_limit(-20)  # nobody publishes: every wait runs out
+    try:
+        again, *_, got = run_chain(*args, chain_all=False)
+    finally:
+        n.lib.gridnet_hip_chain_set_spin_limit(old)
+    assert torch.equal(got[0], want[0])
+    for a, e in zip([again.s_all, again.stats, *([again.saved] if run.rows else [])], kept):
+        assert torch.equal(a, e)
+
+
 def test_the_largest_batch_and_one_more():
     run = run_chain((16, 16, 16), 1, 1, 2, "relu", backward=False)[0]
     batch = 1

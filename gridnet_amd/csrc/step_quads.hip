@@ -57,6 +57,9 @@ constexpr int rows_floats(int plane) { return 6 * plane; }
 constexpr int window_floats(int plane) { return rows_floats(plane) + kSides; }
 // the four waves' windows: 16 floats past a multiple of 64, so that the pieces of a row, one for each wave, go to different banks
 constexpr int kForwardFloats = window_floats(kPlaneForward) + 16;
+// The residual form, forward: h and n = LayerNorm(h) of a block's own cells, [2][row][sample][cell], for h + (result - n).  In registers
+// (h requested with the window, a second time) they made 7 to 12 of them spill: 64^3, batch 128, eight iterations, 295 -> 275 us, with silu 380 -> 335.
+constexpr int kBack = 512;
 // gamma and beta of the workgroup's rows and of the entries beyond their ends
 constexpr int kAffineRows = kWinRows * kWaves * 8, kAffine = kAffineRows + kWinRows * 4;
 // Deltas by cell, [row][4 cells][4 samples], zeros around the block: row (i, j) is number 5 (i + 1) + j + 1, the row behind
@@ -208,9 +211,10 @@ struct QuadFetch {
     // LN: normalised on the way, with the statistics of the thread's sample.  The LDS places are worked out here, from a thread
     // number that the compiler cannot see through: it would keep them in registers that the loops have no room for.
     // An end goes to [row][side][sample], in the forward to [row][sample][side].
-    template <bool LN, int PLANE>
+    // BACK: the blocks' own cells, as they are and normalised, to back[block][2][row][sample][cell].
+    template <bool LN, int PLANE, bool BACK = false>
     __device__ __forceinline__ void commit(float *windows, int stride, const Buf &v, const float *affine, float mean,
-                                           float rstd) const {
+                                           float rstd, float *back = nullptr) const {
         constexpr int SIDE = PLANE == kPlaneForward ? 1 : 4, SAMPLE = PLANE == kPlaneForward ? 2 : 1;
         const int t = opaque(threadIdx.x), m = t & 3, s = t >> 2 & 3;
         float *win = windows + m * stride;
@@ -225,6 +229,14 @@ struct QuadFetch {
                     const quad g = load_quad(gb), b = load_quad(gb + 4);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) val[q] = fmaf((val[q] - mean) * rstd, g[q], b[q]);
+                }
+                if (BACK) {
+                    const int i = r / 6 - 1, j = r % 6 - 1;
+                    if ((unsigned)i < 4u && (unsigned)j < 4u) {
+                        float *to = back + m * kBack + (4 * i + j) * 16 + s * 4;
+                        *reinterpret_cast<quad *>(to) = v.rows[e];
+                        *reinterpret_cast<quad *>(to + 256) = val;
+                    }
                 }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) val[q] = where & 1 ? val[q] : 0.f;
@@ -308,7 +320,7 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
                int nchunk, int chunk_len, LnFold ln) {
     constexpr int PLANE = kPlaneForward, WINDOW = kForwardFloats;
     constexpr int SIDE_WEIGHTS = 16 * 18;  // [row][neighbour row][side]
-    __shared__ __attribute__((aligned(16))) float lds[kWaves * (WINDOW + SIDE_WEIGHTS) + kAffine];
+    __shared__ __attribute__((aligned(16))) float lds[kWaves * (WINDOW + SIDE_WEIGHTS + (RES ? kBack : 0)) + kAffine];
     QuadWork work;
     if (!work.find(ln.walk_reverse ? reversed_on_its_xcd(blockIdx.x, gridDim.x) : blockIdx.x, M, N, K, nchunk, chunk_len, B))
         return;
@@ -316,6 +328,7 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
     const QuadFetch fx(work, M, N, K);
     float *win = lds + work.wave * WINDOW, *affine = lds + kWaves * WINDOW;
     float *ends = affine + kAffine + work.wave * SIDE_WEIGHTS + pl.row * 18;
+    float *back = affine + kAffine + kWaves * SIDE_WEIGHTS;
     const long cells = (long)M * N * K;
     const bool ln_in = ln.x_stats != nullptr;
     const int first = pl.own - pl.k;  // cell 0 of the lane's row; pl.k is the lane's sample
@@ -337,7 +350,6 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
         fx.pack_affine(affine, pre, beta);
     }
     wait_global_loads();
-    quad raw = {0.f, 0.f, 0.f, 0.f}, raw_next = raw;  // RES: h of the owned cells
     auto fetch_group = [&](int s) {
         const int mine = min(s + fx.sample(), work.end - 1) - s;  // past the end: the last sample again
         fx.fetch(x + s * cells, 4u * (unsigned)mine * (unsigned)cells, pre);
@@ -346,10 +358,9 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
             mean = st.x;
             rstd = st.y;
         }
-        if (RES) raw_next = load_quad(at_cell(x + s * cells, (min(s + pl.k, work.end - 1) - s) * (int)cells + first));
     };
     fetch_group(work.first);
-    quad cur, stored = raw;
+    quad cur, stored = {0.f, 0.f, 0.f, 0.f};
     int done = -1;  // the first of the samples in `stored`: a group's result leaves behind the wait for the next one's window
     const auto store_group = [&] {
         if (done >= 0 && done + pl.k < work.end)
@@ -357,16 +368,15 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
     };
     for (int s = work.first; s < work.end; s += kGroup) {
         lds_barrier();  // gamma and beta; the windows are free
-        if (ln_in) fx.template commit<true, PLANE>(lds, WINDOW, pre, affine, mean, rstd);
+        if (RES) fx.template commit<true, PLANE, true>(lds, WINDOW, pre, affine, mean, rstd, back);  // with statistics always
+        else if (ln_in) fx.template commit<true, PLANE>(lds, WINDOW, pre, affine, mean, rstd);
         else fx.template commit<false, PLANE>(lds, WINDOW, pre, affine, mean, rstd);
-        if (RES) raw = raw_next;
         lds_barrier();
         if (work.active) store_group();
         if (s + kGroup < work.end) fetch_group(s + kGroup);
         if (!work.active) continue;
         float *own = win + pl.rows00 + PLANE + 16;
         cur = load_quad(own);
-        const quad base = cur;
         quad u0 = bv;
 #pragma unroll
         for (int n = 0; n < 9; ++n) {  // the entries beyond the row's ends: the same for every iteration
@@ -401,7 +411,10 @@ void quads_fwd(const float *__restrict__ weight, const float *__restrict__ bias,
             if (it + 1 < inner) *reinterpret_cast<quad *>(own) = cur;
             wave_order();
         }
-        if (RES) cur = raw + (cur - base);
+        if (RES) {
+            const float *from = back + work.wave * kBack + pl.row * 16 + pl.k * 4;
+            cur = load_quad(from) + (cur - load_quad(from + 256));
+        }
         stored = cur;
         done = s;
         if (ln.y_part) {  // (mean, M2) of the block's 64 cells, by the lanes of a sample

@@ -375,6 +375,21 @@ size_t gridnet_hip_fused_workspace_bytes(int B, int M, int N, int K, int inner, 
     return slabs ? (need + 255) / 256 * 256 + slabs : need;
 }
 
+int gridnet_hip_fused_route(int B, int M, int N, int K, int inner, int block_size, int residual, int backward,
+                            size_t workspace_bytes) {
+    StepArgs a{};
+    a.dtype = GRIDNET_F32; a.B = B; a.M = M; a.N = N; a.K = K; a.inner = inner;
+    a.block_size = block_size; a.activation = GRIDNET_ACT_RELU;
+    a.ln.gamma = (const float *)&a;  // only whether there is one matters, here and below
+    a.ln.residual = residual != 0;
+    a.ln.y_raw = residual == 2 ? nullptr : (const float *)&a;
+    if (!has_blocks(B, M, N, K, block_size) || M % block_size || N % block_size || K % block_size || inner < 1 ||
+        (long)M * N * K * 27 >= (1L << 31) || !step_fast_supports(a, backward != 0))
+        return -1;
+    if (backward) give_slabs(a, (void *)256, workspace_bytes, fused_backward_dsum(a) + fused_backward_parts(a));
+    return step_fast_route(a, backward != 0);
+}
+
 static int fused_forward(int dtype, const void *weight, const void *bias, const void *scale,
                          const void *gamma, const void *beta, const void *x, const void *x_stats,
                          void *y_raw, void *y_stats, int B, int M, int N, int K, int inner,

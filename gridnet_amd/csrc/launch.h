@@ -155,6 +155,7 @@ int step_backward_f64(const StepArgs &a, hipStream_t st);
 bool step_fast_supports(const StepArgs &a, bool backward);
 size_t step_fast_backward_workspace(const StepArgs &a);   // what the backward cannot do without
 size_t step_fast_slab_bytes(const StepArgs &a);           // room for the gradient copies of a split batch
+int step_fast_route(const StepArgs &a, bool backward);    // enum gridnet_route: the kernels that take it
 int step_forward_fast(const StepArgs &a, hipStream_t st);
 int step_backward_fast(const StepArgs &a, hipStream_t st);
 // partial statistics per (block, batch element) that the kernels above write when asked to

@@ -2220,15 +2220,25 @@ size_t step_fast_slab_bytes(const StepArgs &a) {
     return std::max(quads, (size_t)chunks * kStepSlabPlanes * a.M * a.N * a.K * sizeof(float));
 }
 
+int step_fast_route(const StepArgs &a, bool backward) {
+    // one inner iteration: a plain stencil, by whole rows
+    if (backward ? bwd_rows_supports(a) : fwd_rows_supports(a)) return GRIDNET_ROUTE_ROWS;
+    if (step_quads_supports(a, backward)) return GRIDNET_ROUTE_QUADS;
+    return !backward && walks_pairs(a) ? GRIDNET_ROUTE_PAIRS : GRIDNET_ROUTE_BLOCKS;
+}
 int step_forward_fast(const StepArgs &a, hipStream_t st) {
-    if (fwd_rows_supports(a)) return fwd_rows_launch(a, st);  // one inner iteration: a plain stencil, by whole rows
-    if (step_quads_supports(a, false)) return step_quads_forward(a, st);
-    return dispatch<false>(a, st);
+    switch (step_fast_route(a, false)) {
+        case GRIDNET_ROUTE_ROWS: return fwd_rows_launch(a, st);
+        case GRIDNET_ROUTE_QUADS: return step_quads_forward(a, st);
+        default: return dispatch<false>(a, st);
+    }
 }
 int step_backward_fast(const StepArgs &a, hipStream_t st) {
-    if (bwd_rows_supports(a)) return bwd_rows_launch(a, st);  // one inner iteration: by whole rows
-    if (step_quads_supports(a, true)) return step_quads_backward(a, st);
-    return dispatch<true>(a, st);
+    switch (step_fast_route(a, true)) {
+        case GRIDNET_ROUTE_ROWS: return bwd_rows_launch(a, st);
+        case GRIDNET_ROUTE_QUADS: return step_quads_backward(a, st);
+        default: return dispatch<true>(a, st);
+    }
 }
 
 }  // namespace gridnet

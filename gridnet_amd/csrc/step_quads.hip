@@ -815,11 +815,32 @@ static bool covers(const StepArgs &a) {
     return a.dtype == GRIDNET_F32 && a.block_size == 4 && !a.normalize && a.inner >= 2 && a.B >= kGroup &&
            a.ln.gamma && (long)a.M * a.N * a.K <= 1L << 26;
 }
-// Forward of a chain's step, leaky_relu, us, step_fwd_fast -> quads_fwd: 64^3, batch 128, eight iterations, 476 -> 280
-// (with silu 435 -> 327); batch 4, 42 -> 23; batch 5, four, 45 -> 25; 32^3, batch 128, 50 -> 33; batch 4, 12.2 -> 11.1.
+// The forward's rule.  Few samples of few blocks are left to step_fwd_fast, which spreads each over a wave with one cell per thread
+// (few_for_slots).  So are rows of one block, where three waves of four have no block (with a batch that is no multiple of four
+// places of the fourth are empty, too), as soon as the chip has more than a few rounds of waves -- until then idle ones cost nothing --
+// and rows of two, or of more with a batch of five, where there are more rounds still and the workgroups are more than the chip holds.
+// Forward of a chain's step, leaky_relu, statistics included, from a graph, us, step_fwd_fast -> quads_fwd: 16 x 16 x 4, batch 6,
+// two iterations, 5.9 -> 7.9; 32 x 32 x 12, batch 7 (1344 pairs of block and sample), 7.7 -> 8.1; 16 x 16 x 64, batch 6 (1536), 9.2 ->
+// 8.5; 32 x 32 x 20, batch 5 (1600), 11.4 -> 8.3; 64 x 64 x 44, batch 13, 40 -> 25; 64^3, batch 9, eight, 57 -> 37.  Rows of one block,
+// 128 x 128 x 4: batch 12 (four rounds), two iterations, 23.4 -> 21.1, eight 29.2 -> 29.1; batch 13 (five and a third), 23.4 -> 24.4, eight
+// 29.5 -> 35.8; batch 128, eight, 117 -> 174; 64 x 64 x 4, batch 128, 42 -> 48; batch 64 (five and a third), two, 23.4 -> 21.0.  Of
+// two: 128 x 128 x 8, batch 16, eight, 42.8 -> 39.3; batch 64, two, 60 -> 65, eight 114 -> 103, with silu, batch 128, 217 -> 247; but 64 x 64 x 8, batch
+// 128 (256 workgroups), 67 -> 52.  Over 2000 grids of 16 to 128 cells a side, K from 4, batch 4 to 128, two to eight iterations, the
+// better kernel every time would be 0.1 % faster than the rule and quads_fwd everywhere 4 % slower; with silu and in the residual
+// form the same to 0.1 %.
+constexpr int kFewestPairs = 6;                    // per CU
+constexpr int kForwardPerCu = 3;                   // workgroups, a wave of each on every SIMD
+constexpr int kMostRoundsOfOne = 5, kMostRoundsOfTwo = 8;
+static bool fills_places(const StepArgs &a) {
+    const long cus = plan_device_cus(), groups = quad_groups(a), pairs = (long)(a.M / 4) * (a.N / 4) * (a.K / 4) * a.B;
+    const long waves = groups * kWaves * ((a.B + kGroup - 1) / kGroup), round = kForwardPerCu * kWaves * cus;
+    if (pairs <= kFewestPairs * cus) return false;
+    if (10 * pairs <= 3 * waves * kGroup && waves > kMostRoundsOfOne * round) return false;
+    return !(2 * pairs <= waves * kGroup && waves > kMostRoundsOfTwo * round && groups > kForwardPerCu * cus);
+}
 bool step_quads_supports(const StepArgs &a, bool backward) {
     if (!covers(a)) return false;
-    if (!backward) return true;
+    if (!backward) return fills_places(a);
     if (!a.ln.y_raw) return false;  // no LayerNorm behind the step
     int nchunk, chunk_len;
     return a.inner <= kMostIterations && cross_rows_supports(a) &&

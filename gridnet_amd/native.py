@@ -39,6 +39,7 @@ EXPORTS = (
     "gridnet_hip_layernorm_forward",
     "gridnet_hip_layernorm_backward",
     "gridnet_hip_fused_workspace_bytes",
+    "gridnet_hip_fused_route",
     "gridnet_hip_fused_forward_chain_merges",
     "gridnet_hip_fused_forward_chain_workspace_bytes",
     "gridnet_hip_fused_forward_chain",
@@ -108,6 +109,8 @@ def _load():
     lib.gridnet_hip_layernorm_backward.argtypes = [i, p, p, p, p, p, p, p, p, i, l, i, p, z, p]
     lib.gridnet_hip_fused_workspace_bytes.restype = z
     lib.gridnet_hip_fused_workspace_bytes.argtypes = [i, i, i, i, i, i, i]
+    lib.gridnet_hip_fused_route.restype = i
+    lib.gridnet_hip_fused_route.argtypes = [i, i, i, i, i, i, i, i, z]
     lib.gridnet_hip_fused_forward_chain_merges.restype = i
     lib.gridnet_hip_fused_forward_chain_merges.argtypes = [i] * 7
     lib.gridnet_hip_fused_forward_chain_workspace_bytes.restype = z

@@ -67,7 +67,7 @@ enum gridnet_flags {
 };
 
 /* Library build id (monotonic integer) -- lets a binding check it loaded what it expects. */
-#define GRIDNET_HIP_VERSION 10
+#define GRIDNET_HIP_VERSION 11
 int gridnet_hip_version(void);
 
 /* Thread-local message of the last non-zero status returned on this thread ("" if none). */
@@ -201,6 +201,16 @@ int gridnet_hip_layernorm_backward(int dtype, const void *dy, const void *x, con
  */
 size_t gridnet_hip_fused_workspace_bytes(int B, int M, int N, int K, int inner, int block_size,
                                          int backward);
+
+/* Which kernels take a fused step of these sizes on the current device: GRIDNET_ROUTE_BLOCKS, by blocks;
+ * GRIDNET_ROUTE_ROWS, by whole grid rows (one inner iteration); GRIDNET_ROUTE_PAIRS, 8^3 blocks, two samples per
+ * pass; GRIDNET_ROUTE_QUADS, 4^3 blocks, four samples to a wave.  The results agree to rounding; this is for those who
+ * profile or test one of them.  residual: 1 for the residual form, 2 for the last step of its loop (y_raw == NULL in
+ * gridnet_hip_fused_backward_residual).  workspace_bytes: what the backward is handed, copies of the gradients included
+ * (the forward's choice does not depend on it).  -1: not a fused step.  Needs no device; without one, 256 compute units. */
+enum gridnet_route { GRIDNET_ROUTE_BLOCKS = 0, GRIDNET_ROUTE_ROWS = 1, GRIDNET_ROUTE_PAIRS = 2, GRIDNET_ROUTE_QUADS = 3 };
+int gridnet_hip_fused_route(int B, int M, int N, int K, int inner, int block_size, int residual, int backward,
+                            size_t workspace_bytes);
 
 /* y_raw = step(LayerNorm(x; x_stats, gamma, beta)), y_stats = statistics of y_raw.
  * x_stats == NULL: x is used as it is (the first step of a chain). */

@@ -5,16 +5,20 @@ import pytest
 import torch
 
 from helpers import ATOL, RTOL, assert_close, make_acts, make_params
+from test_routes import BLOCKS, QUADS, route
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# forward: the rows' blocks in workgroups of four, three, two and one; one, two and more groups of samples, the last one of
-# every size; two to nine iterations.  The backward is this file's where the last column says so: a walk of 32 at least, groups
-# that are nearly full, more than half of the places of its waves taken
+# the rows' blocks in workgroups of four, three, two and one; one, two and more groups of samples, the last one of
+# every size; two to nine iterations.  The forward is this file's with more than six pairs of block and sample to a CU, the
+# backward where the last column says so: a walk of 32 at least, groups that are nearly full, more than half of the places of
+# its waves taken
 @pytest.mark.parametrize("shape,batch,inner,quads", [
     ((4, 4, 4), 4, 2, False), ((4, 8, 12), 5, 3, False), ((8, 8, 20), 7, 2, False), ((8, 4, 36), 6, 9, False),
+    ((32, 32, 4), 25, 3, False), ((32, 32, 8), 14, 2, False), ((32, 32, 12), 11, 9, False), ((32, 32, 20), 5, 2, False),
+    ((20, 28, 28), 7, 3, False),
     ((32, 32, 32), 16, 8, True), ((32, 32, 32), 31, 7, True), ((16, 16, 16), 256, 4, True), ((32, 32, 36), 32, 2, True),
     ((40, 44, 44), 16, 2, True), ((40, 44, 44), 4, 8, True), ((40, 44, 44), 16, 9, False), ((48, 48, 60), 16, 2, True)], ids=str)
 @pytest.mark.parametrize("residual", [False, True], ids=["chain", "residual"])
@@ -24,6 +28,9 @@ def test_chain_against_the_oracle(shape, batch, inner, quads, residual, activati
     from oracle.network import network_forward_backward
 
     print(f"quads, chain {shape} B={batch} inner={inner} residual={residual} {activation} backward here: {quads}", flush=True)
+    pairs = batch * shape[0] * shape[1] * shape[2] // 64
+    assert (route(shape, batch, inner, 4, residual) == QUADS) == (pairs > 6 * 256)
+    assert (route(shape, batch, inner, 4, residual, backward=1) == QUADS) == quads
     g = torch.Generator().manual_seed(3)
     w, b, r = make_params(shape, seed=11)
     if inner >= 7:
@@ -52,6 +59,7 @@ def test_an_infinite_gradient_stays_within_the_taps_reach():
     params = [*make_params(shape, seed=11), *((a + 0.2 * torch.randn(shape, generator=g)) for a in (1, 0))]
     x, gy = (make_acts(batch, shape, seed=s) for s in (12, 13))
     run = BodyRunner(*(t.to(DEV) for t in params), batch, inner, 1, 4, "tanh", fused=True, outer_residual=True)
+    assert route(shape, batch, inner, 4, 1, backward=1) == QUADS and route(shape, batch, inner, 4, 2, backward=1) == BLOCKS
     run.forward(x.to(DEV))
     bad = gy.clone()
     bad[5][at] = float("inf")

@@ -25,3 +25,13 @@ def route(shape, batch, inner, block_size, residual=0, backward=0, workspace=Non
 @pytest.mark.parametrize("residual", [0, 1])
 def test_forward_of_small_blocks(shape, batch, inner, want, residual):
     assert route(shape, batch, inner, 4, residual) == want
+
+
+# the backward: a walk of 32 at least, groups of four samples that are nearly full, half of the places of its waves taken, seven tenths
+# where there are three rounds of them
+@pytest.mark.parametrize("shape,batch,inner,want", [
+    ((64, 64, 64), 8, 2, BLOCKS), ((64, 64, 64), 16, 2, QUADS), ((64, 64, 64), 5, 4, BLOCKS), ((64, 64, 64), 4, 8, QUADS),
+    ((40, 40, 40), 32, 4, BLOCKS), ((44, 44, 44), 32, 4, QUADS), ((52, 52, 52), 32, 4, QUADS), ((64, 64, 64), 32, 9, BLOCKS),
+    ((128, 56, 36), 100, 5, BLOCKS), ((56, 80, 52), 16, 6, BLOCKS), ((80, 80, 40), 20, 4, BLOCKS), ((80, 80, 48), 20, 4, QUADS)], ids=str)
+def test_backward_of_small_blocks(shape, batch, inner, want):
+    assert [route(shape, batch, inner, 4, residual, backward=1) for residual in (0, 1, 2)] == [want, want, BLOCKS]

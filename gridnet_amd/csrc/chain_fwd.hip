@@ -241,8 +241,11 @@ __device__ __forceinline__ void merge_words(const ChainFwdArgs &a, const unsigne
 // S from the raw cells as they come in, G and H once per launch.  c is the mean of 32 of the block's values: S and
 // (mean - c) G then are of the size of the normalised sum, and the result is as exact as that (errors against 64 bits over eleven
 // kinds of chain, six seeds each: 1.00 times those of normalising first).  Per step of 64: 32^3, batch 1, 3.6 -> 2.5 us, batch 8,
-// 5.8 -> 3.9; 64^3, batch 1, 7.5 -> 6.8.  With one inner iteration only: the backward of more recomputes the step from its normalised
-// input, and the forward keeps to its operations.  (A wave of its own for the statistics, nine to a workgroup: two workgroups no
+// 5.8 -> 3.9; 64^3, batch 1, 7.5 -> 6.8.  With one inner iteration only: of more the statistics are a small part.  The backward by
+// whole rows of 16, 32 or 64 cells reads the pre-activations that are kept here; the other ones form them again from the
+// normalised input, with other last bits, so that a cell within rounding of a kink can have the derivative of the side that the forward
+// did not take.  The value is continuous there, and against 64 bits nothing changes: with relu, 16 x 24 x 40, batch 4, eight steps,
+// one chain of 200 had a cell on the wrong side, and one when the forward normalised first.  (A wave of its own for the statistics, nine to a workgroup: two workgroups no
 // longer fit a CU, although the occupancy query says that they do.)
 template <int ACT, bool ONE> __global__ __launch_bounds__(kCfThreads) __attribute__((amdgpu_waves_per_eu(4))) void chain_fwd(ChainFwdArgs a) {
     __shared__ float win[2][kWindow];

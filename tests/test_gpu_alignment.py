@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from helpers import assert_close, make_acts, make_params
+from test_routes import QUADS, route
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -101,19 +102,26 @@ def test_layernorm_with_tensors_at_odd_addresses():
         assert_close(g.cpu(), e.cpu(), what=name)
 
 
-def test_fused_chain_with_tensors_at_odd_addresses():
+# 8^3 blocks, and 4^3 with four samples to a wave: one parameter set, then one for each step
+@pytest.mark.parametrize("shape,bs,batch,separate", [((16, 16, 16), 8, 4, False), ((32, 32, 36), 4, 32, False),
+                                                     ((32, 32, 36), 4, 32, True)], ids=str)
+def test_fused_chain_with_tensors_at_odd_addresses(shape, bs, batch, separate):
     """The chain with the LayerNorm folded into the step kernels, all buffers one element off."""
     from gridnet_amd.runner import BodyRunner
 
-    shape, bs, inner, outer, batch = (16, 16, 16), 8, 2, 3, 4
-    print("odd addresses: fused chain", flush=True)
+    inner, outer = 2, 3
+    print(f"odd addresses: fused chain {shape} bs={bs} separate={separate}", flush=True)
+    if bs == 4:
+        assert [route(shape, batch, inner, bs, backward=d) for d in (0, 1)] == [QUADS, QUADS]
     w, b, r = make_params(shape, seed=71)
+    if separate:
+        w, b, r = ([t * f for f in (1.0, 0.9, 1.1)] for t in (w, b, r))
     gamma, beta = 1 + 0.1 * make_acts(1, shape, seed=72)[0], 0.1 * make_acts(1, shape, seed=73)[0]
     x, gy = make_acts(batch, shape, seed=74), make_acts(batch, shape, seed=75)
 
     def call(place):
-        run = BodyRunner(*(place(t.to(DEV)) for t in (w, b, r, gamma, beta)), batch, inner, outer, bs,
-                         "silu", backward=True, fused=True)
+        put = [[place(s.to(DEV)) for s in t] if isinstance(t, list) else place(t.to(DEV)) for t in (w, b, r, gamma, beta)]
+        run = BodyRunner(*put, batch, inner, outer, bs, "silu", backward=True, fused=True)
         if place is odd:  # the workspaces too: four bytes past the allocator's alignment
             for name in ("fw_ws", "fb_ws", "ln_ws", "bw_ws"):
                 nbytes = getattr(run, name).numel()
@@ -122,7 +130,7 @@ def test_fused_chain_with_tensors_at_odd_addresses():
         y = run.forward(place(x.to(DEV)))
         grads = run.backward(place(gy.to(DEV)))
         torch.cuda.synchronize()
-        return [y.clone()] + [g.clone() for g in grads]
+        return [y.clone()] + [torch.stack(g) if isinstance(g, list) else g.clone() for g in grads]
 
     for i, (g, e) in enumerate(zip(call(odd), call(even))):
         assert_close(g.cpu(), e.cpu(), what=f"output {i}")

@@ -6,19 +6,21 @@ import pytest
 import torch
 
 from helpers import make_acts, make_params
+from test_routes import BLOCKS, PAIRS, route
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("shape,batch,inner", [
-    ((40, 40, 40), 63, 2), ((40, 40, 40), 64, 3), ((40, 40, 40), 65, 2),  # in pairs, in pairs, one by one
-    ((48, 32, 40), 71, 3), ((64, 40, 48), 17, 2), ((16, 24, 8), 5, 2)], ids=str)
-def test_against_oracle(shape, batch, inner):
+@pytest.mark.parametrize("shape,batch,inner,pairs", [
+    ((40, 40, 40), 63, 2, True), ((40, 40, 40), 64, 3, True), ((40, 40, 40), 65, 2, False),
+    ((48, 32, 40), 71, 3, False), ((64, 40, 48), 17, 2, True), ((16, 24, 8), 5, 2, True)], ids=str)
+def test_against_oracle(shape, batch, inner, pairs):
     from gridnet_amd.runner import BodyRunner
     from oracle.network import network_forward
 
     print(f"forward {shape} B={batch} inner={inner}", flush=True)
+    assert route(shape, batch, inner, 8) == (PAIRS if pairs else BLOCKS)
     g = torch.Generator().manual_seed(3)
     params = [*make_params(shape, seed=1), 1 + 0.2 * torch.randn(shape, generator=g), 0.2 * torch.randn(shape, generator=g)]
     x = make_acts(batch, shape, seed=2)

@@ -48,6 +48,31 @@ def test_chain_against_the_oracle(shape, batch, inner, quads, residual, activati
         assert_close(a, e, RTOL, ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)
 
 
+@pytest.mark.parametrize("room,want", [(4, QUADS), (3, QUADS), (2, BLOCKS), (0, BLOCKS)], ids=str)
+def test_backward_with_room_for_fewer_chunks(room, want):
+    """A batch in four chunks with room for the gradients of three: three longer ones.  Two would fill half of the places only, and the
+    step goes to the general kernels."""
+    from gridnet_amd import native as n
+    from gridnet_amd.runner import BodyRunner
+    from oracle.network import network_forward_backward
+
+    shape, batch, inner = (32, 32, 32), 64, 4
+    nbytes = n.lib.gridnet_hip_fused_workspace_bytes(batch, *shape, inner, 4, 1) - (4 - room) * 31 * 32 ** 3 * 4
+    print(f"quads, backward {shape} B={batch} inner={inner}, room for {room} chunks", flush=True)
+    assert route(shape, batch, inner, 4, backward=1, workspace=nbytes) == want
+    g = torch.Generator().manual_seed(3)
+    params = [*make_params(shape, seed=11), *((a + 0.2 * torch.randn(shape, generator=g)) for a in (1, 0))]
+    x, gy = (make_acts(batch, shape, seed=s) for s in (12, 13))
+    run = BodyRunner(*(t.to(DEV) for t in params), batch, inner, 1, 4, "silu", fused=True)
+    run.fb_ws_bytes, run.fb_ws = nbytes, torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+    run.forward(x.to(DEV))
+    got = run.backward(gy.to(DEV))
+    want = network_forward_backward([t.double() for t in params], x.double(), gy.double(), inner_iterations=inner,
+                                    outer_iterations=1, block_size=4, activation="silu")[1:]
+    for name, a, e in zip("dweight dbias dscale dgamma dbeta dx".split(), got, want):
+        assert_close(a, e, RTOL, ATOL * max(1.0, e.pow(2).mean().sqrt().item()), name)
+
+
 def test_an_infinite_gradient_stays_within_the_taps_reach():
     """The last step of the residual loop has no LayerNorm behind it that would spread a non-finite gradient over its sample."""
     from gridnet_amd.runner import BodyRunner

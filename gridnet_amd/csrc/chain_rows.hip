@@ -20,7 +20,9 @@
 //     11 us forward and 24 us backward: everybody waits for that wave at the barrier.
 // 32^3, batch 256, silu, per step: forward 27.5 us, backward 67.7, at 4.2 to 4.3 TB/s where a copy
 // reaches 4.6 (with the kernel that merges 29.1 + 68.4, and with the chunks of a tube on several CUs, 30.4 and 69.0; fwd_rows, bwd_rows and cross_rows with theirs: 28.1 + 4.4,
-// 59.3 + 8.0 + 23.4).  Gated, tanh: 55.7 and 85.8 + 4.9 (op by op the whole training step took 21.3 ms, 9.1 now).
+// 59.3 + 8.0 + 23.4).  The bytes are not what binds: a fifth of the backward's taken away brought 0.7 % of the training step, two sevenths
+// of the gated one's nothing; the vector ALU is 46 to 50 % busy at two waves per SIMD, and 17 and 8 us of a step do not grow with the
+// batch.  Gated, tanh: 55.7 and 85.8 + 4.9 (op by op the whole training step took 21.3 ms, 9.1 now).
 
 #include <algorithm>
 

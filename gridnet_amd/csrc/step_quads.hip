@@ -8,7 +8,8 @@
 //
 // Forward (quads_fwd): lane (row, sample) has the row's 108 weights and does 90 multiply-adds for its four cells in an
 // iteration, where step_fwd_fast does 108 and reads twice as much from LDS.  It is bound by the vector ALU: 102 instructions of a
-// loop of 112.  A step of 64^3, batch 128, eight iterations, leaky_relu: 457 -> 254 us, statistics included.
+// loop of 112.  A step of 64^3, batch 128, eight iterations, leaky_relu: 395 -> 243 us under the
+// profiler, 392 -> 246 from a graph with the statistics.
 //
 // Backward (quads_bwd): there are no registers for that three times over (weights, mirrored weights and gradients).  The
 // fp32 matrix instruction v_mfma_f32_4x4x1_16b does what a row sends to a row for four samples at once, sixteen products of
@@ -17,8 +18,8 @@
 // four entries are 36 instructions; the band (cell k reads entries k - 1, k, k + 1) fills ten of sixteen places, the rest multiplies
 // zeros.  They run on the vector ALU's multipliers, not beside them (8 cycles each, to which a multiply-add of another wave
 // adds its own), so an iteration's 108 there and back cost what the 324 multiply-adds they stand for do; what they save is half of
-// the LDS traffic, half of the other instructions and all of the registers that step_bwd_fast spills in its loops.  The same step:
-// 1053 -> 830 us (860 to 950 on other boxes).  What bounds it: the vector ALU, by counters 44 % of the time in matrix and 18 % in
+// the LDS traffic, half of the other instructions and all of the registers that step_bwd_fast spills in its loops.  The same step under the
+// profiler: 1057 -> 875 us (903 on another box).  What bounds it: the vector ALU, by counters 44 % of the time in matrix and 18 % in
 // other instructions; two waves per SIMD do not fill the waits between dependent matrix instructions; and a clock of 2.0 to 2.2 GHz.
 //
 // A wave's registers come in two layouts there:
@@ -132,8 +133,8 @@ struct QuadWork {
 // Where a lane sits in its wave's block.  The LDS serves a 16-byte read sixteen lanes at a time: lanes 0-3, 12-15, 20-23
 // and 24-27 together, then the others of the lower half wave, and so on.  Those are given the four rows of a plane, which lie side by
 // side.  With row = lane / 4 they came from two planes, and every read took eight cycles instead of four (counted): the LDS was
-// busy for 70 % of the forward and 61 % of the backward, four tenths of it with conflicts.  Now 48 and 40 %; a step of 64^3, batch
-// 128, eight iterations, forward 324 -> 312 us by events, backward 1 % less: the vector ALU and its clock bind it, not the LDS.
+// busy for 70 % of the forward and 61 % of the backward, four tenths of it with conflicts.  Now 45 and 40 %, and a step of 64^3, batch
+// 128, eight iterations is 1 to 4 % faster forward and 1 % backward: the vector ALU and its clock bind it, not the LDS.
 template <int PLANE> struct QuadPlace {
     int lane, row, k;        // k is the cell or the sample
     int i, j;                // of the row in the block
